@@ -138,3 +138,28 @@ def test_bad_arguments(tracea_gpu):
         tracea_gpu.linear(torch.zeros(2, 4, 8, device="cuda"), torch.zeros(3, 8, 8, device="cuda"))
     with pytest.raises(capi.TraceaError, match="residual"):
         tracea_gpu.linear(torch.zeros(2, 4, 8, device="cuda"), torch.zeros(8, 8, device="cuda"), epilogue="residual")
+
+
+@pytest.mark.parametrize("dtype", ["f16", "bf16", "f32"])
+@pytest.mark.parametrize("b,m,k,n", [(2, 1, 8, 8), (5, 65, 72, 64), (3, 128, 1024, 136), (16, 64, 512, 72), (2, 33, 2048, 24)])
+@pytest.mark.parametrize("w_layout", ["kn", "nk"])
+def test_linear_batches_in_one_launch(tracea_gpu, dtype, b, m, k, n, w_layout):
+    """Every batch with weights of its own goes out as one launch: tile edges in M and N, a K below one tile and one
+    long enough to be split, weights stored [K,N] and [N,K], batches of `a` and the output evenly spaced with a gap.
+    Tolerances as above: fp32 sums over k, half storage rounded once."""
+    tdt, rnd, _ = TYPES[dtype]
+    rng = np.random.default_rng(b * m + k)
+    a = rnd(rng.standard_normal((b, m, k)) / np.sqrt(k))
+    w = rnd(rng.standard_normal((b, k, n)))
+    bias = rng.standard_normal(n).astype(np.float32)
+    dw = _dev(w, tdt) if w_layout == "kn" else _dev(w.transpose(0, 2, 1), tdt).transpose(1, 2)
+    da = torch.zeros(b, m + 2, k, device="cuda", dtype=tdt)
+    da[:, :m] = _dev(a, tdt)
+    out = torch.full((b, m + 1, n), 7.0, device="cuda", dtype=torch.float32)
+    for _ in range(2):  # the second call meets the split counters the first one left
+        tracea_gpu.linear(da[:, :m], dw, bias=torch.from_numpy(bias).cuda(), epilogue="bias+relu", out=out[:, :m])
+    got = out.cpu().numpy()
+    assert (got[:, m] == 7.0).all(), "rows between the batches are not the call's"
+    for i in range(b):
+        ref = np.maximum(oracle.gemm_f64(a[i], w[i]) + bias[None, :], 0.0)
+        assert_close_scaled(got[i, :m], ref, 1e-4 if dtype == "f32" else tol_half(k, dtype), "linear batch %d" % i)

@@ -594,6 +594,8 @@ __global__ void __launch_bounds__(WM *WN * 64) contraction_kernel(const Contract
   asm volatile("" ::"s"(args.A), "s"(args.B), "s"(args.M), "s"(args.N), "s"(args.K), "s"(args.lda), "s"(args.ldb),
                "s"(args.a_bytes), "s"(args.b_bytes), "s"(args.grid_m), "s"(args.grid_n), "s"(args.k_split),
                "s"(args.fuse_ws), "s"(args.group_m), "s"(args.tile_list), "s"(args.epi.n_ops));
+  constexpr bool BATCHED = !CONV && BM * BN <= 128 * 128;  // blockIdx.z may name one of several products
+  if constexpr (BATCHED) asm volatile("" ::"s"(args.batch_a), "s"(args.batch_b), "s"(args.batch_rows));
   if constexpr (CONV && BATCH_ARGS) {
     asm volatile("" ::"s"(args.h_in), "s"(args.w_in), "s"(args.c_in), "s"(args.h_out), "s"(args.w_out), "s"(args.s_sz),
                  "s"(args.stride_h), "s"(args.stride_w), "s"(args.pad_h), "s"(args.pad_w), "s"(args.dil_h), "s"(args.dil_w),
@@ -650,6 +652,12 @@ __global__ void __launch_bounds__(WM *WN * 64) contraction_kernel(const Contract
 
   const unsigned short *Ag = (const unsigned short *)args.A;
   const unsigned short *Bg = (const unsigned short *)args.B;
+  if constexpr (BATCHED) {
+    const long long z = (long long)blockIdx.z;
+    Ag += z * args.batch_a;
+    Bg += z * args.batch_b;
+    zrow += z * args.batch_rows;
+  }
   // all phases of a transposed convolution in one launch: blockIdx.z names the phase
   int pad_h = args.pad_h, pad_w = args.pad_w, o_a = args.o_a, o_b = args.o_b;
   if constexpr (CONV) {
@@ -803,7 +811,7 @@ __global__ void __launch_bounds__(WM *WN * 64) contraction_kernel(const Contract
   const int wave_u = __builtin_amdgcn_readfirstlane(wave);
   constexpr unsigned OOB = 0x80000000u;
   __amdgpu_buffer_rsrc_t rsrc_a = __builtin_amdgcn_make_buffer_rsrc(
-      (void *)args.A, 0, (int)args.a_bytes, 0x00020000);
+      (void *)Ag, 0, (int)args.a_bytes, 0x00020000);
   __amdgpu_buffer_rsrc_t rsrc_b = __builtin_amdgcn_make_buffer_rsrc(
       (void *)Bg, 0, (int)args.b_bytes, 0x00020000);
   unsigned a_voff[NA], b_voff[NB];
@@ -1412,7 +1420,8 @@ __global__ void __launch_bounds__(WM *WN * 64) contraction_kernel(const Contract
       const unsigned splits = gridDim.y;
       constexpr unsigned TILE_BYTES = BM * BN * 4, WAVE_BYTES = TM * TN * 4;
       __amdgpu_buffer_rsrc_t rsrc_ws = __builtin_amdgcn_make_buffer_rsrc((void *)args.fuse_ws, 0, 0x7fffffff, 0x00020000);
-      const unsigned first = blockIdx.x * splits * TILE_BYTES + wave * WAVE_BYTES + lane * 16;
+      const unsigned tile = BATCHED ? blockIdx.z * gridDim.x + blockIdx.x : blockIdx.x;
+      const unsigned first = tile * splits * TILE_BYTES + wave * WAVE_BYTES + lane * 16;
       const unsigned mine = first + blockIdx.y * TILE_BYTES;
 #pragma unroll
       for (int i = 0; i < FM; ++i)
@@ -1426,11 +1435,11 @@ __global__ void __launch_bounds__(WM *WN * 64) contraction_kernel(const Contract
           }
       __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
       __syncthreads();
-      if (tid == 0) s_ticket = __hip_atomic_fetch_add(args.fuse_count + blockIdx.x, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (tid == 0) s_ticket = __hip_atomic_fetch_add(args.fuse_count + tile, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       __syncthreads();
       if (s_ticket != splits - 1) return;
       // (back to zero for the next launch on this stream)
-      if (tid == 0) __hip_atomic_store(args.fuse_count + blockIdx.x, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (tid == 0) __hip_atomic_store(args.fuse_count + tile, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 #pragma unroll
       for (int i = 0; i < FM; ++i)
 #pragma unroll
@@ -1612,7 +1621,7 @@ int launch_contraction(const ContractionArgs &a, bool conv, int dtype, bool b_nc
   const bool listed = !conv && a.tile_list != nullptr;  // one workgroup per record, no split grid
   const dim3 grid((unsigned)(listed ? a.tile_count : a.grid_m * a.grid_n),
                   (unsigned)(!listed && a.k_split > 0 ? (a.K + a.k_split - 1) / a.k_split : 1),
-                  (unsigned)(conv && a.phases > 1 ? a.phases : 1)),
+                  (unsigned)(conv ? (a.phases > 1 ? a.phases : 1) : (a.batch > 1 ? a.batch : 1))),
       block(WM * WN * 64);
 #define TRACEA_LAUNCH(DTV, CONVV, NCV)                                                       \
   do {                                                                                       \

@@ -430,14 +430,19 @@ inline bool conv_only(const ContractionVariant &v) { return v.pipeline >= 4; }
 
 constexpr int kOneLaunchMaxSplits = 4;  // finest split that runs as one launch (see launch_maybe_split)
 
-int choose_split(const ContractionVariant &v, int M, int N, int K, int *k_split, int min_tiles = 4) {
-  const long long tiles = (long long)((M + v.bm - 1) / v.bm) * ((N + v.bn - 1) / v.bn);
+// The members that run several products of one shape in one launch (ContractionArgs::batch): the small tiles.  A
+// product that fills the device with 256x256 tiles has nothing to gain from company.
+inline bool takes_batches(const ContractionVariant &v) { return !conv_only(v) && v.bm * v.bn <= 128 * 128; }
+
+int choose_split(const ContractionVariant &v, int M, int N, int K, int *k_split, int min_tiles = 4, int batch = 1) {
+  const long long tiles = (long long)((M + v.bm - 1) / v.bm) * ((N + v.bn - 1) / v.bn) * batch;
   const int nk = (K + v.bk - 1) / v.bk;
   const long long cus = device_limits().cus;
   if (v.bk >= 128 && min_tiles == 4) min_tiles = 2;  // (a range is at least 256 deep, whatever the K tile)
   if (conv_only(v) || tiles * 2 > cus || nk < 2 * min_tiles) return 1;
   long long splits = cus / tiles;
   if (splits > nk / min_tiles) splits = nk / min_tiles;  // at least min_tiles K tiles per range
+  if (batch > 1 && splits > kOneLaunchMaxSplits) splits = kOneLaunchMaxSplits;  // (a batch has no reduction kernel)
   if (splits < 2) return 1;
   const int per = (int)((nk + splits - 1) / splits);
   *k_split = per * v.bk;
@@ -453,7 +458,7 @@ int choose_split(const ContractionVariant &v, int M, int N, int K, int *k_split,
 // The slot rate is calibrated on the 4096^3 GEMM (256x256 tiles, one round, 120 us);
 // the estimate then reads 52.8 / 25.9 us for a 3x3 convolution on N32 7x7x512 with
 // unsplit 64x64 tiles / 128x128 tiles split four ways, where 53.7 / 29.6 us were measured.
-int select_contraction_variant(int m, int n, int k, bool conv, bool b_ncontig) {
+int select_contraction_variant(int m, int n, int k, bool conv, bool b_ncontig, int batch) {
   (void)conv;
   const DeviceLimits &dev = device_limits();
   const double cus = (double)dev.cus, slot_rate = dev.slot_rate;  // multiply-accumulates per microsecond and CU at efficiency 1
@@ -462,9 +467,10 @@ int select_contraction_variant(int m, int n, int k, bool conv, bool b_ncontig) {
   for (int i = 0; i < contraction_variant_count(); ++i) {
     const ContractionVariant &v = contraction_variant(i);
     if (conv_only(v)) continue;  // needs the convolution geometry: see plan_conv_patch
-    const double gm = (double)((m + v.bm - 1) / v.bm), gn = (double)((n + v.bn - 1) / v.bn);
+    if (batch > 1 && !takes_batches(v)) continue;
+    const double gm = (double)((m + v.bm - 1) / v.bm) * batch, gn = (double)((n + v.bn - 1) / v.bn);
     int k_split = 0;
-    const int splits = g_split_k_enabled.load() ? choose_split(v, m, n, k, &k_split) : 1;
+    const int splits = g_split_k_enabled.load() ? choose_split(v, m, n, k, &k_split, 4, batch) : 1;
     const double units = gm * gn * splits;
     const double k_per = splits > 1 ? (double)k_split : (double)(k > 0 ? k : 1);
     const double exact = units / cus > 1.0 ? units / cus : 1.0;
@@ -519,7 +525,7 @@ int select_contraction_variant(int m, int n, int k, bool conv, bool b_ncontig) {
     double cost = rounds * (double)v.bm * (double)v.bn * k_per / (slot_rate * prior);
     // (a coarse split on a tile up to 128x128 runs as one launch, see launch_maybe_split: about a microsecond less)
     const bool one_launch = splits <= kOneLaunchMaxSplits && v.bm * v.bn <= 128 * 128 && v.mfma == 32 && g_split_k_one_launch.load();
-    if (splits > 1) cost += (one_launch ? 3.0 : 4.0) + (double)splits * m * n * 4.0 / 3.0e6;
+    if (splits > 1) cost += (one_launch ? 3.0 : 4.0) + (double)splits * m * n * batch * 4.0 / 3.0e6;
     if (best < 0 || cost < best_cost) {
       best_cost = cost;
       best = i;
@@ -710,7 +716,8 @@ TraceaStatus launch_maybe_split(const char *what, const ContractionVariant &v, C
                                 const EpilogueChain &chain, bool conv, int dtype, bool b_ncontig, int device,
                                 hipStream_t stream, bool static_only = false) {
   int k_split = 0;
-  const int splits = g_split_k_enabled.load() ? choose_split(v, args.M, args.N, args.K, &k_split) : 1;
+  const int batch = args.batch > 1 ? args.batch : 1;
+  const int splits = g_split_k_enabled.load() ? choose_split(v, args.M, args.N, args.K, &k_split, 4, batch) : 1;
   t_last_split_launches = 1;
   // One launch: the tile's last workgroup sums the partial products and runs the chain (tiles up to
   // 128x128: the larger kernels do not carry the code; never for the entry point that must not allocate).
@@ -718,7 +725,7 @@ TraceaStatus launch_maybe_split(const char *what, const ContractionVariant &v, C
   // one CU, where the reduction kernel spreads them over the device.  Measured, 20 launches in a graph:
   // 2 ranges 6.6 us against 7.6, 4 ranges 7.2-7.8 against 8.0-9.3, 9 ranges 8.9 against 7.7, 18 ranges
   // 12.8 against 8.5.
-  const long long tiles = (long long)args.grid_m * args.grid_n;
+  const long long tiles = (long long)args.grid_m * args.grid_n * batch;
   if (splits > 1 && splits <= kOneLaunchMaxSplits && g_split_k_one_launch.load() && !static_only && v.bm * v.bn <= 128 * 128 && v.mfma == 32 && args.phases <= 1 &&
       args.out_map == 0 && args.tile_list == nullptr && tiles <= kFuseTiles) {
     const size_t bytes = (size_t)tiles * (size_t)splits * (size_t)(v.bm * v.bn) * 4;
@@ -736,7 +743,7 @@ TraceaStatus launch_maybe_split(const char *what, const ContractionVariant &v, C
     }
   }
   TraceaStatus ws = TRACEA_SUCCESS;
-  void *scratch = split_workspace(what, static_only, device, stream, splits, args.M, args.N, &ws);
+  void *scratch = batch > 1 ? nullptr : split_workspace(what, static_only, device, stream, splits, args.M, args.N, &ws);
   if (ws != TRACEA_SUCCESS) return ws;
   t_last_splits = scratch != nullptr ? splits : 1;
   if (scratch == nullptr) {
@@ -761,20 +768,71 @@ TraceaStatus launch_maybe_split(const char *what, const ContractionVariant &v, C
 }
 
 // ---- GEMM ----------------------------------------------------------------------
+// Several products of one shape, `count` of them, operand z at the given multiples of z elements behind the views.
+struct GemmBatch {
+  int count = 1;
+  long long a = 0, b = 0, c = 0;
+};
+
+// What the half-precision tile kernels read in place.
+struct HalfLayout {
+  bool ok, b_kcontig;
+};
+HalfLayout half_layout(const View &a, const View &b, const View &c) {
+  HalfLayout l{false, false};
+  if (!is_half(a.dtype) || b.dtype != a.dtype || a.shape[1] <= 0) return l;
+  const bool a_ok = a.stride[1] == 1 && a.stride[0] % 8 == 0 && a.shape[1] % 8 == 0 && aligned(a.ptr, 16);
+  const bool b_ncontig = b.stride[1] == 1 && b.stride[0] % 8 == 0 && b.shape[1] % 8 == 0 && aligned(b.ptr, 16);
+  l.b_kcontig = b.stride[0] == 1 && b.stride[1] % 8 == 0 && aligned(b.ptr, 16);
+  l.ok = a_ok && (l.b_kcontig || b_ncontig) && c.stride[1] == 1;
+  return l;
+}
+// What the fp32 tile kernels read in place.  (N itself may be ragged where B is read through a buffer descriptor,
+// i.e. below 2 GiB: a piece that starts inside N is read whole -- what lies behind N in the row only reaches output
+// columns that are never stored, and behind the last row the descriptor returns zeros -- and the epilogue stores by
+// valid channels.)
+bool f32_layout(const View &a, const View &b, const View &c) {
+  const long long K = a.shape[1], N = b.shape[1];
+  return a.dtype == TRACEA_DTYPE_FLOAT32 && b.dtype == TRACEA_DTYPE_FLOAT32 && c.dtype == TRACEA_DTYPE_FLOAT32 && K > 0 &&
+         a.stride[1] == 1 && b.stride[1] == 1 && c.stride[1] == 1 && K % 4 == 0 &&
+         (N % 4 == 0 || ((K - 1) * b.stride[0] + N) * 4 < (1ll << 31)) && a.stride[0] % 4 == 0 && b.stride[0] % 4 == 0 &&
+         aligned(a.ptr, 16) && aligned(b.ptr, 16);
+}
+
+// True when run_gemm takes the batch in one launch: operands of every product as the tile kernels read them and below
+// 2 GiB, output batches a whole number of rows apart, and a product too small to fill the device on its own -- one of
+// 256 or more 256x256 tiles runs faster on those, which take no batch.  Sixteen products of 128x512x512 in f16: 16
+// launches of 8.4 us each, 135 us a call, against one of 9 us.
+bool gemm_batch_in_one_launch(const View &a, const View &b, const View &c, const GemmBatch &batch) {
+  const long long M = a.shape[0], K = a.shape[1], N = b.shape[1];
+  const bool f32 = f32_layout(a, b, c);
+  const HalfLayout half = half_layout(a, b, c);
+  if (!f32 && !half.ok) return false;
+  const int step = f32 ? 4 : 8, esz = f32 ? 4 : 2;
+  const long long a_extent = ((M - 1) * a.stride[0] + K) * esz;
+  const long long b_extent = half.ok && half.b_kcontig ? ((N - 1) * b.stride[1] + K) * esz : ((K - 1) * b.stride[0] + N) * esz;
+  if (a_extent >= (1ll << 31) || b_extent >= (1ll << 31)) return false;
+  if (batch.a % step != 0 || batch.b % step != 0 || c.stride[0] <= 0 || batch.c % c.stride[0] != 0 || batch.count > 65535) return false;
+  if (!f32) {
+    const int forced = forced_variant("gemm");
+    if (forced >= 0 && !takes_batches(contraction_variant(forced))) return false;
+    if (((M + 255) / 256) * ((N + 255) / 256) >= device_limits().cus) return false;
+  }
+  return true;
+}
+
 TraceaStatus run_gemm(const View &a, const View &b, const View &c, const EpilogueChain &chain,
-                      hipStream_t stream, bool static_only = false) {
+                      hipStream_t stream, bool static_only = false, const GemmBatch &batch = GemmBatch()) {
   const long long M = a.shape[0], K = a.shape[1], N = b.shape[1];
   t_last_contraction = -1;
   if (M == 0 || N == 0) return TRACEA_SUCCESS;
   DeviceScope scope(c.device);
   if (scope.err != hipSuccess) return hip_status("hipSetDevice", (int)scope.err);
 
-  if (is_half(a.dtype) && b.dtype == a.dtype && K > 0) {
-    const bool a_ok = a.stride[1] == 1 && a.stride[0] % 8 == 0 && K % 8 == 0 && aligned(a.ptr, 16);
-    const bool b_kcontig = b.stride[0] == 1 && b.stride[1] % 8 == 0 && aligned(b.ptr, 16);
-    const bool b_ncontig = b.stride[1] == 1 && b.stride[0] % 8 == 0 && N % 8 == 0 && aligned(b.ptr, 16);
-    const bool c_ok = c.stride[1] == 1;
-    if (a_ok && (b_kcontig || b_ncontig) && c_ok) {
+  {
+    const HalfLayout half = half_layout(a, b, c);
+    const bool b_kcontig = half.b_kcontig;
+    if (half.ok) {
       ContractionArgs args{};
       args.A = a.ptr; args.B = b.ptr; args.C = c.ptr;
       args.M = (int)M; args.N = (int)N; args.K = (int)K;
@@ -783,9 +841,17 @@ TraceaStatus run_gemm(const View &a, const View &b, const View &c, const Epilogu
       args.ldc = c.stride[0];
       args.out_dtype = c.dtype;
       args.epi = chain;
-      char key[160];
-      snprintf(key, sizeof(key), "gemm_%lld_%lld_%lld_%s", M, N, K, tuning_device_name());
-      int vi = pick_contraction("gemm", key, (int)M, (int)N, (int)K, false, a.dtype, !b_kcontig);
+      int vi;
+      if (batch.count > 1) {
+        args.batch = batch.count;
+        args.batch_a = batch.a; args.batch_b = batch.b; args.batch_rows = batch.c / c.stride[0];
+        vi = forced_variant("gemm");
+        if (vi < 0) vi = select_contraction_variant((int)M, (int)N, (int)K, false, !b_kcontig, batch.count);
+      } else {
+        char key[160];
+        snprintf(key, sizeof(key), "gemm_%lld_%lld_%lld_%s", M, N, K, tuning_device_name());
+        vi = pick_contraction("gemm", key, (int)M, (int)N, (int)K, false, a.dtype, !b_kcontig);
+      }
       if (vi < 0) return fail(TRACEA_UNKNOWN_ERROR, "gemm: no kernel variant available");
       // direct-to-LDS variants address operands with 32-bit byte offsets below 2 GiB
       const long long a_extent = ((M - 1) * a.stride[0] + K) * 2;
@@ -800,14 +866,12 @@ TraceaStatus run_gemm(const View &a, const View &b, const View &c, const Epilogu
       return launch_maybe_split("gemm launch", v, args, chain, false, a.dtype, !b_kcontig, c.device, stream, static_only);
     }
   }
-  if (a.dtype == TRACEA_DTYPE_FLOAT32 && b.dtype == TRACEA_DTYPE_FLOAT32 && c.dtype == TRACEA_DTYPE_FLOAT32 && K > 0 &&
-      a.stride[1] == 1 && b.stride[1] == 1 && c.stride[1] == 1 && K % 4 == 0 &&
-      (N % 4 == 0 || ((K - 1) * b.stride[0] + N) * 4 < (1ll << 31)) &&
-      a.stride[0] % 4 == 0 && b.stride[0] % 4 == 0 && aligned(a.ptr, 16) && aligned(b.ptr, 16)) {
-    // (N itself may be ragged where B is read through a buffer descriptor, i.e. below 2 GiB: a piece that starts
-    // inside N is read whole -- what lies behind N in the row only reaches output columns that are never stored,
-    // and behind the last row the descriptor returns zeros -- and the epilogue stores by valid channels)
+  if (f32_layout(a, b, c)) {
     ContractionArgs args{};
+    if (batch.count > 1) {
+      args.batch = batch.count;
+      args.batch_a = batch.a; args.batch_b = batch.b; args.batch_rows = batch.c / c.stride[0];
+    }
     args.A = a.ptr; args.B = b.ptr; args.C = c.ptr;
     args.M = (int)M; args.N = (int)N; args.K = (int)K;
     args.lda = a.stride[0]; args.ldb = b.stride[0]; args.ldc = c.stride[0];
@@ -825,7 +889,8 @@ TraceaStatus run_gemm(const View &a, const View &b, const View &c, const Epilogu
     // 3072^3 558 / 441, 2048^3 134.7 / 133.4, 4096^3 972 / 1033.  (A 128x64 tile was never the fastest:
     // 477 at 3072^3, 1003 at 4096^3.)
     static const ContractionVariant f32_tile128 = {"f32_128x128x16", 128, 128, 16, 2, 2, 1, 0, 0, nullptr, 32};
-    const long long tiles128 = ((M + 127) / 128) * ((N + 127) / 128), tiles64 = ((M + 63) / 64) * ((N + 63) / 64);
+    const long long tiles128 = ((M + 127) / 128) * ((N + 127) / 128) * batch.count,
+                    tiles64 = ((M + 63) / 64) * ((N + 63) / 64) * batch.count;
     const long long ncu = device_limits().cus;
     int tile = args.a_bytes != 0 && (double)((tiles64 + ncu - 1) / ncu) * 1.06 < (double)((tiles128 + ncu - 1) / ncu) * 4.0 ? 64 : 128;
     int k_split = 0, splits = 1;
@@ -862,7 +927,7 @@ TraceaStatus run_gemm(const View &a, const View &b, const View &c, const Epilogu
         splits = (nk + per - 1) / per;
       }
     } else {
-      splits = g_split_k_enabled.load() ? choose_split(f32_tile128, (int)M, (int)N, (int)K, &k_split, 4) : 1;
+      splits = g_split_k_enabled.load() ? choose_split(f32_tile128, (int)M, (int)N, (int)K, &k_split, 4, batch.count) : 1;
     }
     const long long tiles = tile == 128 ? tiles128 : tiles64;
     const size_t tile_elts = tile == 128 ? 128 * 128 : 64 * 64;
@@ -881,7 +946,7 @@ TraceaStatus run_gemm(const View &a, const View &b, const View &c, const Epilogu
       }
     }
     TraceaStatus ws = TRACEA_SUCCESS;
-    void *scratch = split_workspace("gemm_f32 launch", static_only, c.device, stream, splits, M, N, &ws);
+    void *scratch = batch.count > 1 ? nullptr : split_workspace("gemm_f32 launch", static_only, c.device, stream, splits, M, N, &ws);
     if (ws != TRACEA_SUCCESS) return ws;
     t_last_splits = scratch != nullptr ? splits : 1;
     if (scratch == nullptr) {
@@ -1334,6 +1399,10 @@ TraceaStatus dispatch_linear(const TraceaTensorView &ta, const TraceaTensorView 
     a2.shape[0] = c2.shape[0] = B * M;
     return run_gemm(a2, w2, c2, chain, stream);
   }
+  GemmBatch batch;
+  batch.count = (int)std::min(B, 65536ll);
+  batch.a = a.stride[0]; batch.b = shared ? 0 : w.stride[0]; batch.c = c.stride[0];
+  if (B > 1 && gemm_batch_in_one_launch(a2, w2, c2, batch)) return run_gemm(a2, w2, c2, chain, stream, false, batch);
   for (long long b = 0; b < B; ++b) {
     View ab = a2, wb = w2, cb = c2;
     ab.ptr = (char *)a.ptr + b * a.stride[0] * elem_size(a.dtype);

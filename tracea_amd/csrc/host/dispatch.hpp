@@ -115,7 +115,7 @@ TraceaStatus dispatch_clock_probe(void *out, int32_t samples, int32_t gap, void 
 
 // Heuristic choice among the feasible contraction variants (used when neither a
 // forced variant nor a tuning-cache entry decides).  Returns -1 if none fits.
-int select_contraction_variant(int m, int n, int k, bool conv, bool b_ncontig = false);
+int select_contraction_variant(int m, int n, int k, bool conv, bool b_ncontig = false, int batch = 1);
 
 // TraceaResult builders: strings are malloc'ed, released by tracea_free_string.
 struct PipelineConfig;

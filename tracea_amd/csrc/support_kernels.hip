@@ -201,11 +201,13 @@ __global__ void __launch_bounds__(256) gemm_f32_dma_kernel(const ContractionArgs
   const int K = args.k_split > 0 ? min(args.K, kb + args.k_split) : args.K;
   // one-launch split: see the block in front of the epilogue
   const bool fused = args.k_split > 0 && args.fuse_ws != nullptr;
-  const long long zrow = args.k_split > 0 && !fused ? (long long)blockIdx.y * M : 0ll;
+  const long long zrow = (args.k_split > 0 && !fused ? (long long)blockIdx.y * M : 0ll) + (long long)blockIdx.z * args.batch_rows;
+  const float *Ag = (const float *)args.A + (long long)blockIdx.z * args.batch_a;
+  const float *Bg = (const float *)args.B + (long long)blockIdx.z * args.batch_b;
 
   constexpr unsigned OOB = 0x80000000u;
-  __amdgpu_buffer_rsrc_t rsrc_a = __builtin_amdgcn_make_buffer_rsrc((void *)args.A, 0, (int)args.a_bytes, 0x00020000);
-  __amdgpu_buffer_rsrc_t rsrc_b = __builtin_amdgcn_make_buffer_rsrc((void *)args.B, 0, (int)args.b_bytes, 0x00020000);
+  __amdgpu_buffer_rsrc_t rsrc_a = __builtin_amdgcn_make_buffer_rsrc((void *)Ag, 0, (int)args.a_bytes, 0x00020000);
+  __amdgpu_buffer_rsrc_t rsrc_b = __builtin_amdgcn_make_buffer_rsrc((void *)Bg, 0, (int)args.b_bytes, 0x00020000);
   // TM pieces of A and TN of B per thread and K tile
   unsigned a_voff[TM], b_voff[TN];
   int a_kcol[TM], b_krow[TN];
@@ -408,7 +410,8 @@ __global__ void __launch_bounds__(256) gemm_f32_dma_kernel(const ContractionArgs
     const unsigned splits = gridDim.y;
     constexpr unsigned TILE_BYTES = BM * BN * 4, WAVE_BYTES = TILE_BYTES / 4;
     __amdgpu_buffer_rsrc_t rsrc_ws = __builtin_amdgcn_make_buffer_rsrc((void *)args.fuse_ws, 0, 0x7fffffff, 0x00020000);
-    const unsigned first = blockIdx.x * splits * TILE_BYTES + wave_u * WAVE_BYTES + lane * 16;
+    const unsigned tile = blockIdx.z * gridDim.x + blockIdx.x;
+    const unsigned first = tile * splits * TILE_BYTES + wave_u * WAVE_BYTES + lane * 16;
     const unsigned mine = first + blockIdx.y * TILE_BYTES;
 #pragma unroll
     for (int i = 0; i < TM; ++i)
@@ -422,10 +425,10 @@ __global__ void __launch_bounds__(256) gemm_f32_dma_kernel(const ContractionArgs
         }
     __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): the stores are acknowledged
     __syncthreads();
-    if (tid == 0) s_ticket = __hip_atomic_fetch_add(args.fuse_count + blockIdx.x, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (tid == 0) s_ticket = __hip_atomic_fetch_add(args.fuse_count + tile, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     __syncthreads();
     if (s_ticket != splits - 1) return;
-    if (tid == 0) __hip_atomic_store(args.fuse_count + blockIdx.x, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (tid == 0) __hip_atomic_store(args.fuse_count + tile, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
@@ -462,7 +465,8 @@ int launch_gemm_f32(const ContractionArgs &a, int tile, hipStream_t stream) {
   args.grid_n = (a.N + edge - 1) / edge;
   args.group_m = 4;
   const unsigned splits = a.k_split > 0 ? (unsigned)((a.K + a.k_split - 1) / a.k_split) : 1u;
-  const dim3 grid((unsigned)(args.grid_m * args.grid_n), splits);
+  const dim3 grid((unsigned)(args.grid_m * args.grid_n), splits, (unsigned)(a.batch > 1 ? a.batch : 1));
+  if (!dma && a.batch > 1) return (int)hipErrorInvalidValue;  // (the register-staged twin takes one product)
   if (!dma) hipLaunchKernelGGL(gemm_f32_kernel, grid, dim3(256), 0, stream, args);
   else if (tile == 64) hipLaunchKernelGGL((gemm_f32_dma_kernel<1, 1, 4, 1>), grid, dim3(256), 0, stream, args);
   else if (tile == 6432) hipLaunchKernelGGL((gemm_f32_dma_kernel<1, 1, 4, 2>), grid, dim3(256), 0, stream, args);
