@@ -198,7 +198,7 @@ TraceaStatus tracea_low_rank_mlp(TraceaTensorView x, TraceaTensorView a, TraceaT
 
 /* ---- FlashAttention-2 forward: reference include/tracea.hpp:147-149,
  * src/interface/c_bindings.rs:443-495.  q,k,v,o [B,H,S,D], f16 or bf16, D <= 128.
- * The kernels read D = 64 or 128 with a contiguous head dimension, other strides
+ * The kernels read a D that is a multiple of 8 with a contiguous head dimension, other strides
  * multiples of 8 elements and bases on 16 bytes in place.  Any other D from 1 to
  * 128 (the reference compiles its kernel for the head dimension at hand:
  * src/kernels/attention/cuda_emitter.rs:39-58) and any other strides or bases

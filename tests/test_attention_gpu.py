@@ -277,3 +277,29 @@ def test_other_head_dimensions_and_unaligned_tensors_run_from_padded_copies(trac
     got = tracea_gpu.attention(qt, kw[..., :64], vo, causal=False, out=out_wide[..., 3:67])
     assert_close_scaled(got.float().cpu().numpy(), want, _tol(d, dtype), "unaligned tensors")
     assert (out_wide[..., :3] == 7.0).all() and (out_wide[..., 67:] == 7.0).all()   # nothing written beside the result
+
+
+@pytest.mark.parametrize("dtype", ["bf16", "f16"])
+@pytest.mark.parametrize("d", [8, 40, 56, 72, 96, 104, 120])
+def test_head_dimensions_that_are_multiples_of_8_run_in_place(tracea_gpu, dtype, d):
+    """The members that stop at the tensors' last column: head dimensions on either side of their 32-wide blocks and of
+    the tile widths, one and several tiles, a length inside a tile.  The tensors are column slices of larger ones full
+    of NaN, which neither the score product nor the result may take in, and the columns beside the result stay."""
+    from tracea_amd import capi
+    tdt, rnd = (torch.bfloat16, round_bf16) if dtype == "bf16" else (torch.float16, round_f16)
+    for (b, h, s) in [(1, 2, 1), (2, 1, 77), (1, 2, 300), (1, 1, 640)]:
+        q, k, v = _inputs(b, h, s, d, 13 * s + d, rnd)
+
+        def inside(x):  # [B,S,H,D+8] storage, seen as [B,H,S,D]
+            big = torch.full((b, s, h, d + 8), float("nan"), device="cuda", dtype=tdt)
+            view = big[..., :d].transpose(1, 2)
+            if x is not None:
+                view.copy_(_dev(x, tdt))
+            return big, view
+        for causal in (False, True):
+            want = oracle.attention_bhsd(q, k, v, 1.0 / np.sqrt(d), causal)
+            big, out = inside(None)
+            tracea_gpu.attention(inside(q)[1], inside(k)[1], inside(v)[1], causal=causal, out=out)
+            assert "part" in capi.last_variant("attention")
+            assert_close_scaled(out.float().cpu().numpy(), want, _tol(d, dtype), "D=%d S=%d causal=%s %s" % (d, s, causal, dtype))
+            assert torch.isnan(big[..., d:].float()).all()

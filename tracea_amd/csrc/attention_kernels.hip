@@ -413,9 +413,20 @@ constexpr bool fa2_pipe_parks_queries(int d, int qb, int items, bool shift) { re
 // phase B.  K(u+2) is requested by every wave at the barrier that opens slot 2u, V(u+1) at the one that opens
 // slot 2u+1; a request has two slots to land, and a barrier waits for the one before last.  Eight waves, one
 // query block per workgroup, two-stage rings, no causal mask (waves would differ in their number of tiles).
-template <int DT, int D, bool EARLY_MAX, int WAVES, int NSTG, int QB, int ITEMS = 1, bool SHIFT = false, bool PP = false>
+//
+// DU: head dimensions between the two tile widths.  The tensors have a.D <= DU columns (a multiple of 8); the tiles keep
+// the row pitch of D = 64 or 128, columns from a.D on are requested out of range (zeros, no memory traffic), and
+// the products run over DU columns only: DU / 16 k-steps of the score product, DU / 32 blocks of O.  0: exactly D
+// columns, no tests anywhere.  Such a call used to copy Q, K and V into padded tensors, run the kernel for D on them and
+// copy the result back: B2 H16 S1000 D96 causal 4 copies of 11-15 us each around a kernel of 20 us, 70 us a
+// call, against 19 us.
+template <int DT, int D, bool EARLY_MAX, int WAVES, int NSTG, int QB, int ITEMS = 1, bool SHIFT = false, bool PP = false, int DU = 0>
 __global__ void __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(QB == 1 ? 2 : 1, QB == 1 ? 2 : 1)))
 fa2_fwd_pipe_kernel(const AttentionArgs a) {
+  constexpr bool PART = DU > 0;
+  constexpr int DC = PART ? DU : D;  // columns the products run over
+  static_assert(!PART || (DU <= D && DU % 32 == 0 && EARLY_MAX && SHIFT && !PP && ITEMS == 1 && QB == 1), "partial head dimensions exist in the default form only");
+  const int d_cols = PART ? a.D : D;  // columns the tensors have
   static_assert(!PP || (EARLY_MAX && WAVES == 8 && NSTG == 2 && QB == 1 && ITEMS == 1), "the half-iteration offset exists for eight waves, one block, two stages");
   static_assert(!SHIFT || EARLY_MAX, "the shifted score product exists in the two-phase form only");
   constexpr bool PARK = fa2_pipe_parks_queries(D, QB, ITEMS, SHIFT);
@@ -426,8 +437,8 @@ fa2_fwd_pipe_kernel(const AttentionArgs a) {
   constexpr int ROW_BYTES = D * 2;
   constexpr int CH = D / 8;
   constexpr int TILE_BYTES = FA_BKV * ROW_BYTES;
-  constexpr int KS = D / 16;
-  constexpr int DB = D / 32;
+  constexpr int KS = DC / 16;
+  constexpr int DB = DC / 32;
   constexpr int RPI = 64 / CH;                 // tile rows per wave-wide load instruction
   constexpr int NI = FA_BKV / (RPI * WAVES); // load instructions per wave per tensor per tile
   constexpr int RP = 256 / ROW_BYTES > 0 ? 256 / ROW_BYTES : 1;
@@ -505,7 +516,16 @@ fa2_fwd_pipe_kernel(const AttentionArgs a) {
       const int qr = mine < S ? mine : S - 1;
       const unsigned short *qp = Qg + (long long)qr * a.q_ss + g * 8;
 #pragma unroll
-      for (int ks = 0; ks < NK; ++ks) dst[qi][ks] = prescale(*(const u32x4 *)(qp + ks * 16));
+      for (int ks = 0; ks < NK; ++ks) {
+        if constexpr (PART) {
+          const bool in = ks * 16 + g * 8 < d_cols;
+          const u32x4 raw = *(const u32x4 *)(in ? qp + ks * 16 : qp - g * 8);
+          const u32x4 zero4 = {0u, 0u, 0u, 0u};
+          dst[qi][ks] = prescale(in ? raw : zero4);
+        } else {
+          dst[qi][ks] = prescale(*(const u32x4 *)(qp + ks * 16));
+        }
+      }
     }
   };
 #pragma unroll
@@ -526,9 +546,9 @@ fa2_fwd_pipe_kernel(const AttentionArgs a) {
 
   // Buffer views of this (batch, head) slice: rows 0..S-1; anything beyond reads as zero.
   __amdgpu_buffer_rsrc_t rsrc_k = __builtin_amdgcn_make_buffer_rsrc(
-      (void *)Kg, 0, (int)(((long long)(S - 1) * a.k_ss + D) * 2), 0x00020000);
+      (void *)Kg, 0, (int)(((long long)(S - 1) * a.k_ss + d_cols) * 2), 0x00020000);
   __amdgpu_buffer_rsrc_t rsrc_v = __builtin_amdgcn_make_buffer_rsrc(
-      (void *)Vg, 0, (int)(((long long)(S - 1) * a.v_ss + D) * 2), 0x00020000);
+      (void *)Vg, 0, (int)(((long long)(S - 1) * a.v_ss + d_cols) * 2), 0x00020000);
   // Load instruction i of this wave covers tile rows (i*WAVES + wave)*RPI + lane/CH; the lane's
   // LDS slot is 16-byte column lane%CH of that row, so it fetches the global column that the
   // swizzle of the tensor maps there.
@@ -539,6 +559,11 @@ fa2_fwd_pipe_kernel(const AttentionArgs a) {
     const int p = lane % CH;
     k_voff[i] = (unsigned)(row * (int)a.k_ss * 2 + ((p ^ ((row / RP) & (CH - 1))) << 4));
     v_voff[i] = (unsigned)(row * (int)a.v_ss * 2 + ((p ^ (((row / RP) % WIN) << 2)) << 4));
+    if constexpr (PART) {
+      // (out of range whatever tile offset is added: a slice ends below 2 GiB)
+      if (((p ^ ((row / RP) & (CH - 1))) << 3) >= d_cols) k_voff[i] = 0x80000000u;
+      if (((p ^ (((row / RP) % WIN) << 2)) << 3) >= d_cols) v_voff[i] = 0x80000000u;
+    }
   }
   auto load_k = [&](int t, unsigned char *dst) __attribute__((always_inline)) {
     const unsigned adv = (unsigned)t * (unsigned)(FA_BKV * 2) * (unsigned)a.k_ss;
@@ -926,8 +951,8 @@ fa2_fwd_pipe_kernel(const AttentionArgs a) {
       // ---- phase A: S^T(t+1) = K(t+1) Q^T  with  P(t) = exp2(S(t)*scale - m), row sums ----
       // chunk ks: the 2*QB MFMAs of k-step ks (operands read one chunk ahead) and
       // 32*QB/KS of the 32*QB exponentials
-      constexpr int EPC = 32 * QB / KS;  // exponentials per chunk
-      static_assert((32 * QB) % KS == 0 && (EPC == 4 || EPC == 8 || EPC == 16), "exponentials must divide over the k-steps");
+      constexpr int EPC = (32 * QB + KS - 1) / KS;  // most exponentials of a chunk
+      static_assert(KS >= 2 && KS <= 8 * QB, "exponentials must divide over the k-steps");
       __builtin_amdgcn_sched_barrier(0);
       // The wave runs this phase at raised priority: a SIMD holds two waves (of two workgroups, or of one
       // eight-wave workgroup) that are not in step, and the one inside its exponentials -- the vector ALU's
@@ -964,7 +989,9 @@ fa2_fwd_pipe_kernel(const AttentionArgs a) {
         }
 #pragma unroll
         for (int j = 0; j < EPC; ++j) {
-          const int idx = ks * EPC + j;  // 0..32*QB-1 over (query block, blk, element): block idx/32, blk (idx%32)/16
+          // 0..32*QB-1 over (query block, blk, element): block idx/32, blk (idx%32)/16
+          const int idx = (ks * 32 * QB) / KS + j;
+          if (idx >= ((ks + 1) * 32 * QB) / KS) continue;
           const int qi = idx >> 5, w = idx & 31;
           const float x = SHIFT ? __builtin_amdgcn_exp2f(cur[qi][w >> 4][w & 15])
                                 : __builtin_amdgcn_exp2f(fmaf(cur[qi][w >> 4][w & 15], a.scale_log2, -m_run[qi]));
@@ -1240,7 +1267,7 @@ fa2_fwd_pipe_kernel(const AttentionArgs a) {
           asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1" : "+v"(e0), "+v"(o0));
           asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1" : "+v"(e1), "+v"(o1));
           const u32x4 row16 = {e0, e1, o0, o1};
-          if (q_mine[qi] < S) *(u32x4 *)(orow + d * 32 + (vp * 2 + g) * 8) = row16;
+          if (q_mine[qi] < S && (!PART || d * 32 + (vp * 2 + g) * 8 < d_cols)) *(u32x4 *)(orow + d * 32 + (vp * 2 + g) * 8) = row16;
         }
     }
     tb += ntiles;
@@ -1250,7 +1277,7 @@ fa2_fwd_pipe_kernel(const AttentionArgs a) {
   __builtin_amdgcn_s_waitcnt(0x0f70);
 }
 
-template <int D, bool EARLY_MAX, int WAVES, int NSTG, int QB = 1, int ITEMS = 1, bool SHIFT = false, bool PP = false>
+template <int D, bool EARLY_MAX, int WAVES, int NSTG, int QB = 1, int ITEMS = 1, bool SHIFT = false, bool PP = false, int DU = 0>
 static int launch_fa2_pipe(const AttentionArgs &a, int dtype, hipStream_t stream) {
   if (PP && a.causal) return (int)hipErrorInvalidValue;  // (its feasibility test keeps such a call away)
   // the K and V rings (O leaves from registers), and where they are parked half of the next block's queries
@@ -1261,7 +1288,7 @@ static int launch_fa2_pipe(const AttentionArgs &a, int dtype, hipStream_t stream
   const dim3 grid((unsigned)(nqb / ITEMS * a.B * a.H)), block(WAVES * 64);
 #define TRACEA_FA_LAUNCH(DTV)                                                                  \
   do {                                                                                         \
-    auto kfn = fa2_fwd_pipe_kernel<DTV, D, EARLY_MAX, WAVES, NSTG, QB, ITEMS, SHIFT, PP>;      \
+    auto kfn = fa2_fwd_pipe_kernel<DTV, D, EARLY_MAX, WAVES, NSTG, QB, ITEMS, SHIFT, PP, DU>;  \
     static bool attr_done = false;                                                             \
     if (!attr_done) {                                                                          \
       hipError_t e = hipFuncSetAttribute((const void *)kfn,                                    \
@@ -1290,6 +1317,11 @@ static bool slice_fits(const AttentionArgs &a) {
 // (the running maximum is taken over raw scores, which needs a positive scale)
 static bool feasible_pipe_d128(const AttentionArgs &a) { return a.D == 128 && a.scale_log2 > 0.0f && slice_fits(a); }
 static bool feasible_pipe_d64(const AttentionArgs &a) { return a.D == 64 && a.scale_log2 > 0.0f && slice_fits(a); }
+// (the members for tensors of at most DU columns; the one with the fewest comes first in the table)
+template <int LO, int DU>
+static bool feasible_part(const AttentionArgs &a) {
+  return a.D > LO && a.D <= DU && a.D % 8 == 0 && a.D != 64 && a.D != 128 && a.scale_log2 > 0.0f && slice_fits(a);
+}
 // (the members whose wave groups run half an iteration apart: no causal mask)
 static bool feasible_dense_d128(const AttentionArgs &a) { return !a.causal && feasible_pipe_d128(a); }
 static bool feasible_dense_d64(const AttentionArgs &a) { return !a.causal && feasible_pipe_d64(a); }
@@ -1363,6 +1395,10 @@ static const AttentionVariant kAttentionVariants[] = {
     {"fa2_q128_kv64_d128_u16", FA_BQ, FA_BKV, FA_WAVES, 2, &launch_fa2<128, false>, &feasible_d128, 32, 1},
     {"fa2_q128_kv64_d64_tr", FA_BQ, FA_BKV, FA_WAVES, 2, &launch_fa2<64, true>, &feasible_d64, 32, 1},
     {"fa2_q128_kv64_d64_u16", FA_BQ, FA_BKV, FA_WAVES, 2, &launch_fa2<64, false>, &feasible_d64, 32, 1},
+    // head dimensions off 64 and 128
+    {"fa2_q128_kv64_part64", 128, FA_BKV, 4, 2, &launch_fa2_pipe<64, true, 4, 2, 1, 1, true, false, 64>, &feasible_part<0, 64>, 32, 1},
+    {"fa2_q128_kv64_part96", 128, FA_BKV, 4, 2, &launch_fa2_pipe<128, true, 4, 2, 1, 1, true, false, 96>, &feasible_part<64, 96>, 32, 1},
+    {"fa2_q128_kv64_part128", 128, FA_BKV, 4, 2, &launch_fa2_pipe<128, true, 4, 2, 1, 1, true, false, 128>, &feasible_part<96, 128>, 32, 1},
 };
 
 int attention_variant_count() { return (int)(sizeof(kAttentionVariants) / sizeof(kAttentionVariants[0])); }

@@ -2521,12 +2521,16 @@ TraceaStatus dispatch_attention(const TraceaTensorView &tq, const TraceaTensorVi
   if (!(scale == scale) || std::isinf(scale))
     return fail(TRACEA_INVALID_PARAMS, "tracea_attention: scale is not finite");
   const View *views[4] = {&q, &k, &v, &o};
-  bool in_place = D == 64 || D == 128;
+  // (any other multiple of 8 runs in place too, on the members that stop at the tensors' last column: those take a
+  // positive scale and K/V slices below 2 GiB, tiles requested past the end included)
+  const long long reach = S + 4 * 64;
+  bool in_place = D == 64 || D == 128 ||
+                  (D % 8 == 0 && scale > 0.0f && (reach * k.stride[2] + D) * 2 < (1ll << 31) && (reach * v.stride[2] + D) * 2 < (1ll << 31));
   for (const View *t : views)
     if (t->stride[3] != 1 || t->stride[2] % 8 != 0 || t->stride[1] % 8 != 0 || t->stride[0] % 8 != 0 || !aligned(t->ptr, 16))
       in_place = false;
   if (!in_place) {
-    // Head dimensions other than 64 and 128 (the kernels' two), and tensors the kernels cannot read in place
+    // Head dimensions that are no multiple of 8, and tensors the kernels cannot read in place
     // (head dimension strided, other strides off a multiple of 8 elements, bases off 16 bytes): Q, K and V are
     // copied into dense [B,H,S,Dp] tensors, Dp = 64 or 128, zeros behind the data -- they add nothing to a score
     // and give zero output columns -- the kernels run on those with the caller's scale, and the first D columns
@@ -2542,7 +2546,7 @@ TraceaStatus dispatch_attention(const TraceaTensorView &tq, const TraceaTensorVi
     if (buf == nullptr)
       return fail(TRACEA_UNSUPPORTED_CONFIG,
                   "tracea_attention: head dim %lld / these strides need padded copies, and no buffer for them can be had "
-                  "(stream under capture, or above 1 GiB); in place: head dim 64 or 128, contiguous, other strides "
+                  "(stream under capture, or above 1 GiB); in place: head dim a multiple of 8, contiguous, other strides "
                   "multiples of 8 elements, bases 16-byte aligned", D);
     hipStream_t stream = (hipStream_t)params.stream;
     const View *src[3] = {&q, &k, &v};
