@@ -341,3 +341,29 @@ def test_ragged_sizes_and_strided_operands_run_from_padded_copies(tracea_gpu, sh
             assert_close_scaled(got, want, tol_half(k, dtype), "%s %s" % (dtype, tag))
         got = tracea_gpu.gemm(xa, xb, out_dtype=torch.float32).cpu().numpy()
         assert np.abs(got - ref16).max() <= 1e-4 * max(1.0, np.abs(ref16).max()), dtype + " with fp32 output"
+
+
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+@pytest.mark.parametrize("m", [1, 8, 9, 16, 17, 40, 48])
+def test_products_of_a_few_rows(tracea_gpu, dtype, m):
+    """The kernel for at most 48 rows: both layouts of B, row counts on either side of its 8-row loads and 16-row blocks,
+    widths and depths off its tiles (one piece of K, a K tail of 8, more pieces than ring stages, more waves than pieces),
+    the narrow and the wide form (N 11008), a chain, rows of A and C with a gap, rows behind the last one untouched."""
+    from tracea_amd import capi
+    tdt, rnd = (torch.float16, round_f16) if dtype == "f16" else (torch.bfloat16, round_bf16)
+    for (n, k) in [(8, 8), (24, 72), (136, 1096), (1000, 4104), (48, 8192), (11008, 264)]:
+        rng = np.random.default_rng(m + 3 * n + 7 * k)
+        a = rnd(rng.standard_normal((m, k)) / np.sqrt(k))
+        b = rnd(rng.standard_normal((k, n)))
+        bias = rng.standard_normal(n).astype(np.float32)
+        res = rnd(rng.standard_normal((m, n)))
+        ref = np.maximum(oracle.gemm_f64(a, b) + bias[None, :] + res, 0.0)
+        da = torch.full((m, k + 8), float("nan"), device="cuda", dtype=tdt)
+        da[:, :k] = _dev(a, tdt)
+        ops = [(capi.OP_BIAS_ADD, _dev(bias)), (capi.OP_RESIDUAL_ADD, _dev(res, tdt)), (capi.OP_RELU,)]
+        for tag, db in (("K-contiguous", _dev(np.ascontiguousarray(b.T), tdt).t()), ("N-contiguous", _dev(b, tdt))):
+            out = torch.full((m + 1, n + 4), 7.0, device="cuda", dtype=tdt)
+            tracea_gpu.gemm_ex(da[:, :k], db, ops, out=out[:m, :n])
+            got = out.float().cpu().numpy()
+            assert_close_scaled(got[:m, :n], ref, tol_half(k, dtype), "%s %s" % (tag, (m, n, k)))
+            assert (got[m] == 7.0).all() and (got[:, n:] == 7.0).all(), "outside the output"

@@ -131,6 +131,12 @@ struct ContractionVariant {
 int contraction_variant_count();
 const ContractionVariant &contraction_variant(int i);
 
+// Half-precision GEMM of at most kGemmRowsMax rows (operands below 2 GiB, a_bytes / b_bytes
+// set); takes a batch.
+constexpr int kGemmRowsMax = 48;
+bool gemm_rows_pays(const ContractionArgs &args, bool b_ncontig, int cus);  // ahead of the tile kernels on this problem
+int launch_gemm_rows(const ContractionArgs &args, int dtype, bool b_ncontig, int cus, hipStream_t stream);
+
 // fp32 MFMA GEMM (row-major A [M,K], row-major B [K,N]).
 int launch_gemm_f32(const ContractionArgs &args, int tile, hipStream_t stream);  // tile: 128, 64 or 6432 (64x64 with K tiles of 32)
 // Any dtype/stride combination, no alignment requirement (VALU, slow).

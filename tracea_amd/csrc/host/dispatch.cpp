@@ -821,8 +821,18 @@ bool gemm_batch_in_one_launch(const View &a, const View &b, const View &c, const
   return true;
 }
 
+// The kernel for products of a few rows splits K over the waves of a workgroup, so the switches of the split along K
+// hold for it too; a forced variant or a tuning-cache record of the problem wins over it, as over every rule.
+bool rows_kernel_wanted(long long M, long long N, long long K, int dtype, bool b_ncontig) {
+  if (!g_split_k_enabled.load() || !g_split_k_one_launch.load() || forced_variant("gemm") >= 0) return false;
+  char key[160];
+  snprintf(key, sizeof(key), "gemm_%lld_%lld_%lld_%s", M, N, K, tuning_device_name());
+  return tuning_cache_lookup_variant(key, dtype, b_ncontig) < 0;
+}
+
 TraceaStatus run_gemm(const View &a, const View &b, const View &c, const EpilogueChain &chain,
                       hipStream_t stream, bool static_only = false, const GemmBatch &batch = GemmBatch()) {
+  static thread_local bool in_padded = false;  // this call multiplies padded copies of another call's operands
   const long long M = a.shape[0], K = a.shape[1], N = b.shape[1];
   t_last_contraction = -1;
   if (M == 0 || N == 0) return TRACEA_SUCCESS;
@@ -841,10 +851,24 @@ TraceaStatus run_gemm(const View &a, const View &b, const View &c, const Epilogu
       args.ldc = c.stride[0];
       args.out_dtype = c.dtype;
       args.epi = chain;
-      int vi;
+      // direct-to-LDS variants address operands with 32-bit byte offsets below 2 GiB
+      const long long a_extent = ((M - 1) * a.stride[0] + K) * 2;
+      const long long b_extent = b_kcontig ? ((N - 1) * b.stride[1] + K) * 2 : ((K - 1) * b.stride[0] + N) * 2;
+      const bool small = a_extent < (1ll << 31) && b_extent < (1ll << 31);
+      args.a_bytes = (unsigned)(small ? a_extent : 0);
+      args.b_bytes = (unsigned)(small ? b_extent : 0);
       if (batch.count > 1) {
         args.batch = batch.count;
         args.batch_a = batch.a; args.batch_b = batch.b; args.batch_rows = batch.c / c.stride[0];
+      }
+      if (M <= kGemmRowsMax && small && !in_padded && gemm_rows_pays(args, !b_kcontig, (int)device_limits().cus) &&
+          rows_kernel_wanted(M, N, K, a.dtype, !b_kcontig)) {
+        t_last_splits = 4;  // (the four waves of a workgroup)
+        t_last_split_launches = 1;
+        return hip_status("gemm launch", launch_gemm_rows(args, a.dtype, !b_kcontig, (int)device_limits().cus, stream));
+      }
+      int vi;
+      if (batch.count > 1) {
         vi = forced_variant("gemm");
         if (vi < 0) vi = select_contraction_variant((int)M, (int)N, (int)K, false, !b_kcontig, batch.count);
       } else {
@@ -853,14 +877,8 @@ TraceaStatus run_gemm(const View &a, const View &b, const View &c, const Epilogu
         vi = pick_contraction("gemm", key, (int)M, (int)N, (int)K, false, a.dtype, !b_kcontig);
       }
       if (vi < 0) return fail(TRACEA_UNKNOWN_ERROR, "gemm: no kernel variant available");
-      // direct-to-LDS variants address operands with 32-bit byte offsets below 2 GiB
-      const long long a_extent = ((M - 1) * a.stride[0] + K) * 2;
-      const long long b_extent = b_kcontig ? ((N - 1) * b.stride[1] + K) * 2 : ((K - 1) * b.stride[0] + N) * 2;
-      const bool small = a_extent < (1ll << 31) && b_extent < (1ll << 31);
       vi = resolve_variant(vi, false, !small, K % contraction_variant(vi).bk == 0, !b_kcontig);
       const ContractionVariant &v = contraction_variant(vi);
-      args.a_bytes = (unsigned)(small ? a_extent : 0);
-      args.b_bytes = (unsigned)(small ? b_extent : 0);
       fill_grid(&args, v);
       t_last_contraction = vi;
       return launch_maybe_split("gemm launch", v, args, chain, false, a.dtype, !b_kcontig, c.device, stream, static_only);
@@ -972,7 +990,6 @@ TraceaStatus run_gemm(const View &a, const View &b, const View &c, const Epilogu
   // the any-layout kernel on the vector ALU (fp32 1000 x 900 x 1030: 794 us there).  Half precision: both as
   // K-contiguous rows (a row-major B is transposed on the way); fp32: A by rows, B row-major.  Not for the entry
   // point that must not allocate, nor while the buffer cannot grow (a stream under capture).
-  static thread_local bool in_padded = false;
   const bool same_half = is_half(a.dtype) && b.dtype == a.dtype;
   const bool all_f32 = a.dtype == TRACEA_DTYPE_FLOAT32 && b.dtype == TRACEA_DTYPE_FLOAT32 && c.dtype == TRACEA_DTYPE_FLOAT32;
   if (!in_padded && !static_only && K > 0 && (same_half || all_f32) && c.stride[1] == 1 && M < (1ll << 31) && N < (1ll << 31) &&
