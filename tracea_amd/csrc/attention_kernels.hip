@@ -402,6 +402,8 @@ fa2_fwd_kernel(const AttentionArgs a) {
 // spent on the shift.  The maximum of a tile is taken of z: while it stays below FA_RESCALE_TAU the reference
 // stays; when it moves, the tile's z are lowered by the step and O and the row sum rescaled.  Costs 16
 // registers per query block (the -m block), which the paired members at head dimension 128 do not have.
+// (two query blocks per wave, and four waves on the rings of two key groups at head dimension 128, are alone on their CU)
+constexpr int fa2_pipe_waves_per_simd(int waves, int qb, int kg) { return qb > 1 || (kg > 1 && waves == 4) ? 1 : 2; }
 constexpr bool fa2_pipe_parks_queries(int d, int qb, int items, bool shift) { return items > 1 && shift && d == 128 && qb == 1; }
 //
 // PP: the two waves of a SIMD half an iteration apart.  Phase A of an iteration (exponentials of tile t under
@@ -420,8 +422,15 @@ constexpr bool fa2_pipe_parks_queries(int d, int qb, int items, bool shift) { re
 // columns, no tests anywhere.  Such a call used to copy Q, K and V into padded tensors, run the kernel for D on them and
 // copy the result back: B2 H16 S1000 D96 causal 4 copies of 11-15 us each around a kernel of 20 us, 70 us a
 // call, against 19 us.
-template <int DT, int D, bool EARLY_MAX, int WAVES, int NSTG, int QB, int ITEMS = 1, bool SHIFT = false, bool PP = false, int DU = 0>
-__global__ void __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(QB == 1 ? 2 : 1, QB == 1 ? 2 : 1)))
+//
+// KG: the waves of a workgroup in KG groups that share the keys of one query block: group g takes tiles g, g + KG, ... on
+// K/V rings of its own, and group 0 adds up the partial results (each with its own reference value) through LDS at
+// the end.  For launches that leave CUs idle, where the serial walk over the keys is the time (a SIMD
+// needs 0.6 us per tile and wave, as many waves as it has): replayed graphs, H12 S1024 D64 causal 13.3 -> 10.1 us with 64
+// queries and four groups, H8 S2048 D64 causal 21.9 -> 13.6, H12 S1024 D128 causal 18.4 -> 15.2 with two groups.
+template <int DT, int D, bool EARLY_MAX, int WAVES, int NSTG, int QB, int ITEMS = 1, bool SHIFT = false, bool PP = false, int DU = 0, int KG = 1>
+__global__ void __launch_bounds__(WAVES * 64)
+__attribute__((amdgpu_waves_per_eu(fa2_pipe_waves_per_simd(WAVES, QB, KG), fa2_pipe_waves_per_simd(WAVES, QB, KG))))
 fa2_fwd_pipe_kernel(const AttentionArgs a) {
   constexpr bool PART = DU > 0;
   constexpr int DC = PART ? DU : D;  // columns the products run over
@@ -432,18 +441,20 @@ fa2_fwd_pipe_kernel(const AttentionArgs a) {
   constexpr bool PARK = fa2_pipe_parks_queries(D, QB, ITEMS, SHIFT);
   static_assert(QB == 1 || (QB == 2 && EARLY_MAX), "two query blocks per wave exist in the two-phase form only");
   static_assert(ITEMS == 1 || (ITEMS == 2 && EARLY_MAX), "pairs of query blocks exist in the two-phase form only");
+  static_assert(KG == 1 || (WAVES % KG == 0 && EARLY_MAX && SHIFT && NSTG == 2 && QB == 1 && ITEMS == 1 && !PP), "groups over the keys exist in the default form only");
+  constexpr int QW = WAVES / KG;  // waves per query block
   constexpr int WQ = 32 * QB;  // queries per wave
-  constexpr int BQ = WQ * WAVES;
+  constexpr int BQ = WQ * QW;
   constexpr int ROW_BYTES = D * 2;
   constexpr int CH = D / 8;
   constexpr int TILE_BYTES = FA_BKV * ROW_BYTES;
   constexpr int KS = DC / 16;
   constexpr int DB = DC / 32;
   constexpr int RPI = 64 / CH;                 // tile rows per wave-wide load instruction
-  constexpr int NI = FA_BKV / (RPI * WAVES); // load instructions per wave per tensor per tile
+  constexpr int NI = FA_BKV / (RPI * QW); // load instructions per wave per tensor per tile
   constexpr int RP = 256 / ROW_BYTES > 0 ? 256 / ROW_BYTES : 1;
   constexpr int WIN = ROW_BYTES / 64;
-  static_assert(D % 32 == 0 && FA_BKV % (RPI * WAVES) == 0, "unsupported head dim");
+  static_assert(D % 32 == 0 && FA_BKV % (RPI * QW) == 0, "unsupported head dim");
 
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   static_assert(NSTG == 2 || NSTG == 3 || NSTG == 4, "ring depth");
@@ -452,11 +463,13 @@ fa2_fwd_pipe_kernel(const AttentionArgs a) {
   // K(t+3), K(t+4), V(t+2), V(t+3): half the barriers and waits per key, and a request has two tiles to land.
   constexpr bool PAIR_SYNC = NSTG == 4;
   static_assert(!PAIR_SYNC || (EARLY_MAX && ITEMS == 1 && !PP), "the two-tile barrier exists for one query block per workgroup");
-  unsigned char *const sKbase = smem;                      // NSTG stages
-  unsigned char *const sVbase = smem + NSTG * TILE_BYTES;  // NSTG stages
-
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, wave_wg = tid >> 6;
+  const int kg = KG == 1 ? 0 : __builtin_amdgcn_readfirstlane(wave_wg / QW);  // this wave's group over the keys
+  const int wave = KG == 1 ? wave_wg : wave_wg - kg * QW;                     // its place in the group
   const int wave_u = __builtin_amdgcn_readfirstlane(wave);
+  unsigned char *const sKbase = smem + kg * (2 * NSTG * TILE_BYTES);  // NSTG stages
+  unsigned char *const sVbase = sKbase + NSTG * TILE_BYTES;           // NSTG stages
+
   const int lrow = lane & 31, g = lane >> 5;
   const int grp = wave_u >> 2;  // (PP) 0: waves 0-3, 1: waves 4-7, one phase behind
 
@@ -549,13 +562,13 @@ fa2_fwd_pipe_kernel(const AttentionArgs a) {
       (void *)Kg, 0, (int)(((long long)(S - 1) * a.k_ss + d_cols) * 2), 0x00020000);
   __amdgpu_buffer_rsrc_t rsrc_v = __builtin_amdgcn_make_buffer_rsrc(
       (void *)Vg, 0, (int)(((long long)(S - 1) * a.v_ss + d_cols) * 2), 0x00020000);
-  // Load instruction i of this wave covers tile rows (i*WAVES + wave)*RPI + lane/CH; the lane's
+  // Load instruction i of this wave covers tile rows (i*QW + wave)*RPI + lane/CH; the lane's
   // LDS slot is 16-byte column lane%CH of that row, so it fetches the global column that the
   // swizzle of the tensor maps there.
   unsigned k_voff[NI], v_voff[NI];
 #pragma unroll
   for (int i = 0; i < NI; ++i) {
-    const int row = (i * WAVES + wave) * RPI + lane / CH;
+    const int row = (i * QW + wave) * RPI + lane / CH;
     const int p = lane % CH;
     k_voff[i] = (unsigned)(row * (int)a.k_ss * 2 + ((p ^ ((row / RP) & (CH - 1))) << 4));
     v_voff[i] = (unsigned)(row * (int)a.v_ss * 2 + ((p ^ (((row / RP) % WIN) << 2)) << 4));
@@ -566,22 +579,23 @@ fa2_fwd_pipe_kernel(const AttentionArgs a) {
     }
   }
   auto load_k = [&](int t, unsigned char *dst) __attribute__((always_inline)) {
-    const unsigned adv = (unsigned)t * (unsigned)(FA_BKV * 2) * (unsigned)a.k_ss;
+    const unsigned adv = (unsigned)(t * KG + kg) * (unsigned)(FA_BKV * 2) * (unsigned)a.k_ss;
 #pragma unroll
     for (int i = 0; i < NI; ++i)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(
-          rsrc_k, (__attribute__((address_space(3))) void *)(dst + (i * WAVES + wave_u) * RPI * ROW_BYTES),
+          rsrc_k, (__attribute__((address_space(3))) void *)(dst + (i * QW + wave_u) * RPI * ROW_BYTES),
           16, (int)(k_voff[i] + adv), 0, 0, 0);
   };
   auto load_v = [&](int t, unsigned char *dst) __attribute__((always_inline)) {
-    const unsigned adv = (unsigned)t * (unsigned)(FA_BKV * 2) * (unsigned)a.v_ss;
+    const unsigned adv = (unsigned)(t * KG + kg) * (unsigned)(FA_BKV * 2) * (unsigned)a.v_ss;
 #pragma unroll
     for (int i = 0; i < NI; ++i)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(
-          rsrc_v, (__attribute__((address_space(3))) void *)(dst + (i * WAVES + wave_u) * RPI * ROW_BYTES),
+          rsrc_v, (__attribute__((address_space(3))) void *)(dst + (i * QW + wave_u) * RPI * ROW_BYTES),
           16, (int)(v_voff[i] + adv), 0, 0, 0);
   };
 
+  int tiles_all = 0;  // of the query block
   auto tiles_of = [&](int first_query) __attribute__((always_inline)) -> int {
     int n = (S + FA_BKV - 1) / FA_BKV;
     if (a.causal) {
@@ -589,7 +603,8 @@ fa2_fwd_pipe_kernel(const AttentionArgs a) {
       const int need = last_q / FA_BKV + 1;
       n = need < n ? need : n;
     }
-    return n;
+    tiles_all = n;
+    return (n + KG - 1) / KG;  // (tiles of a group: the same count for all, the last ones may lie past the end)
   };
   int ntiles = tiles_of(q0);
   // tb: K/V tiles of the items before the current one.  Tile t of an item lives in ring stage (tb + t) % NSTG,
@@ -627,9 +642,25 @@ fa2_fwd_pipe_kernel(const AttentionArgs a) {
   // iteration before (NSTG = 3), none (NSTG = 2)
   constexpr int FLIGHT = PAIR_SYNC ? 0 : (NSTG - 2) * 2 * NI;
   constexpr int WAIT_TILES = (FLIGHT & 15) | (7 << 4) | (15 << 8) | ((FLIGHT >> 4) << 14);
-  load_k(0, sKbase);
-  load_v(0, sVbase);
-  load_k(1, sKbase + TILE_BYTES);
+  // (KG > 1: tiles of this group that exist, and the queries in front of the tiles: a wave walks few tiles and the start
+  // is a good part of its time, so it waits for its queries and K(0) alone and requests nothing it does not need)
+  const int group_tiles = KG == 1 ? 0 : (tiles_all - kg + KG - 1) / KG;
+  u32x4 q_raw[KG > 1 ? KS : 1];
+  if constexpr (KG > 1) {
+    const int qr = q_wave0 + lrow < S ? q_wave0 + lrow : S - 1;
+    const unsigned short *qp = Qg + (long long)qr * a.q_ss;
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) q_raw[ks] = *(const u32x4 *)(qp + (!PART || ks * 16 + g * 8 < d_cols ? ks * 16 + g * 8 : 0));
+    __builtin_amdgcn_sched_barrier(0);
+    if (group_tiles > 0) {
+      load_k(0, sKbase);
+      load_v(0, sVbase);
+    }
+  } else {
+    load_k(0, sKbase);
+    load_v(0, sVbase);
+    load_k(1, sKbase + TILE_BYTES);
+  }
   if constexpr (PAIR_SYNC) {
     load_k(2, sKbase + 2 * TILE_BYTES);
     load_v(1, sVbase + TILE_BYTES);
@@ -639,7 +670,13 @@ fa2_fwd_pipe_kernel(const AttentionArgs a) {
     load_k(2, sKbase + 2 * TILE_BYTES);
   }
   __builtin_amdgcn_sched_barrier(0);
-  load_q(q0, qf, std::integral_constant<int, KS>{});
+  if constexpr (KG > 1) {
+    const u32x4 zero4 = {0u, 0u, 0u, 0u};
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) qf[0][ks] = prescale(!PART || ks * 16 + g * 8 < d_cols ? q_raw[ks] : zero4);
+  } else {
+    load_q(q0, qf, std::integral_constant<int, KS>{});
+  }
   // The second item's queries travel with the first tiles.  PARK: the upper half of their k-steps waits in LDS
   // behind the rings (fetched there directly, each lane's fragment in a slot of its own) instead of in
   // registers: the 16 registers that the -m block of SHIFT needs at head dimension 128.
@@ -706,7 +743,7 @@ fa2_fwd_pipe_kernel(const AttentionArgs a) {
   };
   auto take_max = [&](int tile, auto edge_tag, f32x16 (&s)[QB][2]) -> bool {
     constexpr bool EDGE = decltype(edge_tag)::value;
-    const int kv0 = tile * FA_BKV;
+    const int kv0 = (tile * KG + kg) * FA_BKV;
     bool moved = false;
     float mxs[QB];
 #pragma unroll
@@ -841,7 +878,7 @@ fa2_fwd_pipe_kernel(const AttentionArgs a) {
 #pragma unroll
     for (int i = 0; i < NI; ++i)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(
-          rsrc, (__attribute__((address_space(3))) void *)(dst + (i * WAVES + wave_u) * RPI * ROW_BYTES), 16,
+          rsrc, (__attribute__((address_space(3))) void *)(dst + (i * QW + wave_u) * RPI * ROW_BYTES), 16,
           (int)(voff[i] + adv), 0, 0, 0);
   };
   auto head_of = [&](int tt) __attribute__((always_inline)) {
@@ -868,8 +905,8 @@ fa2_fwd_pipe_kernel(const AttentionArgs a) {
       asm volatile("" ::: "memory");
       __builtin_amdgcn_s_barrier();
       asm volatile("" ::: "memory");
-      load_k(ahead(tt + NSTG), sKbase + ((tb + tt) % NSTG) * TILE_BYTES);
-      load_v(ahead(tt + NSTG - 1), sVbase + ((tb + tt + NSTG - 1) % NSTG) * TILE_BYTES);
+      if (KG == 1 || tt + NSTG < group_tiles) load_k(ahead(tt + NSTG), sKbase + ((tb + tt) % NSTG) * TILE_BYTES);
+      if (KG == 1 || tt + NSTG - 1 < group_tiles) load_v(ahead(tt + NSTG - 1), sVbase + ((tb + tt + NSTG - 1) % NSTG) * TILE_BYTES);
     }
   };
   auto mid_of = [&](int tt) __attribute__((always_inline)) {
@@ -898,15 +935,15 @@ fa2_fwd_pipe_kernel(const AttentionArgs a) {
   // request r of iteration tt: r < NI a piece of K(tt+NSTG), else a piece of V(tt+NSTG-1)
   auto request_nth = [&](int tt, int r) __attribute__((always_inline)) {
     if (r < NI) {
-      const unsigned adv = (unsigned)ahead(tt + NSTG) * (unsigned)(FA_BKV * 2) * (unsigned)a.k_ss;
+      const unsigned adv = (unsigned)(ahead(tt + NSTG) * KG + kg) * (unsigned)(FA_BKV * 2) * (unsigned)a.k_ss;
       unsigned char *dst = sKbase + ((tb + tt) % NSTG) * TILE_BYTES;
       __builtin_amdgcn_raw_ptr_buffer_load_lds(
-          rsrc_k, (__attribute__((address_space(3))) void *)(dst + (r * WAVES + wave_u) * RPI * ROW_BYTES), 16, (int)(k_voff[r] + adv), 0, 0, 0);
+          rsrc_k, (__attribute__((address_space(3))) void *)(dst + (r * QW + wave_u) * RPI * ROW_BYTES), 16, (int)(k_voff[r] + adv), 0, 0, 0);
     } else {
-      const unsigned adv = (unsigned)ahead(tt + NSTG - 1) * (unsigned)(FA_BKV * 2) * (unsigned)a.v_ss;
+      const unsigned adv = (unsigned)(ahead(tt + NSTG - 1) * KG + kg) * (unsigned)(FA_BKV * 2) * (unsigned)a.v_ss;
       unsigned char *dst = sVbase + ((tb + tt + NSTG - 1) % NSTG) * TILE_BYTES;
       __builtin_amdgcn_raw_ptr_buffer_load_lds(
-          rsrc_v, (__attribute__((address_space(3))) void *)(dst + ((r - NI) * WAVES + wave_u) * RPI * ROW_BYTES), 16,
+          rsrc_v, (__attribute__((address_space(3))) void *)(dst + ((r - NI) * QW + wave_u) * RPI * ROW_BYTES), 16,
           (int)(v_voff[r - NI] + adv), 0, 0, 0);
     }
   };
@@ -1018,7 +1055,7 @@ fa2_fwd_pipe_kernel(const AttentionArgs a) {
       // ---- phase B: O^T += V^T(t) P^T(t)  with  the running maximum of tile t+1 ----
       // chunk kk: the DB*QB MFMAs of key block kk (operand reads one fragment ahead) and
       // the maximum over 8 of the 32 scores of S(t+1) of each query block
-      const int kv0n = (t + 1) * FA_BKV;
+      const int kv0n = ((t + 1) * KG + kg) * FA_BKV;
       float mx[QB];
 #pragma unroll
       for (int qi = 0; qi < QB; ++qi) mx[qi] = -INFINITY;
@@ -1141,18 +1178,33 @@ fa2_fwd_pipe_kernel(const AttentionArgs a) {
     }
   }
   // (a later item finds its first tiles requested by the item before it, and published by that item's last barrier)
-  __builtin_amdgcn_s_waitcnt(WAIT_TILES);
-  __syncthreads();
+  if constexpr (KG > 1) {
+    __builtin_amdgcn_s_waitcnt(0x0f70 | (NI & 15));  // K(0); V(0) may be on its way
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    if (group_tiles > 1) load_k(1, sKbase + TILE_BYTES);
+  } else {
+    __builtin_amdgcn_s_waitcnt(WAIT_TILES);
+    __syncthreads();
+  }
   scores(sKbase + (tb % NSTG) * TILE_BYTES, s_cur);
 
   // Interior tiles first, then the edge tiles (they are the last ones: the tail of
   // the sequence and, under a causal mask, the tiles that reach the diagonal of
   // this wave's queries), each in a loop of its own with a single body.
   int first_edge = ntiles;
-  if (ntiles * FA_BKV > S) first_edge = ntiles - 1;
-  if (a.causal) {
-    const int fe = (q_wave0 + 1) / FA_BKV;  // first tile with kv0 + 63 > q_wave0
-    first_edge = fe < first_edge ? fe : first_edge;
+  if constexpr (KG == 1) {
+    if (ntiles * FA_BKV > S) first_edge = ntiles - 1;
+    if (a.causal) {
+      const int fe = (q_wave0 + 1) / FA_BKV;  // first tile with kv0 + 63 > q_wave0
+      first_edge = fe < first_edge ? fe : first_edge;
+    }
+  } else {
+    int fe = S / FA_BKV;  // the first tile with a key past the end, then the group's first tile from there on
+    if (a.causal && (q_wave0 + 1) / FA_BKV < fe) fe = (q_wave0 + 1) / FA_BKV;
+    first_edge = fe > kg ? (fe - kg + KG - 1) / KG : 0;
+    first_edge = first_edge < ntiles ? first_edge : ntiles;
   }
   first_edge = __builtin_amdgcn_readfirstlane(first_edge);
   if constexpr (EARLY_MAX) {
@@ -1208,14 +1260,18 @@ fa2_fwd_pipe_kernel(const AttentionArgs a) {
     // product: full iterations while tile t+1 has a key for the wave, the softmax and P.V of the last such
     // tile, and then only the workgroup's barriers and tile requests.  (Per block of 128 queries under a
     // causal mask that is one and a half iterations of two of the four waves and half an iteration of the others.)
-    const int last_live = wave_last_key / FA_BKV;
+    // (a group's first tile may already lie past every key of the wave: last_live is then -1)
+    const int last_live = KG == 1 ? wave_last_key / FA_BKV : (wave_last_key / FA_BKV - kg + KG) / KG - 1;
     for (; t < last_live; ++t) {
       head_wait(t);
       iteration(t, std::true_type{});
     }
-    head_of(t);
-    last_live_iteration(t);
-    for (++t; t < ntiles; ++t) {
+    if (KG == 1 || last_live >= 0) {
+      head_of(t);
+      last_live_iteration(t);
+      ++t;
+    }
+    for (; t < ntiles; ++t) {
       head_of(t);
       mid_of(t);
     }
@@ -1233,6 +1289,54 @@ fa2_fwd_pipe_kernel(const AttentionArgs a) {
       load_k(ahead(t + NSTG), sKbase + ((tb + t) % NSTG) * TILE_BYTES);
       load_v(ahead(t + NSTG - 1), sVbase + ((tb + t + NSTG - 1) % NSTG) * TILE_BYTES);
       iteration(t, std::true_type{});
+    }
+  }
+  if constexpr (KG > 1) {
+    // Each wave's O, its share of the row sum and its reference value, 16 bytes per lane at a time (1 KB a row); a query
+    // none of whose keys a group has seen carries no reference there.
+    constexpr int ROWS = DB * 4 + 1;
+    __builtin_amdgcn_s_waitcnt(0x0f70);  // (look-ahead requests past the end still write the rings)
+    __syncthreads();
+    f32x4 *const part = (f32x4 *)smem + lane;
+    if (kg > 0) {
+      f32x4 *const dst = part + ((kg - 1) * QW + wave_u) * (ROWS * 64);
+      const f32x4 sums = {l_run[0], kg * FA_BKV <= last_key[0] + g * 4 ? m_run[0] : -INFINITY, 0.0f, 0.0f};
+      dst[DB * 4 * 64] = sums;
+#pragma unroll
+      for (int d = 0; d < DB; ++d)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) dst[(d * 4 + e) * 64] = f32x4{o[0][d][e * 4], o[0][d][e * 4 + 1], o[0][d][e * 4 + 2], o[0][d][e * 4 + 3]};
+    }
+    __syncthreads();
+    if (kg > 0) return;
+    float l_g[KG], m_g[KG], m_all = m_run[0];
+    l_g[0] = l_run[0];
+    m_g[0] = m_run[0];
+#pragma unroll
+    for (int z = 1; z < KG; ++z) {
+      const f32x4 sums = part[((z - 1) * QW + wave_u) * (ROWS * 64) + DB * 4 * 64];
+      l_g[z] = sums[0];
+      m_g[z] = sums[1];
+      m_all = fmaxf(m_all, sums[1]);
+    }
+    l_run[0] = 0.0f;
+#pragma unroll
+    for (int z = 0; z < KG; ++z) {
+      const float f = __builtin_amdgcn_exp2f(m_g[z] - m_all);
+      l_run[0] += l_g[z] * f;
+#pragma unroll
+      for (int d = 0; d < DB; ++d)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          if (z == 0) {
+#pragma unroll
+            for (int x = 0; x < 4; ++x) o[0][d][e * 4 + x] *= f;
+          } else {
+            const f32x4 v = part[((z - 1) * QW + wave_u) * (ROWS * 64) + (d * 4 + e) * 64];
+#pragma unroll
+            for (int x = 0; x < 4; ++x) o[0][d][e * 4 + x] += v[x] * f;
+          }
+        }
     }
   }
   {
@@ -1277,18 +1381,19 @@ fa2_fwd_pipe_kernel(const AttentionArgs a) {
   __builtin_amdgcn_s_waitcnt(0x0f70);
 }
 
-template <int D, bool EARLY_MAX, int WAVES, int NSTG, int QB = 1, int ITEMS = 1, bool SHIFT = false, bool PP = false, int DU = 0>
+template <int D, bool EARLY_MAX, int WAVES, int NSTG, int QB = 1, int ITEMS = 1, bool SHIFT = false, bool PP = false, int DU = 0, int KG = 1>
 static int launch_fa2_pipe(const AttentionArgs &a, int dtype, hipStream_t stream) {
   if (PP && a.causal) return (int)hipErrorInvalidValue;  // (its feasibility test keeps such a call away)
   // the K and V rings (O leaves from registers), and where they are parked half of the next block's queries
-  constexpr size_t lds = 2 * (size_t)NSTG * FA_BKV * D * 2 +
+  constexpr size_t lds = KG * 2 * (size_t)NSTG * FA_BKV * D * 2 +
                          (fa2_pipe_parks_queries(D, QB, ITEMS, SHIFT) ? (size_t)WAVES * (D / 32) * 1024 : 0);
-  const int nqb = (a.S + 32 * QB * WAVES - 1) / (32 * QB * WAVES);
+  constexpr int bq = 32 * QB * (WAVES / KG);
+  const int nqb = (a.S + bq - 1) / bq;
   if (nqb % ITEMS != 0) return (int)hipErrorInvalidValue;  // (feasible_pairs keeps such a call away)
   const dim3 grid((unsigned)(nqb / ITEMS * a.B * a.H)), block(WAVES * 64);
 #define TRACEA_FA_LAUNCH(DTV)                                                                  \
   do {                                                                                         \
-    auto kfn = fa2_fwd_pipe_kernel<DTV, D, EARLY_MAX, WAVES, NSTG, QB, ITEMS, SHIFT, PP, DU>;  \
+    auto kfn = fa2_fwd_pipe_kernel<DTV, D, EARLY_MAX, WAVES, NSTG, QB, ITEMS, SHIFT, PP, DU, KG>; \
     static bool attr_done = false;                                                             \
     if (!attr_done) {                                                                          \
       hipError_t e = hipFuncSetAttribute((const void *)kfn,                                    \
@@ -1310,8 +1415,8 @@ namespace tracea_amd {
 
 // The buffer loads address a (batch, head) slice with 32-bit byte offsets.
 static bool slice_fits(const AttentionArgs &a) {
-  const long long k_ext = ((long long)(a.S - 1 + 4 * FA_BKV) * a.k_ss + a.D) * 2;  // (tiles up to 3 past the end are requested)
-  const long long v_ext = ((long long)(a.S - 1 + 4 * FA_BKV) * a.v_ss + a.D) * 2;
+  const long long k_ext = ((long long)(a.S - 1 + 16 * FA_BKV) * a.k_ss + a.D) * 2;  // (tiles past the end are requested: up to 3, 12 with four groups)
+  const long long v_ext = ((long long)(a.S - 1 + 16 * FA_BKV) * a.v_ss + a.D) * 2;
   return k_ext < (1ll << 31) && v_ext < (1ll << 31);
 }
 // (the running maximum is taken over raw scores, which needs a positive scale)
@@ -1395,10 +1500,18 @@ static const AttentionVariant kAttentionVariants[] = {
     {"fa2_q128_kv64_d128_u16", FA_BQ, FA_BKV, FA_WAVES, 2, &launch_fa2<128, false>, &feasible_d128, 32, 1},
     {"fa2_q128_kv64_d64_tr", FA_BQ, FA_BKV, FA_WAVES, 2, &launch_fa2<64, true>, &feasible_d64, 32, 1},
     {"fa2_q128_kv64_d64_u16", FA_BQ, FA_BKV, FA_WAVES, 2, &launch_fa2<64, false>, &feasible_d64, 32, 1},
+    // the keys of a query block shared by groups of waves
+    {"fa2_q64_kv64_d64_k4", 64, FA_BKV, 8, 2, &launch_fa2_pipe<64, true, 8, 2, 1, 1, true, false, 0, 4>, &feasible_pipe_d64, 32, 1, 0, 4},
+    {"fa2_q128_kv64_d64_k2", 128, FA_BKV, 8, 2, &launch_fa2_pipe<64, true, 8, 2, 1, 1, true, false, 0, 2>, &feasible_pipe_d64, 32, 1, 0, 2},
+    {"fa2_q64_kv64_d128_k2", 64, FA_BKV, 4, 2, &launch_fa2_pipe<128, true, 4, 2, 1, 1, true, false, 0, 2>, &feasible_pipe_d128, 32, 1, 0, 2},
+    {"fa2_q128_kv64_d128_k2", 128, FA_BKV, 8, 2, &launch_fa2_pipe<128, true, 8, 2, 1, 1, true, false, 0, 2>, &feasible_pipe_d128, 32, 1, 0, 2},
     // head dimensions off 64 and 128
     {"fa2_q128_kv64_part64", 128, FA_BKV, 4, 2, &launch_fa2_pipe<64, true, 4, 2, 1, 1, true, false, 64>, &feasible_part<0, 64>, 32, 1},
     {"fa2_q128_kv64_part96", 128, FA_BKV, 4, 2, &launch_fa2_pipe<128, true, 4, 2, 1, 1, true, false, 96>, &feasible_part<64, 96>, 32, 1},
     {"fa2_q128_kv64_part128", 128, FA_BKV, 4, 2, &launch_fa2_pipe<128, true, 4, 2, 1, 1, true, false, 128>, &feasible_part<96, 128>, 32, 1},
+    {"fa2_q64_kv64_part64_k4", 64, FA_BKV, 8, 2, &launch_fa2_pipe<64, true, 8, 2, 1, 1, true, false, 64, 4>, &feasible_part<0, 64>, 32, 1, 0, 4},
+    {"fa2_q64_kv64_part96_k2", 64, FA_BKV, 4, 2, &launch_fa2_pipe<128, true, 4, 2, 1, 1, true, false, 96, 2>, &feasible_part<64, 96>, 32, 1, 0, 2},
+    {"fa2_q64_kv64_part128_k2", 64, FA_BKV, 4, 2, &launch_fa2_pipe<128, true, 4, 2, 1, 1, true, false, 128, 2>, &feasible_part<96, 128>, 32, 1, 0, 2},
 };
 
 int attention_variant_count() { return (int)(sizeof(kAttentionVariants) / sizeof(kAttentionVariants[0])); }

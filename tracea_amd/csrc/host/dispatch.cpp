@@ -2540,7 +2540,7 @@ TraceaStatus dispatch_attention(const TraceaTensorView &tq, const TraceaTensorVi
   const View *views[4] = {&q, &k, &v, &o};
   // (any other multiple of 8 runs in place too, on the members that stop at the tensors' last column: those take a
   // positive scale and K/V slices below 2 GiB, tiles requested past the end included)
-  const long long reach = S + 4 * 64;
+  const long long reach = S + 16 * 64;
   bool in_place = D == 64 || D == 128 ||
                   (D % 8 == 0 && scale > 0.0f && (reach * k.stride[2] + D) * 2 < (1ll << 31) && (reach * v.stride[2] + D) * 2 < (1ll << 31));
   for (const View *t : views)
@@ -2601,14 +2601,23 @@ TraceaStatus dispatch_attention(const TraceaTensorView &tq, const TraceaTensorVi
   int vi = forced_variant("attention");
   if (vi >= 0 && !attention_variant(vi).feasible(a)) vi = -1;
   if (vi < 0) vi = tuning_cache_lookup_attention(a);
-  auto member = [&](int block_q, int waves, int items) {
+  auto member = [&](int block_q, int waves, int items, int key_groups = 0) {
     for (int i = 0; i < attention_variant_count(); ++i) {
       const AttentionVariant &v = attention_variant(i);
-      if (v.block_q == block_q && v.waves == waves && v.stages == 2 && v.mfma == 32 && v.items == items && v.offset_groups == 0 && v.feasible(a)) return i;
+      if (v.block_q == block_q && v.waves == waves && v.stages == 2 && v.mfma == 32 && v.items == items && v.offset_groups == 0 && v.key_groups == key_groups &&
+          v.feasible(a))
+        return i;
     }
     return -1;
   };
   const long long cus = device_limits().cus, bh = (long long)(B * H);
+  // Launches that leave CUs idle: the keys of a block shared by groups of waves.  Replayed graphs, default / groups, us:
+  // 64 queries at head dimension up to 64, four groups, H12 S1024 13.3 / 10.1, H8 S2048 21.9 / 13.6, H12 S512 8.4 / 7.7, but
+  // S300 6.8 / 6.9 and S256 6.0 / 6.3; 64 queries at up to 128, two groups, H12 S1024 18.4 / 15.2, S512 11.4 / 10.4, S256
+  // 8.2 / 7.9 (under a causal mask S289 8.3 / 8.9).  Where those blocks of 64 would come in a second round, blocks of 128 on two groups: H8 S4096 D64 43.9 / 39.3
+  // (of 64: 46.3).
+  if (vi < 0 && bh * ((S + 63) / 64) <= cus && S > (D > 64 && !a.causal ? 192 : 384)) vi = D <= 64 ? member(64, 8, 1, 4) : member(64, 4, 1, 2);
+  if (vi < 0 && bh * ((S + 127) / 128) < cus && S > 512) vi = member(128, 8, 1, 2);
   // Two query blocks per workgroup where the pairs alone fill the device: the second block starts on tiles and
   // queries already requested, and under a causal mask a heavy block is paired with a light one.  Sweep over
   // B*H in {8, 32, 128, 512} and S in {512 ... 8192}, replayed graphs: with at least one pair per CU the paired
