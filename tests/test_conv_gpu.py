@@ -625,3 +625,43 @@ def test_random_geometry_on_the_patch_in_lds_members(tracea_gpu, seed):
             assert_close_scaled(y.float().cpu().numpy(), ref, tol_half(fr * fs * c, "f16" if tdt == torch.float16 else "bf16"),
                                 "%s %s" % (member, (n, h, w, c, k, fr, fs, stride, pad, dil, epi)))
     assert len(ran) >= 5 and sum(ran.values()) >= 40, ran
+
+
+PRIVATE_MEMBERS = ["c16x16_c64_w8_w16_ksplit", "c16x32_c64_w8_w16_ksplit", "c32x32_c64_w8_w16_ksplit", "c32x32_c64_w4_w16_ksplit"]
+
+
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+@pytest.mark.parametrize("member", PRIVATE_MEMBERS)
+def test_few_pixels_on_private_rings(tracea_gpu, dtype, member):
+    """The kernel for few output pixels (K dealt to the waves in 64-channel pieces, private rings), forced: one piece of K
+    for eight waves, a piece count off the wave count, tiles cut by the last pixel and the last filter (40, 24, 8),
+    stride, dilation, asymmetric padding, 1x1 and 5x5 filters; bias + ReLU, and BatchNorm + residual + SiLU (table,
+    prefetched residual and the general operators), against torch in double."""
+    from tracea_amd import capi
+    tdt, rnd = (torch.float16, round_f16) if dtype == "f16" else (torch.bfloat16, round_bf16)
+    capi.force_variant("conv2d", member)
+    try:
+        for (n, h, w, c, k, fs, stride, pad, dil) in [(1, 7, 7, 512, 64, 3, 1, 1, 1), (1, 1, 1, 64, 8, 1, 1, 0, 1), (2, 9, 5, 64, 40, 3, 2, 1, 1),
+                                                      (1, 13, 17, 128, 24, 3, 1, 2, 2), (3, 8, 8, 192, 72, 1, 2, 0, 1),
+                                                      (1, 6, 20, 64, 32, 5, 1, (1, 3), 1)]:
+            kg = fs * fs * c
+            rng = np.random.default_rng(h * 31 + w + k)
+            x = rnd(rng.standard_normal((n, h, w, c)))
+            wk = rnd(rng.standard_normal((k, fs, fs, c)) * np.sqrt(2.0 / kg))
+            bias = (rng.standard_normal(k) * 0.1).astype(np.float32)
+            acc = torch.nn.functional.conv2d(torch.from_numpy(x).permute(0, 3, 1, 2).double(), torch.from_numpy(wk).permute(0, 3, 1, 2).double(),
+                                             stride=stride, padding=pad, dilation=dil).permute(0, 2, 3, 1).numpy()
+            y = tracea_gpu.conv2d(_dev(x, tdt), _dev(wk, tdt), bias=_dev(bias), stride=stride, padding=pad, dilation=dil, epilogue="bias+relu")
+            assert capi.last_variant("conv2d") == member, "%s refused %s" % (member, (n, h, w, c))
+            assert_close_scaled(y.float().cpu().numpy(), np.maximum(acc + bias, 0.0), tol_half(kg, dtype), "%s %s" % (member, (n, h, w, c)))
+            bn = [rng.uniform(0.5, 1.5, k).astype(np.float32), rng.standard_normal(k).astype(np.float32),
+                  rng.standard_normal(k).astype(np.float32), rng.uniform(0.5, 1.5, k).astype(np.float32)]
+            res = rnd(rng.standard_normal(acc.shape))
+            want = (acc - bn[2]) / np.sqrt(bn[3] + 1e-5) * bn[0] + bn[1] + res
+            want = want / (1.0 + np.exp(-want))
+            y = tracea_gpu.conv2d_ex(_dev(x, tdt), _dev(wk, tdt), [(capi.OP_BATCHNORM, *[_dev(v) for v in bn], 1e-5),
+                                                                  (capi.OP_RESIDUAL_ADD, _dev(res, tdt)), (capi.OP_SILU,)],
+                                     stride=stride, padding=pad, dilation=dil)
+            assert_close_scaled(y.float().cpu().numpy(), want, tol_half(kg, dtype), "%s chain %s" % (member, (n, h, w, c)))
+    finally:
+        capi.force_variant("conv2d", -1)

@@ -7,6 +7,7 @@
 #include "conv_wave16_kernel.hpp"
 #include "conv_ksplit16_kernel.hpp"
 #include "conv_thin8_kernel.hpp"
+#include "conv_private16_kernel.hpp"
 
 #define TRACEA_CAT2(a, b) a##b
 #define TRACEA_CAT(a, b) TRACEA_CAT2(a, b)
@@ -36,6 +37,9 @@ const ContractionVariant &TRACEA_CAT(contraction_variant_, V_NAME)() {
 #elif V_DIRECT == 10
       (size_t)CT_TABLE_BYTES,  // the patch, sized by the problem, comes on top
       &launch_conv_thin8<V_STAGES>, 16};
+#elif V_DIRECT == 11
+      (size_t)V_WM * V_STAGES * (V_BM + V_BN) * 128 + (size_t)TRACEA_MAX_EPILOGUE_OPS * 2 * V_BN * 4,
+      &launch_conv_private16<V_WM, V_BM, V_BN, V_STAGES>, 16};
 #elif V_DIRECT == 6
       (size_t)V_STAGES * (V_BM + V_BN) * V_BK * 2,
       &launch_contraction<V_BM, V_BN, V_BK, V_WM, V_WN, V_STAGES, 2, 16>, 16};  // pipeline 2 on 16x16x32 MFMAs

@@ -1883,7 +1883,25 @@ void fast_epilogue_form(const EpilogueChain &chain, int dtype, ContractionArgs *
   a->fe = fe;
 }
 
+// Plan of the kernel for few output pixels (pipeline 11): K-contiguous filters, C a multiple of 64 (a piece of K lies in
+// one tap), input and filters below 2 GiB.
+bool plan_conv_private16(const ConvGeometry &g, const ContractionVariant &v, bool w_ncontig, ContractionArgs *a) {
+  const TraceaConvParamsBlock &b = g.block;
+  if (v.pipeline != 11 || w_ncontig || b.c_in % 64 != 0) return false;
+  const long long x_bytes = (long long)b.batch * b.h_in * b.w_in * b.c_in * 2, w_bytes = (long long)g.n_gemm * g.k_gemm * 2;
+  if (x_bytes >= (1ll << 31) || w_bytes >= (1ll << 31)) return false;
+  a->grid_m = (g.m_gemm + v.bm - 1) / v.bm;
+  a->grid_n = (g.n_gemm + v.bn - 1) / v.bn;
+  if ((long long)a->grid_m * a->grid_n >= (1ll << 31)) return false;
+  magic_for_divisor((uint32_t)a->grid_n, (uint64_t)a->grid_m * a->grid_n, &a->gn_m, &a->gn_s);
+  a->group_m = 1;
+  a->a_bytes = (unsigned)x_bytes;
+  a->b_bytes = (unsigned)w_bytes;
+  return true;
+}
+
 bool plan_conv_resident(const ConvGeometry &g, const ContractionVariant &v, bool w_ncontig, ContractionArgs *a) {
+  if (v.pipeline == 11) return plan_conv_private16(g, v, w_ncontig, a);
   if (v.pipeline == 7 || v.pipeline == 8) return plan_conv_wave16(g, v, w_ncontig, a);
   if (v.pipeline == 9) return plan_conv_ksplit16(g, v, w_ncontig, a);
   if (v.pipeline == 10) return plan_conv_thin8(g, v, w_ncontig, a);
@@ -1917,10 +1935,32 @@ TraceaStatus run_conv(const ConvPlan &plan, const EpilogueChain &chain, hipStrea
   // at least 10 pixel blocks.  Measured in a replayed HIP graph against the best other variant: N32
   // 56x56x64->64 14.1 us / 16.7; N64 25.2 / 28.6; N32 64->128 24.5 / 28.8; N8 10.3 / 9.5 (not taken).
   bool resident_chosen = false;
-  // First choice: the kernels on 16x16x32 MFMAs with the patch in LDS and the filter slab resident or in a
+  const bool by_rule = forced_variant("conv2d") < 0 && tuning_cache_lookup_variant(key, plan.x.dtype, plan.w_ncontig) < 0;
+  // Launches of few output pixels: the smallest tile that still comes in one round of workgroups (32x32: on four waves up
+  // to 18 pieces of K, eight beyond), or 32x32 tiles in up to 400 workgroups on four waves from K = 1152 on.  Replayed
+  // graphs, best other kernel / this one, us: one image 56x56 64->64 3x3 7.6 / 5.0, 28x28 128->128 8.7 / 4.8, 14x14
+  // 256->256 6.7 / 4.8, 7x7 512->512 10.2 (two launches) / 7.0, 56x56 64->128 stride 2 7.5 / 4.5, 14x14 256->512 stride 2
+  // 8.5 / 4.9; four images 14x14 256->256 8.9 / 6.9, 28x28 128->128 (392 workgroups) 10.7 / 8.6, 7x7 512->512 12.0 / 8.4;
+  // sixteen images 7x7 512->512 (400) 16.4 / 15.6; but four images 56x56 64->64 (784) 9.4 / 11.8.
+  if (by_rule) {
+    const long long cus = device_limits().cus;
+    const ContractionVariant *best = nullptr;
+    long long best_tile = 0;
+    for (int i = 0; i < contraction_variant_count(); ++i) {
+      const ContractionVariant &cv = contraction_variant(i);
+      ContractionArgs probe = a;
+      if (cv.pipeline != 11 || !plan_conv_private16(g, cv, plan.w_ncontig, &probe)) continue;
+      const long long wgs = (long long)probe.grid_m * probe.grid_n, tile = (long long)cv.bm * cv.bn;
+      if (tile == 32 * 32 && (cv.waves_m == 4) != (wgs > cus || a.K <= 18 * 64)) continue;
+      if (wgs > cus && !(tile == 32 * 32 && wgs <= 400 && a.K >= 1152)) continue;
+      if (best == nullptr || tile < best_tile) { best = &cv; best_tile = tile; vi = i; }
+    }
+    resident_chosen = best != nullptr;
+  }
+  // Next: the kernels on 16x16x32 MFMAs with the patch in LDS and the filter slab resident or in a
   // ring (pipelines 7 to 10), where their plan fits, the launch fills most of the device and a workgroup's
   // tile is at least three quarters of the kernel's largest (smaller tiles leave its waves' blocks empty).
-  if (forced_variant("conv2d") < 0 && tuning_cache_lookup_variant(key, plan.x.dtype, plan.w_ncontig) < 0) {
+  if (by_rule) {
     for (int i = 0; i < contraction_variant_count() && !resident_chosen; ++i) {
       const ContractionVariant &cv = contraction_variant(i);
       if (cv.pipeline < 7 || cv.pipeline > 10) continue;
@@ -1940,7 +1980,7 @@ TraceaStatus run_conv(const ConvPlan &plan, const EpilogueChain &chain, hipStrea
       }
     }
   }
-  if (!resident_chosen && forced_variant("conv2d") < 0 && tuning_cache_lookup_variant(key, plan.x.dtype, plan.w_ncontig) < 0) {
+  if (!resident_chosen && by_rule) {
     for (int i = 0; i < contraction_variant_count() && !resident_chosen; ++i) {
       const ContractionVariant &cv = contraction_variant(i);
       if (cv.pipeline != 5) continue;
@@ -1963,7 +2003,7 @@ TraceaStatus run_conv(const ConvPlan &plan, const EpilogueChain &chain, hipStrea
   // short K (one 56x56x64->64 image: 7.4 us against 8.4).  Everywhere else the streamed
   // 8-wave 128x64 and pipelined 64x64 tiles are as fast or faster.  A tuning-cache entry or
   // a forced variant wins over this rule, and tracea_autotune_conv2d measures every variant.
-  if (!resident_chosen && forced_variant("conv2d") < 0 && tuning_cache_lookup_variant(key, plan.x.dtype, plan.w_ncontig) < 0 && g.stride_h == 1 &&
+  if (!resident_chosen && by_rule && g.stride_h == 1 &&
       g.stride_w == 1 && g.block.r_sz * g.block.s_sz > 1 && a.K % 64 == 0 && a.K / 64 <= 40) {
     const long long hw = (long long)g.block.h_out * g.block.w_out;
     int chosen = -1;
@@ -1989,12 +2029,15 @@ TraceaStatus run_conv(const ConvPlan &plan, const EpilogueChain &chain, hipStrea
   const long long w_extent = (long long)g.n_gemm * g.k_gemm * 2;
   const bool small = x_extent < (1ll << 31) && w_extent < (1ll << 31);
   if (conv_only(contraction_variant(vi)) && plan_conv_resident(g, contraction_variant(vi), plan.w_ncontig, &a)) {
-    if (contraction_variant(vi).pipeline == 5 || contraction_variant(vi).pipeline >= 7) fast_epilogue_form(chain, plan.x.dtype, &a);
+    if (contraction_variant(vi).pipeline == 5 || (contraction_variant(vi).pipeline >= 7 && contraction_variant(vi).pipeline <= 10)) fast_epilogue_form(chain, plan.x.dtype, &a);
     const int e = contraction_variant(vi).launch(a, true, plan.x.dtype, false, stream);
     // a member that refuses the arguments its plan accepted (it launched nothing) gives way to the
     // selector's choice below, like one whose plan failed
     if (e != (int)hipErrorInvalidValue) {
       t_last_conv = vi;
+      // (pipelines 9 and 11 split K over the waves of a workgroup)
+      t_last_splits = contraction_variant(vi).pipeline == 11 ? contraction_variant(vi).waves_m : contraction_variant(vi).pipeline == 9 ? 4 : 1;
+      t_last_split_launches = 1;
       return hip_status("conv2d launch", e);
     }
     (void)hipGetLastError();
