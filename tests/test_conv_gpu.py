@@ -635,7 +635,7 @@ PRIVATE_MEMBERS = ["c16x16_c64_w8_w16_ksplit", "c16x32_c64_w8_w16_ksplit", "c32x
 def test_few_pixels_on_private_rings(tracea_gpu, dtype, member):
     """The kernel for few output pixels (K dealt to the waves in 64-channel pieces, private rings), forced: one piece of K
     for eight waves, a piece count off the wave count, tiles cut by the last pixel and the last filter (40, 24, 8),
-    stride, dilation, asymmetric padding, 1x1 and 5x5 filters; bias + ReLU, and BatchNorm + residual + SiLU (table,
+    stride, dilation, asymmetric padding, 1x1 and 5x5 filters, channels that are no multiple of 64; bias + ReLU, and BatchNorm + residual + SiLU (table,
     prefetched residual and the general operators), against torch in double."""
     from tracea_amd import capi
     tdt, rnd = (torch.float16, round_f16) if dtype == "f16" else (torch.bfloat16, round_bf16)
@@ -643,7 +643,8 @@ def test_few_pixels_on_private_rings(tracea_gpu, dtype, member):
     try:
         for (n, h, w, c, k, fs, stride, pad, dil) in [(1, 7, 7, 512, 64, 3, 1, 1, 1), (1, 1, 1, 64, 8, 1, 1, 0, 1), (2, 9, 5, 64, 40, 3, 2, 1, 1),
                                                       (1, 13, 17, 128, 24, 3, 1, 2, 2), (3, 8, 8, 192, 72, 1, 2, 0, 1),
-                                                      (1, 6, 20, 64, 32, 5, 1, (1, 3), 1)]:
+                                                      (1, 6, 20, 64, 32, 5, 1, (1, 3), 1), (1, 40, 36, 8, 64, 7, 4, 3, 1),
+                                                      (2, 6, 7, 24, 40, 3, 1, 1, 1), (1, 9, 9, 96, 48, 3, 2, 1, 2), (1, 5, 5, 72, 16, 1, 1, 0, 1)]:
             kg = fs * fs * c
             rng = np.random.default_rng(h * 31 + w + k)
             x = rnd(rng.standard_normal((n, h, w, c)))

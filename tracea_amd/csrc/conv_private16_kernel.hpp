@@ -6,7 +6,7 @@
 // zero padding; the sum is formed as one partial sum per wave, added in wave order at the end.
 //
 // A workgroup takes 8 XR output pixels by 16 NB filters and all of K = R*S*C; its waves take the 64-channel pieces of K
-// in turn (C is a multiple of 64, so a piece lies inside one tap and the tap's offsets are scalars).  A piece is 8 XR
+// in turn (with C a multiple of 64 a piece lies inside one tap and the tap's offsets are scalars).  A piece is 8 XR
 // pixel rows and 16 NB filter rows of 128 bytes, requested straight into the wave's ring of DEPTH stages, 8 rows per
 // direct-to-LDS load; pixels outside the image are requested out of range and read as zeros.  No wave waits for
 // another before the partial sums meet in LDS.  What bounds such a launch is latency -- the launch itself (1.8 us),
@@ -19,7 +19,9 @@
 
 namespace tracea_amd {
 
-template <int DT, int WAVES, int XR, int NB, int DEPTH>
+// GEN: any multiple of 8 channels.  A 16-byte column of a piece still lies inside one tap, but the columns of a piece lie in
+// several: tap and channel are worked out per lane, once for each of the two columns its rows are swizzled to.
+template <int DT, int WAVES, int XR, int NB, int DEPTH, bool GEN>
 __global__ void __launch_bounds__(WAVES * 64) conv_private16_kernel(const ContractionArgs args) {
   constexpr int BM = 8 * XR, BN = 16 * NB, MB = XR / 2, NT = WAVES * 64;
   constexpr int BR = 2 * NB, REQS = BR + XR, STAGE = REQS * 1024;
@@ -59,29 +61,39 @@ __global__ void __launch_bounds__(WAVES * 64) conv_private16_kernel(const Contra
     fast_divmod(rem, args.w_m, args.w_s, args.w_out, ho, wo);
     hi0[i] = m < M ? ho * args.stride_h - args.pad_h : -(1 << 28);
     wi0[i] = wo * args.stride_w - args.pad_w;
-    pix[i] = (((img * args.h_in + ho * args.stride_h - args.pad_h) * w_in + wi0[i]) * C + ((lane & 7) ^ ((row >> 1) & 7)) * 8) * 2;
+    pix[i] = (((img * args.h_in + ho * args.stride_h - args.pad_h) * w_in + wi0[i]) * C + (GEN ? 0 : ((lane & 7) ^ ((row >> 1) & 7)) * 8)) * 2;
   }
   unsigned char *const ring = smem + wave * (DEPTH * STAGE);
-  const int pieces = K / 64;
+  const int pieces = GEN ? (K + 63) / 64 : K / 64;
   auto request = [&](int t, int slot) __attribute__((always_inline)) {
     const int p = wave + WAVES * t;
     const bool live = p < pieces;
     const int k0 = live ? p * 64 : 0;
-    int rf, rem, sf, ci;
-    fast_divmod(k0, args.sc_m, args.sc_s, args.s_sz * C, rf, rem);
-    fast_divmod(rem, args.c_m, args.c_s, C, sf, ci);
-    const int dh = rf * args.dil_h, dw = sf * args.dil_w;
-    const int off = ((dh * w_in + dw) * C + ci) * 2;
+    // (rows of even and odd loads: the swizzle of a row repeats every 16 rows)
+    constexpr int NK = GEN ? 2 : 1;
+    int dh[NK], dw[NK], off[NK];
+    bool in[NK];
+#pragma unroll
+    for (int e = 0; e < NK; ++e) {
+      const int k = GEN ? k0 + ((lane & 7) ^ ((e * 4 + (lane >> 4)) & 7)) * 8 : k0;
+      int rf, rem, sf, ci;
+      fast_divmod(k, args.sc_m, args.sc_s, args.s_sz * C, rf, rem);
+      fast_divmod(rem, args.c_m, args.c_s, C, sf, ci);
+      dh[e] = rf * args.dil_h;
+      dw[e] = sf * args.dil_w;
+      off[e] = ((dh[e] * w_in + dw[e]) * C + ci) * 2;
+      in[e] = GEN ? live & (k < K) : live;
+    }
     unsigned char *dst = ring + slot * STAGE;
 #pragma unroll
     for (int i = 0; i < BR; ++i)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_b, (__attribute__((address_space(3))) void *)(dst + i * 1024), 16,
-                                               (int)(live ? b_voff[i] : OOB), k0 * 2, 0, 0);
+                                               (int)(in[i % NK] ? b_voff[i] : OOB), k0 * 2, 0, 0);
 #pragma unroll
     for (int i = 0; i < XR; ++i) {
-      const bool ok = live & ((unsigned)(hi0[i] + dh) < (unsigned)args.h_in) & ((unsigned)(wi0[i] + dw) < (unsigned)w_in);
+      const bool ok = in[i % NK] & ((unsigned)(hi0[i] + dh[i % NK]) < (unsigned)args.h_in) & ((unsigned)(wi0[i] + dw[i % NK]) < (unsigned)w_in);
       __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_a, (__attribute__((address_space(3))) void *)(dst + (BR + i) * 1024), 16,
-                                               (int)(ok ? (unsigned)(pix[i] + off) : OOB), 0, 0, 0);
+                                               (int)(ok ? (unsigned)(pix[i] + off[i % NK]) : OOB), 0, 0, 0);
     }
   };
 #pragma unroll
@@ -208,13 +220,13 @@ int launch_conv_private16(const ContractionArgs &a, bool conv, int dtype, bool b
   constexpr int XR = BM / 8, NB = BN / 16;
   constexpr int lds = WAVES * DEPTH * (2 * NB + XR) * 1024 + TRACEA_MAX_EPILOGUE_OPS * 2 * BN * 4;
   static_assert(lds <= 160 * 1024, "rings and table must fit LDS");
-  if (!conv || b_ncontig || a.c_in % 64 != 0 || a.a_bytes == 0 || a.b_bytes == 0 || a.grid_m != (a.M + BM - 1) / BM ||
+  if (!conv || b_ncontig || a.c_in % 8 != 0 || a.a_bytes == 0 || a.b_bytes == 0 || a.grid_m != (a.M + BM - 1) / BM ||
       a.grid_n != (a.N + BN - 1) / BN)
     return (int)hipErrorInvalidValue;
   const dim3 grid((unsigned)(a.grid_m * a.grid_n)), block(WAVES * 64);
-#define TRACEA_LAUNCH_CP(DTV)                                                                              \
+#define TRACEA_LAUNCH_CP(DTV, GENV)                                                                          \
   do {                                                                                                     \
-    auto kfn = conv_private16_kernel<DTV, WAVES, XR, NB, DEPTH>;                                           \
+    auto kfn = conv_private16_kernel<DTV, WAVES, XR, NB, DEPTH, GENV>;                                     \
     static bool attr_done = false;                                                                         \
     if (!attr_done) {                                                                                      \
       hipError_t e = hipFuncSetAttribute((const void *)kfn, hipFuncAttributeMaxDynamicSharedMemorySize, lds); \
@@ -224,8 +236,10 @@ int launch_conv_private16(const ContractionArgs &a, bool conv, int dtype, bool b
     hipLaunchKernelGGL(kfn, grid, block, lds, stream, a);                                                  \
     return (int)hipGetLastError();                                                                         \
   } while (0)
-  if (dtype == DT_F16) TRACEA_LAUNCH_CP(DT_F16);
-  else TRACEA_LAUNCH_CP(DT_BF16);
+  const bool gen = a.c_in % 64 != 0;
+  if (dtype == DT_F16) { if (gen) TRACEA_LAUNCH_CP(DT_F16, true); else TRACEA_LAUNCH_CP(DT_F16, false); }
+  else { if (gen) TRACEA_LAUNCH_CP(DT_BF16, true); else TRACEA_LAUNCH_CP(DT_BF16, false); }
+  return (int)hipErrorInvalidValue;
 #undef TRACEA_LAUNCH_CP
 }
 

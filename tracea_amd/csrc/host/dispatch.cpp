@@ -1883,11 +1883,10 @@ void fast_epilogue_form(const EpilogueChain &chain, int dtype, ContractionArgs *
   a->fe = fe;
 }
 
-// Plan of the kernel for few output pixels (pipeline 11): K-contiguous filters, C a multiple of 64 (a piece of K lies in
-// one tap), input and filters below 2 GiB.
+// Plan of the kernel for few output pixels (pipeline 11): K-contiguous filters, input and filters below 2 GiB.
 bool plan_conv_private16(const ConvGeometry &g, const ContractionVariant &v, bool w_ncontig, ContractionArgs *a) {
   const TraceaConvParamsBlock &b = g.block;
-  if (v.pipeline != 11 || w_ncontig || b.c_in % 64 != 0) return false;
+  if (v.pipeline != 11 || w_ncontig || b.c_in % 8 != 0) return false;
   const long long x_bytes = (long long)b.batch * b.h_in * b.w_in * b.c_in * 2, w_bytes = (long long)g.n_gemm * g.k_gemm * 2;
   if (x_bytes >= (1ll << 31) || w_bytes >= (1ll << 31)) return false;
   a->grid_m = (g.m_gemm + v.bm - 1) / v.bm;
