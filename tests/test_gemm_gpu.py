@@ -367,3 +367,39 @@ def test_products_of_a_few_rows(tracea_gpu, dtype, m):
             got = out.float().cpu().numpy()
             assert_close_scaled(got[:m, :n], ref, tol_half(k, dtype), "%s %s" % (tag, (m, n, k)))
             assert (got[m] == 7.0).all() and (got[:, n:] == 7.0).all(), "outside the output"
+
+
+# one element in a row or column, K off and on the 64-deep tiles, a last row of B within 8 elements of the end in the tile
+# before the last (N 3), two groups of waves with an even and an odd number of K tiles, 128x128 tiles (1409 x 1423)
+@pytest.mark.parametrize("shape", [(1, 9, 8), (8, 1, 9), (65, 3, 66), (63, 65, 64), (64, 64, 73), (3, 130, 127), (70, 67, 321),
+                                   (129, 65, 577), (1409, 1423, 71)])
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+def test_operands_at_any_element_alignment(tracea_gpu, dtype, shape):
+    """The kernel that reads ragged rows in place: pitches and first elements on every residue that matters, both layouts
+    of B, infinities and NaN in the gaps behind the rows and behind the operands, nothing written outside the output."""
+    from tracea_amd import capi
+    m, n, k = shape
+    tdt, rnd = (torch.float16, round_f16) if dtype == "f16" else (torch.bfloat16, round_bf16)
+    rng = np.random.default_rng(m + 3 * n + 7 * k)
+    a = rnd(rng.standard_normal((m, k)) / np.sqrt(k))
+    b = rnd(rng.standard_normal((k, n)))
+    bias = rng.standard_normal(n).astype(np.float32)
+    ref = np.maximum(oracle.gemm_f64(a, b) + bias[None, :], 0.0)
+
+    def placed(x, gap, first, junk):
+        rows, cols = x.shape
+        flat = torch.full((first + rows * (cols + gap) + 16,), junk, device="cuda", dtype=tdt)
+        v = torch.as_strided(flat, (rows, cols), (cols + gap, 1), first)
+        v.copy_(_dev(np.ascontiguousarray(x), tdt))
+        return v
+
+    for gap, first in ((0, 1), (1, 0), (3, 2), (5, 7)):
+        for junk in (float("nan"), float("inf")):
+            da = placed(a, gap, first, junk)
+            for tag, db in (("row-major B", placed(b, gap, first, junk)), ("column-major B", placed(b.T, gap, first, junk).t())):
+                out = torch.full((m + 1, n + 3), 7.0, device="cuda", dtype=tdt)
+                tracea_gpu.gemm(da, db, bias=_dev(bias), epilogue="bias+relu", out=out[:m, :n])
+                assert capi.last_variant("gemm") in ("t64x64x64_w2x2", "t128x128x64_w2x2"), "ran from copies"
+                got = out.float().cpu().numpy()
+                assert_close_scaled(got[:m, :n], ref, tol_half(k, dtype), "%s gap %d first %d" % (tag, gap, first))
+                assert (got[m] == 7.0).all() and (got[:, n:] == 7.0).all(), "outside the output"

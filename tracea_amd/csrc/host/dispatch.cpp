@@ -830,6 +830,55 @@ bool rows_kernel_wanted(long long M, long long N, long long K, int dtype, bool b
   return tuning_cache_lookup_variant(key, dtype, b_ncontig) < 0;
 }
 
+// What the kernel for operands at any element alignment reads in place: rows that do not overlap, of A along K and of B
+// along N or K, extents that hold a 16-byte piece and stay below 2 GiB.
+bool ragged_layout(const View &a, const View &b, const View &c) {
+  const long long M = a.shape[0], K = a.shape[1], N = b.shape[1];
+  if (!is_half(a.dtype) || b.dtype != a.dtype || K <= 0 || c.stride[1] != 1 || a.stride[1] != 1) return false;
+  if ((((uintptr_t)a.ptr | (uintptr_t)b.ptr) & 1) != 0 || a.stride[0] < K) return false;
+  const bool kn = b.stride[1] == 1 && b.stride[0] >= N;
+  if (!kn && (b.stride[0] != 1 || b.stride[1] < K)) return false;
+  const long long cap = 1ll << 30;  // elements
+  if (a.stride[0] >= cap || b.stride[0] >= cap || b.stride[1] >= cap) return false;
+  const long long a_extent = (M - 1) * a.stride[0] + K;
+  const long long b_extent = kn ? (K - 1) * b.stride[0] + N : (N - 1) * b.stride[1] + K;
+  return a_extent >= 8 && a_extent < cap && b_extent >= 8 && b_extent < cap;
+}
+
+// As for products of a few rows, a forced variant or a tuning record wins over the rule (the record of the padded
+// problem, which is what those run).
+bool ragged_kernel_wanted(long long M, long long N, long long K, int dtype) {
+  if (forced_variant("gemm") >= 0) return false;
+  char key[160];
+  snprintf(key, sizeof(key), "gemm_%lld_%lld_%lld_%s", M, N, (K + 31) / 32 * 32, tuning_device_name());
+  return tuning_cache_lookup_variant(key, dtype, false) < 0;
+}
+
+// Its tile and the groups of waves that share K, or 0 where padded copies and the tile kernels are ahead.  f16, us,
+// B by rows, in place (replayed graphs) / from copies (eager):
+//   128x128 tiles for at least half a round of them (1600x1600x501 12.6 against 15.7 on 64x64, 1400x1400x501 12.4
+//   against 11.3), up to four rounds (4001^3 215 / 239, with B by columns 215 / 210; 6001^3 729-862 / 663-762);
+//   two groups where 64x64 tiles leave CUs idle and K is long enough to deal (1000x900x1030 11.8 against 13.1 with one
+//   group, 300x300x301 7.4 against 7.5, 129x257x203 8.2 against 7.5; 1400x1400x501, two rounds, 14.1 against 11.3);
+//   copies where a few workgroups would walk a long K that the tile kernels split over the device (100x100x2501 16.0 /
+//   17.1, x4001 22.4 / 17.5; 300x300x3001 18.1 / 24.0, x6001 35.6 / 34.4; 500x500x9001 49.9 / 62.1).
+int ragged_tile(long long M, long long N, long long K, int *groups) {
+  const long long tiles128 = ((M + 127) / 128) * ((N + 127) / 128), tiles64 = ((M + 63) / 64) * ((N + 63) / 64);
+  const long long cus = device_limits().cus;
+  *groups = 1;
+  if (tiles128 > cus * 4) return 0;
+  if (tiles128 * 2 >= cus) return 128;
+  if (tiles64 * 120 < K - 2500) return 0;
+  if (tiles64 <= cus && K > 256) *groups = 2;
+  return 64;
+}
+
+int variant_index(const char *name) {
+  for (int i = 0; i < contraction_variant_count(); ++i)
+    if (strcmp(contraction_variant(i).name, name) == 0) return i;
+  return -1;
+}
+
 TraceaStatus run_gemm(const View &a, const View &b, const View &c, const EpilogueChain &chain,
                       hipStream_t stream, bool static_only = false, const GemmBatch &batch = GemmBatch()) {
   static thread_local bool in_padded = false;  // this call multiplies padded copies of another call's operands
@@ -984,8 +1033,31 @@ TraceaStatus run_gemm(const View &a, const View &b, const View &c, const Epilogu
     t_last_split_launches = 2;
     return hip_status("split-K reduction launch", launch_splitk_reduce(r, stream));
   }
-  // Operands the tile kernels cannot read as they lie -- a K (or the N of a row-major B) that is not a whole
-  // number of 16-byte pieces, rows that do not start on 16 bytes, strides along K -- are copied once into
+  if (!in_padded && ragged_layout(a, b, c) && ragged_kernel_wanted(M, N, K, a.dtype)) {
+    ContractionArgs args{};
+    int groups = 1;
+    const int tile = ragged_tile(M, N, K, &groups);
+    if (tile != 0) {
+      const bool b_ncontig = b.stride[1] == 1 && b.stride[0] >= N;
+      args.A = a.ptr; args.B = b.ptr; args.C = c.ptr;
+      args.M = (int)M; args.N = (int)N; args.K = (int)K;
+      args.lda = a.stride[0]; args.ldb = b_ncontig ? b.stride[0] : b.stride[1]; args.ldc = c.stride[0];
+      args.out_dtype = c.dtype;
+      args.epi = chain;
+      args.a_bytes = (unsigned)(((M - 1) * args.lda + K) * 2);
+      args.b_bytes = (unsigned)((b_ncontig ? (K - 1) * args.ldb + N : (N - 1) * args.ldb + K) * 2);
+      // (reported as the member on the same tiles that stages them through registers too)
+      static const int staged = variant_index("t64x64x64_w2x2"), staged128 = variant_index("t128x128x64_w2x2");
+      const int vi = tile == 64 ? staged : staged128;
+      fill_grid(&args, contraction_variant(vi));
+      t_last_contraction = vi;
+      t_last_splits = groups;
+      t_last_split_launches = 1;
+      return hip_status("gemm launch", launch_gemm_ragged(args, a.dtype, b_ncontig, tile, groups, stream));
+    }
+  }
+  // Operands none of these kernels reads in place -- fp32 with a K that is not a whole number of 16-byte pieces or rows
+  // that do not start on 16 bytes, strides along K, and half precision where ragged_tile says so -- are copied once into
   // padded, zero-filled rows and multiplied from there: two copy launches in front of a tile kernel instead of
   // the any-layout kernel on the vector ALU (fp32 1000 x 900 x 1030: 794 us there).  Half precision: both as
   // K-contiguous rows (a row-major B is transposed on the way); fp32: A by rows, B row-major.  Not for the entry
