@@ -265,3 +265,27 @@ def test_filter_cache_reuses_the_regrouped_bank_until_it_is_cleared(tracea_gpu):
     finally:
         capi.lib().tracea_set_conv_transpose_filter_cache(0)
         capi.lib().tracea_conv_transpose_filter_cache_clear()
+
+
+# like phases in one launch (2x2 and 4x4 at stride 2), unlike ones (3x3, 5x3 at 3x2), one phase (stride 1); K tiles of one
+# and of several to a tap (C 64, 128, 192), K off the 64-column tiles, more rows than one tile
+@pytest.mark.parametrize("shape", [(1, 5, 6, 64, 24, 4, 4, 2, 1, 0), (2, 9, 7, 128, 72, 3, 3, 2, 1, 1), (1, 6, 6, 192, 40, 2, 2, 2, 0, 0),
+                                   (2, 7, 5, 64, 136, 3, 3, 1, 1, 0), (1, 4, 6, 64, 16, 5, 3, (3, 2), (2, 1), (2, 1)),
+                                   (3, 17, 15, 256, 64, 4, 4, 2, 1, 0), (1, 3, 3, 1024, 8, 2, 2, 2, 0, 0)])
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+def test_filters_read_in_place(tracea_gpu, shape, dtype):
+    """[C,R,S,K] banks that the phase kernels read where they lie: dense, and with NaN in a gap between
+    the input channels; then the same call with the bank in an order that is regrouped."""
+    n, h, w, c, k, r, s, stride, pad, opad = shape
+    tdt, rounder = (torch.float16, round_f16) if dtype == "f16" else (torch.bfloat16, round_bf16)
+    x, wt = _operands(shape, 5, rounder)
+    bias = np.random.default_rng(6).standard_normal(k).astype(np.float32)
+    want = np.maximum(oracle.conv_transpose2d_nhwc(x, wt, stride, pad, opad) + bias, 0.0)
+    wide = torch.full((c, r * s * k + 8), float("nan"), device="cuda", dtype=tdt)
+    wide[:, :r * s * k] = _dev(wt, tdt).reshape(c, -1)
+    for tag, bank, layout in (("dense", _dev(wt, tdt), "crsk"),
+                              ("gap", torch.as_strided(wide, (c, r, s, k), (r * s * k + 8, s * k, k, 1)), "crsk"),
+                              ("regrouped", _dev(wt.transpose(3, 1, 2, 0), tdt), "krsc")):
+        y = tracea_gpu.conv_transpose2d(_dev(x, tdt), bank, bias=_dev(bias), stride=stride, padding=pad, output_padding=opad,
+                                        epilogue="bias+relu", weight_layout=layout)
+        assert_close_scaled(y.float().cpu().numpy(), want, tol_half(c * r * s, dtype), tag)

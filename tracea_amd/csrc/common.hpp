@@ -70,6 +70,12 @@ struct ContractionArgs {
   int phases;
   long long phase_b_stride;
   int phase_pad_h[4], phase_pad_w[4];
+  // b_taps != 0 (N-contiguous B, c_in a multiple of the K tile, below 2 GiB): the filter bank of a transposed
+  // convolution read where it lies.  The filters of tap (r, s) of the phase start (b_rmax - r) * b_tap_r + (s_sz - 1 - s) *
+  // b_tap_s elements behind B, ldb elements from one input channel to the next; phases > 1: phase (o_a, o_b) starts
+  // phase_b_h[o_a] + phase_b_w[o_b] elements behind B (phase_b_stride is not used)
+  int b_taps, b_rmax, b_tap_r, b_tap_s;
+  int phase_b_h[4], phase_b_w[4];
   // patch-resident convolution (pipeline 4) only: filter rows, M tiles per image,
   // padded row width W + 2 pad_w, 16-byte chunks per patch pixel (odd), patch
   // load iterations per thread, LDS bytes reserved for the patch, and the

@@ -668,7 +668,11 @@ __global__ void __launch_bounds__(WM *WN * 64) contraction_kernel(const Contract
       // selects, not an index: a run-time index into the kernel arguments can move them to scratch memory
       pad_h = o_a == 0 ? args.phase_pad_h[0] : o_a == 1 ? args.phase_pad_h[1] : o_a == 2 ? args.phase_pad_h[2] : args.phase_pad_h[3];
       pad_w = o_b == 0 ? args.phase_pad_w[0] : o_b == 1 ? args.phase_pad_w[1] : o_b == 2 ? args.phase_pad_w[2] : args.phase_pad_w[3];
-      Bg += (long long)z * args.phase_b_stride;
+      if (B_NCONTIG && args.b_taps != 0)
+        Bg += (o_a == 0 ? args.phase_b_h[0] : o_a == 1 ? args.phase_b_h[1] : o_a == 2 ? args.phase_b_h[2] : args.phase_b_h[3]) +
+              (o_b == 0 ? args.phase_b_w[0] : o_b == 1 ? args.phase_b_w[1] : o_b == 2 ? args.phase_b_w[2] : args.phase_b_w[3]);
+      else
+        Bg += (long long)z * args.phase_b_stride;
     }
   }
 
@@ -851,6 +855,15 @@ __global__ void __launch_bounds__(WM *WN * 64) contraction_kernel(const Contract
       dh = rf * args.dil_h;
       dw = sf * args.dil_w;
     }
+    int b_soff = (int)((long long)k0 * args.ldb * 2);  // (N-contiguous B)
+    if constexpr (CONV && B_NCONTIG) {
+      if (args.b_taps != 0) {  // the K tile lies in one tap
+        int rf, rem, sf, c0;
+        fast_divmod(k0, args.sc_m, args.sc_s, args.s_sz * args.c_in, rf, rem);
+        fast_divmod(rem, args.c_m, args.c_s, args.c_in, sf, c0);
+        b_soff = ((args.b_rmax - rf) * args.b_tap_r + (args.s_sz - 1 - sf) * args.b_tap_s + c0 * (int)args.ldb) * 2;
+      }
+    }
 #pragma unroll
     for (int i = 0; i < NA; ++i) {
       if (i < lo || i >= hi) continue;
@@ -887,7 +900,7 @@ __global__ void __launch_bounds__(WM *WN * 64) contraction_kernel(const Contract
         // hardware's range check, so the row is tested here
         const unsigned voff = k0 + (tid + i * NT) / NB_CH < K ? b_voff[i] : OOB;
         __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_b, (__attribute__((address_space(3))) void *)dst, 16,
-                                                 (int)voff, (int)((long long)k0 * args.ldb * 2), 0, 0);
+                                                 (int)voff, b_soff, 0, 0);
       }
     }
   };

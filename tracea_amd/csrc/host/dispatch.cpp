@@ -459,7 +459,6 @@ int choose_split(const ContractionVariant &v, int M, int N, int K, int *k_split,
 // the estimate then reads 52.8 / 25.9 us for a 3x3 convolution on N32 7x7x512 with
 // unsplit 64x64 tiles / 128x128 tiles split four ways, where 53.7 / 29.6 us were measured.
 int select_contraction_variant(int m, int n, int k, bool conv, bool b_ncontig, int batch) {
-  (void)conv;
   const DeviceLimits &dev = device_limits();
   const double cus = (double)dev.cus, slot_rate = dev.slot_rate;  // multiply-accumulates per microsecond and CU at efficiency 1
   int best = -1;
@@ -468,6 +467,7 @@ int select_contraction_variant(int m, int n, int k, bool conv, bool b_ncontig, i
     const ContractionVariant &v = contraction_variant(i);
     if (conv_only(v)) continue;  // needs the convolution geometry: see plan_conv_patch
     if (batch > 1 && !takes_batches(v)) continue;
+    if (conv && v.mfma == 16) continue;  // (a convolution would run on the twin: resolve_variant)
     const double gm = (double)((m + v.bm - 1) / v.bm) * batch, gn = (double)((n + v.bn - 1) / v.bn);
     int k_split = 0;
     const int splits = g_split_k_enabled.load() ? choose_split(v, m, n, k, &k_split, 4, batch) : 1;
@@ -508,7 +508,8 @@ int select_contraction_variant(int m, int n, int k, bool conv, bool b_ncontig, i
     // 107.8): the eight-wave 16x16x32 member runs this layout.  (Before the transposing reads were written as
     // instructions the compiler put a vmcnt(0) in front of each one that followed a tile request: 128-132 and
     // 209 us for the two 16x16x32 members.)
-    if (b_ncontig && !conv && v.bm * v.bn >= 256 * 256 && v.waves_m * v.waves_n == 4) prior *= 0.8;
+    // (convolutions, eight waves too: N8 48x48 512->256 4x4 s2 transposed 118.4 us on 256x256 tiles, 106.5 on 128x128)
+    if (b_ncontig && v.bm * v.bn >= 256 * 256 && (conv || v.waves_m * v.waves_n == 4)) prior *= 0.8;
     {
       // A CU with fewer than 8 resident waves (one 4-wave workgroup, the launch too small or
       // the tile's LDS too large for a second) hides less latency.  The fourth root is fitted
@@ -2385,12 +2386,21 @@ TraceaStatus run_conv_transpose_by_phase(const ConvTransposePlan &plan, const Ep
         }
       total += (long long)K * pr.taps * ps.taps * C;
     }
+  // A bank whose output channels lie side by side (the reference's [C*R*S, K] rows among them) is read where it lies, as
+  // an N-contiguous B, by the direct-to-LDS kernels when a K tile lies inside a tap: no regrouping launch.  Same sums in
+  // the same order.  Replayed graphs, regrouped / in place, us: N8 32x32 512->256 4x4 s2 52.1 / 46.7, N8 64x64 256->128
+  // 51.4 / 49.7, N1 16x16 512->512 22.8 / 16.2, N2 20x20 128->64 11.5 / 7.7, N8 32x32 128->128 2x2 11.6 / 8.6, N8 40x40
+  // 512->128 3x3 s1 37.5 / 36.5.  (A cached bank stays what it was.)
+  const long long w_reach = (C - 1) * w.stride[3] + (R - 1) * w.stride[1] + (S - 1) * w.stride[2] + K;
+  const bool in_place = !g_ct_filter_cache.load() && w.stride[0] == 1 && K % 8 == 0 && C % 64 == 0 && aligned(w.ptr, 16) &&
+                        w.stride[1] >= 0 && w.stride[2] >= 0 && w.stride[3] > 0 && w.stride[1] % 8 == 0 && w.stride[2] % 8 == 0 &&
+                        w.stride[3] % 8 == 0 && w_reach * 2 < (1ll << 31) && (long long)N * H * W * C * 2 < (1ll << 31);
   // The regrouped filters live in the per-(device, stream) scratch buffer that split-K launches use
   // (no launch of this path splits K, and work on one stream is ordered); a bank beyond its 64 MiB
   // cap, or a first use while the stream is being captured, takes a stream-ordered allocation.
   hipError_t e = hipSuccess;
   void *filt = nullptr;
-  bool pooled = true, regroup = true;
+  bool pooled = true, regroup = !in_place;
   if (g_ct_filter_cache.load()) {
     // cached copy of this bank: built once (the stream is drained before the copy is published, so that
     // calls on other streams may read it), then no helper launch and no allocation per call
@@ -2421,7 +2431,7 @@ TraceaStatus run_conv_transpose_by_phase(const ConvTransposePlan &plan, const Ep
       }
     }
   }
-  if (filt == nullptr) {
+  if (!in_place && filt == nullptr) {
     filt = splitk_scratch(out.device, stream, (size_t)total * 2 + 256);
     pooled = filt != nullptr;
     if (!pooled) {
@@ -2454,10 +2464,11 @@ TraceaStatus run_conv_transpose_by_phase(const ConvTransposePlan &plan, const Ep
       }
       ContractionArgs c{};
       c.A = x.ptr;
-      c.B = (const unsigned short *)filt + phase_off[(size_t)a * sw + b];
+      if (in_place) c.B = (const unsigned short *)w.ptr + (uniform ? 0 : pr.first_tap * w.stride[1] + ps.first_tap * w.stride[2]);
+      else c.B = (const unsigned short *)filt + phase_off[(size_t)a * sw + b];
       c.C = out.ptr;
       c.M = (int)m; c.N = K; c.K = (int)kg;
-      c.ldb = kg; c.ldc = plan.ldc;
+      c.ldb = in_place ? w.stride[3] : kg; c.ldc = plan.ldc;
       c.out_dtype = out.dtype;
       c.h_in = H; c.w_in = W; c.c_in = C;
       c.h_out = pr.out; c.w_out = ps.out; c.s_sz = ps.taps;
@@ -2475,22 +2486,34 @@ TraceaStatus run_conv_transpose_by_phase(const ConvTransposePlan &plan, const Ep
         c.phase_b_stride = (long long)K * kg;
         for (int i = 0; i < sh; ++i) c.phase_pad_h[i] = phase_axis(i, sh, plan.pad_h, R, Ho).pad;
         for (int i = 0; i < sw; ++i) c.phase_pad_w[i] = phase_axis(i, sw, plan.pad_w, S, Wo).pad;
+        for (int i = 0; i < sh; ++i) c.phase_b_h[i] = phase_axis(i, sh, plan.pad_h, R, Ho).first_tap * (int)w.stride[1];
+        for (int i = 0; i < sw; ++i) c.phase_b_w[i] = phase_axis(i, sw, plan.pad_w, S, Wo).first_tap * (int)w.stride[2];
       }
       c.epi = chain;
       // uniform phases go out as one launch: the selector sees the rows of all of them
       // (VAE layer 65.2 -> 53.8 us on 128x128 tiles instead of 128x64)
       const long long m_launch = uniform ? (long long)c.M * sh * sw : (long long)c.M;
-      int vi = select_contraction_variant((int)(m_launch < (1ll << 31) - 1 ? m_launch : (1ll << 31) - 1), c.N, c.K, true);
+      int vi = select_contraction_variant((int)(m_launch < (1ll << 31) - 1 ? m_launch : (1ll << 31) - 1), c.N, c.K, true, in_place);
       if (vi < 0) { st = fail(TRACEA_UNKNOWN_ERROR, "tracea_conv_transpose2d: no kernel variant available"); break; }
-      const long long w_extent = (long long)K * kg * 2;
+      const long long w_extent = in_place ? w_reach * 2 : (long long)K * kg * 2;
       const bool small = x_extent < (1ll << 31) && w_extent < (1ll << 31);
-      vi = resolve_variant(vi, true, !small, true, false);
+      vi = resolve_variant(vi, true, !small, true, in_place);
+      if (in_place) {
+        // (a K tile that would reach over a tap, or a member that stages through registers: a 64-deep direct one)
+        if (contraction_variant(vi).pipeline < 2 || C % contraction_variant(vi).bk != 0) {
+          vi = variant_index(contraction_variant(vi).bm >= 128 ? "t128x64x64_w4x2_p2" : "t64x64x64_w2x2_p2");
+        }
+        c.b_taps = 1;
+        c.b_rmax = pr.taps - 1;
+        c.b_tap_r = (int)(sh * w.stride[1]);
+        c.b_tap_s = (int)(sw * w.stride[2]);
+      }
       const ContractionVariant &v = contraction_variant(vi);
       c.a_bytes = (unsigned)(small ? x_extent : 0);
       c.b_bytes = (unsigned)(small ? w_extent : 0);
       fill_grid(&c, v);
       t_last_conv = vi;
-      st = hip_status("conv_transpose2d phase launch", v.launch(c, true, x.dtype, false, stream));
+      st = hip_status("conv_transpose2d phase launch", v.launch(c, true, x.dtype, in_place, stream));
     }
   if (!pooled) {
     e = hipFreeAsync(filt, stream);
