@@ -163,3 +163,17 @@ def test_linear_batches_in_one_launch(tracea_gpu, dtype, b, m, k, n, w_layout):
     for i in range(b):
         ref = np.maximum(oracle.gemm_f64(a[i], w[i]) + bias[None, :], 0.0)
         assert_close_scaled(got[i, :m], ref, 1e-4 if dtype == "f32" else tol_half(k, dtype), "linear batch %d" % i)
+
+
+@pytest.mark.parametrize("b,m,k,n", [(34, 2, 1024, 72), (8, 70, 1024, 136), (40, 130, 700, 260), (48, 64, 2040, 64)])
+def test_linear_f32_batch_is_as_exact_as_its_products_one_by_one(tracea_gpu, b, m, k, n):
+    """A batch fills the device with one workgroup per tile where a single product splits K into ranges; its sums are
+    formed over ranges as short all the same.  Bound: the error against 64 bits of the products one by one, with a tenth
+    for the order of the additions."""
+    g = torch.Generator().manual_seed(b * m + k)
+    a = torch.randn(b, m, k, generator=g).cuda()
+    w = (torch.randn(b, k, n, generator=g) / k ** 0.5).cuda()
+    one_launch = tracea_gpu.linear(a, w)
+    singles = torch.stack([tracea_gpu.gemm(a[i], w[i]) for i in range(b)])
+    ref = torch.stack([a[i].double() @ w[i].double() for i in range(b)])
+    assert (one_launch.double() - ref).norm() <= 1.1 * (singles.double() - ref).norm()

@@ -98,7 +98,7 @@ struct ContractionArgs {
   } fe;
   EpilogueChain epi;
   // batch > 1: grid.z = batch products of one shape in one launch (half-precision tiles up to 128x128 and the fp32
-  // direct-to-LDS kernel); product z reads A + z*batch_a and B + z*batch_b (elements) and writes the rows from
+  // kernel on 64x64); product z reads A + z*batch_a and B + z*batch_b (elements) and writes the rows from
   // z*batch_rows of C on.  Not combined with a tile list or a split that needs the reduction kernel.
   int batch;
   long long batch_a, batch_b, batch_rows;

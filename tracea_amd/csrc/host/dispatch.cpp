@@ -800,6 +800,18 @@ bool f32_layout(const View &a, const View &b, const View &c) {
          aligned(a.ptr, 16) && aligned(b.ptr, 16);
 }
 
+// Two tile shapes for fp32, 128x128x16 and (direct-to-LDS form only) 64x64x16.  A CU works through its
+// share of the tiles at one 128x128 tile per 4 units of time or one 64x64 tile per 1.06 units
+// (the small tile reads its operands from LDS twice as often): the shape whose busiest CU
+// finishes first is taken.  Measured, 128 / 64, in us: 1024^3 68 / 24.7, 1536^3 102 / 77,
+// 3072^3 558 / 441, 2048^3 134.7 / 133.4, 4096^3 972 / 1033.  (A 128x64 tile was never the fastest:
+// 477 at 3072^3, 1003 at 4096^3.)
+bool f32_small_tiles(long long M, long long N) {
+  const long long tiles128 = ((M + 127) / 128) * ((N + 127) / 128), tiles64 = ((M + 63) / 64) * ((N + 63) / 64);
+  const long long ncu = device_limits().cus;
+  return (double)((tiles64 + ncu - 1) / ncu) * 1.06 < (double)((tiles128 + ncu - 1) / ncu) * 4.0;
+}
+
 // True when run_gemm takes the batch in one launch: operands of every product as the tile kernels read them and below
 // 2 GiB, output batches a whole number of rows apart, and a product too small to fill the device on its own -- one of
 // 256 or more 256x256 tiles runs faster on those, which take no batch.  Sixteen products of 128x512x512 in f16: 16
@@ -814,7 +826,10 @@ bool gemm_batch_in_one_launch(const View &a, const View &b, const View &c, const
   const long long b_extent = half.ok && half.b_kcontig ? ((N - 1) * b.stride[1] + K) * esz : ((K - 1) * b.stride[0] + N) * esz;
   if (a_extent >= (1ll << 31) || b_extent >= (1ll << 31)) return false;
   if (batch.a % step != 0 || batch.b % step != 0 || c.stride[0] <= 0 || batch.c % c.stride[0] != 0 || batch.count > 65535) return false;
-  if (!f32) {
+  if (f32) {
+    // (the batch runs on 64x64 tiles: a product that is ahead on the larger ones is large enough to go alone)
+    if (!f32_small_tiles(M, N)) return false;
+  } else {
     const int forced = forced_variant("gemm");
     if (forced >= 0 && !takes_batches(contraction_variant(forced))) return false;
     if (((M + 255) / 256) * ((N + 255) / 256) >= device_limits().cus) return false;
@@ -950,17 +965,10 @@ TraceaStatus run_gemm(const View &a, const View &b, const View &c, const Epilogu
       args.a_bytes = (unsigned)a_extent;
       args.b_bytes = (unsigned)b_extent;
     }
-    // Two tile shapes, 128x128x16 and (direct-to-LDS form only) 64x64x16.  A CU works through its
-    // share of the tiles at one 128x128 tile per 4 units of time or one 64x64 tile per 1.06 units
-    // (the small tile reads its operands from LDS twice as often): the shape whose busiest CU
-    // finishes first is taken.  Measured, 128 / 64, in us: 1024^3 68 / 24.7, 1536^3 102 / 77,
-    // 3072^3 558 / 441, 2048^3 134.7 / 133.4, 4096^3 972 / 1033.  (A 128x64 tile was never the fastest:
-    // 477 at 3072^3, 1003 at 4096^3.)
     static const ContractionVariant f32_tile128 = {"f32_128x128x16", 128, 128, 16, 2, 2, 1, 0, 0, nullptr, 32};
-    const long long tiles128 = ((M + 127) / 128) * ((N + 127) / 128) * batch.count,
-                    tiles64 = ((M + 63) / 64) * ((N + 63) / 64) * batch.count;
+    const long long tiles128 = ((M + 127) / 128) * ((N + 127) / 128), tiles64 = ((M + 63) / 64) * ((N + 63) / 64) * batch.count;
     const long long ncu = device_limits().cus;
-    int tile = args.a_bytes != 0 && (double)((tiles64 + ncu - 1) / ncu) * 1.06 < (double)((tiles128 + ncu - 1) / ncu) * 4.0 ? 64 : 128;
+    int tile = args.a_bytes != 0 && (batch.count > 1 || f32_small_tiles(M, N)) ? 64 : 128;  // (a batch: gemm_batch_in_one_launch)
     int k_split = 0, splits = 1;
     t_last_split_launches = 1;
     const bool can_fuse = args.a_bytes != 0 && !static_only && g_split_k_enabled.load() && g_split_k_one_launch.load();
@@ -995,7 +1003,7 @@ TraceaStatus run_gemm(const View &a, const View &b, const View &c, const Epilogu
         splits = (nk + per - 1) / per;
       }
     } else {
-      splits = g_split_k_enabled.load() ? choose_split(f32_tile128, (int)M, (int)N, (int)K, &k_split, 4, batch.count) : 1;
+      splits = g_split_k_enabled.load() ? choose_split(f32_tile128, (int)M, (int)N, (int)K, &k_split, 4) : 1;
     }
     const long long tiles = tile == 128 ? tiles128 : tiles64;
     const size_t tile_elts = tile == 128 ? 128 * 128 : 64 * 64;

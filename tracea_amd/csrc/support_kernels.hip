@@ -182,7 +182,11 @@ __global__ void __launch_bounds__(256) gemm_f32_kernel(const ContractionArgs arg
 // out of range (they write zeros to a stage nobody multiplies), so that the
 // count of outstanding requests a wave waits on is the same in every iteration.
 // ---------------------------------------------------------------------------
-template <int TM, int TN, int STAGES, int KSUB, int FIRST_T = 1>
+// BATCH: products of one shape along grid.z (one product's instantiation carries none of it: 0.7 % at 1024^3).  A batch
+// fills the device without splitting K, so its accumulators hand their sums over every 256 k, as the up to four ranges
+// of 256 and more of a single product on these tiles do: 34 products of 2x72x1024 were off by 2.4e-7 in one chain,
+// 2.1e-7 launched one by one and here.  (On 64x64 tiles only: the larger ones have no registers for the handed-over sums.)
+template <int TM, int TN, int STAGES, int KSUB, bool BATCH, int FIRST_T = 1>
 __global__ void __launch_bounds__(256) gemm_f32_dma_kernel(const ContractionArgs args) {
   constexpr int BM = 64 * TM, BN = 64 * TN, BK = F32_BK * KSUB;  // a stage holds KSUB sub-tiles of 16 k, each [A][B]
   constexpr int A_STAGE = BM * F32_BK * 4, B_STAGE = F32_BK * BN * 4, SUB = A_STAGE + B_STAGE, STAGE = KSUB * SUB;
@@ -201,9 +205,13 @@ __global__ void __launch_bounds__(256) gemm_f32_dma_kernel(const ContractionArgs
   const int K = args.k_split > 0 ? min(args.K, kb + args.k_split) : args.K;
   // one-launch split: see the block in front of the epilogue
   const bool fused = args.k_split > 0 && args.fuse_ws != nullptr;
-  const long long zrow = (args.k_split > 0 && !fused ? (long long)blockIdx.y * M : 0ll) + (long long)blockIdx.z * args.batch_rows;
-  const float *Ag = (const float *)args.A + (long long)blockIdx.z * args.batch_a;
-  const float *Bg = (const float *)args.B + (long long)blockIdx.z * args.batch_b;
+  long long zrow = args.k_split > 0 && !fused ? (long long)blockIdx.y * M : 0ll;
+  const float *Ag = (const float *)args.A, *Bg = (const float *)args.B;
+  if constexpr (BATCH) {
+    zrow += (long long)blockIdx.z * args.batch_rows;
+    Ag += (long long)blockIdx.z * args.batch_a;
+    Bg += (long long)blockIdx.z * args.batch_b;
+  }
 
   constexpr unsigned OOB = 0x80000000u;
   __amdgpu_buffer_rsrc_t rsrc_a = __builtin_amdgcn_make_buffer_rsrc((void *)Ag, 0, (int)args.a_bytes, 0x00020000);
@@ -266,6 +274,12 @@ __global__ void __launch_bounds__(256) gemm_f32_dma_kernel(const ContractionArgs
   f32x16 acc_odd;
 #pragma unroll
   for (int e = 0; e < 16; ++e) acc_odd[e] = 0.0f;
+  static_assert(!BATCH || ONE, "one block per wave");
+  f32x16 total;  // BATCH: what the accumulators have handed over
+  if constexpr (BATCH) {
+#pragma unroll
+    for (int e = 0; e < 16; ++e) total[e] = 0.0f;
+  }
 
   const int lrow = lane & 31, lhalf = lane >> 5;
   // A: row wm*32TM + i*32 + lrow, 16-byte columns 2h and 2h+1 (k = 8h .. 8h+7)
@@ -388,6 +402,17 @@ __global__ void __launch_bounds__(256) gemm_f32_dma_kernel(const ContractionArgs
   for (int kt = 0; kt < nk; kt += 2) {
     step(kt, af0, bf0, af1, bf1);
     if (kt + 1 < nk) step(kt + 1, af1, bf1, af0, bf0);
+    if constexpr (BATCH) {
+      constexpr int HAND_OVER = 256 / BK;  // (even: after the second step of a pair)
+      if ((kt + 2) % HAND_OVER == 0) {
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+          total[e] += acc[0][0][e] + acc_odd[e];
+          acc[0][0][e] = 0.0f;
+          acc_odd[e] = 0.0f;
+        }
+      }
+    }
   }
   // requests past the end of K may still be writing zeros where the epilogue stages, and the last operand reads
   // (of a tile nobody multiplies) may still be writing their registers
@@ -398,6 +423,10 @@ __global__ void __launch_bounds__(256) gemm_f32_dma_kernel(const ContractionArgs
   if constexpr (ONE) {
 #pragma unroll
     for (int e = 0; e < 16; ++e) acc[0][0][e] += acc_odd[e];
+  }
+  if constexpr (BATCH) {
+#pragma unroll
+    for (int e = 0; e < 16; ++e) acc[0][0][e] = total[e] + acc[0][0][e];
   }
 
   // One-launch split along K, as in the half-precision kernels: every workgroup leaves its partial product in
@@ -410,7 +439,7 @@ __global__ void __launch_bounds__(256) gemm_f32_dma_kernel(const ContractionArgs
     const unsigned splits = gridDim.y;
     constexpr unsigned TILE_BYTES = BM * BN * 4, WAVE_BYTES = TILE_BYTES / 4;
     __amdgpu_buffer_rsrc_t rsrc_ws = __builtin_amdgcn_make_buffer_rsrc((void *)args.fuse_ws, 0, 0x7fffffff, 0x00020000);
-    const unsigned tile = blockIdx.z * gridDim.x + blockIdx.x;
+    const unsigned tile = BATCH ? blockIdx.z * gridDim.x + blockIdx.x : blockIdx.x;
     const unsigned first = tile * splits * TILE_BYTES + wave_u * WAVE_BYTES + lane * 16;
     const unsigned mine = first + blockIdx.y * TILE_BYTES;
 #pragma unroll
@@ -466,11 +495,14 @@ int launch_gemm_f32(const ContractionArgs &a, int tile, hipStream_t stream) {
   args.group_m = 4;
   const unsigned splits = a.k_split > 0 ? (unsigned)((a.K + a.k_split - 1) / a.k_split) : 1u;
   const dim3 grid((unsigned)(args.grid_m * args.grid_n), splits, (unsigned)(a.batch > 1 ? a.batch : 1));
-  if (!dma && a.batch > 1) return (int)hipErrorInvalidValue;  // (the register-staged twin takes one product)
-  if (!dma) hipLaunchKernelGGL(gemm_f32_kernel, grid, dim3(256), 0, stream, args);
-  else if (tile == 64) hipLaunchKernelGGL((gemm_f32_dma_kernel<1, 1, 4, 1>), grid, dim3(256), 0, stream, args);
-  else if (tile == 6432) hipLaunchKernelGGL((gemm_f32_dma_kernel<1, 1, 4, 2>), grid, dim3(256), 0, stream, args);
-  else hipLaunchKernelGGL((gemm_f32_dma_kernel<2, 2, 2, 1>), grid, dim3(256), 0, stream, args);
+  if (a.batch > 1) {
+    if (!dma || tile == 128) return (int)hipErrorInvalidValue;  // (those forms take one product)
+    if (tile == 64) hipLaunchKernelGGL((gemm_f32_dma_kernel<1, 1, 4, 1, true>), grid, dim3(256), 0, stream, args);
+    else hipLaunchKernelGGL((gemm_f32_dma_kernel<1, 1, 4, 2, true>), grid, dim3(256), 0, stream, args);
+  } else if (!dma) hipLaunchKernelGGL(gemm_f32_kernel, grid, dim3(256), 0, stream, args);
+  else if (tile == 64) hipLaunchKernelGGL((gemm_f32_dma_kernel<1, 1, 4, 1, false>), grid, dim3(256), 0, stream, args);
+  else if (tile == 6432) hipLaunchKernelGGL((gemm_f32_dma_kernel<1, 1, 4, 2, false>), grid, dim3(256), 0, stream, args);
+  else hipLaunchKernelGGL((gemm_f32_dma_kernel<2, 2, 2, 1, false>), grid, dim3(256), 0, stream, args);
   return (int)hipGetLastError();
 }
 
