@@ -329,13 +329,14 @@ void tracea_set_split_k(int32_t enabled);
 void tracea_set_split_k_one_launch(int32_t enabled);
 int32_t tracea_last_split_k_launches(void);
 /* tracea_conv_transpose2d runs as one stride-1 convolution per output phase (stride_h * stride_w
- * launches on a regrouped copy of the filter bank, the outputs written in place) when every phase
+ * launches on the filter bank or a regrouped copy of it, the outputs written in place) when every phase
  * has taps and no negative padding and the input is dense half-precision NHWC with a multiple of 8
  * channels; otherwise, and always after tracea_set_conv_transpose_by_phase(0), as a GEMM to fp32
  * partial products followed by a gather.  The two formulations agree within the tolerance of the
  * operator (fp32 accumulation in a different order). */
 void tracea_set_conv_transpose_by_phase(int32_t enabled);
-/* The by-phase formulation regroups the filter bank at every call (one helper launch).  With the filter
+/* The by-phase formulation regroups the filter bank at every call (one helper launch), except a bank whose output
+ * channels lie side by side with a multiple of 64 input channels, which it reads where it lies.  With the filter
  * cache on, the regrouped bank of a (device, filter pointer, shape, strides, stride, padding) is built once,
  * kept in device memory of its own and reused by later calls, which then launch nothing but the phase
  * convolutions and allocate nothing: for callers whose filters do not change between calls (inference).
