@@ -304,3 +304,25 @@ def test_head_dimensions_that_are_multiples_of_8_run_in_place(tracea_gpu, dtype,
             assert "part" in capi.last_variant("attention")
             assert_close_scaled(out.float().cpu().numpy(), want, _tol(d, dtype), "D=%d S=%d causal=%s %s" % (d, s, causal, dtype))
             assert torch.isnan(big[..., d:].float()).all()
+
+
+@pytest.mark.parametrize("d", [64, 96, 40])
+def test_rows_stored_backwards_run_from_copies(tracea_gpu, d):
+    """K and V with a negative row stride (the C ABI's strides are signed): the kernels reach a slice's rows by unsigned
+    offsets from its first one, so such a call runs from copies, for every head dimension."""
+    import ctypes as C
+
+    from tracea_amd import capi
+    b, h, s = 2, 3, 130
+    q, k, v = _inputs(b, h, s, d, 17 * d, round_f16)
+    want = oracle.attention_bhsd(q, k, v, 1.0 / np.sqrt(d), True)
+    dq, dk, dv = _dev(q, torch.float16), _dev(k[:, :, ::-1].copy(), torch.float16), _dev(v[:, :, ::-1].copy(), torch.float16)
+    out = torch.empty_like(dq)
+
+    def backwards(t):
+        return capi.View(t.data_ptr() + (s - 1) * d * 2, (b, h, s, d), (h * s * d, s * d, -d, 1), capi.F16, 0)
+    vq, vo = (capi.View(t.data_ptr(), (b, h, s, d), None, capi.F16, 0) for t in (dq, out))
+    vk, vv = backwards(dk), backwards(dv)
+    capi.check("tracea_attention", capi.lib().tracea_attention(vq.c, vk.c, vv.c, C.byref(vo.c), capi.AttentionParams(1, 0, 0.0, None)))
+    torch.cuda.synchronize()
+    assert_close_scaled(out.float().cpu().numpy(), want, _tol(d, "f16"), "backwards D=%d" % d)

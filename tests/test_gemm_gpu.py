@@ -403,3 +403,25 @@ def test_operands_at_any_element_alignment(tracea_gpu, dtype, shape):
                 got = out.float().cpu().numpy()
                 assert_close_scaled(got[:m, :n], ref, tol_half(k, dtype), "%s gap %d first %d" % (tag, gap, first))
                 assert (got[m] == 7.0).all() and (got[:, n:] == 7.0).all(), "outside the output"
+
+
+@pytest.mark.parametrize("shape", [(40, 64, 64), (130, 72, 96), (33, 67, 45)])
+@pytest.mark.parametrize("dtype", ["f16", "f32"])
+def test_rows_stored_backwards_run_from_copies(tracea_gpu, dtype, shape):
+    """A and B with negative row strides (the C ABI's strides are signed): the tile kernels reach an operand's rows by
+    unsigned offsets from its first one, so such a product runs from copies."""
+    from tracea_amd import capi
+    m, n, k = shape
+    tdt, rnd, code = (torch.float16, round_f16, capi.F16) if dtype == "f16" else (torch.float32, lambda x: np.asarray(x, np.float32), capi.F32)
+    rng = np.random.default_rng(m + n)
+    a = rnd(rng.standard_normal((m, k)) / np.sqrt(k))
+    b = rnd(rng.standard_normal((k, n)))
+    ref = oracle.gemm_f64(a, b)
+    da, db, out = _dev(a[::-1].copy(), tdt), _dev(b[::-1].copy(), tdt), torch.empty(m, n, device="cuda", dtype=torch.float32)
+    esz = da.element_size()
+    va = capi.View(da.data_ptr() + (m - 1) * k * esz, (m, k), (-k, 1), code, 0)
+    vb = capi.View(db.data_ptr() + (k - 1) * n * esz, (k, n), (-n, 1), code, 0)
+    vc = capi.View(out.data_ptr(), (m, n), None, capi.F32, 0)
+    capi.check("tracea_gemm", capi.lib().tracea_gemm(va.c, vb.c, None, None, C.byref(vc.c), capi.GemmParams(capi.EPI_IDENTITY, None)))
+    torch.cuda.synchronize()
+    assert np.abs(out.cpu().numpy() - ref).max() <= 1e-4 * max(1.0, np.abs(ref).max())

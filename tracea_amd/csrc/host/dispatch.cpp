@@ -782,6 +782,7 @@ struct HalfLayout {
 HalfLayout half_layout(const View &a, const View &b, const View &c) {
   HalfLayout l{false, false};
   if (!is_half(a.dtype) || b.dtype != a.dtype || a.shape[1] <= 0) return l;
+  if (a.stride[0] < 0 || b.stride[0] < 0 || b.stride[1] < 0) return l;  // (offsets and extents are unsigned from the first row on)
   const bool a_ok = a.stride[1] == 1 && a.stride[0] % 8 == 0 && a.shape[1] % 8 == 0 && aligned(a.ptr, 16);
   const bool b_ncontig = b.stride[1] == 1 && b.stride[0] % 8 == 0 && b.shape[1] % 8 == 0 && aligned(b.ptr, 16);
   l.b_kcontig = b.stride[0] == 1 && b.stride[1] % 8 == 0 && aligned(b.ptr, 16);
@@ -795,7 +796,7 @@ HalfLayout half_layout(const View &a, const View &b, const View &c) {
 bool f32_layout(const View &a, const View &b, const View &c) {
   const long long K = a.shape[1], N = b.shape[1];
   return a.dtype == TRACEA_DTYPE_FLOAT32 && b.dtype == TRACEA_DTYPE_FLOAT32 && c.dtype == TRACEA_DTYPE_FLOAT32 && K > 0 &&
-         a.stride[1] == 1 && b.stride[1] == 1 && c.stride[1] == 1 && K % 4 == 0 &&
+         a.stride[1] == 1 && b.stride[1] == 1 && c.stride[1] == 1 && K % 4 == 0 && a.stride[0] >= 0 && b.stride[0] >= 0 &&
          (N % 4 == 0 || ((K - 1) * b.stride[0] + N) * 4 < (1ll << 31)) && a.stride[0] % 4 == 0 && b.stride[0] % 4 == 0 &&
          aligned(a.ptr, 16) && aligned(b.ptr, 16);
 }
@@ -1205,7 +1206,8 @@ TraceaStatus dispatch_gemm_tiles(const TraceaTensorView &ta, const TraceaTensorV
   const bool a_ok = a.stride[1] == 1 && a.stride[0] % 8 == 0 && K % 8 == 0 && aligned(a.ptr, 16);
   const bool b_kcontig = b.stride[0] == 1 && b.stride[1] % 8 == 0 && aligned(b.ptr, 16);
   const bool b_ncontig = b.stride[1] == 1 && b.stride[0] % 8 == 0 && N % 8 == 0 && aligned(b.ptr, 16);
-  if (!(is_half(a.dtype) && b.dtype == a.dtype && a_ok && (b_kcontig || b_ncontig) && c.stride[1] == 1))
+  const bool forward = a.stride[0] >= 0 && b.stride[0] >= 0 && b.stride[1] >= 0;  // (unsigned offsets, as in half_layout)
+  if (!(is_half(a.dtype) && b.dtype == a.dtype && a_ok && forward && (b_kcontig || b_ncontig) && c.stride[1] == 1))
     return fail(TRACEA_UNSUPPORTED_CONFIG,
                 "%s: needs fp16 or bf16 operands of one type, 16-byte aligned, K-contiguous A with K and the row "
                 "stride multiples of 8, B contiguous along K or N, unit column stride of C", what);
@@ -2688,6 +2690,8 @@ TraceaStatus dispatch_attention(const TraceaTensorView &tq, const TraceaTensorVi
   const long long reach = S + 16 * 64;
   bool in_place = D == 64 || D == 128 ||
                   (D % 8 == 0 && scale > 0.0f && (reach * k.stride[2] + D) * 2 < (1ll << 31) && (reach * v.stride[2] + D) * 2 < (1ll << 31));
+  // (rows of K and V are reached by unsigned offsets from the slice's first row)
+  if (k.stride[2] < 0 || v.stride[2] < 0) in_place = false;
   for (const View *t : views)
     if (t->stride[3] != 1 || t->stride[2] % 8 != 0 || t->stride[1] % 8 != 0 || t->stride[0] % 8 != 0 || !aligned(t->ptr, 16))
       in_place = false;
