@@ -326,3 +326,15 @@ def test_rows_stored_backwards_run_from_copies(tracea_gpu, d):
     capi.check("tracea_attention", capi.lib().tracea_attention(vq.c, vk.c, vv.c, C.byref(vo.c), capi.AttentionParams(1, 0, 0.0, None)))
     torch.cuda.synchronize()
     assert_close_scaled(out.float().cpu().numpy(), want, _tol(d, "f16"), "backwards D=%d" % d)
+
+
+@pytest.mark.parametrize("d", [40, 96])
+def test_result_over_the_keys(tracea_gpu, d):
+    """The result written over K, then over V: their other readers must not see it."""
+    b, h, s = 1, 4, 700
+    q, k, v = _inputs(b, h, s, d, d, round_f16)
+    want = oracle.attention_bhsd(q, k, v, 1.0 / np.sqrt(d), False)
+    for which in (1, 2):
+        t = [_dev(x, torch.float16) for x in (q, k, v)]
+        tracea_gpu.attention(*t, out=t[which])
+        assert_close_scaled(t[which].float().cpu().numpy(), want, _tol(d, "f16"), "over operand %d" % which)

@@ -666,3 +666,17 @@ def test_few_pixels_on_private_rings(tracea_gpu, dtype, member):
             assert_close_scaled(y.float().cpu().numpy(), want, tol_half(kg, dtype), "%s chain %s" % (member, (n, h, w, c)))
     finally:
         capi.force_variant("conv2d", -1)
+
+
+@pytest.mark.parametrize("hw", [7, 14])
+def test_pointwise_convolution_over_its_input(tracea_gpu, hw):
+    """1x1 filters, 64 channels to 64, the output written over the input: a tile of 64 filters has read its pixels before it
+    writes them, smaller ones share them between workgroups and leave such calls alone."""
+    rng = np.random.default_rng(hw)
+    x = round_f16(rng.standard_normal((1, hw, hw, 64)))
+    w = round_f16(rng.standard_normal((64, 1, 1, 64)) / 8)
+    want = x.reshape(-1, 64).astype(np.float64) @ w.reshape(64, 64).T.astype(np.float64)
+    for _ in range(3):
+        t = _dev(x, torch.float16)
+        tracea_gpu.conv2d(t, _dev(w, torch.float16), out=t)
+        assert_close_scaled(t.float().cpu().numpy().reshape(-1, 64), want, tol_half(64, "f16"), "in place")

@@ -177,3 +177,25 @@ def test_linear_f32_batch_is_as_exact_as_its_products_one_by_one(tracea_gpu, b, 
     singles = torch.stack([tracea_gpu.gemm(a[i], w[i]) for i in range(b)])
     ref = torch.stack([a[i].double() @ w[i].double() for i in range(b)])
     assert (one_launch.double() - ref).norm() <= 1.1 * (singles.double() - ref).norm()
+
+
+@pytest.mark.parametrize("dtype", ["f16", "f32"])
+def test_linear_batches_that_share_memory_keep_their_order(tracea_gpu, dtype):
+    """Output batches on one another: the last product stays.  An output over the input: each product reads its own rows."""
+    tdt, rnd, _ = TYPES[dtype]
+    tol = 1e-4 if dtype == "f32" else tol_half(64, dtype)
+    rng = np.random.default_rng(4)
+    b, m, k = 6, 60, 64
+    a = rnd(rng.standard_normal((b, m, k)) / np.sqrt(k))
+    w = rnd(rng.standard_normal((b, k, k)))
+    one = torch.empty(m, k, device="cuda", dtype=tdt)
+    tracea_gpu.linear(_dev(a, tdt), _dev(w, tdt), out=one.expand(b, m, k))
+    assert_close_scaled(one.float().cpu().numpy(), oracle.gemm_f64(a[-1], w[-1]), tol, "last batch")
+    rows = torch.empty(m + b - 1, k, device="cuda", dtype=tdt)  # batch i on rows i .. i + m - 1
+    tracea_gpu.linear(_dev(a, tdt), _dev(w, tdt), out=rows.as_strided((b, m, k), (k, k, 1)))
+    want = np.concatenate([oracle.gemm_f64(a[i], w[i])[:1] for i in range(b - 1)] + [oracle.gemm_f64(a[-1], w[-1])])
+    assert_close_scaled(rows.float().cpu().numpy(), want, tol, "overlapping batches")
+    x = _dev(a, tdt)
+    tracea_gpu.linear(x, _dev(w, tdt), out=x)
+    for i in range(b):
+        assert_close_scaled(x[i].float().cpu().numpy(), oracle.gemm_f64(a[i], w[i]), tol, "in place")

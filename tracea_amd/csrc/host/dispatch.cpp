@@ -10,6 +10,7 @@
 #include <algorithm>
 #include <atomic>
 #include <cmath>
+#include <cstdlib>
 #include <cstring>
 #include <map>
 #include <mutex>
@@ -57,6 +58,44 @@ bool is_half(int dt) { return dt == TRACEA_DTYPE_FLOAT16 || dt == TRACEA_DTYPE_B
 bool is_float_type(int dt) { return dt == TRACEA_DTYPE_FLOAT32 || is_half(dt); }
 int elem_size(int dt) { return dt == TRACEA_DTYPE_FLOAT32 ? 4 : 2; }
 bool aligned(const void *p, size_t a) { return (((uintptr_t)p) & (a - 1)) == 0; }
+
+// Rows of equal length on one pitch, the form of most views: element rows `pitch` apart, `len` elements of each used.
+bool row_form(const View &v, long long *pitch, long long *len) {
+  if (v.rank < 2 || v.stride[v.rank - 1] != 1) return false;
+  // the pitch is the stride of the last dim but one; a [B,H,S,D] view of [B,S,H,D] storage has its heads inside the row
+  *pitch = v.stride[v.rank - 2];
+  *len = v.shape[v.rank - 1];
+  if (*pitch < *len) return false;
+  for (int i = v.rank - 3; i >= 0; --i) {
+    if (v.shape[i] == 1 || v.stride[i] % *pitch == 0) continue;
+    if (v.stride[i] < *len || (*len += (v.shape[i] - 1) * v.stride[i]) > *pitch) return false;
+  }
+  return true;
+}
+
+// Whether two views may share an element (columns of one buffer side by side, a query tensor inside a packed
+// [Q K V] row and the like are told apart).
+bool may_overlap(const View &a, const View &b) {
+  auto span = [](const View &v, uintptr_t *lo, uintptr_t *hi) {
+    long long first = 0, last = 0;
+    for (int i = 0; i < v.rank; ++i) {
+      if (v.shape[i] <= 0) return false;
+      (v.stride[i] < 0 ? first : last) += (v.shape[i] - 1) * v.stride[i];
+    }
+    *lo = (uintptr_t)v.ptr + (uintptr_t)(first * elem_size(v.dtype));
+    *hi = (uintptr_t)v.ptr + (uintptr_t)((last + 1) * elem_size(v.dtype));
+    return true;
+  };
+  uintptr_t alo, ahi, blo, bhi;
+  if (!span(a, &alo, &ahi) || !span(b, &blo, &bhi) || ahi <= blo || bhi <= alo) return false;
+  long long pa, la, pb, lb;
+  if (!row_form(a, &pa, &la) || !row_form(b, &pb, &lb)) return true;
+  pa *= elem_size(a.dtype); la *= elem_size(a.dtype); pb *= elem_size(b.dtype); lb *= elem_size(b.dtype);
+  if (pa != pb) return true;
+  long long d = ((long long)((intptr_t)b.ptr - (intptr_t)a.ptr)) % pa;
+  if (d < 0) d += pa;
+  return d < la || d + lb > pa;
+}
 
 const char *dtype_name(int dt) {
   switch (dt) {
@@ -827,6 +866,8 @@ bool gemm_batch_in_one_launch(const View &a, const View &b, const View &c, const
   const long long b_extent = half.ok && half.b_kcontig ? ((N - 1) * b.stride[1] + K) * esz : ((K - 1) * b.stride[0] + N) * esz;
   if (a_extent >= (1ll << 31) || b_extent >= (1ll << 31)) return false;
   if (batch.a % step != 0 || batch.b % step != 0 || c.stride[0] <= 0 || batch.c % c.stride[0] != 0 || batch.count > 65535) return false;
+  // (products that write what another one reads or writes keep their order: one by one)
+  if (c.stride[0] < N || std::abs(batch.c) / c.stride[0] < M) return false;
   if (f32) {
     // (the batch runs on 64x64 tiles: a product that is ahead on the larger ones is large enough to go alone)
     if (!f32_small_tiles(M, N)) return false;
@@ -927,8 +968,9 @@ TraceaStatus run_gemm(const View &a, const View &b, const View &c, const Epilogu
         args.batch = batch.count;
         args.batch_a = batch.a; args.batch_b = batch.b; args.batch_rows = batch.c / c.stride[0];
       }
+      // (an output that is also an operand works where one workgroup reads all of what it overwrites: not on these tiles)
       if (M <= kGemmRowsMax && small && !in_padded && gemm_rows_pays(args, !b_kcontig, (int)device_limits().cus) &&
-          rows_kernel_wanted(M, N, K, a.dtype, !b_kcontig)) {
+          rows_kernel_wanted(M, N, K, a.dtype, !b_kcontig) && !may_overlap(c, a) && !may_overlap(c, b)) {
         t_last_splits = 4;  // (the four waves of a workgroup)
         t_last_split_launches = 1;
         return hip_status("gemm launch", launch_gemm_rows(args, a.dtype, !b_kcontig, (int)device_limits().cus, stream));
@@ -1043,7 +1085,8 @@ TraceaStatus run_gemm(const View &a, const View &b, const View &c, const Epilogu
     t_last_split_launches = 2;
     return hip_status("split-K reduction launch", launch_splitk_reduce(r, stream));
   }
-  if (!in_padded && ragged_layout(a, b, c) && ragged_kernel_wanted(M, N, K, a.dtype)) {
+  // (an output that is also an operand: the copies below hold what it overwrites)
+  if (!in_padded && ragged_layout(a, b, c) && ragged_kernel_wanted(M, N, K, a.dtype) && !may_overlap(c, a) && !may_overlap(c, b)) {
     ContractionArgs args{};
     int groups = 1;
     const int tile = ragged_tile(M, N, K, &groups);
@@ -1502,7 +1545,7 @@ TraceaStatus dispatch_linear(const TraceaTensorView &ta, const TraceaTensorView 
   GemmBatch batch;
   batch.count = (int)std::min(B, 65536ll);
   batch.a = a.stride[0]; batch.b = shared ? 0 : w.stride[0]; batch.c = c.stride[0];
-  if (B > 1 && gemm_batch_in_one_launch(a2, w2, c2, batch)) return run_gemm(a2, w2, c2, chain, stream, false, batch);
+  if (B > 1 && gemm_batch_in_one_launch(a2, w2, c2, batch) && !may_overlap(c, a) && !may_overlap(c, w)) return run_gemm(a2, w2, c2, chain, stream, false, batch);
   for (long long b = 0; b < B; ++b) {
     View ab = a2, wb = w2, cb = c2;
     ab.ptr = (char *)a.ptr + b * a.stride[0] * elem_size(a.dtype);
@@ -2024,7 +2067,8 @@ TraceaStatus run_conv(const ConvPlan &plan, const EpilogueChain &chain, hipStrea
   // 256->256 6.7 / 4.8, 7x7 512->512 10.2 (two launches) / 7.0, 56x56 64->128 stride 2 7.5 / 4.5, 14x14 256->512 stride 2
   // 8.5 / 4.9; four images 14x14 256->256 8.9 / 6.9, 28x28 128->128 (392 workgroups) 10.7 / 8.6, 7x7 512->512 12.0 / 8.4;
   // sixteen images 7x7 512->512 (400) 16.4 / 15.6; but four images 56x56 64->64 (784) 9.4 / 11.8.
-  if (by_rule) {
+  // (an output that is also the input works where one workgroup reads all of what it overwrites: not on these tiles)
+  if (by_rule && !may_overlap(plan.out, plan.x)) {
     const long long cus = device_limits().cus;
     const ContractionVariant *best = nullptr;
     long long best_tile = 0;
@@ -2404,7 +2448,8 @@ TraceaStatus run_conv_transpose_by_phase(const ConvTransposePlan &plan, const Ep
   const long long w_reach = (C - 1) * w.stride[3] + (R - 1) * w.stride[1] + (S - 1) * w.stride[2] + K;
   const bool in_place = !g_ct_filter_cache.load() && w.stride[0] == 1 && K % 8 == 0 && C % 64 == 0 && aligned(w.ptr, 16) &&
                         w.stride[1] >= 0 && w.stride[2] >= 0 && w.stride[3] > 0 && w.stride[1] % 8 == 0 && w.stride[2] % 8 == 0 &&
-                        w.stride[3] % 8 == 0 && w_reach * 2 < (1ll << 31) && (long long)N * H * W * C * 2 < (1ll << 31);
+                        w.stride[3] % 8 == 0 && w_reach * 2 < (1ll << 31) && (long long)N * H * W * C * 2 < (1ll << 31) &&
+                        !may_overlap(out, w);
   // The regrouped filters live in the per-(device, stream) scratch buffer that split-K launches use
   // (no launch of this path splits K, and work on one stream is ordered); a bank beyond its 64 MiB
   // cap, or a first use while the stream is being captured, takes a stream-ordered allocation.
@@ -2692,6 +2737,8 @@ TraceaStatus dispatch_attention(const TraceaTensorView &tq, const TraceaTensorVi
                   (D % 8 == 0 && scale > 0.0f && (reach * k.stride[2] + D) * 2 < (1ll << 31) && (reach * v.stride[2] + D) * 2 < (1ll << 31));
   // (rows of K and V are reached by unsigned offsets from the slice's first row)
   if (k.stride[2] < 0 || v.stride[2] < 0) in_place = false;
+  // (a result over K or V: the copies hold what it overwrites)
+  if (D != 64 && D != 128 && (may_overlap(o, k) || may_overlap(o, v))) in_place = false;
   for (const View *t : views)
     if (t->stride[3] != 1 || t->stride[2] % 8 != 0 || t->stride[1] % 8 != 0 || t->stride[0] % 8 != 0 || !aligned(t->ptr, 16))
       in_place = false;
