@@ -27,7 +27,7 @@ struct EpilogueChain {
 // Problem description handed to the contraction kernels.  For a convolution
 // the GEMM view is M = batch*h_out*w_out, N = k_out, K = r*s*c_in, A is the
 // NHWC activation tensor and B the filter bank.
-struct ContractionArgs {
+struct ContractionCore {
   const void *A;
   const void *B;
   void *C;
@@ -70,12 +70,6 @@ struct ContractionArgs {
   int phases;
   long long phase_b_stride;
   int phase_pad_h[4], phase_pad_w[4];
-  // b_taps != 0 (N-contiguous B, c_in a multiple of the K tile, below 2 GiB): the filter bank of a transposed
-  // convolution read where it lies.  The filters of tap (r, s) of the phase start (b_rmax - r) * b_tap_r + (s_sz - 1 - s) *
-  // b_tap_s elements behind B, ldb elements from one input channel to the next; phases > 1: phase (o_a, o_b) starts
-  // phase_b_h[o_a] + phase_b_w[o_b] elements behind B (phase_b_stride is not used)
-  int b_taps, b_rmax, b_tap_r, b_tap_s;
-  int phase_b_h[4], phase_b_w[4];
   // patch-resident convolution (pipeline 4) only: filter rows, M tiles per image,
   // padded row width W + 2 pad_w, 16-byte chunks per patch pixel (odd), patch
   // load iterations per thread, LDS bytes reserved for the patch, and the
@@ -97,9 +91,21 @@ struct ContractionArgs {
     long long res_ld;
   } fe;
   EpilogueChain epi;
-  // batch > 1: grid.z = batch products of one shape in one launch (half-precision tiles up to 128x128 and the fp32
-  // kernel on 64x64); product z reads A + z*batch_a and B + z*batch_b (elements) and writes the rows from
-  // z*batch_rows of C on.  Not combined with a tile list or a split that needs the reduction kernel.
+};
+
+// ... and what few launches add: the kernels that do not read it take the block above, whose size and offsets every
+// launch pays for (with these fields in one block 3072x1024x768 11.46 us against 11.26).
+struct ContractionArgs : ContractionCore {
+  // b_taps != 0 (N-contiguous B, c_in a multiple of the K tile, below 2 GiB): the filter bank of a transposed
+  // convolution read where it lies.  The filters of tap (r, s) of the phase start (b_rmax - r) * b_tap_r + (s_sz - 1 - s) *
+  // b_tap_s elements behind B, ldb elements from one input channel to the next; phases > 1: phase (o_a, o_b) starts
+  // phase_b_h[o_a] + phase_b_w[o_b] elements behind B (phase_b_stride is not used)
+  int b_taps, b_rmax, b_tap_r, b_tap_s;
+  int phase_b_h[4], phase_b_w[4];
+  // batch > 1: grid.z = batch products of one shape in one launch (half-precision tiles up to 128x128 on direct-to-LDS
+  // loads, the few-row kernel and the fp32 kernel on 64x64); product z reads A + z*batch_a and B + z*batch_b (elements)
+  // and writes the rows from z*batch_rows of C on.  Not combined with a tile list or a split that needs the reduction
+  // kernel.
   int batch;
   long long batch_a, batch_b, batch_rows;
 };

@@ -390,7 +390,7 @@ __device__ __forceinline__ void apply_epilogue_tab(float (&v)[8], long long m, i
 // the chain is made of bias / scale-shift / BatchNorm / ReLU / one residual.
 // Whether that holds is the same for the whole workgroup, so it is decided
 // once and the row loops are emitted twice, each behind a uniform branch.
-__device__ __forceinline__ bool chain_is_simple(const ChainPlan &plan, const ContractionArgs &args, int n0, int bn) {
+__device__ __forceinline__ bool chain_is_simple(const ChainPlan &plan, const ContractionCore &args, int n0, int bn) {
   bool ok = n0 + bn <= args.N && (args.ldc & 7) == 0 && (((uintptr_t)args.C) & 15) == 0;
 #pragma unroll
   for (int o = 0; o < TRACEA_MAX_EPILOGUE_OPS; ++o) {
@@ -413,7 +413,7 @@ __device__ __forceinline__ bool chain_is_simple(const ChainPlan &plan, const Con
 // row_of(r) gives the output row of staged row r, or -1 if it does not exist.
 // F32OUT: C holds fp32 (two 16-byte stores per lane and row) instead of DT.
 template <int DT, int TN, bool F32OUT = false, typename RowOf>
-__device__ __forceinline__ void simple_rows(const float *stage, int lane, int n, const ContractionArgs &args,
+__device__ __forceinline__ void simple_rows(const float *stage, int lane, int n, const ContractionCore &args,
                                             const ChainPlan &plan, const float *tab, int bn, RowOf row_of) {
   constexpr int EP_PITCH = TN + 4, LPR = TN / 8, RPI = 64 / LPR, NIT = 32 / RPI;
   constexpr int GROUP = NIT < 4 ? NIT : 4;
@@ -511,7 +511,7 @@ __device__ __forceinline__ void simple_rows(const float *stage, int lane, int n,
 // of tile indices, then the run is laid out in column-major groups of
 // `group_m` tile rows, which gives every XCD a compact rectangle of C and
 // therefore a small set of A and B panels to keep in its L2.
-__device__ __forceinline__ void tile_coordinates(const ContractionArgs &a, int &tile_m,
+__device__ __forceinline__ void tile_coordinates(const ContractionCore &a, int &tile_m,
                                                  int &tile_n) {
   int bid = blockIdx.x;
   const int total = a.grid_m * a.grid_n;
@@ -566,8 +566,11 @@ struct Sequenced {
 
 // ---- the kernel -----------------------------------------------------------------
 // MS: the MFMA shape, 32 (v_mfma_f32_32x32x16) or 16 (v_mfma_f32_16x16x32; GEMM on pipeline 2 only).
-template <int DT, int BM, int BN, int BK, int WM, int WN, int NS, int PIPE, int MS, bool CONV, bool B_NCONTIG>
-__global__ void __launch_bounds__(WM *WN * 64) contraction_kernel(const ContractionArgs args) {
+// EXT: what few launches need and the others do not carry.  GEMM: blockIdx.z names one of several products (batch_*; in
+// every kernel these three fields cost 3072x1024x768 11.22 us against 10.95, 1536x1536x2048 23.6 against 23.4).
+// Convolution: a bank in place (b_taps; in every kernel with an N-contiguous B, N8 56x56 128->512 1x1 17.0 against 16.6).
+template <int DT, int BM, int BN, int BK, int WM, int WN, int NS, int PIPE, int MS, bool CONV, bool B_NCONTIG, bool EXT>
+__global__ void __launch_bounds__(WM *WN * 64) contraction_kernel(const std::conditional_t<EXT, ContractionArgs, ContractionCore> args) {
   static_assert(MS == 32 || (MS == 16 && PIPE == 2 && !CONV && BK % 32 == 0), "the 16x16x32 form exists for a GEMM on pipeline 2");
   constexpr int NT = WM * WN * 64;
   constexpr int CH = BK / 8;       // 16-byte pieces per tile row
@@ -594,7 +597,8 @@ __global__ void __launch_bounds__(WM *WN * 64) contraction_kernel(const Contract
   asm volatile("" ::"s"(args.A), "s"(args.B), "s"(args.M), "s"(args.N), "s"(args.K), "s"(args.lda), "s"(args.ldb),
                "s"(args.a_bytes), "s"(args.b_bytes), "s"(args.grid_m), "s"(args.grid_n), "s"(args.k_split),
                "s"(args.fuse_ws), "s"(args.group_m), "s"(args.tile_list), "s"(args.epi.n_ops));
-  constexpr bool BATCHED = !CONV && BM * BN <= 128 * 128;  // blockIdx.z may name one of several products
+  constexpr bool BATCHED = EXT && !CONV, TAPS = EXT && CONV;
+  static_assert(!TAPS || (B_NCONTIG && PIPE >= 2), "a bank is read in place with direct-to-LDS loads");
   if constexpr (BATCHED) asm volatile("" ::"s"(args.batch_a), "s"(args.batch_b), "s"(args.batch_rows));
   if constexpr (CONV && BATCH_ARGS) {
     asm volatile("" ::"s"(args.h_in), "s"(args.w_in), "s"(args.c_in), "s"(args.h_out), "s"(args.w_out), "s"(args.s_sz),
@@ -668,7 +672,7 @@ __global__ void __launch_bounds__(WM *WN * 64) contraction_kernel(const Contract
       // selects, not an index: a run-time index into the kernel arguments can move them to scratch memory
       pad_h = o_a == 0 ? args.phase_pad_h[0] : o_a == 1 ? args.phase_pad_h[1] : o_a == 2 ? args.phase_pad_h[2] : args.phase_pad_h[3];
       pad_w = o_b == 0 ? args.phase_pad_w[0] : o_b == 1 ? args.phase_pad_w[1] : o_b == 2 ? args.phase_pad_w[2] : args.phase_pad_w[3];
-      if (B_NCONTIG && args.b_taps != 0)
+      if constexpr (TAPS)
         Bg += (o_a == 0 ? args.phase_b_h[0] : o_a == 1 ? args.phase_b_h[1] : o_a == 2 ? args.phase_b_h[2] : args.phase_b_h[3]) +
               (o_b == 0 ? args.phase_b_w[0] : o_b == 1 ? args.phase_b_w[1] : o_b == 2 ? args.phase_b_w[2] : args.phase_b_w[3]);
       else
@@ -856,13 +860,11 @@ __global__ void __launch_bounds__(WM *WN * 64) contraction_kernel(const Contract
       dw = sf * args.dil_w;
     }
     int b_soff = (int)((long long)k0 * args.ldb * 2);  // (N-contiguous B)
-    if constexpr (CONV && B_NCONTIG) {
-      if (args.b_taps != 0) {  // the K tile lies in one tap
-        int rf, rem, sf, c0;
-        fast_divmod(k0, args.sc_m, args.sc_s, args.s_sz * args.c_in, rf, rem);
-        fast_divmod(rem, args.c_m, args.c_s, args.c_in, sf, c0);
-        b_soff = ((args.b_rmax - rf) * args.b_tap_r + (args.s_sz - 1 - sf) * args.b_tap_s + c0 * (int)args.ldb) * 2;
-      }
+    if constexpr (TAPS) {  // the K tile lies in one tap (a tile past the end of K in none: its requests are out of range)
+      int rf, rem, sf, c0;
+      fast_divmod(k0, args.sc_m, args.sc_s, args.s_sz * args.c_in, rf, rem);
+      fast_divmod(rem, args.c_m, args.c_s, args.c_in, sf, c0);
+      b_soff = k0 < K ? ((args.b_rmax - rf) * args.b_tap_r + (args.s_sz - 1 - sf) * args.b_tap_s + c0 * (int)args.ldb) * 2 : 0;
     }
 #pragma unroll
     for (int i = 0; i < NA; ++i) {
@@ -1433,7 +1435,8 @@ __global__ void __launch_bounds__(WM *WN * 64) contraction_kernel(const Contract
       const unsigned splits = gridDim.y;
       constexpr unsigned TILE_BYTES = BM * BN * 4, WAVE_BYTES = TM * TN * 4;
       __amdgpu_buffer_rsrc_t rsrc_ws = __builtin_amdgcn_make_buffer_rsrc((void *)args.fuse_ws, 0, 0x7fffffff, 0x00020000);
-      const unsigned tile = BATCHED ? blockIdx.z * gridDim.x + blockIdx.x : blockIdx.x;
+      unsigned tile = blockIdx.x;
+      if constexpr (BATCHED) tile += blockIdx.z * gridDim.x;
       const unsigned first = tile * splits * TILE_BYTES + wave * WAVE_BYTES + lane * 16;
       const unsigned mine = first + blockIdx.y * TILE_BYTES;
 #pragma unroll
@@ -1630,15 +1633,18 @@ template <int BM, int BN, int BK, int WM, int WN, int NS, int PIPE, int MS = 32>
 int launch_contraction(const ContractionArgs &a, bool conv, int dtype, bool b_ncontig,
                        hipStream_t stream) {
   if (MS == 16 && conv) return (int)hipErrorInvalidValue;  // (the dispatcher sends convolutions to the 32x32x16 twin)
+  const bool ext = conv ? a.b_taps != 0 : a.batch > 1;
+  constexpr bool BATCHES = PIPE >= 2 && BM * BN <= 128 * 128, TAPS = PIPE >= 2 && MS == 32;
+  if (ext && !(conv ? TAPS && b_ncontig : BATCHES)) return (int)hipErrorInvalidValue;
   constexpr size_t lds = (size_t)NS * (BM + BN) * BK * 2;
   const bool listed = !conv && a.tile_list != nullptr;  // one workgroup per record, no split grid
   const dim3 grid((unsigned)(listed ? a.tile_count : a.grid_m * a.grid_n),
                   (unsigned)(!listed && a.k_split > 0 ? (a.K + a.k_split - 1) / a.k_split : 1),
                   (unsigned)(conv ? (a.phases > 1 ? a.phases : 1) : (a.batch > 1 ? a.batch : 1))),
       block(WM * WN * 64);
-#define TRACEA_LAUNCH(DTV, CONVV, NCV)                                                       \
+#define TRACEA_LAUNCH(DTV, CONVV, NCV, EXTV)                                                 \
   do {                                                                                       \
-    auto kfn = contraction_kernel<DTV, BM, BN, BK, WM, WN, NS, PIPE, MS, (CONVV) && MS == 32, NCV>; \
+    auto kfn = contraction_kernel<DTV, BM, BN, BK, WM, WN, NS, PIPE, MS, (CONVV) && MS == 32, NCV, EXTV>; \
     static bool attr_done = false;                                                           \
     if (!attr_done) {                                                                        \
       hipError_t e = hipFuncSetAttribute((const void *)kfn,                                  \
@@ -1649,15 +1655,20 @@ int launch_contraction(const ContractionArgs &a, bool conv, int dtype, bool b_nc
     hipLaunchKernelGGL(kfn, grid, block, lds, stream, a);                                    \
     return (int)hipGetLastError();                                                           \
   } while (0)
-  if (dtype == DT_F16) {
-    if (conv) { if (b_ncontig) TRACEA_LAUNCH(DT_F16, true, true); else TRACEA_LAUNCH(DT_F16, true, false); }
-    else      { if (b_ncontig) TRACEA_LAUNCH(DT_F16, false, true); else TRACEA_LAUNCH(DT_F16, false, false); }
-  } else {
-    if (conv) { if (b_ncontig) TRACEA_LAUNCH(DT_BF16, true, true); else TRACEA_LAUNCH(DT_BF16, true, false); }
-    else      { if (b_ncontig) TRACEA_LAUNCH(DT_BF16, false, true); else TRACEA_LAUNCH(DT_BF16, false, false); }
-  }
+#define TRACEA_LAUNCH_FORM(DTV)                                                              \
+  do {                                                                                       \
+    if (conv) {                                                                              \
+      if (!b_ncontig) TRACEA_LAUNCH(DTV, true, false, false);                                \
+      if (ext) TRACEA_LAUNCH(DTV, true, true, TAPS);                                         \
+      TRACEA_LAUNCH(DTV, true, true, false);                                                 \
+    }                                                                                        \
+    if (b_ncontig) { if (ext) TRACEA_LAUNCH(DTV, false, true, BATCHES); else TRACEA_LAUNCH(DTV, false, true, false); } \
+    if (ext) TRACEA_LAUNCH(DTV, false, false, BATCHES); else TRACEA_LAUNCH(DTV, false, false, false); \
+  } while (0)
+  if (dtype == DT_F16) TRACEA_LAUNCH_FORM(DT_F16);
+  TRACEA_LAUNCH_FORM(DT_BF16);
+#undef TRACEA_LAUNCH_FORM
 #undef TRACEA_LAUNCH
-  return (int)hipErrorInvalidValue;
 }
 
 }  // namespace tracea_amd

@@ -34,7 +34,7 @@ constexpr int CK_TABLE_BYTES = TRACEA_MAX_EPILOGUE_OPS * 2 * 64 * 4;
 constexpr int CK_STAGE_BYTES = 64 * 256;  // 64 filters x 128 channels
 
 template <int DT, int CIN, int NPB, int RING>
-__global__ void __launch_bounds__(CK_THREADS) conv_ksplit16_kernel(const ContractionArgs args) {
+__global__ void __launch_bounds__(CK_THREADS) conv_ksplit16_kernel(const ContractionCore args) {
   constexpr int NT = CK_THREADS, BN = 64, NW = NT / 64;
   constexpr int CPT = CIN / 128;  // stages (128-channel chunks) per filter tap
   static_assert(CIN % 256 == 0 && RING >= 3 && NPB >= 1 && NPB <= 8, "unsupported shape");

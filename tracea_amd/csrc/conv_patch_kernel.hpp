@@ -24,7 +24,7 @@
 namespace tracea_amd {
 
 template <int DT, int TM, int BN, int WM, int WN, int NSB, bool FULL>
-__global__ void __launch_bounds__(WM *WN * 64) conv_patch_kernel(const ContractionArgs args) {
+__global__ void __launch_bounds__(WM *WN * 64) conv_patch_kernel(const ContractionCore args) {
   constexpr int NT = WM * WN * 64;
   constexpr int BK = 64, CH = 8, ROW_BYTES = 128, RP = 2;  // filter tile: BN rows x 64 k, XOR-swizzled
   constexpr int TMW = TM / WM, TN = BN / WN, FM = TMW / 32, FN = TN / 32;

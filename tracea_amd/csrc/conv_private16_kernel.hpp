@@ -22,7 +22,7 @@ namespace tracea_amd {
 // GEN: any multiple of 8 channels.  A 16-byte column of a piece still lies inside one tap, but the columns of a piece lie in
 // several: tap and channel are worked out per lane, once for each of the two columns its rows are swizzled to.
 template <int DT, int WAVES, int XR, int NB, int DEPTH, bool GEN>
-__global__ void __launch_bounds__(WAVES * 64) conv_private16_kernel(const ContractionArgs args) {
+__global__ void __launch_bounds__(WAVES * 64) conv_private16_kernel(const ContractionCore args) {
   constexpr int BM = 8 * XR, BN = 16 * NB, MB = XR / 2, NT = WAVES * 64;
   constexpr int BR = 2 * NB, REQS = BR + XR, STAGE = REQS * 1024;
   constexpr int NBLK = (MB * NB + WAVES - 1) / WAVES;  // blocks of the output a wave finishes

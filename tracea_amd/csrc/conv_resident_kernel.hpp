@@ -49,7 +49,7 @@ constexpr int RS_TABLE_BYTES = TRACEA_MAX_EPILOGUE_OPS * 2 * 64 * 4;
 
 // KS: 16-wide k-steps (K / 16); KPT: k-steps per filter tap (C / 16).
 template <int DT, int KS, int KPT>
-__global__ void __launch_bounds__(RS_THREADS) conv_resident_kernel(const ContractionArgs args) {
+__global__ void __launch_bounds__(RS_THREADS) conv_resident_kernel(const ContractionCore args) {
   constexpr int NT = RS_THREADS, BN = 64, NW = NT / 64;
   constexpr int CPB = rs_cpb(KS), FIT = rs_filter_iters(KS);
 

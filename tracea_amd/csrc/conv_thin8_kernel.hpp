@@ -44,7 +44,7 @@ __host__ __device__ constexpr int ct_aux_bytes(int r, int p_tm, int patch_bytes)
 }
 
 template <int DT, int R>
-__global__ void __launch_bounds__(CT_THREADS) conv_thin8_kernel(const ContractionArgs args) {
+__global__ void __launch_bounds__(CT_THREADS) conv_thin8_kernel(const ContractionCore args) {
   constexpr int NT = CT_THREADS, BN = 64, NW = NT / 64, C = 8, PBW = 2, STEPS = 2 * R;
   asm volatile("" ::"s"(args.A), "s"(args.B), "s"(args.N), "s"(args.ldb), "s"(args.b_bytes), "s"(args.grid_n), "s"(args.h_in),
                "s"(args.w_in), "s"(args.h_out), "s"(args.w_out), "s"(args.s_sz), "s"(args.stride_h), "s"(args.stride_w));

@@ -51,7 +51,7 @@ constexpr int cw_ring_stage_bytes(int cin) { return cw_ring_iters(cin) * 256 * 1
 inline int cw_resident_filter_bytes(int k) { return 64 * k * 2; }
 
 template <int DT, int CIN, int PBW, int RING, int WK = 4>
-__global__ void __launch_bounds__(CW_THREADS) conv_wave16_kernel(const ContractionArgs args) {
+__global__ void __launch_bounds__(CW_THREADS) conv_wave16_kernel(const ContractionCore args) {
   static_assert(WK == 4 || (WK == 8 && RING == 0), "eight multiplying waves only with the resident filter slab");
   static_assert(RING != 0 || CIN == 64, "the resident slab's layout: one load instruction per thread and tap");
   constexpr int NT = CW_THREADS, BN = 64, NW = NT / 64;

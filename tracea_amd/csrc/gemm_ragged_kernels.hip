@@ -43,7 +43,7 @@ constexpr int ragged_group_bytes(int t) { return t * (t + 4) * 4 > t * 512 ? t *
 
 // T: rows and columns of the tile; WN: waves side by side (two rows of them); KN: B by rows (else by columns)
 template <int DT, int T, int WN, int GROUPS, int DEPTH, bool KN>
-__global__ void __launch_bounds__(GROUPS * WN * 128) gemm_ragged_kernel(const ContractionArgs args) {
+__global__ void __launch_bounds__(GROUPS * WN * 128) gemm_ragged_kernel(const ContractionCore args) {
   constexpr int GT = WN * 128;                // threads of a group
   constexpr int NP = T * 8 / GT;              // 16-byte pieces per thread, operand and K tile of 64
   constexpr int OPERAND = T * 128, STAGE = 2 * OPERAND;

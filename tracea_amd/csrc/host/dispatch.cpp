@@ -469,9 +469,9 @@ inline bool conv_only(const ContractionVariant &v) { return v.pipeline >= 4; }
 
 constexpr int kOneLaunchMaxSplits = 4;  // finest split that runs as one launch (see launch_maybe_split)
 
-// The members that run several products of one shape in one launch (ContractionArgs::batch): the small tiles.  A
-// product that fills the device with 256x256 tiles has nothing to gain from company.
-inline bool takes_batches(const ContractionVariant &v) { return !conv_only(v) && v.bm * v.bn <= 128 * 128; }
+// The members that run several products of one shape in one launch (ContractionArgs::batch): the small tiles on
+// direct-to-LDS loads.  A product that fills the device with 256x256 tiles has nothing to gain from company.
+inline bool takes_batches(const ContractionVariant &v) { return !conv_only(v) && v.pipeline >= 2 && v.bm * v.bn <= 128 * 128; }
 
 int choose_split(const ContractionVariant &v, int M, int N, int K, int *k_split, int min_tiles = 4, int batch = 1) {
   const long long tiles = (long long)((M + v.bm - 1) / v.bm) * ((N + v.bn - 1) / v.bn) * batch;

@@ -28,7 +28,7 @@ constexpr int F32_BM = 128, F32_BN = 128, F32_BK = 16, F32_PITCH = 132;
 // scratch memory (488 bytes per lane) and kept 192 registers: 1024^3 took 46.6 us that way and
 // 32.9 us this way (128x128 tiles), 4096^3 1194 -> 979 us.
 template <int ROWS, int FM, int FN>
-__device__ __forceinline__ void f32_tile_epilogue(const f32x16 (&acc)[FM][FN], float *stage, const ContractionArgs &args,
+__device__ __forceinline__ void f32_tile_epilogue(const f32x16 (&acc)[FM][FN], float *stage, const ContractionCore &args,
                                                   int m_wave, int n_wave, long long zrow, int lane) {
   static_assert(ROWS == 32 || ROWS == 16, "a 32-row block is staged whole or in two halves");
   constexpr int W = 32 * FN, CH = 8 * FN;  // floats and 16-byte chunks per staged row
@@ -66,7 +66,7 @@ __device__ __forceinline__ void f32_tile_epilogue(const f32x16 (&acc)[FM][FN], f
   });
 }
 
-__global__ void __launch_bounds__(256) gemm_f32_kernel(const ContractionArgs args) {
+__global__ void __launch_bounds__(256) gemm_f32_kernel(const ContractionCore args) {
   __shared__ float As[F32_BK][F32_PITCH];
   __shared__ float Bs[F32_BK][F32_PITCH];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -187,7 +187,7 @@ __global__ void __launch_bounds__(256) gemm_f32_kernel(const ContractionArgs arg
 // of 256 and more of a single product on these tiles do: 34 products of 2x72x1024 were off by 2.4e-7 in one chain,
 // 2.1e-7 launched one by one and here.  (On 64x64 tiles only: the larger ones have no registers for the handed-over sums.)
 template <int TM, int TN, int STAGES, int KSUB, bool BATCH, int FIRST_T = 1>
-__global__ void __launch_bounds__(256) gemm_f32_dma_kernel(const ContractionArgs args) {
+__global__ void __launch_bounds__(256) gemm_f32_dma_kernel(const std::conditional_t<BATCH, ContractionArgs, ContractionCore> args) {
   constexpr int BM = 64 * TM, BN = 64 * TN, BK = F32_BK * KSUB;  // a stage holds KSUB sub-tiles of 16 k, each [A][B]
   constexpr int A_STAGE = BM * F32_BK * 4, B_STAGE = F32_BK * BN * 4, SUB = A_STAGE + B_STAGE, STAGE = KSUB * SUB;
   constexpr int B_PITCH = BN * 4, B_PIECES = BN / 4;  // bytes and 16-byte pieces per k row of B
