@@ -399,7 +399,7 @@ def test_operands_at_any_element_alignment(tracea_gpu, dtype, shape):
             for tag, db in (("row-major B", placed(b, gap, first, junk)), ("column-major B", placed(b.T, gap, first, junk).t())):
                 out = torch.full((m + 1, n + 3), 7.0, device="cuda", dtype=tdt)
                 tracea_gpu.gemm(da, db, bias=_dev(bias), epilogue="bias+relu", out=out[:m, :n])
-                assert capi.last_variant("gemm") in ("t64x64x64_w2x2", "t128x128x64_w2x2"), "ran from copies"
+                assert capi.last_variant("gemm").endswith("_any"), "ran from copies"
                 got = out.float().cpu().numpy()
                 assert_close_scaled(got[:m, :n], ref, tol_half(k, dtype), "%s gap %d first %d" % (tag, gap, first))
                 assert (got[m] == 7.0).all() and (got[:, n:] == 7.0).all(), "outside the output"

@@ -166,3 +166,44 @@ def test_tuner_cli_writes_the_reference_record(tracea_gpu, cache_file, tmp_path)
     assert r.returncode == 0, r.stderr
     rec = json.loads(out.read_text())
     assert rec["kernel"] == "attention" and rec["problem"]["causal"] is True
+
+
+def test_a_record_speaks_for_the_kernels_it_was_measured_against(tracea_gpu, cache_file):
+    """The kernel for a few rows is a candidate of every search, so a tuned call runs the winner over all; a record that was
+    not measured against it (older ones, planted ones) does not displace it, nor does a record of the single product
+    decide a batch in one launch, nor one of the padded copies' product a ragged call that needs no copies."""
+    from tracea_amd import capi, tuner as T
+    names = capi.variants("gemm")
+    key = "gemm_16_512_512_%s" % _device_name()
+    a, b = torch.randn(16, 512, device="cuda").half(), torch.randn(512, 512, device="cuda").half().t()
+
+    def ran():
+        tracea_gpu.gemm(a, b)
+        return capi.last_variant("gemm")
+
+    for tune in (lambda: json.loads(capi.take_result(capi.lib().tracea_tune_gemm(16, 512, 512))[2]),
+                 lambda: T.autotune_gemm(16, 512, 512, iterations=0)[0]):
+        cfg = tune()
+        assert json.loads(cache_file.read_text())[key]["few_rows_measured"] == 1
+        assert ran() == names[T.variant_for_config(cfg)]
+        T.cache_reload()                                    # as a later process reads it
+        assert ran() == names[T.variant_for_config(cfg)]
+        cache_file.unlink()
+        T.cache_reload()
+
+    tile = [c for c in T.propose_gemm_configs(16, 512, 512) if c["m_tile"] == 64][0]
+    tile_name = names[T.variant_for_config(tile)]
+
+    def plant(key, **tags):
+        cache_file.write_text(json.dumps({key: dict(config=tile, score=1.0, timestamp=1, **tags)}))
+        T.cache_reload()
+
+    plant(key)
+    assert ran().endswith("_rows")
+    plant(key, few_rows_measured=1)
+    assert ran() == tile_name
+    tracea_gpu.linear(a.expand(3, 16, 512), torch.randn(3, 512, 512, device="cuda").half().transpose(1, 2))
+    assert capi.last_variant("gemm").endswith("_rows")
+    plant("gemm_100_90_1056_%s" % _device_name())
+    tracea_gpu.gemm(torch.randn(100, 1030, device="cuda").half(), torch.randn(1030, 90, device="cuda").half())
+    assert capi.last_variant("gemm").endswith("_any")

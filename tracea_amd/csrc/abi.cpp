@@ -195,7 +195,7 @@ int32_t tracea_select_variant(const char *op, int64_t m, int64_t n, int64_t k) {
     return -1;
   const bool conv = !strcmp(op, "conv2d");
   if (!conv && strcmp(op, "gemm") != 0) return -1;
-  return select_contraction_variant((int)m, (int)n, (int)k, conv);
+  return conv ? select_contraction_variant((int)m, (int)n, (int)k, true) : select_gemm_variant((int)m, (int)n, (int)k);
 }
 
 TraceaStatus tracea_conv_params_pack(int32_t n, int32_t h, int32_t w, int32_t c, int32_t k,

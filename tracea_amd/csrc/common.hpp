@@ -134,6 +134,8 @@ struct ContractionVariant {
                  // (the build's mode 6 is pipeline 2 with mfma = 16)
                  // 5: convolution only: input patch and filter bank both resident in LDS
                  //    (conv_resident_kernel.hpp); bm = most pixels per workgroup, K = 16 * stages exactly
+                 // 7 to 11: convolution only (contraction_variants.def)
+                 // 12, 13 (kPipelineRows, kPipelineAny): GEMM only, the kernels of launch_gemm_rows and launch_gemm_ragged
   size_t lds_bytes;
   // launch: returns hipError_t as int
   int (*launch)(const ContractionArgs &, bool conv, int dtype, bool b_ncontig, hipStream_t);
@@ -142,6 +144,7 @@ struct ContractionVariant {
 
 int contraction_variant_count();
 const ContractionVariant &contraction_variant(int i);
+constexpr int kPipelineRows = 12, kPipelineAny = 13;
 
 // Half-precision GEMM of at most kGemmRowsMax rows (operands below 2 GiB, a_bytes / b_bytes
 // set); takes a batch.

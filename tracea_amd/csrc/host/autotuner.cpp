@@ -66,7 +66,7 @@ std::vector<PipelineConfig> propose_contraction(uint32_t m, uint32_t n, uint32_t
     if (i == pick) continue;
     const ContractionVariant &v = contraction_variant(i);
     if (v.lds_bytes > hw.shared_memory_per_block) continue;
-    if (v.pipeline >= 4 && !conv) continue;  // patch-resident kernels compute convolutions only
+    if (v.pipeline >= 4 && v.pipeline < kPipelineRows && !conv) continue;  // patch-resident kernels compute convolutions only
     out.push_back(config_for_contraction_variant(i));
   }
   return out;
@@ -141,6 +141,7 @@ PipelineConfig AutoTuner::optimize_v2(const std::string &key, const std::vector<
   e.timestamp = (uint64_t)std::chrono::duration_cast<std::chrono::seconds>(
                     std::chrono::system_clock::now().time_since_epoch())
                     .count();
+  e.few_rows_measured = few_rows_measured;
   tuning_cache_put(key, e, true);
   has_best = true;
   best_config = best;

@@ -879,15 +879,6 @@ bool gemm_batch_in_one_launch(const View &a, const View &b, const View &c, const
   return true;
 }
 
-// The kernel for products of a few rows splits K over the waves of a workgroup, so the switches of the split along K
-// hold for it too; a forced variant or a tuning-cache record of the problem wins over it, as over every rule.
-bool rows_kernel_wanted(long long M, long long N, long long K, int dtype, bool b_ncontig) {
-  if (!g_split_k_enabled.load() || !g_split_k_one_launch.load() || forced_variant("gemm") >= 0) return false;
-  char key[160];
-  snprintf(key, sizeof(key), "gemm_%lld_%lld_%lld_%s", M, N, K, tuning_device_name());
-  return tuning_cache_lookup_variant(key, dtype, b_ncontig) < 0;
-}
-
 // What the kernel for operands at any element alignment reads in place: rows that do not overlap, of A along K and of B
 // along N or K, extents that hold a 16-byte piece and stay below 2 GiB.
 bool ragged_layout(const View &a, const View &b, const View &c) {
@@ -901,15 +892,6 @@ bool ragged_layout(const View &a, const View &b, const View &c) {
   const long long a_extent = (M - 1) * a.stride[0] + K;
   const long long b_extent = kn ? (K - 1) * b.stride[0] + N : (N - 1) * b.stride[1] + K;
   return a_extent >= 8 && a_extent < cap && b_extent >= 8 && b_extent < cap;
-}
-
-// As for products of a few rows, a forced variant or a tuning record wins over the rule (the record of the padded
-// problem, which is what those run).
-bool ragged_kernel_wanted(long long M, long long N, long long K, int dtype) {
-  if (forced_variant("gemm") >= 0) return false;
-  char key[160];
-  snprintf(key, sizeof(key), "gemm_%lld_%lld_%lld_%s", M, N, (K + 31) / 32 * 32, tuning_device_name());
-  return tuning_cache_lookup_variant(key, dtype, false) < 0;
 }
 
 // Its tile and the groups of waves that share K, or 0 where padded copies and the tile kernels are ahead.  f16, us,
@@ -937,6 +919,33 @@ int variant_index(const char *name) {
   return -1;
 }
 
+// The member of a GEMM kernel outside the tile family (its first one, or the one on tiles of `tile` rows).
+int other_gemm_member(int pipeline, int tile = 0) {
+  for (int i = contraction_variant_count() - 1; i >= 0; --i)
+    if (contraction_variant(i).pipeline == pipeline && (tile == 0 || contraction_variant(i).bm == tile)) return i;
+  return -1;
+}
+
+TraceaStatus run_gemm_any_alignment(const View &a, const View &b, const View &c, const EpilogueChain &chain, int tile, int groups, hipStream_t stream) {
+  const long long M = a.shape[0], K = a.shape[1], N = b.shape[1];
+  const bool b_ncontig = b.stride[1] == 1 && b.stride[0] >= N;
+  ContractionArgs args{};
+  args.A = a.ptr; args.B = b.ptr; args.C = c.ptr;
+  args.M = (int)M; args.N = (int)N; args.K = (int)K;
+  args.lda = a.stride[0]; args.ldb = b_ncontig ? b.stride[0] : b.stride[1]; args.ldc = c.stride[0];
+  args.out_dtype = c.dtype;
+  args.epi = chain;
+  args.a_bytes = (unsigned)(((M - 1) * args.lda + K) * 2);
+  args.b_bytes = (unsigned)((b_ncontig ? (K - 1) * args.ldb + N : (N - 1) * args.ldb + K) * 2);
+  static const int member64 = other_gemm_member(kPipelineAny, 64), member128 = other_gemm_member(kPipelineAny, 128);
+  const int vi = tile == 64 ? member64 : member128;
+  fill_grid(&args, contraction_variant(vi));
+  t_last_contraction = vi;
+  t_last_splits = groups;
+  t_last_split_launches = 1;
+  return hip_status("gemm launch", launch_gemm_ragged(args, a.dtype, b_ncontig, tile, groups, stream));
+}
+
 TraceaStatus run_gemm(const View &a, const View &b, const View &c, const EpilogueChain &chain,
                       hipStream_t stream, bool static_only = false, const GemmBatch &batch = GemmBatch()) {
   static thread_local bool in_padded = false;  // this call multiplies padded copies of another call's operands
@@ -946,6 +955,10 @@ TraceaStatus run_gemm(const View &a, const View &b, const View &c, const Epilogu
   DeviceScope scope(c.device);
   if (scope.err != hipSuccess) return hip_status("hipSetDevice", (int)scope.err);
 
+  // (a forced variant wins over every rule; the kernel for any alignment takes whole 16-byte pieces as well)
+  const int forced = forced_variant("gemm"), forced_pipeline = forced >= 0 ? contraction_variant(forced).pipeline : -1;
+  if (forced_pipeline == kPipelineAny && batch.count == 1 && ragged_layout(a, b, c) && !may_overlap(c, a) && !may_overlap(c, b))
+    return run_gemm_any_alignment(a, b, c, chain, contraction_variant(forced).bm, 1, stream);
   {
     const HalfLayout half = half_layout(a, b, c);
     const bool b_kcontig = half.b_kcontig;
@@ -968,22 +981,31 @@ TraceaStatus run_gemm(const View &a, const View &b, const View &c, const Epilogu
         args.batch = batch.count;
         args.batch_a = batch.a; args.batch_b = batch.b; args.batch_rows = batch.c / c.stride[0];
       }
-      // (an output that is also an operand works where one workgroup reads all of what it overwrites: not on these tiles)
-      if (M <= kGemmRowsMax && small && !in_padded && gemm_rows_pays(args, !b_kcontig, (int)device_limits().cus) &&
-          rows_kernel_wanted(M, N, K, a.dtype, !b_kcontig) && !may_overlap(c, a) && !may_overlap(c, b)) {
-        t_last_splits = 4;  // (the four waves of a workgroup)
-        t_last_split_launches = 1;
-        return hip_status("gemm launch", launch_gemm_rows(args, a.dtype, !b_kcontig, (int)device_limits().cus, stream));
-      }
-      int vi;
-      if (batch.count > 1) {
-        vi = forced_variant("gemm");
-        if (vi < 0) vi = select_contraction_variant((int)M, (int)N, (int)K, false, !b_kcontig, batch.count);
-      } else {
+      // a forced variant, else the tuner's record of the problem (a batch in one launch is another one: no record)
+      int vi = forced;
+      bool rows_measured = false;
+      if (vi < 0 && batch.count == 1) {
         char key[160];
         snprintf(key, sizeof(key), "gemm_%lld_%lld_%lld_%s", M, N, K, tuning_device_name());
-        vi = pick_contraction("gemm", key, (int)M, (int)N, (int)K, false, a.dtype, !b_kcontig);
+        vi = tuning_cache_lookup_variant(key, a.dtype, !b_kcontig, &rows_measured);
+        if (vi >= 0 && contraction_variant(vi).pipeline == kPipelineAny && ragged_layout(a, b, c) && !may_overlap(c, a) && !may_overlap(c, b))
+          return run_gemm_any_alignment(a, b, c, chain, contraction_variant(vi).bm, 1, stream);
       }
+      // A few rows: splits K over the waves of a workgroup, so the switches of the split along K hold for it too.  An
+      // output that is also an operand works where one workgroup reads all of what it overwrites: not on these tiles.
+      if (M <= kGemmRowsMax && small && !in_padded && g_split_k_enabled.load() && g_split_k_one_launch.load()) {
+        static const int rows = other_gemm_member(kPipelineRows);
+        const bool by_rule = forced < 0 && (vi < 0 || !rows_measured) && gemm_rows_pays(args, !b_kcontig, (int)device_limits().cus);
+        if ((vi == rows || by_rule) && !may_overlap(c, a) && !may_overlap(c, b)) {
+          t_last_contraction = rows;
+          t_last_splits = 4;  // (the four waves of a workgroup)
+          t_last_split_launches = 1;
+          return hip_status("gemm launch", launch_gemm_rows(args, a.dtype, !b_kcontig, (int)device_limits().cus, stream));
+        }
+      }
+      // (a record of one of the two that cannot run the call: by rule)
+      if (forced < 0 && vi >= 0 && contraction_variant(vi).pipeline >= kPipelineRows) vi = -1;
+      if (vi < 0) vi = select_contraction_variant((int)M, (int)N, (int)K, false, !b_kcontig, batch.count);
       if (vi < 0) return fail(TRACEA_UNKNOWN_ERROR, "gemm: no kernel variant available");
       vi = resolve_variant(vi, false, !small, K % contraction_variant(vi).bk == 0, !b_kcontig);
       const ContractionVariant &v = contraction_variant(vi);
@@ -1086,28 +1108,11 @@ TraceaStatus run_gemm(const View &a, const View &b, const View &c, const Epilogu
     return hip_status("split-K reduction launch", launch_splitk_reduce(r, stream));
   }
   // (an output that is also an operand: the copies below hold what it overwrites)
-  if (!in_padded && ragged_layout(a, b, c) && ragged_kernel_wanted(M, N, K, a.dtype) && !may_overlap(c, a) && !may_overlap(c, b)) {
-    ContractionArgs args{};
+  // (a record of the padded copies' product says nothing about this road: it holds where the copies are taken)
+  if (!in_padded && forced < 0 && ragged_layout(a, b, c) && !may_overlap(c, a) && !may_overlap(c, b)) {
     int groups = 1;
     const int tile = ragged_tile(M, N, K, &groups);
-    if (tile != 0) {
-      const bool b_ncontig = b.stride[1] == 1 && b.stride[0] >= N;
-      args.A = a.ptr; args.B = b.ptr; args.C = c.ptr;
-      args.M = (int)M; args.N = (int)N; args.K = (int)K;
-      args.lda = a.stride[0]; args.ldb = b_ncontig ? b.stride[0] : b.stride[1]; args.ldc = c.stride[0];
-      args.out_dtype = c.dtype;
-      args.epi = chain;
-      args.a_bytes = (unsigned)(((M - 1) * args.lda + K) * 2);
-      args.b_bytes = (unsigned)((b_ncontig ? (K - 1) * args.ldb + N : (N - 1) * args.ldb + K) * 2);
-      // (reported as the member on the same tiles that stages them through registers too)
-      static const int staged = variant_index("t64x64x64_w2x2"), staged128 = variant_index("t128x128x64_w2x2");
-      const int vi = tile == 64 ? staged : staged128;
-      fill_grid(&args, contraction_variant(vi));
-      t_last_contraction = vi;
-      t_last_splits = groups;
-      t_last_split_launches = 1;
-      return hip_status("gemm launch", launch_gemm_ragged(args, a.dtype, b_ncontig, tile, groups, stream));
-    }
+    if (tile != 0) return run_gemm_any_alignment(a, b, c, chain, tile, groups, stream);
   }
   // Operands none of these kernels reads in place -- fp32 with a K that is not a whole number of 16-byte pieces or rows
   // that do not start on 16 bytes, strides along K, and half precision where ragged_tile says so -- are copied once into
@@ -1153,6 +1158,19 @@ TraceaStatus run_gemm(const View &a, const View &b, const View &c, const Epilogu
   g.epi = chain;
   return hip_status("gemm_generic launch", launch_gemm_generic(g, stream));
 }
+
+}  // namespace
+
+int select_gemm_variant(int m, int n, int k) {
+  ContractionArgs args{};
+  args.M = m; args.N = n; args.K = k;
+  if (m <= kGemmRowsMax && k % 8 == 0 && (long long)n * k < (1ll << 30) && g_split_k_enabled.load() && g_split_k_one_launch.load() &&
+      gemm_rows_pays(args, false, (int)device_limits().cus))
+    return other_gemm_member(kPipelineRows);
+  return select_contraction_variant(m, n, k, false);
+}
+
+namespace {
 
 TraceaStatus gemm_common(const TraceaTensorView &ta, const TraceaTensorView &tb,
                          TraceaTensorView *tc, View *a, View *b, View *c) {

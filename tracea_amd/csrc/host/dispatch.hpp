@@ -116,6 +116,8 @@ TraceaStatus dispatch_clock_probe(void *out, int32_t samples, int32_t gap, void 
 // Heuristic choice among the feasible contraction variants (used when neither a
 // forced variant nor a tuning-cache entry decides).  Returns -1 if none fits.
 int select_contraction_variant(int m, int n, int k, bool conv, bool b_ncontig = false, int batch = 1);
+// ... and for a half-precision product with a K-contiguous B, the kernel for a few rows among the choices.
+int select_gemm_variant(int m, int n, int k);
 
 // TraceaResult builders: strings are malloc'ed, released by tracea_free_string.
 struct PipelineConfig;

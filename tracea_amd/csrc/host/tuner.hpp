@@ -182,6 +182,7 @@ class AutoTuner {
   float best_score = 0.0f;
   std::string hardware_id;
   TuningStats stats;
+  bool few_rows_measured = false;  // set by the measuring function, kept in the record (CacheEntry)
 
   explicit AutoTuner(const HardwareProfile &profile);
 

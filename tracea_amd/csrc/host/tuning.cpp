@@ -52,6 +52,7 @@ void load_locked() {
     if (const Json *t = kv.second.find("timestamp")) e.timestamp = (uint64_t)t->num;
     if (const Json *t = kv.second.find("operand_dtype")) e.operand_dtype = t->str;
     if (const Json *t = kv.second.find("b_layout")) e.b_layout = t->str;
+    if (const Json *t = kv.second.find("few_rows_measured")) e.few_rows_measured = t->num != 0;
     g_cache[kv.first] = e;
   }
 }
@@ -68,6 +69,7 @@ void save_locked() {
     e.set("timestamp", Json::make_num((double)kv.second.timestamp));
     if (!kv.second.operand_dtype.empty()) e.set("operand_dtype", Json::make_str(kv.second.operand_dtype));
     if (!kv.second.b_layout.empty()) e.set("b_layout", Json::make_str(kv.second.b_layout));
+    if (kv.second.few_rows_measured) e.set("few_rows_measured", Json::make_num(1));
     root.set(kv.first, e);
   }
   std::ofstream f(path);
@@ -185,9 +187,10 @@ void tuning_history_reload() {
   g_hist_loaded = false;
 }
 
-int tuning_cache_lookup_variant(const std::string &key, int dtype, bool b_ncontig) {
+int tuning_cache_lookup_variant(const std::string &key, int dtype, bool b_ncontig, bool *few_rows_measured) {
   CacheEntry e;
   if (!tuning_cache_get(key, &e) || !e.matches(dtype, b_ncontig)) return -1;
+  if (few_rows_measured != nullptr) *few_rows_measured = e.few_rows_measured;
   return contraction_variant_for_config(e.config);
 }
 
@@ -487,15 +490,16 @@ TraceaResult tune_gemm(size_t m, size_t n, size_t k) {
   if (!bench.init(m, n, k)) return failure("tune_gemm: " + bench.error);
   int best = -1;
   float best_tflops = 0.0f;
+  CacheEntry e;
   for (int i = 0; i < contraction_variant_count(); ++i) {
     const float tf = bench.measure(i);
+    if (tf > 0.0f && contraction_variant(i).pipeline == kPipelineRows) e.few_rows_measured = true;
     if (tf > best_tflops) {
       best_tflops = tf;
       best = i;
     }
   }
   if (best < 0) return failure("tune_gemm: no variant ran: " + bench.error);
-  CacheEntry e;
   e.config = config_for_contraction_variant(best);
   e.score = best_tflops;
   e.timestamp = now_seconds();
@@ -546,6 +550,7 @@ TraceaResult autotune_gemm(size_t m, size_t n, size_t k, uint32_t iterations) {
   if (!gemm_dims_ok(m, n, k)) return failure("autotune_gemm: dimensions must be positive, K a multiple of 8");
   GemmBenchmark bench;
   bool ready = false;
+  AutoTuner tuner(HardwareProfile::mi355x());
   auto measure = [&](const PipelineConfig &cfg) -> float {
     const int vi = contraction_variant_for_config(cfg);
     if (vi < 0) return 0.0f;
@@ -553,9 +558,10 @@ TraceaResult autotune_gemm(size_t m, size_t n, size_t k, uint32_t iterations) {
       if (!bench.init(m, n, k)) return 0.0f;
       ready = true;
     }
-    return bench.measure(vi);
+    const float tf = bench.measure(vi);
+    if (tf > 0.0f && contraction_variant(vi).pipeline == kPipelineRows) tuner.few_rows_measured = true;
+    return tf;
   };
-  AutoTuner tuner(HardwareProfile::mi355x());
   tuner.hardware_id = tuning_device_name();
   PipelineConfig best;
   if (iterations == 0) {
@@ -572,6 +578,7 @@ TraceaResult autotune_gemm(size_t m, size_t n, size_t k, uint32_t iterations) {
       e.config = best;
       e.score = tuner.best_score;
       e.timestamp = now_seconds();
+      e.few_rows_measured = tuner.few_rows_measured;
       tuning_cache_put(key, e, true);
     }
   }

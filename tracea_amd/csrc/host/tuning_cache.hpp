@@ -20,6 +20,9 @@ struct CacheEntry {
   // f16 with a K-contiguous B, which is what every tuner of this path measures.
   std::string operand_dtype;  // "f16" | "bf16"
   std::string b_layout;       // "k_contiguous" | "n_contiguous"
+  // The kernel for products of a few rows took part in the measurement.  Records from before it was a candidate, and
+  // budgeted searches that did not reach it, cannot speak against it: where the rule takes it they do not count.
+  bool few_rows_measured = false;
   bool matches(int dtype, bool b_ncontig) const {
     const std::string d = operand_dtype.empty() ? "f16" : operand_dtype;
     const std::string l = b_layout.empty() ? "k_contiguous" : b_layout;
@@ -55,7 +58,8 @@ void tuning_history_reload();
 
 // Index of the contraction variant a cached config names, or -1; a record measured on other operands
 // (element type, layout of B) than the caller's does not count.
-int tuning_cache_lookup_variant(const std::string &key, int dtype = DT_F16, bool b_ncontig = false);
+// `few_rows_measured`, if given, receives the record's field of that name.
+int tuning_cache_lookup_variant(const std::string &key, int dtype = DT_F16, bool b_ncontig = false, bool *few_rows_measured = nullptr);
 
 // PipelineConfig <-> kernel variant
 PipelineConfig config_for_contraction_variant(int index);
