@@ -305,7 +305,10 @@ TraceaStatus tracea_linear(TraceaTensorView a, TraceaTensorView w, const TraceaT
  * over more workgroups; fp32 partial products go to a
  * scratch buffer the library keeps per (device, stream) (grown on demand up to 64 MiB, never
  * while the stream is being captured, never freed) and a second kernel sums them and applies
- * the operator chain.  On by default; tracea_set_split_k(0) turns it off.
+ * the operator chain.  The kernels for products of a few rows, for GEMM operands at any alignment and for
+ * convolutions of a few output pixels split K over the waves of a workgroup instead, without a workspace.
+ * On by default; tracea_set_split_k(0) turns all of it off (the patch-in-LDS convolutions of the 14x14 and 7x7
+ * stages, whose waves divide K by design, remain).
  * tracea_last_split_k: K ranges of the calling thread's latest gemm / conv2d launch (1: not split).
  * Half-precision launches on tiles up to 128x128 and fp32 launches that are split at most four ways need no second kernel: every workgroup leaves its partial
  * product in the scratch buffer and takes a ticket from a per-tile counter (4 bytes per tile, per (device,

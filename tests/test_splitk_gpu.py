@@ -260,3 +260,25 @@ def test_fp32_gemm_split_matches_float64(tracea_gpu, split_switch, shape):
     assert capi.lib().tracea_last_split_k() >= 2
     assert got.dtype == torch.float32
     np.testing.assert_allclose(got.cpu().numpy(), want, rtol=0, atol=1e-4 * np.sqrt(k))
+
+
+def test_the_switch_reaches_the_splits_over_waves(tracea_gpu, split_switch):
+    """K split over the waves of a workgroup: a few rows, operands at any alignment, a convolution of a few pixels."""
+    capi = split_switch
+    rng = np.random.default_rng(8)
+
+    def half(*shape, scale=1.0):
+        return _dev(round_f16(rng.standard_normal(shape) * scale), torch.float16)
+    rows, wide = half(16, 1024, scale=1 / 32), half(1024, 512)
+    ragged, odd = half(70, 1001, scale=1 / 32), half(1001, 90)
+    x, w = half(1, 28, 28, 128), half(128, 3, 3, 128, scale=1 / 34)
+    for op, call in (("gemm", lambda: tracea_gpu.gemm(rows, wide)), ("gemm", lambda: tracea_gpu.gemm(ragged, odd)),
+                     ("conv2d", lambda: tracea_gpu.conv2d(x, w, padding=1))):
+        split = call()
+        assert capi.lib().tracea_last_split_k() >= 2 and capi.lib().tracea_last_split_k_launches() == 1
+        name = capi.last_variant(op)
+        capi.lib().tracea_set_split_k(0)
+        whole = call()
+        assert capi.lib().tracea_last_split_k() == 1, name
+        capi.lib().tracea_set_split_k(1)
+        assert_close_scaled(split.float().cpu().numpy(), whole.float().cpu().numpy(), 2.0 ** -10, name)

@@ -1112,6 +1112,7 @@ TraceaStatus run_gemm(const View &a, const View &b, const View &c, const Epilogu
   if (!in_padded && forced < 0 && ragged_layout(a, b, c) && !may_overlap(c, a) && !may_overlap(c, b)) {
     int groups = 1;
     const int tile = ragged_tile(M, N, K, &groups);
+    if (!g_split_k_enabled.load()) groups = 1;
     if (tile != 0) return run_gemm_any_alignment(a, b, c, chain, tile, groups, stream);
   }
   // Operands none of these kernels reads in place -- fp32 with a K that is not a whole number of 16-byte pieces or rows
@@ -2085,8 +2086,9 @@ TraceaStatus run_conv(const ConvPlan &plan, const EpilogueChain &chain, hipStrea
   // 256->256 6.7 / 4.8, 7x7 512->512 10.2 (two launches) / 7.0, 56x56 64->128 stride 2 7.5 / 4.5, 14x14 256->512 stride 2
   // 8.5 / 4.9; four images 14x14 256->256 8.9 / 6.9, 28x28 128->128 (392 workgroups) 10.7 / 8.6, 7x7 512->512 12.0 / 8.4;
   // sixteen images 7x7 512->512 (400) 16.4 / 15.6; but four images 56x56 64->64 (784) 9.4 / 11.8.
-  // (an output that is also the input works where one workgroup reads all of what it overwrites: not on these tiles)
-  if (by_rule && !may_overlap(plan.out, plan.x)) {
+  // (an output that is also the input works where one workgroup reads all of what it overwrites: not on these tiles; K is
+  // split over the waves, so the switch of the split along K holds)
+  if (by_rule && g_split_k_enabled.load() && !may_overlap(plan.out, plan.x)) {
     const long long cus = device_limits().cus;
     const ContractionVariant *best = nullptr;
     long long best_tile = 0;
