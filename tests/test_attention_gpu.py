@@ -61,17 +61,23 @@ def test_small_and_edge_lengths(tracea_gpu, variant, d, dtype):
         capi.force_variant("attention", -1)
 
 
-@pytest.mark.parametrize("variant", FAMILY, ids=lambda v: "_".join(v))
+# members whose waves share the keys of a block in groups, by head dimension
+GROUPED = [(64, "q64_kv64_d64_k4"), (64, "q128_kv64_d64_k2"), (128, "q64_kv64_d128_k2"), (128, "q128_kv64_d128_k2"),
+           (40, "q64_kv64_part64_k4"), (96, "q64_kv64_part96_k2"), (120, "q64_kv64_part128_k2")]
+
+
+@pytest.mark.parametrize("d,name", [(128, v) for v in FAMILY] + [m for m in GROUPED if m[0] != 128],
+                         ids=lambda v: v if isinstance(v, str) else str(v) if isinstance(v, int) else "_".join(v))
 @pytest.mark.parametrize("dom_mod8", [1, 5])
-def test_dominant_key_needs_the_true_running_maximum(tracea_gpu, variant, dom_mod8):
-    """One key scores about 2^250 times the others for every query row that can see it; the exact output is that
-    key's V row.
+def test_dominant_key_needs_the_true_running_maximum(tracea_gpu, d, name, dom_mod8):
+    """One key scores about 2^250 times the others (2^140 at head dimension 40) for every query row that can see it; the
+    exact output is that key's V row.
     In the kernels a query's keys are split between lanes l and l+32 (keys with kv % 8 in 0..3 and in
     4..7); a running maximum that is consistent between the two but not the true one cancels out of an
     ordinary softmax and passes every comparison with the oracle, yet here exp2 of (score - too small a
     maximum) overflows.  The dominant key is placed once in each half."""
     from tracea_amd import capi
-    b, h, s, d = 1, 2, 384, 128
+    b, h, s = 1, 2, 384
     rng = np.random.default_rng(77 + dom_mod8)
     q = np.zeros((b, h, s, d), np.float32)
     k = round_bf16(rng.standard_normal((b, h, s, d)) * 0.05)
@@ -79,8 +85,8 @@ def test_dominant_key_needs_the_true_running_maximum(tracea_gpu, variant, dom_mo
     q[...] = 4.0
     # a single dominant key per run, visible to every row (under the causal mask: to the rows at or after it)
     gk = 64 * 2 + 8 * 3 + dom_mod8          # tile 2, lane-half chosen by dom_mod8
-    k[:, :, gk, :] = 4.0                    # q.k = 128 * 16 = 2048; others ~ N(0, (4*0.05)^2 * 128) ~ +-2.3
-    name = _member(capi, variant, d)
+    k[:, :, gk, :] = 4.0                    # q.k = 16 d, 2048 at d = 128; others ~ N(0, (4*0.05)^2 * d) ~ +-2.3
+    name = _member(capi, name, d) if isinstance(name, tuple) else "fa2_" + name
     capi.force_variant("attention", name)
     try:
         for causal in (False, True):
@@ -98,18 +104,20 @@ def test_dominant_key_needs_the_true_running_maximum(tracea_gpu, variant, dom_mo
         capi.force_variant("attention", -1)
 
 
-@pytest.mark.parametrize("variant", [("q128", "pipe2"), ("q128", "m16"), ("q256", "s2_pipe2"), ("q128", "pipe")], ids=lambda v: "_".join(v))
+@pytest.mark.parametrize("d,name", [(128, "q128_kv64_d128_pipe2"), (128, "q128_kv64_d128_m16"), (128, "q256_kv64_d128_s2_pipe2"),
+                                    (128, "q128_kv64_d128_pipe")] + GROUPED, ids=lambda v: str(v))
 @pytest.mark.parametrize("dtype", ["bf16", "f16"])
 @pytest.mark.parametrize("step", [0.05, 0.11, 0.3])
-def test_scores_that_climb_along_the_sequence(tracea_gpu, variant, dtype, step):
+def test_scores_that_climb_along_the_sequence(tracea_gpu, d, name, dtype, step):
     """The kernels' reference value for the softmax moves only when a tile's maximum is more than 2^8 above
     it.  Here every query's score grows linearly with the key index, by step * 64 per tile in the exponent's
     log2 units (3.2, 7, 19): below the threshold (the reference lags by several tiles and probabilities
     reach 2^8), just under it, and above it (it moves at every tile).  The output must be the oracle's in all
-    three regimes, dense and causal, and at a sequence end inside a tile."""
+    three regimes, dense and causal, and at a sequence end inside a tile.  (Groups of waves over the keys end
+    up with reference values as far apart.)"""
     from tracea_amd import capi
     tdt, rnd = (torch.bfloat16, round_bf16) if dtype == "bf16" else (torch.float16, round_f16)
-    b, h, s, d = 1, 2, 600, 128
+    b, h, s = 1, 2, 600
     rng = np.random.default_rng(int(step * 100))
     # q = (c, 0, 0, ...) + noise, k_j = (j * u, ...) + noise: q.k_j / sqrt(d) * log2(e) = step * j + O(1)
     c = 8.0
@@ -120,7 +128,7 @@ def test_scores_that_climb_along_the_sequence(tracea_gpu, variant, dtype, step):
     k[..., 0] = np.arange(s) * u
     v = rng.standard_normal((b, h, s, d))
     q, k, v = rnd(q), rnd(k), rnd(v)
-    name = _member(capi, variant, d)
+    name = "fa2_" + name
     capi.force_variant("attention", name)
     try:
         for causal in (False, True):
@@ -338,3 +346,39 @@ def test_result_over_the_keys(tracea_gpu, d):
         t = [_dev(x, torch.float16) for x in (q, k, v)]
         tracea_gpu.attention(*t, out=t[which])
         assert_close_scaled(t[which].float().cpu().numpy(), want, _tol(d, "f16"), "over operand %d" % which)
+
+
+UNGROUPED = [(64, "q128_kv64_d64_pipe2"), (64, "q256_kv64_d64_s2_pp"), (128, "q256_kv64_d128_s2_pipe2"), (128, "q128_kv64_d128_pipe2_x2"),
+             (40, "q128_kv64_part64"), (96, "q128_kv64_part96"), (120, "q128_kv64_part128")]
+
+
+@pytest.mark.parametrize("d,member", GROUPED + UNGROUPED, ids=lambda v: str(v))
+@pytest.mark.parametrize("dtype", ["bf16", "f16"])
+def test_first_scores_far_below_zero(tracea_gpu, dtype, d, member):
+    """The reference value of the softmax starts at the maximum of the first tile a group of waves takes, wherever that
+    lies: all scores near -290 in the exponent's log2 units; the first tile near 0 and every later one below -140 (nothing
+    of those reaches the result); and keys masked with -infinity in whole tiles, so that a group's first tile, or all of
+    its tiles, hold no score, with the others near -290."""
+    from tracea_amd import capi
+    tdt, rnd = (torch.bfloat16, round_bf16) if dtype == "bf16" else (torch.float16, round_f16)
+    b, h, s = 1, 2, 1000
+    tile = np.arange(s) // 64
+    low = -200.0 * np.sqrt(d) / 16
+    for what, base in (("all low", np.full(s, low)), ("descending", np.where(tile == 0, 0.0, low / 2 - tile)),
+                       ("a masked tile", np.where(tile == 1, -np.inf, low)), ("one tile", np.where(tile == 0, low, -np.inf))):
+        rng = np.random.default_rng(d)
+        q, k, v = (rng.standard_normal((b, h, s, d)) * 0.5 for _ in range(3))
+        q[..., 0] = 16.0
+        k[..., 0] = base
+        q, k, v = rnd(q), rnd(k), rnd(v)
+        capi.force_variant("attention", "fa2_" + member)
+        try:
+            for causal in (False, True)[:1 if member.endswith("_pp") else 2]:  # (that member takes no causal mask)
+                want = oracle.attention_bhsd(q, k, v, 1.0 / np.sqrt(d), causal)
+                assert np.isfinite(want).all()
+                got = tracea_gpu.attention(_dev(q, tdt), _dev(k, tdt), _dev(v, tdt), causal=causal).float().cpu().numpy()
+                assert capi.last_variant("attention") == "fa2_" + member
+                assert np.isfinite(got).all(), "%s %s causal=%s" % (member, what, causal)
+                assert_close_scaled(got, want, _tol(d, dtype), "%s %s causal=%s" % (member, what, causal))
+        finally:
+            capi.force_variant("attention", -1)

@@ -713,15 +713,21 @@ fa2_fwd_pipe_kernel(const AttentionArgs a) {
   // the whole excess once that exceeds TAU (`force`: by whatever it is -- the first tile's case, whose reference
   // is the arbitrary 0); the tile's z follow, O is rescaled at once, and alpha is the factor the row sum of the
   // earlier tiles takes with the next tile's sum (exactly 1 where nothing moved).  One branch for all of it.
+  // A first reference rescales nothing: O and the sum are zero, and 2^-mw of a first maximum below -128 is infinite.
+  // KG > 1: the first tile with a score above -infinity sets it (a group's share of the keys may begin with
+  // tiles that are -infinity throughout), and a group that saw none has none.
+  bool seen = false;
   auto fold_shift = [&](const float (&mx)[QB], f32x16 (&z)[QB][2], bool force) __attribute__((always_inline)) {
     bool moved = false;
     float step[QB];
 #pragma unroll
     for (int qi = 0; qi < QB; ++qi) {
       const float mw = max_with_lane_xor32(mx[qi]);
-      const bool mv = (force & (mw > -INFINITY)) | (mw > FA_RESCALE_TAU);
+      const bool first = KG > 1 ? !seen : force;
+      const bool mv = (first & (mw > -INFINITY)) | (mw > FA_RESCALE_TAU);
       step[qi] = mv ? mw : 0.0f;
-      alpha[qi] = __builtin_amdgcn_exp2f(-step[qi]);
+      alpha[qi] = first ? 1.0f : __builtin_amdgcn_exp2f(-step[qi]);
+      if constexpr (KG > 1) seen |= mw > -INFINITY;
       m_run[qi] += step[qi];
       moved |= mv;
     }
@@ -762,11 +768,7 @@ fa2_fwd_pipe_kernel(const AttentionArgs a) {
         moved |= lazy_running_max(m_run[qi], mx * a.scale_log2, alpha[qi]);
       }
     }
-    if constexpr (SHIFT) {  // (tile 0 of a block: O and the row sum are still zero, the factor stays 1)
-      fold_shift(mxs, s, true);
-#pragma unroll
-      for (int qi = 0; qi < QB; ++qi) alpha[qi] = 1.0f;
-    }
+    if constexpr (SHIFT) fold_shift(mxs, s, true);  // (tile 0 of a block)
     return moved;
   };
   // alpha is exactly 1 for every lane whose maximum did not move: the 16*DB
@@ -1293,14 +1295,14 @@ fa2_fwd_pipe_kernel(const AttentionArgs a) {
   }
   if constexpr (KG > 1) {
     // Each wave's O, its share of the row sum and its reference value, 16 bytes per lane at a time (1 KB a row); a query
-    // none of whose keys a group has seen carries no reference there.
+    // of which a group has seen no score above -infinity carries no reference there.
     constexpr int ROWS = DB * 4 + 1;
     __builtin_amdgcn_s_waitcnt(0x0f70);  // (look-ahead requests past the end still write the rings)
     __syncthreads();
     f32x4 *const part = (f32x4 *)smem + lane;
     if (kg > 0) {
       f32x4 *const dst = part + ((kg - 1) * QW + wave_u) * (ROWS * 64);
-      const f32x4 sums = {l_run[0], kg * FA_BKV <= last_key[0] + g * 4 ? m_run[0] : -INFINITY, 0.0f, 0.0f};
+      const f32x4 sums = {l_run[0], seen ? m_run[0] : -INFINITY, 0.0f, 0.0f};
       dst[DB * 4 * 64] = sums;
 #pragma unroll
       for (int d = 0; d < DB; ++d)
@@ -1309,9 +1311,9 @@ fa2_fwd_pipe_kernel(const AttentionArgs a) {
     }
     __syncthreads();
     if (kg > 0) return;
-    float l_g[KG], m_g[KG], m_all = m_run[0];
+    float l_g[KG], m_g[KG], m_all = seen ? m_run[0] : -INFINITY;
     l_g[0] = l_run[0];
-    m_g[0] = m_run[0];
+    m_g[0] = m_all;
 #pragma unroll
     for (int z = 1; z < KG; ++z) {
       const f32x4 sums = part[((z - 1) * QW + wave_u) * (ROWS * 64) + DB * 4 * 64];
