@@ -680,3 +680,25 @@ def test_pointwise_convolution_over_its_input(tracea_gpu, hw):
         t = _dev(x, torch.float16)
         tracea_gpu.conv2d(t, _dev(w, torch.float16), out=t)
         assert_close_scaled(t.float().cpu().numpy().reshape(-1, 64), want, tol_half(64, "f16"), "in place")
+
+
+# n, h=w, c, k, r, stride, member: K-split members in one round go first (eight images), not in two (seven, ten); more than two
+# 32x32 tiles per CU; K too long for one wave's walk on 4 and on 32 tiles; taps that share no pixels
+@pytest.mark.parametrize("case", [(8, 14, 256, 256, 3, 1, "c32x64_c256_s4_w16_ksplit"), (7, 14, 256, 256, 3, 1, "c32x32_c64_w4_w16_ksplit"),
+                                  (10, 14, 256, 256, 3, 1, "c32x32_c64_w4_w16_ksplit"), (5, 28, 128, 128, 3, 1, "c32x32_c64_w4_w16_ksplit"),
+                                  (6, 28, 128, 128, 3, 1, "t64x64x128_w2x2_p2"), (1, 4, 1536, 64, 3, 1, "c16x16_c64_w8_w16_ksplit"),
+                                  (1, 4, 2048, 64, 3, 1, "t64x64x128_w2x2_p2"), (1, 14, 2048, 256, 3, 1, "c16x16_c64_w8_w16_ksplit"),
+                                  (2, 28, 4096, 128, 1, 1, "c32x32_c64_w8_w16_ksplit"), (11, 14, 4096, 128, 1, 1, "t64x64x128_w2x2_p2"),
+                                  (11, 28, 384, 128, 3, 2, "t64x64x128_w2x2_p2")])
+def test_rule_for_few_pixels(tracea_gpu, case):
+    """Both sides of the lines of the rule for few output pixels: the member that runs, and its result against torch's fp32
+    convolution on the CPU."""
+    from tracea_amd import capi
+    n, hw, c, k, r, stride, member = case
+    g = torch.Generator().manual_seed(n * hw + c)
+    x = torch.randn(n, hw, hw, c, generator=g).half()
+    w = (torch.randn(k, r, r, c, generator=g) / (r * r * c) ** 0.5).half()
+    y = tracea_gpu.conv2d(x.cuda(), w.cuda(), stride=stride, padding=r // 2)
+    assert capi.last_variant("conv2d") == member
+    want = torch.nn.functional.conv2d(x.float().permute(0, 3, 1, 2), w.float().permute(0, 3, 1, 2), stride=stride, padding=r // 2)
+    assert_close_scaled(y.float().cpu().numpy(), want.permute(0, 2, 3, 1).numpy(), tol_half(r * r * c, "f16"), member)

@@ -2081,28 +2081,35 @@ TraceaStatus run_conv(const ConvPlan &plan, const EpilogueChain &chain, hipStrea
   bool resident_chosen = false;
   const bool by_rule = forced_variant("conv2d") < 0 && tuning_cache_lookup_variant(key, plan.x.dtype, plan.w_ncontig) < 0;
   // Launches of few output pixels: the smallest tile that still comes in one round of workgroups (32x32: on four waves up
-  // to 18 pieces of K, eight beyond), or 32x32 tiles in up to 400 workgroups on four waves from K = 1152 on.  Replayed
-  // graphs, best other kernel / this one, us: one image 56x56 64->64 3x3 7.6 / 5.0, 28x28 128->128 8.7 / 4.8, 14x14
-  // 256->256 6.7 / 4.8, 7x7 512->512 10.2 (two launches) / 7.0, 56x56 64->128 stride 2 7.5 / 4.5, 14x14 256->512 stride 2
-  // 8.5 / 4.9; four images 14x14 256->256 8.9 / 6.9, 28x28 128->128 (392 workgroups) 10.7 / 8.6, 7x7 512->512 12.0 / 8.4;
-  // sixteen images 7x7 512->512 (400) 16.4 / 15.6; but four images 56x56 64->64 (784) 9.4 / 11.8.
+  // to 18 pieces of K, eight beyond).  Replayed graphs, best other kernel / this one, us: one image 56x56 64->64 3x3 7.6 /
+  // 5.0, 28x28 128->128 8.7 / 4.8, 14x14 256->256 6.7 / 4.8, 7x7 512->512 10.2 (two launches) / 7.0, 56x56 64->128 stride
+  // 2 7.5 / 4.5, 14x14 256->512 stride 2 8.5 / 4.9; four images 14x14 256->256 6.4 / 6.3, 7x7 512->512 12.0 / 8.4.  A
+  // wave walks K / 64 / waves pieces where the streamed kernel spreads K over workgroups: up to K = 14336, or 18432 on
+  // 16x16 tiles for half the CUs and more (4x4 -> 64 filters, K 13824 10.8 / 9.8, 16384 10.0 / 10.9, 36864 14.3 / 20.4; 14x14
+  // -> 256, K 18432 14.8 / 12.6, 27648 17.7 / 16.9, 36864 17.9 / 22.2; 7x7 -> 256, 64 workgroups, K 18432 11.1 / 12.4).
   // (an output that is also the input works where one workgroup reads all of what it overwrites: not on these tiles; K is
   // split over the waves, so the switch of the split along K holds)
-  if (by_rule && g_split_k_enabled.load() && !may_overlap(plan.out, plan.x)) {
-    const long long cus = device_limits().cus;
-    const ContractionVariant *best = nullptr;
+  const long long cus = device_limits().cus;
+  const bool few_pixels = by_rule && g_split_k_enabled.load() && !may_overlap(plan.out, plan.x);
+  auto private_wgs = [&](const ContractionVariant &cv) -> long long {  // 0: cannot run the call
+    ContractionArgs probe = a;
+    return cv.pipeline == 11 && plan_conv_private16(g, cv, plan.w_ncontig, &probe) ? (long long)probe.grid_m * probe.grid_n : 0;
+  };
+  if (few_pixels) {
     long long best_tile = 0;
     for (int i = 0; i < contraction_variant_count(); ++i) {
       const ContractionVariant &cv = contraction_variant(i);
-      ContractionArgs probe = a;
-      if (cv.pipeline != 11 || !plan_conv_private16(g, cv, plan.w_ncontig, &probe)) continue;
-      const long long wgs = (long long)probe.grid_m * probe.grid_n, tile = (long long)cv.bm * cv.bn;
-      if (tile == 32 * 32 && (cv.waves_m == 4) != (wgs > cus || a.K <= 18 * 64)) continue;
-      if (wgs > cus && !(tile == 32 * 32 && wgs <= 400 && a.K >= 1152)) continue;
-      if (best == nullptr || tile < best_tile) { best = &cv; best_tile = tile; vi = i; }
+      const long long wgs = private_wgs(cv), tile = (long long)cv.bm * cv.bn;
+      if (wgs == 0 || wgs > cus || (best_tile != 0 && tile >= best_tile)) continue;
+      if (tile == 32 * 32 && (cv.waves_m == 4) != (a.K <= 18 * 64)) continue;
+      if (a.K > (tile == 16 * 16 && wgs * 2 >= cus ? 18432 : 14336)) continue;
+      best_tile = tile;
+      vi = i;
     }
-    resident_chosen = best != nullptr;
+    resident_chosen = best_tile != 0;
   }
+  const bool one_round = resident_chosen;
+  long long next_wgs = 0;  // workgroups of the member the next rule takes
   // Next: the kernels on 16x16x32 MFMAs with the patch in LDS and the filter slab resident or in a
   // ring (pipelines 7 to 10), where their plan fits, the launch fills most of the device and a workgroup's
   // tile is at least three quarters of the kernel's largest (smaller tiles leave its waves' blocks empty).
@@ -2120,10 +2127,32 @@ TraceaStatus run_conv(const ConvPlan &plan, const EpilogueChain &chain, hipStrea
       // against 13.1 on the 32-pixel member)
       if (!plan_conv_resident(g, cv, plan.w_ncontig, &probe)) continue;
       const bool tile_ok = cv.pipeline == 9 && cv.bm > 32 ? probe.p_tm * 5 >= cv.bm * 2 : probe.p_tm * 4 >= cv.bm * 3;
-      if ((long long)probe.grid_m * probe.grid_n * 4 >= enough && tile_ok) {
+      next_wgs = (long long)probe.grid_m * probe.grid_n;
+      if (next_wgs * 4 >= enough && tile_ok) {
         vi = i;
         resident_chosen = true;
       }
+    }
+  }
+  // Up to two workgroups per CU (what its LDS holds) of 32x32 tiles on four waves, from K = 1152 on, unless a K-split member
+  // with the patch in LDS comes in one round.  us, that member or the streamed kernel / this one: eight images 14x14
+  // 256->256 7.2 (one round) / 9.3, seven 11.9 (two) / 9.2, sixteen images 14x14 -> 7x7 256->512 7.4 (one) / 9.3; 28x28
+  // 128->128 four images (392 workgroups) 8.8 / 7.0, five (490) 9.4 / 7.6, six (588) 8.5 / 10.6; 7x7 512->512 eighteen (448) 13.7 /
+  // 13.2, twenty (496) 14.1 / 14.4, twenty-two (544) 16.2 / 19.7.  The streamed kernel splits K over workgroups, so the line
+  // falls with K times the workgroups, and lower where taps do not share their pixels (1x1 filters, a stride): 1024 channels
+  // 28x28 -> 512 3x3 (K 9216, 400) 20.7 / 22.5; stride 2 11x 28x28 384->128 (K 3456, 272) 11.5 / 13.1; 1x1 2048 channels
+  // 392 and 400 workgroups 11.4-14.2 / 12.2-12.5, 496 11.7 / 13.5, 4096 channels (308) 13.7 / 22.8.
+  if (few_pixels && !one_round) {
+    const bool ksplit = resident_chosen && contraction_variant(vi).pipeline == 9;
+    const bool shared = g.stride_h == 1 && g.stride_w == 1 && g.block.r_sz * g.block.s_sz > 1;
+    for (int i = 0; (!resident_chosen || (ksplit && next_wgs > cus)) && i < contraction_variant_count(); ++i) {
+      const ContractionVariant &cv = contraction_variant(i);
+      if (cv.bm * cv.bn != 32 * 32 || cv.waves_m != 4) continue;
+      const long long wgs = private_wgs(cv);
+      if (wgs <= cus || wgs > 2 * cus || a.K < 1152 || (!ksplit && a.K * wgs > cus * (shared ? 9216 : 3300))) continue;
+      vi = i;
+      resident_chosen = true;
+      break;
     }
   }
   if (!resident_chosen && by_rule) {
