@@ -38,3 +38,24 @@ def round_bf16(x):
     u = x.view(np.uint32).astype(np.uint64)
     rounded = ((u + 0x7FFF + ((u >> 16) & 1)) >> 16) << 16
     return rounded.astype(np.uint32).view(np.float32).reshape(x.shape)
+
+
+def launches(call):
+    """GPU operations of one call, counted as the nodes of a captured graph (the call runs twice on the capturing stream
+    first, so that it finds the workspaces it keeps)."""
+    import ctypes as C
+
+    import torch
+    from tracea_amd import capi
+    stream = torch.cuda.Stream()
+    stream.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(stream):
+        call()
+        call()
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph(keep_graph=True)
+        with torch.cuda.graph(graph, stream=stream):
+            call()
+    n = C.c_size_t(0)
+    assert capi.lib().hipGraphGetNodes(C.c_void_p(graph.raw_cuda_graph()), None, C.byref(n)) == 0
+    return n.value

@@ -254,8 +254,9 @@ def test_strided_views_and_error_paths(tracea_gpu):
 @pytest.mark.parametrize("dtype", ["bf16", "f16"])
 def test_other_head_dimensions_and_unaligned_tensors_run_from_padded_copies(tracea_gpu, dtype):
     """Head dimensions off 64 and 128 (the reference compiles its kernel per head dimension:
-    src/kernels/attention/cuda_emitter.rs:39-58), a strided head dimension, odd strides and bases off
-    16 bytes: padded copies, the caller's scale (1/sqrt of the true D by default), result copied out."""
+    src/kernels/attention/cuda_emitter.rs:39-58): multiples of 8 in place, the others, a strided head dimension, odd
+    strides and bases off 16 bytes from padded copies with the result copied out; the caller's scale (1/sqrt of the
+    true D by default) either way."""
     tdt, rnd = (torch.bfloat16, round_bf16) if dtype == "bf16" else (torch.float16, round_f16)
     for (b, h, s, d) in [(2, 3, 77, 32), (1, 2, 200, 80), (2, 2, 130, 96), (1, 1, 64, 8), (1, 2, 33, 1), (1, 2, 150, 127)]:
         q, k, v = _inputs(b, h, s, d, 7 * s + d, rnd)

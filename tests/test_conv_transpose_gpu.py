@@ -9,7 +9,7 @@ import numpy as np
 import pytest
 
 import oracle
-from helpers import assert_close_scaled, round_f16, round_bf16, tol_half
+from helpers import assert_close_scaled, launches, round_f16, round_bf16, tol_half
 
 torch = pytest.importorskip("torch")
 pytestmark = pytest.mark.gpu
@@ -275,7 +275,7 @@ def test_filter_cache_reuses_the_regrouped_bank_until_it_is_cleared(tracea_gpu):
 @pytest.mark.parametrize("dtype", ["f16", "bf16"])
 def test_filters_read_in_place(tracea_gpu, shape, dtype):
     """[C,R,S,K] banks that the phase kernels read where they lie: dense, and with NaN in a gap between
-    the input channels; then the same call with the bank in an order that is regrouped."""
+    the input channels; then the same call with the bank in an order that is regrouped, which takes one launch more."""
     n, h, w, c, k, r, s, stride, pad, opad = shape
     tdt, rounder = (torch.float16, round_f16) if dtype == "f16" else (torch.bfloat16, round_bf16)
     x, wt = _operands(shape, 5, rounder)
@@ -283,9 +283,17 @@ def test_filters_read_in_place(tracea_gpu, shape, dtype):
     want = np.maximum(oracle.conv_transpose2d_nhwc(x, wt, stride, pad, opad) + bias, 0.0)
     wide = torch.full((c, r * s * k + 8), float("nan"), device="cuda", dtype=tdt)
     wide[:, :r * s * k] = _dev(wt, tdt).reshape(c, -1)
+    count = {}
     for tag, bank, layout in (("dense", _dev(wt, tdt), "crsk"),
                               ("gap", torch.as_strided(wide, (c, r, s, k), (r * s * k + 8, s * k, k, 1)), "crsk"),
                               ("regrouped", _dev(wt.transpose(3, 1, 2, 0), tdt), "krsc")):
-        y = tracea_gpu.conv_transpose2d(_dev(x, tdt), bank, bias=_dev(bias), stride=stride, padding=pad, output_padding=opad,
-                                        epilogue="bias+relu", weight_layout=layout)
+        dx, dbias = _dev(x, tdt), _dev(bias)
+        y = torch.empty(want.shape, device="cuda", dtype=tdt)
+
+        def call():
+            tracea_gpu.conv_transpose2d(dx, bank, bias=dbias, stride=stride, padding=pad, output_padding=opad, epilogue="bias+relu",
+                                        out=y, weight_layout=layout)
+        call()
         assert_close_scaled(y.float().cpu().numpy(), want, tol_half(c * r * s, dtype), tag)
+        count[tag] = launches(call)
+    assert count["dense"] == count["gap"] == count["regrouped"] - 1, count

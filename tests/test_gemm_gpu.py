@@ -315,9 +315,10 @@ def test_operand_beyond_2gib_takes_the_register_staged_kernels(tracea_gpu, dtype
 
 @pytest.mark.parametrize("shape", [(1000, 900, 1030), (129, 257, 203), (5, 3, 7), (300, 1001, 130), (1, 1, 1), (513, 130, 31)])
 def test_ragged_sizes_and_strided_operands_run_from_padded_copies(tracea_gpu, shape):
-    """A K or N that is not a whole number of 16-byte pieces, and operands strided along K: copied into padded rows
-    and multiplied by the tile kernels (the any-layout kernel on the vector ALU remains for what cannot be copied).
-    fp32 and both half types, B row-major and column-major, a column-major A, with a chain and with fp32 output."""
+    """A K or N that is not a whole number of 16-byte pieces, and operands strided along K: fp32 is copied into padded
+    rows and multiplied by the tile kernels (the any-layout kernel on the vector ALU remains for what cannot be copied),
+    both half types are read in place where their rows lie along K or N (what they copy: the next test).  B row-major and
+    column-major, a column-major A in fp32, with a chain and with fp32 output."""
     from tracea_amd import capi
     m, n, k = shape
     rng = np.random.default_rng(m + 3 * n + 7 * k)
@@ -337,14 +338,42 @@ def test_ragged_sizes_and_strided_operands_run_from_padded_copies(tracea_gpu, sh
         xa, xb = _dev(ha, tdt), _dev(hb, tdt)
         for tag, yb in (("row-major B", xb), ("column-major B", xb.t().contiguous().t())):
             got = tracea_gpu.gemm(xa, yb, bias=dbias, epilogue="bias+relu").float().cpu().numpy()
-            assert capi.last_variant("gemm") is not None, "the tile kernels did not run"
+            # (rows of either operand along K or N are read in place; an operand of fewer than 8 elements is copied)
+            assert capi.last_variant("gemm").endswith("_any") == (min(m, n) * k >= 8), "not the expected road"
             assert_close_scaled(got, want, tol_half(k, dtype), "%s %s" % (dtype, tag))
         got = tracea_gpu.gemm(xa, xb, out_dtype=torch.float32).cpu().numpy()
         assert np.abs(got - ref16).max() <= 1e-4 * max(1.0, np.abs(ref16).max()), dtype + " with fp32 output"
 
 
+# m, n, k, columns of A side by side: A along M with ragged and with whole 16-byte pieces; few tiles and a K too long for a
+# few workgroups' walk; more than four rounds of 128x128 tiles
+@pytest.mark.parametrize("case", [(70, 67, 65, True), (136, 72, 96, True), (9, 8, 1001, True), (100, 100, 16001, False), (4097, 4100, 9, False)])
 @pytest.mark.parametrize("dtype", ["f16", "bf16"])
-@pytest.mark.parametrize("m", [1, 8, 9, 16, 17, 40, 48])
+def test_half_operands_that_run_from_padded_copies(tracea_gpu, dtype, case):
+    """What half precision still copies into padded rows: an A strided along K, and the sizes at which the tile kernels on
+    the copies are ahead of the kernel that reads in place.  Both layouts of B (a row-major one is transposed on the
+    way)."""
+    from tracea_amd import capi
+    m, n, k, columns = case
+    tdt, rnd = (torch.float16, round_f16) if dtype == "f16" else (torch.bfloat16, round_bf16)
+    rng = np.random.default_rng(m + 3 * n + 7 * k)
+    a = rnd(rng.standard_normal((m, k), dtype=np.float32) / np.sqrt(k))
+    b = rnd(rng.standard_normal((k, n), dtype=np.float32))
+    bias = rng.standard_normal(n).astype(np.float32)
+    want = np.maximum(oracle.gemm_f64(a, b) + bias[None, :], 0.0)
+    da = _dev(np.ascontiguousarray(a.T), tdt).t() if columns else _dev(a, tdt)
+    for tag, db in (("row-major B", _dev(b, tdt)), ("column-major B", _dev(np.ascontiguousarray(b.T), tdt).t())):
+        got = tracea_gpu.gemm(da, db, bias=_dev(bias), epilogue="bias+relu").float().cpu().numpy()
+        name = capi.last_variant("gemm")
+        assert name is not None and not name.endswith(("_any", "_rows")), "%s: %s" % (tag, name)
+        assert_close_scaled(got, want, tol_half(k, dtype), tag)
+
+
+ROWS = "t48x64x64_w1x4_w16_rows"
+
+
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+@pytest.mark.parametrize("m", [1, 8, 9, 16, 17, 25, 32, 40, 48])
 def test_products_of_a_few_rows(tracea_gpu, dtype, m):
     """The kernel for at most 48 rows: both layouts of B, row counts on either side of its 8-row loads and 16-row blocks,
     widths and depths off its tiles (one piece of K, a K tail of 8, more pieces than ring stages, more waves than pieces),
@@ -362,11 +391,19 @@ def test_products_of_a_few_rows(tracea_gpu, dtype, m):
         da[:, :k] = _dev(a, tdt)
         ops = [(capi.OP_BIAS_ADD, _dev(bias)), (capi.OP_RESIDUAL_ADD, _dev(res, tdt)), (capi.OP_RELU,)]
         for tag, db in (("K-contiguous", _dev(np.ascontiguousarray(b.T), tdt).t()), ("N-contiguous", _dev(b, tdt))):
-            out = torch.full((m + 1, n + 4), 7.0, device="cuda", dtype=tdt)
-            tracea_gpu.gemm_ex(da[:, :k], db, ops, out=out[:m, :n])
-            got = out.float().cpu().numpy()
-            assert_close_scaled(got[:m, :n], ref, tol_half(k, dtype), "%s %s" % (tag, (m, n, k)))
-            assert (got[m] == 7.0).all() and (got[:, n:] == 7.0).all(), "outside the output"
+            # by rule (few workgroups over a long K go to the tile kernels), and on this kernel whatever the rule says
+            for forced in (False, True):
+                out = torch.full((m + 1, n + 4), 7.0, device="cuda", dtype=tdt)
+                capi.force_variant("gemm", ROWS if forced else -1)
+                try:
+                    tracea_gpu.gemm_ex(da[:, :k], db, ops, out=out[:m, :n])
+                finally:
+                    capi.force_variant("gemm", -1)
+                ruled = k <= 4096 and m <= 32 or n == 11008 if tag == "N-contiguous" else True
+                assert (capi.last_variant("gemm") == ROWS) == (forced or ruled), capi.last_variant("gemm")
+                got = out.float().cpu().numpy()
+                assert_close_scaled(got[:m, :n], ref, tol_half(k, dtype), "%s %s" % (tag, (m, n, k)))
+                assert (got[m] == 7.0).all() and (got[:, n:] == 7.0).all(), "outside the output"
 
 
 # one element in a row or column, K off and on the 64-deep tiles, a last row of B within 8 elements of the end in the tile

@@ -7,7 +7,7 @@ import numpy as np
 import pytest
 
 import oracle
-from helpers import assert_close_scaled, round_bf16, round_f16, tol_half
+from helpers import assert_close_scaled, launches, round_bf16, round_f16, tol_half
 
 torch = pytest.importorskip("torch")
 pytestmark = pytest.mark.gpu
@@ -156,8 +156,12 @@ def test_linear_batches_in_one_launch(tracea_gpu, dtype, b, m, k, n, w_layout):
     da = torch.zeros(b, m + 2, k, device="cuda", dtype=tdt)
     da[:, :m] = _dev(a, tdt)
     out = torch.full((b, m + 1, n), 7.0, device="cuda", dtype=torch.float32)
+    dbias = torch.from_numpy(bias).cuda()
     for _ in range(2):  # the second call meets the split counters the first one left
-        tracea_gpu.linear(da[:, :m], dw, bias=torch.from_numpy(bias).cuda(), epilogue="bias+relu", out=out[:, :m])
+        tracea_gpu.linear(da[:, :m], dw, bias=dbias, epilogue="bias+relu", out=out[:, :m])
+    # (fp32 weights stored [N,K] have no kernel of their own: product by product, from copies)
+    launched = launches(lambda: tracea_gpu.linear(da[:, :m], dw, bias=dbias, epilogue="bias+relu", out=out[:, :m]))
+    assert (launched == 1) == (dtype != "f32" or w_layout == "kn"), launched
     got = out.cpu().numpy()
     assert (got[:, m] == 7.0).all(), "rows between the batches are not the call's"
     for i in range(b):
