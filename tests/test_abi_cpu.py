@@ -126,6 +126,15 @@ def test_variant_table():
     assert l.tracea_force_variant(b"gemm", -1) == 0
 
 
+# 256x256 tiles in part of a round, in one and a bit, in three full ones; a layer of few tiles
+@pytest.mark.parametrize("shape", [(13068, 768, 6400, "t256x256x64_w2x4_p2"), (9016, 1024, 2304, "t256x256x64_w2x4_p2"),
+                                   (25600, 640, 2880, "t128x128x64_w2x2_p2"), (73728, 256, 2048, "t128x128x64_w2x2_p2"),
+                                   (98304, 512, 1152, "t256x256x64_w2x4_p2"), (10000, 256, 576, "t128x64x64_w4x2_p2")])
+def test_tiles_of_streamed_convolutions(shape):
+    m, n, k, member = shape
+    assert capi.variants("conv2d")[capi.lib().tracea_select_variant(b"conv2d", m, n, k)] == member
+
+
 def test_tune_without_runtime_reports_failure():
     l = capi.lib()
     l.tracea_shutdown()

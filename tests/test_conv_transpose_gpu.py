@@ -297,3 +297,22 @@ def test_filters_read_in_place(tracea_gpu, shape, dtype):
         assert_close_scaled(y.float().cpu().numpy(), want, tol_half(c * r * s, dtype), tag)
         count[tag] = launches(call)
     assert count["dense"] == count["gap"] == count["regrouped"] - 1, count
+
+
+# n, h=w, c, k, r, stride, pad, read in place: two sides of the line in work per CU, like and unlike phases; 128x128 tiles with K
+# tiles of 128 on a short and on a long K
+@pytest.mark.parametrize("case", [(5, 40, 512, 256, 4, 2, 1, True), (4, 48, 512, 256, 4, 2, 1, False), (8, 48, 512, 256, 3, 2, 1, False),
+                                  (8, 20, 512, 256, 4, 2, 1, True), (8, 40, 512, 256, 3, 1, 1, False)])
+def test_rule_for_filters_in_place(tracea_gpu, case):
+    """Large layers regroup a bank that small ones read where it lies: told by the launches of the same call with the bank in an
+    order that is always regrouped.  Both calls form the same fp32 sums up to their order."""
+    n, hw, c, k, r, stride, pad, in_place = case
+    g = torch.Generator(device="cuda").manual_seed(n * hw)
+    x = torch.randn(n, hw, hw, c, device="cuda", generator=g).half()
+    w = (torch.randn(c, r, r, k, device="cuda", generator=g) * (stride / (r * c ** 0.5))).half()
+    banks, out, count = {"crsk": w, "krsc": w.permute(3, 1, 2, 0).contiguous()}, {}, {}
+    for layout, bank in banks.items():
+        out[layout] = tracea_gpu.conv_transpose2d(x, bank, stride=stride, padding=pad, weight_layout=layout)
+        count[layout] = launches(lambda: tracea_gpu.conv_transpose2d(x, bank, stride=stride, padding=pad, out=out[layout], weight_layout=layout))
+    assert count["krsc"] - count["crsk"] == (1 if in_place else 0), count
+    assert_close_scaled(out["crsk"].float().cpu().numpy(), out["krsc"].float().cpu().numpy(), 2.0 ** -10, "layouts agree")

@@ -547,8 +547,14 @@ int select_contraction_variant(int m, int n, int k, bool conv, bool b_ncontig, i
     // 107.8): the eight-wave 16x16x32 member runs this layout.  (Before the transposing reads were written as
     // instructions the compiler put a vmcnt(0) in front of each one that followed a tile request: 128-132 and
     // 209 us for the two 16x16x32 members.)
-    // (convolutions, eight waves too: N8 48x48 512->256 4x4 s2 transposed 118.4 us on 256x256 tiles, 106.5 on 128x128)
-    if (b_ncontig && v.bm * v.bn >= 256 * 256 && (conv || v.waves_m * v.waves_n == 4)) prior *= 0.8;
+    if (b_ncontig && v.bm * v.bn >= 256 * 256 && v.waves_m * v.waves_n == 4) prior *= 0.8;
+    // Convolutions: 256x256 tiles are ahead by 1.2 of 128x128 ones at equal use of the CUs, and by more in one round, where
+    // three of the smaller tiles on a CU (two fit at a time) take as long as four; behind in a second round that is
+    // nearly empty.  Eight waves go before four for either layout of the filters.  Fitted on 107 shapes, every
+    // member timed for both layouts: the choice is 2 % behind the best member on average (worst 1.2 times).  us, 256x256 on
+    // eight waves / 128x128: M 13068 N 768 K 6400 (0.6 rounds) 131 / 184, M 9016 N 1024 K 2304 60 / 72, M 25600 N 640 K 2880
+    // (1.2 rounds) 138 / 105, M 73728 N 256 K 2304 125 / 109, M 98304 N 512 K 1152 (3 rounds) 117 / 140.
+    if (conv && v.bm * v.bn >= 256 * 256) prior *= (units <= cus ? 1.15 : 0.85) * (v.waves_m * v.waves_n == 4 ? 0.95 : 1.0);
     {
       // A CU with fewer than 8 resident waves (one 4-wave workgroup, the launch too small or
       // the tile's LDS too large for a second) hides less latency.  The fourth root is fitted
@@ -2489,13 +2495,36 @@ TraceaStatus run_conv_transpose_by_phase(const ConvTransposePlan &plan, const Ep
         }
       total += (long long)K * pr.taps * ps.taps * C;
     }
+  // Phases that are alike but for their padding (even filter extents divided by the stride: the 4x4
+  // stride-2 decoder layer) go out as one launch with the phase in blockIdx.z.
+  bool uniform = sh <= 4 && sw <= 4 && sh * sw > 1;
+  for (int a = 1; a < sh && uniform; ++a) {
+    const PhaseAxis p0 = phase_axis(0, sh, plan.pad_h, R, Ho), pa = phase_axis(a, sh, plan.pad_h, R, Ho);
+    uniform = p0.taps == pa.taps && p0.out == pa.out;
+  }
+  for (int b = 1; b < sw && uniform; ++b) {
+    const PhaseAxis p0 = phase_axis(0, sw, plan.pad_w, S, Wo), pb = phase_axis(b, sw, plan.pad_w, S, Wo);
+    uniform = p0.taps == pb.taps && p0.out == pb.out;
+  }
   // A bank whose output channels lie side by side (the reference's [C*R*S, K] rows among them) is read where it lies, as
   // an N-contiguous B, by the direct-to-LDS kernels when a K tile lies inside a tap: no regrouping launch.  Same sums in
   // the same order.  Replayed graphs, regrouped / in place, us: N8 32x32 512->256 4x4 s2 52.1 / 46.7, N8 64x64 256->128
   // 51.4 / 49.7, N1 16x16 512->512 22.8 / 16.2, N2 20x20 128->64 11.5 / 7.7, N8 32x32 128->128 2x2 11.6 / 8.6, N8 40x40
-  // 512->128 3x3 s1 37.5 / 36.5.  (A cached bank stays what it was.)
+  // 512->128 3x3 s1 37.5 / 36.5.  (A cached bank stays what it was.)  Not where reading an
+  // N-contiguous B costs more than the 5 us of the regrouping launch, a few percent of the kernel: from 70e6
+  // multiply-accumulates per CU on (N5 40x40 512->256 4x4 s2, 66e6, 48.8 / 45.6, N4 48x48, 75e6, 57.0 / 62.9, N6 40x40, 79e6,
+  // 58.7 / 63.9, N8 48x48, 151e6, 112.7 / 121.3, N8 48x48 512->192 98.0 / 107.7, 3x3 s2 512->256, 85e6, 100.4 / 105.3; level at N8 48x48 256->256, 75e6, and N8
+  // 44x44 512->256, 127e6), and earlier where the K-contiguous choice is 128x128 tiles with K tiles of 128, whose
+  // N-contiguous form is 14 to 19 % behind (K 4608, N8 40x40 512->256 3x3 s1 52.1 / 57.0; K 2048, N8 20x20 512->256 31.7 / 30.4).
+  const long long k_most = (long long)C * ((R + sh - 1) / sh) * ((S + sw - 1) / sw);
+  const long long m_most = (long long)N * ((Ho + sh - 1) / sh) * ((Wo + sw - 1) / sw) * (uniform ? sh * sw : 1);
+  bool slow_in_place = (double)N * Ho * Wo * K * C * R * S / (sh * sw) > (double)device_limits().cus * 70e6;
+  if (!slow_in_place && k_most > 2560 && k_most < (1ll << 31) && m_most < (1ll << 31)) {
+    const int vk = select_contraction_variant((int)m_most, K, (int)k_most, true);
+    slow_in_place = vk >= 0 && contraction_variant(vk).bk == 128 && contraction_variant(vk).bm * contraction_variant(vk).bn >= 128 * 128;
+  }
   const long long w_reach = (C - 1) * w.stride[3] + (R - 1) * w.stride[1] + (S - 1) * w.stride[2] + K;
-  const bool in_place = !g_ct_filter_cache.load() && w.stride[0] == 1 && K % 8 == 0 && C % 64 == 0 && aligned(w.ptr, 16) &&
+  const bool in_place = !g_ct_filter_cache.load() && !slow_in_place && w.stride[0] == 1 && K % 8 == 0 && C % 64 == 0 && aligned(w.ptr, 16) &&
                         w.stride[1] >= 0 && w.stride[2] >= 0 && w.stride[3] > 0 && w.stride[1] % 8 == 0 && w.stride[2] % 8 == 0 &&
                         w.stride[3] % 8 == 0 && w_reach * 2 < (1ll << 31) && (long long)N * H * W * C * 2 < (1ll << 31) &&
                         !may_overlap(out, w);
@@ -2546,17 +2575,6 @@ TraceaStatus run_conv_transpose_by_phase(const ConvTransposePlan &plan, const Ep
   f.out = filt;
   TraceaStatus st = regroup ? hip_status("phase filter launch", launch_phase_filters(f, stream)) : TRACEA_SUCCESS;
   const long long x_extent = (long long)N * H * W * C * 2;
-  // Phases that are alike but for their padding (even filter extents divided by the stride: the 4x4
-  // stride-2 decoder layer) go out as one launch with the phase in blockIdx.z.
-  bool uniform = sh <= 4 && sw <= 4 && sh * sw > 1;
-  for (int a = 1; a < sh && uniform; ++a) {
-    const PhaseAxis p0 = phase_axis(0, sh, plan.pad_h, R, Ho), pa = phase_axis(a, sh, plan.pad_h, R, Ho);
-    uniform = p0.taps == pa.taps && p0.out == pa.out;
-  }
-  for (int b = 1; b < sw && uniform; ++b) {
-    const PhaseAxis p0 = phase_axis(0, sw, plan.pad_w, S, Wo), pb = phase_axis(b, sw, plan.pad_w, S, Wo);
-    uniform = p0.taps == pb.taps && p0.out == pb.out;
-  }
   for (int a = 0; a < sh && st == TRACEA_SUCCESS; ++a)
     for (int b = 0; b < sw && st == TRACEA_SUCCESS; ++b) {
       if (uniform && (a > 0 || b > 0)) continue;  // phase (0, 0) launched all of them
