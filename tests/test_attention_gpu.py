@@ -383,3 +383,18 @@ def test_first_scores_far_below_zero(tracea_gpu, dtype, d, member):
                 assert_close_scaled(got, want, _tol(d, dtype), "%s %s causal=%s" % (member, what, causal))
         finally:
             capi.force_variant("attention", -1)
+
+
+# heads, keys, head dimension, member: one workgroup per CU exactly (256), both sides of the lines in S, numbers of workgroups that
+# no 8 divides, up to one per CU (231, 252, 148) and beyond (290: a causal launch keeps its order there)
+@pytest.mark.parametrize("case", [(32, 1024, 64, "q128_kv64_d64_k2"), (40, 640, 64, "q128_kv64_d64_pipe2"), (24, 1024, 128, "q128_kv64_d128_pipe2"),
+                                  (21, 700, 128, "q64_kv64_d128_k2"), (36, 400, 128, "q64_kv64_d128_k2"), (37, 450, 96, "q128_kv64_part96"),
+                                  (29, 1200, 64, "q128_kv64_d64_pipe2"), (3, 130, 64, "q128_kv64_d64_pipe2")])
+@pytest.mark.parametrize("causal", [False, True])
+def test_rule_and_block_order(tracea_gpu, case, causal):
+    from tracea_amd import capi
+    h, s, d, member = case
+    q, k, v = _inputs(1, h, s, d, h + s, round_f16)
+    got = tracea_gpu.attention(_dev(q, torch.float16), _dev(k, torch.float16), _dev(v, torch.float16), causal=causal)
+    assert capi.last_variant("attention") == "fa2_" + member
+    assert_close_scaled(got.float().cpu().numpy(), oracle.attention_bhsd(q, k, v, 1.0 / np.sqrt(d), causal), _tol(d, "f16"), str(case))

@@ -2874,13 +2874,18 @@ TraceaStatus dispatch_attention(const TraceaTensorView &tq, const TraceaTensorVi
     return -1;
   };
   const long long cus = device_limits().cus, bh = (long long)(B * H);
-  // Launches that leave CUs idle: the keys of a block shared by groups of waves.  Replayed graphs, default / groups, us:
-  // 64 queries at head dimension up to 64, four groups, H12 S1024 13.3 / 10.1, H8 S2048 21.9 / 13.6, H12 S512 8.4 / 7.7, but
-  // S300 6.8 / 6.9 and S256 6.0 / 6.3; 64 queries at up to 128, two groups, H12 S1024 18.4 / 15.2, S512 11.4 / 10.4, S256
-  // 8.2 / 7.9 (under a causal mask S289 8.3 / 8.9).  Where those blocks of 64 would come in a second round, blocks of 128 on two groups: H8 S4096 D64 43.9 / 39.3
-  // (of 64: 46.3).
-  if (vi < 0 && bh * ((S + 63) / 64) <= cus && S > (D > 64 && !a.causal ? 192 : 384)) vi = D <= 64 ? member(64, 8, 1, 4) : member(64, 4, 1, 2);
-  if (vi < 0 && bh * ((S + 127) / 128) < cus && S > 512) vi = member(128, 8, 1, 2);
+  // Launches that leave CUs idle: the keys of a block shared by groups of waves.  Replayed graphs, default / groups, us.
+  // Blocks of 64 queries, at head dimension up to 64 on four groups: H12 S1024 13.3 / 10.1, H8 S2048 21.9 / 13.6, H12 S512
+  // 8.4 / 7.7, H36 S400 8.7 / 8.6, but S300 7.7 / 8.1 and S256 6.9 / 7.5; above on two: H12 S1024 D128 18.4 / 15.2, S512
+  // 11.4 / 10.4, dense S256 9.0 / 8.6 (under a causal mask S300 9.4 / 10.0), D96 S512 10.5 / 10.3, but S400 9.6 / 9.8.
+  // Where those blocks would come in a second round, blocks of 128 on two groups: H8 S4096 D64 47.8 / 45.1, causal 40.3 /
+  // 35.3, H31 S1024 15.6 / 15.3, but S640 10.6 / 10.7; D128 H8 S4096 71.4 / 70.0, causal 56.9 / 52.5, H16 S1536 causal
+  // 24.3 / 23.3, dense 25.5 / 25.6, but H24 S1024 19.0 / 19.6 and H40 S640 14.7 / 15.7.
+  const long long blocks64 = bh * ((S + 63) / 64), blocks128 = bh * ((S + 127) / 128);
+  const long long from64 = D <= 64 ? 384 : D < 128 ? 448 : a.causal ? 384 : 192;
+  const long long from128 = D <= 64 ? 640 : a.causal ? 1280 : 1792;
+  if (vi < 0 && blocks64 <= cus && S > from64) vi = D <= 64 ? member(64, 8, 1, 4) : member(64, 4, 1, 2);
+  if (vi < 0 && blocks128 <= cus && S > from128) vi = member(128, 8, 1, 2);
   // Two query blocks per workgroup where the pairs alone fill the device: the second block starts on tiles and
   // queries already requested, and under a causal mask a heavy block is paired with a light one.  Sweep over
   // B*H in {8, 32, 128, 512} and S in {512 ... 8192}, replayed graphs: with at least one pair per CU the paired
