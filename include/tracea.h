@@ -339,7 +339,8 @@ int32_t tracea_last_split_k_launches(void);
  * operator (fp32 accumulation in a different order). */
 void tracea_set_conv_transpose_by_phase(int32_t enabled);
 /* The by-phase formulation regroups the filter bank at every call (one helper launch), except a bank whose output
- * channels lie side by side with a multiple of 64 input channels, which it reads where it lies.  With the filter
+ * channels lie side by side with a multiple of 64 input channels, which it reads where it lies (not for large layers,
+ * where the regrouped bank is faster by more than the launch takes).  With the filter
  * cache on, the regrouped bank of a (device, filter pointer, shape, strides, stride, padding) is built once,
  * kept in device memory of its own and reused by later calls, which then launch nothing but the phase
  * convolutions and allocate nothing: for callers whose filters do not change between calls (inference).

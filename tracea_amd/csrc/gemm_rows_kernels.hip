@@ -91,7 +91,7 @@ __global__ void __launch_bounds__(WAVES * 64) gemm_rows_kernel(const Contraction
     }
   }
   const int pieces = (K + 63) / 64;
-  const int mine = (pieces - wave + WAVES - 1) / WAVES;  // pieces wave, wave + 8, ...
+  const int mine = (pieces - wave + WAVES - 1) / WAVES;  // pieces wave, wave + WAVES, ...
 #pragma unroll
   for (int t = 0; t < DEPTH; ++t) request(t, t);
   int slot = 0;
