@@ -2035,11 +2035,15 @@ void fast_epilogue_form(const EpilogueChain &chain, int dtype, ContractionArgs *
 }
 
 // Plan of the kernel for few output pixels (pipeline 11): K-contiguous filters, input and filters below 2 GiB.
+bool conv_private16_takes(const ConvGeometry &g, bool w_ncontig) {
+  const TraceaConvParamsBlock &b = g.block;
+  return !w_ncontig && b.c_in % 8 == 0 && (long long)b.batch * b.h_in * b.w_in * b.c_in * 2 < (1ll << 31) &&
+         (long long)g.n_gemm * g.k_gemm * 2 < (1ll << 31);
+}
 bool plan_conv_private16(const ConvGeometry &g, const ContractionVariant &v, bool w_ncontig, ContractionArgs *a) {
   const TraceaConvParamsBlock &b = g.block;
-  if (v.pipeline != 11 || w_ncontig || b.c_in % 8 != 0) return false;
+  if (v.pipeline != 11 || !conv_private16_takes(g, w_ncontig)) return false;
   const long long x_bytes = (long long)b.batch * b.h_in * b.w_in * b.c_in * 2, w_bytes = (long long)g.n_gemm * g.k_gemm * 2;
-  if (x_bytes >= (1ll << 31) || w_bytes >= (1ll << 31)) return false;
   a->grid_m = (g.m_gemm + v.bm - 1) / v.bm;
   a->grid_n = (g.n_gemm + v.bn - 1) / v.bn;
   if ((long long)a->grid_m * a->grid_n >= (1ll << 31)) return false;
@@ -2096,10 +2100,11 @@ TraceaStatus run_conv(const ConvPlan &plan, const EpilogueChain &chain, hipStrea
   // (an output that is also the input works where one workgroup reads all of what it overwrites: not on these tiles; K is
   // split over the waves, so the switch of the split along K holds)
   const long long cus = device_limits().cus;
-  const bool few_pixels = by_rule && g_split_k_enabled.load() && !may_overlap(plan.out, plan.x);
-  auto private_wgs = [&](const ContractionVariant &cv) -> long long {  // 0: cannot run the call
-    ContractionArgs probe = a;
-    return cv.pipeline == 11 && plan_conv_private16(g, cv, plan.w_ncontig, &probe) ? (long long)probe.grid_m * probe.grid_n : 0;
+  // (32x32 tiles beyond two per CU: no member, and nothing more to ask of the launch)
+  const bool few_pixels = by_rule && g_split_k_enabled.load() && conv_private16_takes(g, plan.w_ncontig) &&
+                          ((a.M + 31ll) / 32) * ((a.N + 31ll) / 32) <= 2 * cus && !may_overlap(plan.out, plan.x);
+  auto private_wgs = [&](const ContractionVariant &cv) -> long long {  // 0: another kernel
+    return cv.pipeline == 11 ? ((a.M + cv.bm - 1ll) / cv.bm) * ((a.N + cv.bn - 1ll) / cv.bn) : 0;
   };
   if (few_pixels) {
     long long best_tile = 0;
