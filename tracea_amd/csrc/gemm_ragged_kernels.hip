@@ -7,8 +7,10 @@
 // four waves may share a tile: they take the K tiles in turn, each with stages and sums of its own, added through LDS at
 // the end.  M 1000 N 900 K 1030 11.8 us (f16, replayed graph) against 24.7 from padded copies of both operands.
 //
-// Bound by the address path: a load off a dword takes a cycle per lane where an aligned one takes four lanes (M = N =
-// 100, K 5000 on one workgroup per CU and four groups: 0.19 us per K tile on rows that start on a dword, 0.38 off it).
+// Bound by the walk over K: nine rounds per group at that size, each a store to LDS, a barrier and a multiply, with the
+// matrix pipe busy for 8 % of the launch and a third of the wave cycles waiting on an instruction.  Of that the address
+// path is about 3 us: a load off a dword takes a cycle per lane where an aligned one takes four lanes (M = N = 100, K 5000
+// on one workgroup per CU and four groups: 0.19 us per K tile on rows that start on a dword, 0.38 off it).
 // Aligned loads of the dwords around a piece, joined in registers, cost the same cycles again (32 us against 33 there,
 // 43 against 33 with one group).
 //
