@@ -398,3 +398,25 @@ def test_rule_and_block_order(tracea_gpu, case, causal):
     got = tracea_gpu.attention(_dev(q, torch.float16), _dev(k, torch.float16), _dev(v, torch.float16), causal=causal)
     assert capi.last_variant("attention") == "fa2_" + member
     assert_close_scaled(got.float().cpu().numpy(), oracle.attention_bhsd(q, k, v, 1.0 / np.sqrt(d), causal), _tol(d, "f16"), str(case))
+
+
+# Causal launches beyond one workgroup per CU take the last query block of 64 heads at a time first.  One group of heads and a
+# smaller one, several groups with 4 heads left, numbers that 4 but not 8 divides, and one that keeps the old order (67): each
+# head's rows are the bits that a launch of that head alone gives, so every block ran once and in its place.
+@pytest.mark.parametrize("b,h,s", [(1, 12, 2900), (1, 36, 1030), (1, 68, 600), (2, 66, 300), (3, 64, 200), (1, 67, 600)])
+@pytest.mark.parametrize("d", [64, 96, 128])
+def test_heaviest_blocks_first(tracea_gpu, b, h, s, d):
+    from tracea_amd import capi
+    g = torch.Generator(device="cuda").manual_seed(b * h + s + d)
+    q, k, v = (torch.randn(b, h, s, d, device="cuda", generator=g).half() for _ in range(3))
+    out = torch.full_like(q, float("nan"))
+    capi.force_variant("attention", "fa2_q128_kv64_part96" if d == 96 else "fa2_q128_kv64_d%d_pipe2" % d)
+    try:
+        tracea_gpu.attention(q, k, v, causal=True, out=out)
+        for bi in range(b):
+            for hi in range(0, h, 5 if h > 12 else 1):
+                one = [t[bi:bi + 1, hi:hi + 1] for t in (q, k, v)]
+                assert torch.equal(tracea_gpu.attention(*one, causal=True)[0, 0], out[bi, hi]), (bi, hi)
+    finally:
+        capi.force_variant("attention", -1)
+    assert not torch.isnan(out).any()

@@ -484,8 +484,21 @@ fa2_fwd_pipe_kernel(const AttentionArgs a) {
   const bool runs = (total & 7) == 0 || !a.causal || total <= 256;
   const int xcd = blockIdx.x & 7;
   const int vid = runs ? xcd * (total >> 3) + min(xcd, total & 7) + ((int)blockIdx.x >> 3) : (int)blockIdx.x;
-  const int bh = vid / per_bh;
-  const int slot = vid - bh * per_bh;
+  // Under a causal mask and beyond one workgroup per CU: the last query block of every head, then the one before, and so on,
+  // so that what is left at the end is the lightest (B4 H12 S1500 D128 39.1 -> 35.5 us, B2 H32 S1400 D64 30.5 -> 24.3).  Heads
+  // that are a multiple of 4 in number keep to one or two XCDs so (others would visit all: B3 H31 S4096 D128 489 us against
+  // 365 in pairs), 64 of them at a time, whose K and V an XCD's L2 then serves (all 256 at once: B8 H32 S2048 D128 333 us
+  // against 279).
+  const int heads = a.B * a.H;
+  int bh, slot;
+  if (ITEMS == 1 && a.causal && total > 256 && (heads & 3) == 0) {
+    const int first = (int)blockIdx.x / (64 * per_bh) * 64, r = (int)blockIdx.x - first * per_bh, n = min(64, heads - first);
+    slot = r / n;
+    bh = first + r - slot * n;
+  } else {
+    bh = vid / per_bh;
+    slot = vid - bh * per_bh;
+  }
   // the query block of item i: alone, from the last block to the first; in pairs, a heavy and a light one
   // under a causal mask and two neighbours otherwise
   auto item_block = [&](int i) __attribute__((always_inline)) -> int {

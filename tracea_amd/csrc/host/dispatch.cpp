@@ -2891,15 +2891,22 @@ TraceaStatus dispatch_attention(const TraceaTensorView &tq, const TraceaTensorVi
   const long long from128 = D <= 64 ? 640 : a.causal ? 1280 : 1792;
   if (vi < 0 && blocks64 <= cus && S > from64) vi = D <= 64 ? member(64, 8, 1, 4) : member(64, 4, 1, 2);
   if (vi < 0 && blocks128 <= cus && S > from128) vi = member(128, 8, 1, 2);
-  // Two query blocks per workgroup where the pairs alone fill the device: the second block starts on tiles and
-  // queries already requested, and under a causal mask a heavy block is paired with a light one.  Sweep over
-  // B*H in {8, 32, 128, 512} and S in {512 ... 8192}, replayed graphs: with at least one pair per CU the paired
-  // member wins or ties (causal B4 H32 S4096 D128 585 -> 553 us, B1 H32 S2048 63.8 -> 52.2; dense B4 H32 S4096
-  // 1002 -> 980 on eight waves), with fewer it loses (causal B1 H32 S1024 26.2 -> 30.1).
-  // (Dense attention no longer takes the pairs by rule: with the softmax shift folded into the score product,
+  // Under a causal mask, up to two workgroups per CU over a long sequence: the last block's walk over its keys is longer than
+  // a SIMD's share of all the work, so two groups share that as well.  H12 S4096 D64 45.2 / 36.7, D128 67.7 / 58.0, H8 S8192
+  // D64 95.5 / 79.0, H32 S2048 27.2 / 26.5 and 42.1 / 41.7, but H36 S1500 20.3 / 21.5, H40 S1024 14.3 / 15.1.
+  if (vi < 0 && a.causal && S >= 2048 && blocks128 > cus && blocks128 <= 2 * cus) vi = member(128, 8, 1, 2);
+  // Two query blocks per workgroup, a heavy one paired with a light one, fill the device evenly where their number is a
+  // multiple of two per CU, and start the second block on tiles already requested.  Single blocks, the heaviest first,
+  // need no such number.  Replayed graphs, pairs / single blocks, us: B4 H12 S1500 D64 29.0 / 22.2, D128 44.7 / 35.5, B4 H32
+  // S700 D128 32.4 / 29.6, B2 H18 S4096 D64 114.1 / 88.2, B4 H32 S4096 D128 492.7 / 487.9, B8 H32 S2048 280.7 / 278.6; in
+  // full rounds over short sequences the pairs keep ahead: B8 H32 S512 D64 19.8 / 21.2, D128 32.1 / 33.1, S1024 D128 82.8 / 84.7.
+  // Heads that are no multiple of 4 come in their old order, and in pairs wherever these fill the device (B3 H31 S2048 D128
+  // 105.6 against 136.8 with the heaviest blocks of all heads first).
+  // (Dense attention does not take the pairs by rule: with the softmax shift folded into the score product,
   // which the paired members at head dimension 128 have no registers for, the one-block eight-wave member below
   // is ahead -- B4 H32 S4096 D128 904 us against 964, B8 H32 S2048 D64 294 against 302, same box.)
-  if (vi < 0 && a.causal && bh * (((S + 127) / 128) / 2) >= cus) vi = member(128, 4, 2);
+  const long long pairs = bh * (((S + 127) / 128) / 2);
+  if (vi < 0 && a.causal && pairs >= cus && (bh % 4 != 0 || (S <= 1024 && pairs % (2 * cus) == 0))) vi = member(128, 4, 2);
   // Dense attention over a long sequence with enough workgroups to go round: 256 queries on eight waves share
   // every K/V tile (B4 H32 S4096 D128: 997-999 us against 1013 for 128 queries on four).  Under a causal mask
   // the smaller block wins (584 against 624 us: less masked work on the diagonal, finer load balance).
