@@ -1655,6 +1655,20 @@ TraceaStatus conv_common(const TraceaTensorView &tx, const TraceaTensorView &tw,
   return TRACEA_SUCCESS;
 }
 
+// The most output rows that one of an image's tiles of t pixels spans (tiles start at multiples of t).  The walk over the tiles
+// ends at the first that spans as many as t pixels can.  The plans below ask for it tile size by tile size, and only
+// where the rows of the first tile fit (a filter slab that leaves no room for any patch is refused at once): walked to
+// the end for every size, a call of 4x 112x112 64->128 5x5 or 7x7 waited 213 us for the host beside kernels of 34 and 52.
+long long most_rows_spanned(int hw, int w_out, int t) {
+  const int most = (t - 2 + w_out) / w_out + 1;
+  int rows = 1;
+  for (int p0 = 0; p0 < hw && rows < most; p0 += t) {
+    const int span = (std::min(p0 + t, hw) - 1) / w_out - p0 / w_out + 1;
+    rows = std::max(rows, span);
+  }
+  return rows;
+}
+
 // Fills the patch-resident convolution fields of `a` for variant `v` and sets
 // the grid; false when the kernel cannot run this problem (then nothing the
 // caller relies on has been changed).
@@ -1748,12 +1762,7 @@ bool plan_conv_filter_resident(const ConvGeometry &g, const ContractionVariant &
   long long rows = 0, iters = 0, patch_bytes = 0;
   for (;;) {
     // most output rows one of the image's tiles spans (tiles start at multiples of tm_fit), then padded input rows
-    long long out_rows = 1;
-    for (int p0 = 0; p0 < hw; p0 += tm_fit) {
-      const int last = (p0 + tm_fit < hw ? p0 + tm_fit : hw) - 1;
-      const long long span = last / b.w_out - p0 / b.w_out + 1;
-      if (span > out_rows) out_rows = span;
-    }
+    const long long out_rows = most_rows_spanned(hw, b.w_out, tm_fit);
     rows = (out_rows - 1) * g.stride_h + (long long)(b.r_sz - 1) * g.dil_h + 1;
     iters = (rows * seg + 7) / 8;
     patch_bytes = (rows * pw * cpp + 1) * 16;  // (+1: the repeated first part behind the last pixel)
@@ -1819,13 +1828,7 @@ bool plan_conv_wave16(const ConvGeometry &g, const ContractionVariant &v, bool w
   const int seg = (int)((pw + ppi - 1) / ppi);
   // LDS bytes of the patch of the worst tile when tiles hold t pixels (tiles start at multiples of t): the
   // most output rows a tile spans, then padded input rows
-  auto patch_for = [&](int t) -> long long {
-    long long out_rows = 1;
-    for (int p0 = 0; p0 < hw; p0 += t) {
-      const int last = (p0 + t < hw ? p0 + t : hw) - 1;
-      const long long span = last / b.w_out - p0 / b.w_out + 1;
-      if (span > out_rows) out_rows = span;
-    }
+  auto patch_of = [&](long long out_rows) -> long long {
     const long long rows = (out_rows - 1) * g.stride_h + (long long)(b.r_sz - 1) * g.dil_h + 1;
     const long long bytes = (rows * pw * cpp + 64) * 16;
     return (bytes + 1023) / 1024 * 1024;
@@ -1833,13 +1836,17 @@ bool plan_conv_wave16(const ConvGeometry &g, const ContractionVariant &v, bool w
   const long long room = (long long)device_limits().lds_bytes - filter_bytes - table_bytes;
   // the largest tile up to the balanced one that fits; failing that (few, wide rows: a smaller tile still
   // straddles two rows) the smallest larger one
+  if (patch_of(1) > room) return false;
+  auto fits = [&](int t) {
+    return patch_of((t - 1) / b.w_out + 1) <= room && patch_of(most_rows_spanned(hw, b.w_out, t)) <= room;
+  };
   int tm_fit = 0;
   for (int t = tm < v.bm ? tm : v.bm; t >= 16 && tm_fit == 0; --t)
-    if (patch_for(t) <= room) tm_fit = t;
+    if (fits(t)) tm_fit = t;
   for (int t = tm + 1; t <= v.bm && t <= hw && tm_fit == 0; ++t)
-    if (patch_for(t) <= room) tm_fit = t;
+    if (fits(t)) tm_fit = t;
   if (tm_fit == 0) return false;
-  const long long patch_bytes = patch_for(tm_fit);
+  const long long patch_bytes = patch_of(most_rows_spanned(hw, b.w_out, tm_fit));
   a->r_sz = b.r_sz;
   a->p_tm = tm_fit;
   a->p_tiles = (hw + tm_fit - 1) / tm_fit;
@@ -1888,22 +1895,20 @@ bool plan_conv_ksplit16(const ConvGeometry &g, const ContractionVariant &v, bool
   const long long row_chunks = pw * cpp;
   if (row_chunks >= (1ll << 20)) return false;
   const int seg = (int)((row_chunks + 63) / 64);
-  auto patch_for = [&](int t) -> long long {
-    long long out_rows = 1;
-    for (int p0 = 0; p0 < hw; p0 += t) {
-      const int last = (p0 + t < hw ? p0 + t : hw) - 1;
-      const long long span = last / b.w_out - p0 / b.w_out + 1;
-      if (span > out_rows) out_rows = span;
-    }
+  auto patch_of = [&](long long out_rows) -> long long {
     const long long rows = (out_rows - 1) * g.stride_h + (long long)(b.r_sz - 1) * g.dil_h + 1;
     return (rows * row_chunks * 16 + 1023) / 1024 * 1024;
   };
   const long long room = (long long)device_limits().lds_bytes - ring_bytes - table_bytes;
+  if (patch_of(1) > room) return false;
+  auto fits = [&](int t) {
+    return patch_of((t - 1) / b.w_out + 1) <= room && patch_of(most_rows_spanned(hw, b.w_out, t)) <= room;
+  };
   int tm_fit = 0;
   for (int t = tm < v.bm ? tm : v.bm; t >= 16 && tm_fit == 0; --t)
-    if (patch_for(t) <= room) tm_fit = t;
+    if (fits(t)) tm_fit = t;
   for (int t = tm + 1; t <= v.bm && t <= hw && tm_fit == 0; ++t)
-    if (patch_for(t) <= room) tm_fit = t;
+    if (fits(t)) tm_fit = t;
   if (tm_fit == 0) return false;
   a->r_sz = b.r_sz;
   a->p_tm = tm_fit;
@@ -1911,7 +1916,7 @@ bool plan_conv_ksplit16(const ConvGeometry &g, const ContractionVariant &v, bool
   a->p_pw = (int)pw;
   a->p_cpp = cpp;
   a->p_iters = 0;
-  a->p_np_bytes = (int)patch_for(tm_fit);
+  a->p_np_bytes = (int)patch_of(most_rows_spanned(hw, b.w_out, tm_fit));
   a->p_seg = seg;
   a->p_ppi = 0;
   magic_for_divisor((uint32_t)cpp, (uint64_t)seg * 64, &a->p_cpp_m, &a->p_cpp_s);
@@ -1949,12 +1954,7 @@ bool plan_conv_thin8(const ConvGeometry &g, const ContractionVariant &v, bool w_
   const int hw = b.h_out * b.w_out;
   const int grid_n = (g.n_gemm + v.bn - 1) / v.bn;
   auto patch_for = [&](int t) -> long long {
-    long long out_rows = 1;
-    for (int p0 = 0; p0 < hw; p0 += t) {
-      const int last = (p0 + t < hw ? p0 + t : hw) - 1;
-      const long long span = last / b.w_out - p0 / b.w_out + 1;
-      if (span > out_rows) out_rows = span;
-    }
+    const long long out_rows = most_rows_spanned(hw, b.w_out, t);
     const long long rows = (out_rows - 1) * g.stride_h + (long long)(b.r_sz - 1) * g.dil_h + 1;
     return (rows * rp * 16 + 1023) / 1024 * 1024;
   };
