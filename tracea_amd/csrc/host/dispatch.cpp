@@ -2898,15 +2898,16 @@ TraceaStatus dispatch_attention(const TraceaTensorView &tq, const TraceaTensorVi
   // Two query blocks per workgroup, a heavy one paired with a light one, fill the device evenly where their number is a
   // multiple of two per CU, and start the second block on tiles already requested.  Single blocks, the heaviest first,
   // need no such number.  Replayed graphs, pairs / single blocks, us: B4 H12 S1500 D64 29.0 / 22.2, D128 44.7 / 35.5, B4 H32
-  // S700 D128 32.4 / 29.6, B2 H18 S4096 D64 114.1 / 88.2, B4 H32 S4096 D128 492.7 / 487.9, B8 H32 S2048 280.7 / 278.6; in
-  // full rounds over short sequences the pairs keep ahead: B8 H32 S512 D64 19.8 / 21.2, D128 32.1 / 33.1, S1024 D128 82.8 / 84.7.
+  // S700 D128 32.4 / 29.6, B2 H18 S4096 D64 114.1 / 88.2, B4 H32 S4096 D128 492.7 / 487.9; in full rounds over sequences up
+  // to 2048 the pairs are ahead or level: B8 H32 S512 D64 19.8 / 21.2, D128 32.1 / 33.1, S1024 D128 82.8 / 84.7, B4 H32 S2048
+  // 135.2 / 135.5.
   // Heads that are no multiple of 4 come in their old order, and in pairs wherever these fill the device (B3 H31 S2048 D128
   // 105.6 against 136.8 with the heaviest blocks of all heads first).
   // (Dense attention does not take the pairs by rule: with the softmax shift folded into the score product,
   // which the paired members at head dimension 128 have no registers for, the one-block eight-wave member below
   // is ahead -- B4 H32 S4096 D128 904 us against 964, B8 H32 S2048 D64 294 against 302, same box.)
   const long long pairs = bh * (((S + 127) / 128) / 2);
-  if (vi < 0 && a.causal && pairs >= cus && (bh % 4 != 0 || (S <= 1024 && pairs % (2 * cus) == 0))) vi = member(128, 4, 2);
+  if (vi < 0 && a.causal && pairs >= cus && (bh % 4 != 0 || (S <= 2048 && pairs % (2 * cus) == 0))) vi = member(128, 4, 2);
   // Dense attention over a long sequence with enough workgroups to go round: 256 queries on eight waves share
   // every K/V tile (B4 H32 S4096 D128: 997-999 us against 1013 for 128 queries on four).  Under a causal mask
   // the smaller block wins (584 against 624 us: less masked work on the diagonal, finer load balance).
