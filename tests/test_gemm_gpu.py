@@ -479,3 +479,32 @@ def test_output_over_an_operand(tracea_gpu, dtype, shape):
         x = _dev(a, tdt)
         tracea_gpu.gemm(x, _dev(b, tdt), out=x)
         assert_close_scaled(x.float().cpu().numpy(), ref, tol_half(n, dtype), "in place %s" % (shape,))
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("kind", ["gelu", "silu", "bias+silu"])
+@pytest.mark.parametrize("n", [128, 120])  # whole tiles (the row body with the short forms) and partial ones (the general one)
+def test_activations_over_the_whole_range(tracea_gpu, dtype, kind, n):
+    """Every row holds one value x in all columns: zero, tiny, the range in which the activation bends, where its exponential
+    leaves fp32, the type's largest, infinities and NaN, against the formula in float64.  Three units of fp32 in the
+    exponential's argument (up to 2^8 before it overflows) and half a unit of the stored type; results below the
+    smallest normal number of fp32 or the type count as that small."""
+    big = torch.finfo(dtype).max
+    x = torch.cat([torch.tensor([0.0, -0.0, big, -big, float("inf"), float("-inf"), float("nan")]), torch.linspace(-20, 20, 641),
+                   torch.tensor([1.0, -1.0]).repeat_interleave(20) * torch.logspace(-6, 4, 20).repeat(2)]).to(dtype)
+    a = torch.zeros(x.numel(), 64, dtype=dtype)
+    a[:, 3] = x
+    b = torch.zeros(64, n, dtype=dtype)
+    b[3] = 1
+    kw = {"bias": torch.zeros(n).cuda()} if "bias" in kind else {}
+    got = tracea_gpu.gemm(a.cuda(), b.cuda(), epilogue=kind, **kw).double().cpu()
+    v = x.double()
+    want = 0.5 * v * (1 + torch.tanh(0.79788456 * (v + 0.044715 * v ** 3))) if kind == "gelu" else v / (1 + torch.exp(-v))
+    v, want = v[:, None].expand_as(got), want[:, None].expand_as(got)
+    assert torch.equal(torch.isnan(got), torch.isnan(want))
+    assert torch.equal(got[torch.isinf(want)], want[torch.isinf(want)])
+    fin = torch.isfinite(want)
+    half_unit = 2.0 ** -11 if dtype == torch.float16 else 2.0 ** -8
+    # (1 + tanh cancels below zero in the general body: an absolute error of two units of fp32 times |x|)
+    bound = want.abs() * (half_unit + 3 * 2.0 ** -16) + v.abs() * 2.0 ** -22 + max(torch.finfo(dtype).tiny * half_unit, 2.0 ** -126)
+    assert bool(((got - want).abs() <= bound)[fin].all())

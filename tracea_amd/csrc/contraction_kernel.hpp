@@ -149,6 +149,23 @@ __device__ __forceinline__ void load_as_float(const void *base, int dtype, long 
   }
 }
 
+// GELU (tanh form) and SiLU for results that are then rounded to 16 bits: 0.5 x (1 + tanh(u)) = x / (1 + exp(-2 u)) with
+// u = 0.79788456 (x + 0.044715 x^3), and x / (1 + exp(-x)), both x / (1 + 2^(x (c1 + c3 x^2))) with the constants below.  The
+// hardware's exp2 and reciprocal, one unit in the last place of fp32 each, in nine instructions a value, where the library's
+// tanhf, expf and the division take some fifty (f16 3328x2560x768 with GELU 47.5 -> 34.9 us,
+// 16384x3072x768 144.5 -> 103.1, where the product alone takes 30.3 and 83.7).  Infinities and NaN come out as from those;
+// the square is held below infinity for SiLU's c3 = 0.
+struct HalfActivation {
+  float c1, c3;
+};
+__device__ __forceinline__ HalfActivation half_activation(int kind) {
+  return kind == TRACEA_EPI_OP_GELU ? HalfActivation{-2.3022082f, -0.10294324f} : HalfActivation{-1.4426950f, 0.0f};
+}
+__device__ __forceinline__ float activate_half(float x, HalfActivation f) {
+  const float t = x * fmaf(f.c3, fminf(x * x, 1e30f), f.c1);
+  return x * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(t));
+}
+
 // Applies one operator to V consecutive channels n..n+V-1 of output row m
 // (fp32 in, fp32 out), reading its operands from global memory.
 template <int V>
@@ -343,7 +360,7 @@ __device__ __forceinline__ ChainPlan chain_plan(const EpilogueChain &chain) {
 // once) over kinds held in one scalar.
 __device__ __forceinline__ void apply_epilogue_tab(float (&v)[8], long long m, int n, int nvalid,
                                                    const EpilogueChain &chain, const ChainPlan &plan,
-                                                   const float *tab, int bn) {
+                                                   const float *tab, int bn, bool half_out) {
 #pragma nounroll
   for (int o = 0; o < plan.n_ops; ++o) {
     const int kind = (int)((plan.kinds >> (4 * o)) & 15u);
@@ -362,32 +379,41 @@ __device__ __forceinline__ void apply_epilogue_tab(float (&v)[8], long long m, i
         for (int e = 0; e < 8; ++e) v[e] = v[e] + a[e];
       } else if (kind == TRACEA_EPI_OP_BIAS_ADD_SILU) {
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          const float x = v[e] + a[e];
-          v[e] = x / (1.0f + expf(-x));
+        for (int e = 0; e < 8; ++e) v[e] = v[e] + a[e];
+        if (half_out) {
+          const HalfActivation f = half_activation(kind);
+#pragma unroll
+          for (int e = 0; e < 8; ++e) v[e] = activate_half(v[e], f);
+        } else {
+#pragma unroll
+          for (int e = 0; e < 8; ++e) v[e] = v[e] / (1.0f + expf(-v[e]));
         }
       } else {
 #pragma unroll
         for (int e = 0; e < 8; ++e) v[e] = v[e] * a[e] + b[e];
       }
+    } else if (half_out && (kind == TRACEA_EPI_OP_GELU || kind == TRACEA_EPI_OP_SILU)) {
+      const HalfActivation f = half_activation(kind);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[e] = activate_half(v[e], f);
     } else if (kind == TRACEA_EPI_OP_RESIDUAL_ADD && o == plan.res_index) {
       float t[8];
       load_as_float<8>(plan.res_ptr, plan.res_dtype, m * plan.res_ld + n, nvalid, t);
 #pragma unroll
       for (int e = 0; e < 8; ++e) v[e] = v[e] + t[e];
     } else {
-      apply_epilogue_one<8>(v, m, n, nvalid, chain.ops[o]);  // GELU, SiLU, a second residual
+      apply_epilogue_one<8>(v, m, n, nvalid, chain.ops[o]);  // GELU and SiLU in fp32, a second residual
     }
   }
 }
 
 // ---- specialised row body ------------------------------------------------------------
 // The general row body above carries every fallback inline (partial channel
-// vectors, unaligned rows, per-element loads and stores, GELU / SiLU): several
+// vectors, unaligned rows, per-element loads and stores, fp32 GELU / SiLU): several
 // thousand instructions and hundreds of branches per row, more than the
 // instruction cache holds.  Nearly every call needs none of it: all 8 channels
 // of every lane exist, rows of C (and of the residual) are 16-byte aligned, and
-// the chain is made of bias / scale-shift / BatchNorm / ReLU / one residual.
+// the chain is made of bias / scale-shift / BatchNorm / ReLU / GELU / SiLU / one residual.
 // Whether that holds is the same for the whole workgroup, so it is decided
 // once and the row loops are emitted twice, each behind a uniform branch.
 __device__ __forceinline__ bool chain_is_simple(const ChainPlan &plan, const ContractionCore &args, int n0, int bn) {
@@ -397,11 +423,22 @@ __device__ __forceinline__ bool chain_is_simple(const ChainPlan &plan, const Con
     const int kind = (int)((plan.kinds >> (4 * o)) & 15u);
     ok = ok && (kind == TRACEA_EPI_OP_NONE || kind == TRACEA_EPI_OP_BIAS_ADD || kind == TRACEA_EPI_OP_RELU ||
                 kind == TRACEA_EPI_OP_SCALE_SHIFT || kind == TRACEA_EPI_OP_BATCHNORM ||
+                (args.out_dtype != DT_F32 && (kind == TRACEA_EPI_OP_GELU || kind == TRACEA_EPI_OP_SILU || kind == TRACEA_EPI_OP_BIAS_ADD_SILU)) ||
                 (kind == TRACEA_EPI_OP_RESIDUAL_ADD && o == plan.res_index));
   }
   if (plan.res_index >= 0)
     ok = ok && plan.res_dtype != DT_F32 && (plan.res_ld & 7) == 0 && (((uintptr_t)plan.res_ptr) & 15) == 0;
   return ok;
+}
+
+__device__ __forceinline__ bool chain_activates(const ChainPlan &plan) {
+  bool any = false;
+#pragma unroll
+  for (int o = 0; o < TRACEA_MAX_EPILOGUE_OPS; ++o) {
+    const int kind = (int)((plan.kinds >> (4 * o)) & 15u);
+    any = any || kind == TRACEA_EPI_OP_GELU || kind == TRACEA_EPI_OP_SILU || kind == TRACEA_EPI_OP_BIAS_ADD_SILU;
+  }
+  return any;
 }
 
 // The specialised path for the 32 staged rows of one accumulator block: the
@@ -412,7 +449,8 @@ __device__ __forceinline__ bool chain_is_simple(const ChainPlan &plan, const Con
 // its staged values and one more per operator, back to back.
 // row_of(r) gives the output row of staged row r, or -1 if it does not exist.
 // F32OUT: C holds fp32 (two 16-byte stores per lane and row) instead of DT.
-template <int DT, int TN, bool F32OUT = false, typename RowOf>
+// ACT: GELU and SiLU among the operators (in every launch's body they cost ResNet-18 at batch 5 one percent).
+template <int DT, int TN, bool F32OUT = false, bool ACT = false, typename RowOf>
 __device__ __forceinline__ void simple_rows(const float *stage, int lane, int n, const ContractionCore &args,
                                             const ChainPlan &plan, const float *tab, int bn, RowOf row_of) {
   constexpr int EP_PITCH = TN + 4, LPR = TN / 8, RPI = 64 / LPR, NIT = 32 / RPI;
@@ -461,13 +499,13 @@ __device__ __forceinline__ void simple_rows(const float *stage, int lane, int n,
             for (int e = 0; e < 8; ++e) v[g][e] = v[g][e] + (float)h[e];
           }
         }
-      } else {  // bias: v + a; scale/shift and BatchNorm: v * a + b
+      } else if (!ACT || (kind != TRACEA_EPI_OP_GELU && kind != TRACEA_EPI_OP_SILU)) {  // bias: v + a; scale/shift and BatchNorm: v * a + b
         const float *pa = tab + (o * 2) * bn;
         const f32x4 a0 = *(const f32x4 *)pa, a1 = *(const f32x4 *)(pa + 4);
         const f32x4 b0 = *(const f32x4 *)(pa + bn), b1 = *(const f32x4 *)(pa + bn + 4);  // zeros for a bias
         const float a[8] = {a0[0], a0[1], a0[2], a0[3], a1[0], a1[1], a1[2], a1[3]};
         const float b[8] = {b0[0], b0[1], b0[2], b0[3], b1[0], b1[1], b1[2], b1[3]};
-        if (kind == TRACEA_EPI_OP_BIAS_ADD) {
+        if (kind == TRACEA_EPI_OP_BIAS_ADD || (ACT && kind == TRACEA_EPI_OP_BIAS_ADD_SILU)) {
 #pragma unroll
           for (int g = 0; g < GROUP; ++g)
 #pragma unroll
@@ -477,6 +515,15 @@ __device__ __forceinline__ void simple_rows(const float *stage, int lane, int n,
           for (int g = 0; g < GROUP; ++g)
 #pragma unroll
             for (int e = 0; e < 8; ++e) v[g][e] = v[g][e] * a[e] + b[e];
+        }
+      }
+      if constexpr (ACT) {  // (chain_is_simple lets these through for 16-bit results only)
+        if (kind == TRACEA_EPI_OP_GELU || kind == TRACEA_EPI_OP_SILU || kind == TRACEA_EPI_OP_BIAS_ADD_SILU) {
+          const HalfActivation f = half_activation(kind);
+#pragma unroll
+          for (int g = 0; g < GROUP; ++g)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) v[g][e] = activate_half(v[g][e], f);
         }
       }
     }
@@ -1600,9 +1647,10 @@ __global__ void __launch_bounds__(WM *WN * 64) contraction_kernel(const std::con
       auto row_of = [&](int r) -> long long { return mb + r < M ? out_row(mb + r) : -1ll; };
       if constexpr (F32_SIMPLE) {
         if (out_f32) simple_rows<DT, TN, true>(stage, lane, n0 + wn * TN + ec, args, plan, tab, BN, row_of);
+        else if (chain_activates(plan)) simple_rows<DT, TN, false, true>(stage, lane, n0 + wn * TN + ec, args, plan, tab, BN, row_of);
         else simple_rows<DT, TN, false>(stage, lane, n0 + wn * TN + ec, args, plan, tab, BN, row_of);
       } else {
-        simple_rows<DT, TN, false>(stage, lane, n0 + wn * TN + ec, args, plan, tab, BN, row_of);
+        simple_rows<DT, TN, false, true>(stage, lane, n0 + wn * TN + ec, args, plan, tab, BN, row_of);  // (one copy, see above)
       }
     } else {
       for (int r = er; r < 32; r += RPI) {
@@ -1619,7 +1667,7 @@ __global__ void __launch_bounds__(WM *WN * 64) contraction_kernel(const std::con
           }
           const int nvalid = N - n;
           const long long row = out_row(m);
-          apply_epilogue_tab(v, row, n, nvalid, args.epi, plan, tab, BN);
+          apply_epilogue_tab(v, row, n, nvalid, args.epi, plan, tab, BN, args.out_dtype != DT_F32);
           store_from_float<8>(args.C, args.out_dtype, row * args.ldc + n, nvalid, v);
         }
       }

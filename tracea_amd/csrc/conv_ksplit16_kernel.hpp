@@ -432,7 +432,7 @@ __global__ void __launch_bounds__(CK_THREADS) conv_ksplit16_kernel(const Contrac
       }
       const int nvalid = N - n;
       const long long m = m_img + pr;
-      apply_epilogue_tab(v, m, n, nvalid, args.epi, plan, table + ec, BN);
+      apply_epilogue_tab(v, m, n, nvalid, args.epi, plan, table + ec, BN, args.out_dtype != DT_F32);
       store_from_float<8>(args.C, args.out_dtype, m * args.ldc + n, nvalid, v);
     }
   }

@@ -279,8 +279,8 @@ __global__ void __launch_bounds__(WM *WN * 64) conv_patch_kernel(const Contracti
     __builtin_amdgcn_wave_barrier();
     if (simple) {
       const int pb = wm * TMW + i * 32;
-      simple_rows<DT, TN>(stage, lane, n0 + wn * TN + ec, args, plan, tab, BN,
-                          [&](int r) -> long long { return pb + r < npix ? m_img + pb + r : -1ll; });
+      auto row_of = [&](int r) -> long long { return pb + r < npix ? m_img + pb + r : -1ll; };
+      simple_rows<DT, TN, false, true>(stage, lane, n0 + wn * TN + ec, args, plan, tab, BN, row_of);  // (a second copy: 133 registers)
     } else {
       for (int r = er; r < 32; r += RPI) {
         const int pr = wm * TMW + i * 32 + r;
@@ -296,7 +296,7 @@ __global__ void __launch_bounds__(WM *WN * 64) conv_patch_kernel(const Contracti
           }
           const int nvalid = N - n;
           const long long m = m_img + pr;
-          apply_epilogue_tab(v, m, n, nvalid, args.epi, plan, tab, BN);
+          apply_epilogue_tab(v, m, n, nvalid, args.epi, plan, tab, BN, args.out_dtype != DT_F32);
           store_from_float<8>(args.C, args.out_dtype, m * args.ldc + n, nvalid, v);
         }
       }
