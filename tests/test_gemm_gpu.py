@@ -508,3 +508,33 @@ def test_activations_over_the_whole_range(tracea_gpu, dtype, kind, n):
     # (1 + tanh cancels below zero in the general body: an absolute error of two units of fp32 times |x|)
     bound = want.abs() * (half_unit + 3 * 2.0 ** -16) + v.abs() * 2.0 ** -22 + max(torch.finfo(dtype).tiny * half_unit, 2.0 ** -126)
     assert bool(((got - want).abs() <= bound)[fin].all())
+
+
+# four to eight elements in an operand, K on and off the 32-deep tiles, a last row of B within 4 elements of the end in the tile
+# before the last (N 1 and 3), two groups of waves with an even and an odd number of K tiles, more tiles than CUs (1100 x 1090)
+@pytest.mark.parametrize("shape", [(1, 5, 4), (4, 1, 33), (2, 3, 34), (65, 3, 66), (63, 65, 64), (64, 64, 95), (3, 130, 127), (70, 67, 321),
+                                   (129, 65, 577), (1100, 1090, 403)])
+def test_fp32_operands_at_any_element_alignment(tracea_gpu, shape):
+    """As above for fp32 with both operands by rows."""
+    m, n, k = shape
+    rng = np.random.default_rng(m + 3 * n + 7 * k)
+    a = (rng.standard_normal((m, k)) / np.sqrt(k)).astype(np.float32)
+    b = rng.standard_normal((k, n)).astype(np.float32)
+    bias = rng.standard_normal(n).astype(np.float32)
+    ref = np.maximum(oracle.gemm_f64(a, b) + bias[None, :], 0.0)
+
+    def placed(x, gap, first, junk):
+        rows, cols = x.shape
+        flat = torch.full((first + rows * (cols + gap) + 16,), junk, device="cuda")
+        v = torch.as_strided(flat, (rows, cols), (cols + gap, 1), first)
+        v.copy_(_dev(x))
+        return v
+
+    for gap, first in ((0, 1), (1, 0), (3, 2), (5, 3)):
+        for junk in (float("nan"), float("inf")):
+            out = torch.full((m + 1, n + 3), 7.0, device="cuda")
+            tracea_gpu.gemm(placed(a, gap, first, junk), placed(b, gap, first, junk), bias=_dev(bias), epilogue="bias+relu", out=out[:m, :n])
+            got = out.cpu().numpy()
+            # (k products and sums rounded to fp32, about 3 in absolute value at most for a row of A of unit length)
+            assert np.abs(got[:m, :n] - ref).max() <= 2.0 ** -24 * 2 * (k + 8) * max(1.0, np.abs(ref).max()), (gap, first)
+            assert (got[m] == 7.0).all() and (got[:, n:] == 7.0).all(), "outside the output"

@@ -154,6 +154,7 @@ int launch_gemm_rows(const ContractionArgs &args, int dtype, bool b_ncontig, int
 // Half-precision GEMM of operands at any element alignment (A by rows, B by rows or by columns, extents from 16 bytes
 // to 2 GiB in a_bytes / b_bytes) on tiles of `tile` (64 or 128) with K dealt to `groups` (1 or, 64 only, 2) groups of waves.
 int launch_gemm_ragged(const ContractionArgs &args, int dtype, bool b_ncontig, int tile, int groups, hipStream_t stream);
+int launch_gemm_ragged_f32(const ContractionArgs &args, int groups, hipStream_t stream);
 
 // fp32 MFMA GEMM (row-major A [M,K], row-major B [K,N]).
 int launch_gemm_f32(const ContractionArgs &args, int tile, hipStream_t stream);  // tile: 128, 64 or 6432 (64x64 with K tiles of 32)

@@ -246,4 +246,165 @@ int launch_gemm_ragged(const ContractionArgs &a, int dtype, bool b_ncontig, int 
   return dtype == DT_F16 ? launch_type<DT_F16>(a, b_ncontig, tile, groups, stream) : launch_type<DT_BF16>(a, b_ncontig, tile, groups, stream);
 }
 
+// The same for fp32, A and B by rows: K tiles of 32 through registers, DEPTH ahead, 64x64 of C per group of four waves, a wave
+// 32x32 of it on 32x32x2 MFMAs.  An MFMA's two k are its lane halves': half g takes k 16 g + j of the tile in MFMA j,
+// so that a lane reads four of them from a row of A at once.  1000x900x1030 28.9 us (replayed graph) against 42.8 from padded
+// copies of both operands, 33x65x16 6.4 against 11.0.  Bound by the walk over K: 0.7 us per K tile and group where a CU
+// has one workgroup, of which the MFMAs' issue is 0.43.  Four groups measured level with two (1000x900x1030).
+//
+// Reads stay inside the extents ((rows - 1) * pitch + row length, at least 4 elements) as above.
+typedef f32x4 f32x4_any __attribute__((aligned(4)));
+
+__device__ __forceinline__ f32x4 drop_front(f32x4 p, unsigned s) {
+  const f32x4 h = {p[1], p[2], p[3], 0.0f};
+  p = (s & 1) ? h : p;
+  const f32x4 w = {p[2], p[3], 0.0f, 0.0f};
+  return (s & 2) ? w : p;
+}
+__device__ __forceinline__ f32x4 keep_front(f32x4 p, int keep) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) p[i] = i < keep ? p[i] : 0.0f;
+  return p;
+}
+
+template <int GROUPS>
+__global__ void __launch_bounds__(GROUPS * 256) gemm_ragged_f32_kernel(const ContractionCore args) {
+  constexpr int T = 64, GT = 256, NP = 2, DEPTH = 4, NT = GROUPS * GT;
+  constexpr int A_PITCH = 36;                  // floats: 16 rows at one column lie in 16 different groups of four banks
+  constexpr int A_FLOATS = T * A_PITCH, STAGE = A_FLOATS + 32 * T, GROUP_FLOATS = 2 * STAGE;
+  constexpr int PITCH = T + 4;
+  static_assert(T * PITCH <= GROUP_FLOATS, "a group's sums go over its stages");
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  const int tid = threadIdx.x % GT, lane = threadIdx.x & 63, wave = tid >> 6;
+  const int group = __builtin_amdgcn_readfirstlane(threadIdx.x / GT);
+  const int wm = wave & 1, wn = wave >> 1, r = lane & 31, g = lane >> 5;
+  int tile_m, tile_n;
+  tile_coordinates(args, tile_m, tile_n);
+  const int m0 = tile_m * T, n0 = tile_n * T;
+  const int M = args.M, N = args.N, K = args.K;
+  const float *A = (const float *)args.A, *B = (const float *)args.B;
+  const unsigned a_last = args.a_bytes / 4 - 4, b_last = args.b_bytes / 4 - 4;  // where the last whole piece starts
+  const unsigned ldb = (unsigned)args.ldb;
+
+  unsigned a_off[NP], b_off[NP], a_dst[NP], b_dst[NP];
+#pragma unroll
+  for (int i = 0; i < NP; ++i) {
+    const int p = tid + i * GT, row = p >> 3, krow = p >> 4, cn = (p & 15) * 4;
+    a_off[i] = (unsigned)min(m0 + row, M - 1) * (unsigned)args.lda + (p & 7) * 4;
+    a_dst[i] = row * A_PITCH + (p & 7) * 4;
+    b_off[i] = (unsigned)krow * ldb + n0 + cn;
+    // (the two halves of a wave read rows 16 apart: the lower 16 rows have their two 32 columns exchanged)
+    b_dst[i] = A_FLOATS + krow * T + (cn ^ ((krow >> 4) << 5));
+  }
+  const int kcol = (tid & 7) * 4;
+
+  f32x4 ra[DEPTH][NP], rb[DEPTH][NP];
+  auto load = [&](int slot, int k0) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < NP; ++i) {
+      ra[slot][i] = *(const f32x4_any *)(A + min(a_off[i] + (unsigned)k0, a_last));
+      rb[slot][i] = *(const f32x4_any *)(B + min(b_off[i] + (unsigned)k0 * ldb, b_last));
+    }
+  };
+  auto store = [&](int slot, float *dst, int k0) __attribute__((always_inline)) {
+    f32x4 va[NP], vb[NP];
+#pragma unroll
+    for (int i = 0; i < NP; ++i) {
+      va[i] = ra[slot][i];
+      vb[i] = rb[slot][i];
+    }
+    if (k0 + 36 > K) {  // (a row of B within 4 elements of the end may need the shift in front of the last tile)
+#pragma unroll
+      for (int i = 0; i < NP; ++i) {
+        const unsigned oa = a_off[i] + (unsigned)k0, ob = b_off[i] + (unsigned)k0 * ldb;
+        va[i] = keep_front(drop_front(va[i], oa - min(oa, a_last)), K - k0 - kcol);
+        vb[i] = keep_front(drop_front(vb[i], ob - min(ob, b_last)), k0 + ((tid + i * GT) >> 4) < K ? 4 : 0);
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < NP; ++i) {
+      *(f32x4 *)(dst + a_dst[i]) = va[i];
+      *(f32x4 *)(dst + b_dst[i]) = vb[i];
+    }
+  };
+
+  f32x16 acc[4] = {};  // four chains of MFMAs: none waits for the one before, and the sums round less
+  float *const stages = (float *)smem + group * GROUP_FLOATS;
+  const int fa_at = (wm * 32 + r) * A_PITCH + g * 16;
+  const int fb_at = A_FLOATS + g * 16 * T + ((wn * 32 + r) ^ (g << 5));
+  auto multiply = [&](const float *st) __attribute__((always_inline)) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const f32x4 fa = *(const f32x4 *)(st + fa_at + j * 4);
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        acc[e] = __builtin_amdgcn_mfma_f32_32x32x2f32(st[fb_at + (j * 4 + e) * T], fa[e], acc[e], 0, 0, 0);
+    }
+  };
+
+  const int rounds = ((K + 31) / 32 + GROUPS - 1) / GROUPS;  // the same for every group, tiles of zeros behind the last one
+  auto k_of = [&](int t) { return min(t * GROUPS + group, rounds * GROUPS) * 32; };
+#pragma unroll
+  for (int d = 0; d < DEPTH; ++d) load(d, k_of(d));
+  auto round = [&](auto slot_c, int t) __attribute__((always_inline)) {
+    constexpr int slot = decltype(slot_c)::value;
+    float *st = stages + (t & 1) * STAGE;
+    store(slot, st, k_of(t));
+    load(slot, k_of(t + DEPTH));
+    // (as above: the stage's last readers passed the previous barrier, the loads stay in flight)
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    multiply(st);
+  };
+  for (int t = 0; t < rounds; ++t) {
+    round(std::integral_constant<int, 0>{}, t);
+    if (++t >= rounds) break;
+    round(std::integral_constant<int, 1>{}, t);
+    if (++t >= rounds) break;
+    round(std::integral_constant<int, 2>{}, t);
+    if (++t >= rounds) break;
+    round(std::integral_constant<int, 3>{}, t);
+  }
+  __syncthreads();
+  // a lane's registers 4 i .. 4 i + 3: row r, columns 8 i + 4 g .. + 3 of the wave's 32x32
+  const f32x16 sum = (acc[0] + acc[1]) + (acc[2] + acc[3]);
+  float *sums = stages + (wm * 32 + r) * PITCH + wn * 32 + g * 4;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) *(f32x4 *)(sums + i * 8) = f32x4{sum[4 * i], sum[4 * i + 1], sum[4 * i + 2], sum[4 * i + 3]};
+  __syncthreads();
+#pragma nounroll
+  for (int p = threadIdx.x; p < T * (T / 4); p += NT) {
+    const int row = p / (T / 4), n = n0 + (p % (T / 4)) * 4, m = m0 + row;
+    if (m >= M || n >= N) continue;
+    const float *src = (const float *)smem + row * PITCH + (p % (T / 4)) * 4;
+    f32x4 s = *(const f32x4 *)src;
+#pragma unroll
+    for (int o = 1; o < GROUPS; ++o) s += *(const f32x4 *)(src + o * GROUP_FLOATS);
+    float v[4] = {s[0], s[1], s[2], s[3]};
+    apply_epilogue<4>(v, m, n, N - n, args.epi);
+    store_from_float<4>(args.C, args.out_dtype, (long long)m * args.ldc + n, N - n, v);
+  }
+}
+
+template <int GROUPS>
+static int launch_f32_one(const ContractionArgs &a, hipStream_t stream) {
+  constexpr int lds = GROUPS * 2 * (64 * 36 + 32 * 64) * 4;
+  auto kfn = gemm_ragged_f32_kernel<GROUPS>;
+  static bool attr_done = false;
+  if (!attr_done) {
+    hipError_t e = hipFuncSetAttribute((const void *)kfn, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    if (e != hipSuccess) return (int)e;
+    attr_done = true;
+  }
+  hipLaunchKernelGGL(kfn, dim3((unsigned)(a.grid_m * a.grid_n)), dim3(GROUPS * 256), lds, stream, a);
+  return (int)hipGetLastError();
+}
+
+int launch_gemm_ragged_f32(const ContractionArgs &a, int groups, hipStream_t stream) {
+  if (a.M < 1 || a.N < 1 || a.K < 1 || a.a_bytes < 16 || a.b_bytes < 16) return (int)hipErrorInvalidValue;
+  return groups == 2 ? launch_f32_one<2>(a, stream) : launch_f32_one<1>(a, stream);
+}
+
 }  // namespace tracea_amd

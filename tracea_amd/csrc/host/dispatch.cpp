@@ -919,6 +919,30 @@ int ragged_tile(long long M, long long N, long long K, int *groups) {
   return 64;
 }
 
+// The same for fp32, A and B by rows.
+bool ragged_f32_layout(const View &a, const View &b, const View &c) {
+  const long long M = a.shape[0], K = a.shape[1], N = b.shape[1];
+  if (a.dtype != TRACEA_DTYPE_FLOAT32 || b.dtype != a.dtype || c.dtype != a.dtype || K <= 0) return false;
+  if (a.stride[1] != 1 || b.stride[1] != 1 || c.stride[1] != 1 || a.stride[0] < K || b.stride[0] < N) return false;
+  if ((((uintptr_t)a.ptr | (uintptr_t)b.ptr) & 3) != 0) return false;
+  const long long cap = 1ll << 29;  // elements
+  if (a.stride[0] >= cap || b.stride[0] >= cap || c.stride[0] < 0) return false;
+  const long long a_extent = (M - 1) * a.stride[0] + K, b_extent = (K - 1) * b.stride[0] + N;
+  return a_extent >= 4 && a_extent < cap && b_extent >= 4 && b_extent < cap;
+}
+
+// Its groups of waves that share K, or 0 where padded copies and the tile kernels are ahead.  us, replayed graphs, from copies /
+// in place: up to one tile per CU on two groups, unless so few workgroups walk a long K that the tile kernels split over the
+// device (33x65x16 11.0 / 6.4 with one group, 6.8 with two; 300x300x301 17.5 / 11.3, 1000x900x1030 42.8 / 28.9, but
+// 64x1000x1001 23.1 / 23.4, 500x500x1999 35.4 / 43.2, 100x100x2501 26.4 / 49.6); above on one group while the copies weigh
+// more than the tile kernels' higher rate (1300x1300x1301 74.0 / 62.6, 1700x900x1999 99.5 / 88.8, 1999x1999x501 65.5 / 53.2, but
+// 1501x1501x301 32.8 / 33.2, 1998x1048x195 26.4 / 27.2).
+int ragged_f32_groups(long long M, long long N, long long K) {
+  const long long tiles = ((M + 63) / 64) * ((N + 63) / 64), cus = device_limits().cus;
+  if (tiles <= cus) return K > 800 + 10 * tiles ? 0 : K > 32 ? 2 : 1;
+  return tiles <= 4 * cus && K > 400 && tiles * K <= cus * 3200 ? 1 : 0;
+}
+
 int variant_index(const char *name) {
   for (int i = 0; i < contraction_variant_count(); ++i)
     if (strcmp(contraction_variant(i).name, name) == 0) return i;
@@ -950,6 +974,23 @@ TraceaStatus run_gemm_any_alignment(const View &a, const View &b, const View &c,
   t_last_splits = groups;
   t_last_split_launches = 1;
   return hip_status("gemm launch", launch_gemm_ragged(args, a.dtype, b_ncontig, tile, groups, stream));
+}
+
+TraceaStatus run_gemm_f32_any_alignment(const View &a, const View &b, const View &c, const EpilogueChain &chain, int groups, hipStream_t stream) {
+  const long long M = a.shape[0], K = a.shape[1], N = b.shape[1];
+  ContractionArgs args{};
+  args.A = a.ptr; args.B = b.ptr; args.C = c.ptr;
+  args.M = (int)M; args.N = (int)N; args.K = (int)K;
+  args.lda = a.stride[0]; args.ldb = b.stride[0]; args.ldc = c.stride[0];
+  args.out_dtype = DT_F32;
+  args.epi = chain;
+  args.a_bytes = (unsigned)(((M - 1) * args.lda + K) * 4);
+  args.b_bytes = (unsigned)(((K - 1) * args.ldb + N) * 4);
+  static const ContractionVariant tile = {"f32_64x64x32", 64, 64, 32, 2, 2, 1, 0, 0, nullptr, 32};
+  fill_grid(&args, tile);
+  t_last_splits = groups;
+  t_last_split_launches = 1;
+  return hip_status("gemm_f32 launch", launch_gemm_ragged_f32(args, groups, stream));
 }
 
 TraceaStatus run_gemm(const View &a, const View &b, const View &c, const EpilogueChain &chain,
@@ -1120,6 +1161,10 @@ TraceaStatus run_gemm(const View &a, const View &b, const View &c, const Epilogu
     const int tile = ragged_tile(M, N, K, &groups);
     if (!g_split_k_enabled.load()) groups = 1;
     if (tile != 0) return run_gemm_any_alignment(a, b, c, chain, tile, groups, stream);
+  }
+  if (!in_padded && ragged_f32_layout(a, b, c) && !may_overlap(c, a) && !may_overlap(c, b)) {
+    const int groups = ragged_f32_groups(M, N, K);
+    if (groups != 0) return run_gemm_f32_any_alignment(a, b, c, chain, g_split_k_enabled.load() ? groups : 1, stream);
   }
   // Operands none of these kernels reads in place -- fp32 with a K that is not a whole number of 16-byte pieces or rows
   // that do not start on 16 bytes, strides along K, and half precision where ragged_tile says so -- are copied once into
