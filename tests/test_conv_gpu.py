@@ -378,6 +378,42 @@ def test_filter_resident_variant_operator_chains(tracea_gpu, member, cin):
         capi.force_variant("conv2d", -1)
 
 
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+@pytest.mark.parametrize("member,cin,r,stride", [(m, c, 3, 1) for m, c in LDS_MEMBERS + KSPLIT_MEMBERS] + [("c128x64_c8_r7_w16_thin", 8, 7, 2)])
+def test_conv_activations_in_the_epilogue_from_registers(tracea_gpu, member, cin, r, stride, dtype):
+    """GELU and SiLU with and without an affine part in front, which the kernels with an epilogue from registers take there,
+    and chains that must not be taken for these: parts before or behind the activation.  Scores from -60 to 60 reach both
+    ends of the activations.  Tolerance: that of the sum and of the stored result's rounding, and as
+    much again for the slopes of two activations (at most 1.13 each) and a second rounding."""
+    from tracea_amd import capi
+    rng = np.random.default_rng(5)
+    td, rnd = (torch.float16, round_f16) if dtype == "f16" else (torch.bfloat16, round_bf16)
+    n, h, w, k = 3, 17, 23, 64
+    x = rnd(rng.standard_normal((n, h, w, cin)))
+    w_rsck = rnd(rng.standard_normal((r, r, cin, k)) * np.sqrt(2.0 / (r * r * cin)))
+    acc = oracle.conv2d_nhwc(x, w_rsck, stride, r // 2, 1)
+    bias = (rng.standard_normal(k) * 20).astype(np.float32)
+    (gamma, beta, mean, var), (scale, shift) = _bn_params(rng, k)
+    res = rnd(rng.standard_normal(acc.shape))
+    dx, dw = _dev(x, td), _dev(w_rsck, td).permute(3, 0, 1, 2).contiguous()
+    O, E = capi, oracle
+    bias_op = ((O.OP_BIAS_ADD, _dev(bias)), (E.EPI_BIAS_ADD, bias))
+    ss = ((O.OP_SCALE_SHIFT, _dev(scale), _dev(shift)), (E.EPI_SCALE_SHIFT, scale, shift))
+    bn = ((O.OP_BATCHNORM, _dev(gamma), _dev(beta), _dev(mean), _dev(var), 1e-5), (E.EPI_BATCHNORM, gamma, beta, mean, var, 1e-5))
+    relu, gelu, silu = ((O.OP_RELU,), (E.EPI_RELU,)), ((O.OP_GELU,), (E.EPI_GELU,)), ((O.OP_SILU,), (E.EPI_SILU,))
+    resid = ((O.OP_RESIDUAL_ADD, _dev(res, td)), (E.EPI_RESIDUAL_ADD, res))
+    capi.force_variant("conv2d", member)
+    try:
+        for chain in ([gelu], [silu], [bias_op, gelu], [bias_op, silu], [ss, gelu], [bn, silu], [relu, gelu], [gelu, relu], [silu, resid],
+                      [resid, silu], [bias_op, silu, gelu], [silu, bias_op], [bias_op, relu, silu]):
+            want = oracle.epilogue_apply(acc, [c[1] for c in chain])
+            y = tracea_gpu.conv2d_ex(dx, dw, [c[0] for c in chain], stride=stride, padding=r // 2)
+            assert capi.last_variant("conv2d") == member
+            assert_close_scaled(y.float().cpu().numpy(), want, 2 * tol_half(r * r * cin, dtype), "%s %s chain %s" % (member, dtype, [c[1][0] for c in chain]))
+    finally:
+        capi.force_variant("conv2d", -1)
+
+
 @pytest.mark.parametrize("kernel", ["t128x64x64_w4x1_p2", "t64x64x64_w2x2_p2", "c256x64_w8x1_s3_patch",
                                     "c448x64_k576_resident", "c400x64_c64_w16_resident", None])
 def test_conv_silu_kinds_through_tracea_conv2d(tracea_gpu, kernel):

@@ -83,7 +83,7 @@ struct ContractionCore {
   unsigned gn_m, gn_s, pt_m, pt_s;
   // pipeline 5 only: the chain in the fast form of conv_resident_kernel.hpp, or sig < 0
   struct FastEpilogue {
-    int sig;                  // bit 0 affine, 1 ReLU, 2 residual, 3 ReLU (in this order); < 0: not of this form
+    int sig;                  // bit 0 affine, 1 ReLU, 2 residual, 3 ReLU (in this order), 4 SiLU or 5 GELU instead of 1 to 3; < 0: not of this form
     int aff_kind, aff_dtype;  // TraceaEpilogueOpKind of the affine part and the DataType of a bias
     const void *p0, *p1, *p2, *p3;
     float epsilon;

@@ -166,6 +166,13 @@ __device__ __forceinline__ float activate_half(float x, HalfActivation f) {
   return x * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(t));
 }
 
+// (as bits of the convolutions' compile-time chain forms)
+constexpr int FORM_SILU = 16, FORM_GELU = 32;
+template <int F>
+__device__ __forceinline__ HalfActivation form_activation() {
+  return half_activation((F & FORM_GELU) != 0 ? TRACEA_EPI_OP_GELU : TRACEA_EPI_OP_SILU);
+}
+
 // Applies one operator to V consecutive channels n..n+V-1 of output row m
 // (fp32 in, fp32 out), reading its operands from global memory.
 template <int V>

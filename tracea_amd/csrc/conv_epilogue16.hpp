@@ -7,7 +7,8 @@
 // order of its emitter, src/emitter/cuda/conv.rs:91-116) everything happens in registers: per pair of
 // filter blocks one v_permlane16_swap per packed register gives every lane 8 consecutive channels of its
 // pixel, one 16-byte store; a residual is fetched in that layout, 16 bytes per lane, and taken back to the
-// accumulators' layout by the same swap.  F: bit 0 affine, 1 first ReLU, 2 residual, 3 second ReLU.
+// accumulators' layout by the same swap.  F: bit 0 affine, 1 first ReLU, 2 residual, 3 second ReLU; 4 SiLU or 5 GELU instead of
+// those three.
 #pragma once
 #include "contraction_kernel.hpp"
 
@@ -16,6 +17,7 @@ namespace tracea_amd {
 template <int DT, int F>
 struct Epilogue16 {
   static constexpr bool AFF = (F & 1) != 0, RELU1 = (F & 2) != 0, RES = (F & 4) != 0, RELU2 = (F & 8) != 0;
+  static constexpr bool ACT = (F & (FORM_SILU | FORM_GELU)) != 0;
   // the chain's last ReLU on the packed halves (one v_pk_max_f16 per two values; rounding is monotonic and
   // keeps zero, so max before or after it is the same value)
   static constexpr bool PK = DT == DT_F16 && (RELU2 || (RELU1 && !RES));
@@ -48,6 +50,10 @@ struct Epilogue16 {
   }
   static __device__ __forceinline__ f32x4 finish(f32x4 v, f32x4 a, f32x4 b, const float (&r)[4]) {
     if constexpr (AFF) v = v * a + b;
+    if constexpr (ACT) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] = activate_half(v[e], form_activation<F>());
+    }
     if constexpr (RELU1_F32) {
 #pragma unroll
       for (int e = 0; e < 4; ++e) v[e] = fmaxf(0.0f, v[e]);
@@ -152,9 +158,12 @@ struct Epilogue16 {
   }
 };
 
-// switch (sig) over the 16 forms: BODY(F) with F a compile-time constant
-#define TRACEA_EPILOGUE16_FORMS(sig, BODY)                                                                              \
+// switch (sig) over the forms: BODY(F) with F a compile-time constant; MORE: further cases
+#define TRACEA_EPILOGUE16_ACTIVATIONS(BODY)                                                                             \
+    case 16: BODY(16); break; case 17: BODY(17); break; case 32: BODY(32); break; case 33: BODY(33); break;
+#define TRACEA_EPILOGUE16_FORMS(sig, BODY, MORE)                                                                        \
   switch (sig) {                                                                                                        \
+    MORE                                                                                                                \
     case 0: BODY(0); break;  case 1: BODY(1); break;  case 2: BODY(2); break;  case 3: BODY(3); break;                  \
     case 4: BODY(4); break;  case 5: BODY(5); break;  case 6: BODY(6); break;  case 7: BODY(7); break;                  \
     case 8: BODY(8); break;  case 9: BODY(9); break;  case 10: BODY(10); break; case 11: BODY(11); break;               \

@@ -396,7 +396,7 @@ __global__ void __launch_bounds__(CK_THREADS) conv_ksplit16_kernel(const Contrac
         });
       };
 #define TRACEA_CK_FORM(F) run_form(std::integral_constant<int, F>{})
-      TRACEA_EPILOGUE16_FORMS(sig, TRACEA_CK_FORM)
+      TRACEA_EPILOGUE16_FORMS(sig, TRACEA_CK_FORM, TRACEA_EPILOGUE16_ACTIVATIONS(TRACEA_CK_FORM))
 #undef TRACEA_CK_FORM
       return;
     }

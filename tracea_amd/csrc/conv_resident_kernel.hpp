@@ -392,6 +392,10 @@ __global__ void __launch_bounds__(RS_THREADS) conv_resident_kernel(const Contrac
 #pragma unroll
             for (int e = 0; e < 8; ++e) v[e] = v[e] * ta[e] + tb[e];
           }
+          if constexpr ((F & (FORM_SILU | FORM_GELU)) != 0) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) v[e] = activate_half(v[e], form_activation<F>());
+          }
           if constexpr (RELU1) {
 #pragma unroll
             for (int e = 0; e < 8; ++e) v[e] = fmaxf(0.0f, v[e]);
@@ -430,12 +434,13 @@ __global__ void __launch_bounds__(RS_THREADS) conv_resident_kernel(const Contrac
       TRACEA_RS_FORM(0) TRACEA_RS_FORM(1) TRACEA_RS_FORM(2) TRACEA_RS_FORM(3) TRACEA_RS_FORM(4) TRACEA_RS_FORM(5)
       TRACEA_RS_FORM(6) TRACEA_RS_FORM(7) TRACEA_RS_FORM(8) TRACEA_RS_FORM(9) TRACEA_RS_FORM(10) TRACEA_RS_FORM(11)
       TRACEA_RS_FORM(12) TRACEA_RS_FORM(13) TRACEA_RS_FORM(14) TRACEA_RS_FORM(15)
+      TRACEA_RS_FORM(16) TRACEA_RS_FORM(17) TRACEA_RS_FORM(32) TRACEA_RS_FORM(33)
 #undef TRACEA_RS_FORM
       default: break;
     }
   } else {
-    // every other case (partial channel groups, unaligned rows, fp32 output, GELU / SiLU, further
-    // residuals): the general operator chain on the staged values
+    // every other case (partial channel groups, unaligned rows, fp32 output, GELU / SiLU among
+    // others, further residuals): the general operator chain on the staged values
     const ChainPlan plan = chain_plan(args.epi);
     for (int idx = tid; idx < npix * (BN / 8); idx += NT) {
       const int pr = idx >> 3;

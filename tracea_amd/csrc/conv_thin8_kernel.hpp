@@ -265,7 +265,7 @@ __global__ void __launch_bounds__(CT_THREADS) conv_thin8_kernel(const Contractio
         }
       };
 #define TRACEA_CT_FORM(F) run_form(std::integral_constant<int, F>{})
-      TRACEA_EPILOGUE16_FORMS(sig, TRACEA_CT_FORM)
+      TRACEA_EPILOGUE16_FORMS(sig, TRACEA_CT_FORM, )
 #undef TRACEA_CT_FORM
     } else {
       // any other chain: accumulators through the staging area, then the general operator loop over whole pixels

@@ -557,7 +557,7 @@ __global__ void __launch_bounds__(CW_THREADS) conv_wave16_kernel(const Contracti
       }
     };
 #define TRACEA_CW_FORM(F) run_form(std::integral_constant<int, F>{})
-    TRACEA_EPILOGUE16_FORMS(form_sig, TRACEA_CW_FORM)
+    TRACEA_EPILOGUE16_FORMS(form_sig, TRACEA_CW_FORM, TRACEA_EPILOGUE16_ACTIVATIONS(TRACEA_CW_FORM))
 #undef TRACEA_CW_FORM
     return;
   }

@@ -2042,11 +2042,15 @@ bool plan_conv_thin8(const ConvGeometry &g, const ContractionVariant &v, bool w_
   return true;
 }
 
-// The operator chain in the fast form of the filter-resident kernel: [affine] [ReLU] [residual] [ReLU],
-// each part at most once and in this order, affine = bias / scale-shift / BatchNorm; every tile has all 64
+// The operator chain in the fast form of the filter-resident kernel: [affine] [ReLU] [residual] [ReLU] or [affine] [GELU or
+// SiLU], each part at most once and in this order, affine = bias / scale-shift / BatchNorm; every tile has all 64
 // channels, output rows and residual rows are 8-byte aligned and addressable with 32-bit byte offsets
 // inside a tile, output and residual have the operand type.  Anything else: sig = -1 (general path).
-void fast_epilogue_form(const EpilogueChain &chain, int dtype, ContractionArgs *a) {
+// activations: whether the kernel has the forms with GELU and SiLU.  The one for 8 channels does not: its epilogue runs once per
+// tile of a persistent workgroup, and four more forms cost the others there (16x 112x112 8->64 7x7 with bias and ReLU 9.85 ->
+// 9.95 us, 10.15 behind a test of their own).  Elsewhere, bias and SiLU, us, before (general path) / now: 32x 56x56 64->64 3x3 18.8 / 12.4,
+// 32x 14x14 256->256 14.8 / 12.2.
+void fast_epilogue_form(const EpilogueChain &chain, int dtype, bool activations, ContractionArgs *a) {
   ContractionArgs::FastEpilogue fe{};
   fe.sig = -1;
   a->fe = fe;
@@ -2055,18 +2059,26 @@ void fast_epilogue_form(const EpilogueChain &chain, int dtype, ContractionArgs *
   int sig = 0, stage = 0;
   for (int o = 0; o < chain.n_ops && ok; ++o) {
     const EpilogueOpDev &op = chain.ops[o];
-    const bool aff = op.kind == TRACEA_EPI_OP_BIAS_ADD || op.kind == TRACEA_EPI_OP_SCALE_SHIFT || op.kind == TRACEA_EPI_OP_BATCHNORM;
+    const bool act = op.kind == TRACEA_EPI_OP_GELU || op.kind == TRACEA_EPI_OP_SILU || op.kind == TRACEA_EPI_OP_BIAS_ADD_SILU;
+    const bool aff = op.kind == TRACEA_EPI_OP_BIAS_ADD || op.kind == TRACEA_EPI_OP_BIAS_ADD_SILU || op.kind == TRACEA_EPI_OP_SCALE_SHIFT ||
+                     op.kind == TRACEA_EPI_OP_BATCHNORM;
     int part;
     if (op.kind == TRACEA_EPI_OP_NONE) continue;
+    else if (act && !activations) { ok = false; break; }
     else if (aff) part = 0;
+    else if (act) part = 1;
     else if (op.kind == TRACEA_EPI_OP_RELU) part = stage <= 2 ? 1 : 3;
     else if (op.kind == TRACEA_EPI_OP_RESIDUAL_ADD) part = 2;
     else { ok = false; break; }
     if (part < stage) { ok = false; break; }
-    sig |= 1 << part;
+    if (aff || !act) sig |= 1 << part;
     stage = part + 1;
+    if (act) {
+      sig |= op.kind == TRACEA_EPI_OP_GELU ? 32 : 16;
+      stage = 4;  // (nothing may follow)
+    }
     if (aff) {
-      fe.aff_kind = op.kind; fe.aff_dtype = op.dtype;
+      fe.aff_kind = op.kind == TRACEA_EPI_OP_BIAS_ADD_SILU ? (int)TRACEA_EPI_OP_BIAS_ADD : op.kind; fe.aff_dtype = op.dtype;
       fe.p0 = op.p0; fe.p1 = op.p1; fe.p2 = op.p2; fe.p3 = op.p3; fe.epsilon = op.epsilon;
     }
     if (part == 2) {
@@ -2260,7 +2272,8 @@ TraceaStatus run_conv(const ConvPlan &plan, const EpilogueChain &chain, hipStrea
   const long long w_extent = (long long)g.n_gemm * g.k_gemm * 2;
   const bool small = x_extent < (1ll << 31) && w_extent < (1ll << 31);
   if (conv_only(contraction_variant(vi)) && plan_conv_resident(g, contraction_variant(vi), plan.w_ncontig, &a)) {
-    if (contraction_variant(vi).pipeline == 5 || (contraction_variant(vi).pipeline >= 7 && contraction_variant(vi).pipeline <= 10)) fast_epilogue_form(chain, plan.x.dtype, &a);
+    if (contraction_variant(vi).pipeline == 5 || (contraction_variant(vi).pipeline >= 7 && contraction_variant(vi).pipeline <= 10)) 
+      fast_epilogue_form(chain, plan.x.dtype, contraction_variant(vi).pipeline != 10, &a);
     const int e = contraction_variant(vi).launch(a, true, plan.x.dtype, false, stream);
     // a member that refuses the arguments its plan accepted (it launched nothing) gives way to the
     // selector's choice below, like one whose plan failed
