@@ -53,3 +53,20 @@ def test_two_workgroups_of_the_headline_kernels_fit_a_cu():
             assert regs <= 256, (name, regs)
         if "conv_patch_kernel" in name and "ELi256ELi64ELi8ELi1E" in name:
             assert regs <= 128, (name, regs)
+
+
+def test_activations_are_kernels_of_their_own():
+    """GELU and SiLU in a row body slow the launches that have none of them, so each half-precision tile kernel exists with and
+    without (the last template argument)."""
+    families = {"contraction_kernel": r"18contraction_kernelI(?:Li\d+E){9}Lb[01]ELb[01]ELb[01]ELb([01])EEE", "conv_patch_kernel": r"17conv_patch_kernelI(?:Li\d+E){6}Lb[01]ELb([01])EEE",
+                "conv_wave16_kernel": r"18conv_wave16_kernelI(?:Li\d+E){5}Lb([01])EEE", "conv_ksplit16_kernel": r"20conv_ksplit16_kernelI(?:Li\d+E){4}Lb([01])EEE",
+                "conv_resident_kernel": r"20conv_resident_kernelI(?:Li\d+E){3}Lb([01])EEE", "conv_thin8_kernel": r"17conv_thin8_kernelI(?:Li\d+E){2}Lb([01])EEE"}
+    res = _resources()
+    for family, pattern in families.items():
+        names = [n for n in res if family + "ILi" in n]
+        assert names, family
+        for n in names:
+            m = re.search(pattern, n)
+            assert m, n
+            twin = n[:m.start(1)] + "10"[int(m.group(1))] + n[m.end(1):]
+            assert twin in res, n

@@ -149,28 +149,54 @@ __device__ __forceinline__ void load_as_float(const void *base, int dtype, long 
   }
 }
 
-// GELU (tanh form) and SiLU for results that are then rounded to 16 bits: 0.5 x (1 + tanh(u)) = x / (1 + exp(-2 u)) with
-// u = 0.79788456 (x + 0.044715 x^3), and x / (1 + exp(-x)), both x / (1 + 2^(x (c1 + c3 x^2))) with the constants below.  The
-// hardware's exp2 and reciprocal, one unit in the last place of fp32 each, in nine instructions a value, where the library's
-// tanhf, expf and the division take some fifty (f16 3328x2560x768 with GELU 47.5 -> 34.9 us,
-// 16384x3072x768 144.5 -> 103.1, where the product alone takes 30.3 and 83.7).  Infinities and NaN come out as from those;
-// the square is held below infinity for SiLU's c3 = 0.
-struct HalfActivation {
-  float c1, c3;
-};
-__device__ __forceinline__ HalfActivation half_activation(int kind) {
-  return kind == TRACEA_EPI_OP_GELU ? HalfActivation{-2.3022082f, -0.10294324f} : HalfActivation{-1.4426950f, 0.0f};
-}
-__device__ __forceinline__ float activate_half(float x, HalfActivation f) {
-  const float t = x * fmaf(f.c3, fminf(x * x, 1e30f), f.c1);
+// GELU (tanh form) for results that are then rounded to 16 bits: 0.5 x (1 + tanh(u)) = x / (1 + exp(-2 u)) with
+// u = 0.79788456 (x + 0.044715 x^3), that is x / (1 + 2^(x (c1 + c3 x^2))) with the constants below.  The hardware's exp2 and
+// reciprocal in eight instructions a value, where the library's tanhf and its branches take some fifty
+// (f16 3328x2560x768 45.2 -> 32.2 us, 16384x3072x768 130.8 -> 92.1).
+// Largest relative error in front of the rounding, this / tanhf: 1.9e-7 / 1.4e-7 from -1e-3 up, 9.7e-7 / 8.5e-4 from -4 to -1, and
+// 9.4e-6 down to -10, where 1 + tanhf cancels to zero.  Below -10 both give zero (the reciprocal of
+// 2^126 and more is flushed), and infinities and NaN come out alike: the square is held below infinity.
+__device__ __forceinline__ float gelu_half(float x) {
+  const float t = x * fmaf(-0.10294324f, fminf(x * x, 1e30f), -2.3022082f);
   return x * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(t));
+}
+__device__ __forceinline__ float silu(float x) { return x / (1.0f + expf(-x)); }
+
+// SiLU in the same way, x / (1 + 2^(x c1)).
+template <int G, int V>
+__device__ __forceinline__ void silu_half(float (&v)[G][V]) {
+#pragma unroll
+  for (int g = 0; g < G; ++g)
+#pragma unroll
+    for (int e = 0; e < V; ++e) v[g][e] = v[g][e] * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(v[g][e] * -1.4426950f));
+}
+template <int G, int V>
+__device__ __forceinline__ void gelu_half(float (&v)[G][V]) {
+#pragma unroll
+  for (int g = 0; g < G; ++g)
+#pragma unroll
+    for (int e = 0; e < V; ++e) v[g][e] = gelu_half(v[g][e]);
 }
 
 // (as bits of the convolutions' compile-time chain forms)
 constexpr int FORM_SILU = 16, FORM_GELU = 32;
-template <int F>
-__device__ __forceinline__ HalfActivation form_activation() {
-  return half_activation((F & FORM_GELU) != 0 ? TRACEA_EPI_OP_GELU : TRACEA_EPI_OP_SILU);
+template <int F, int G, int V>
+__device__ __forceinline__ void form_activation(float (&v)[G][V]) {
+  if constexpr ((F & FORM_GELU) != 0) gelu_half(v);
+  else silu_half(v);
+}
+
+// Whether a launch takes the kernels with GELU and SiLU in their fast row bodies (ACT below): 16-bit results and one of
+// them in the chain.  They are kernels of their own because in every launch's body they cost the others: with bias and ReLU
+// 16 products of 128x512x512 took 6.60 us instead of 6.53, 16x 56x56 32->64 3x3 8.98 instead of 8.81, 8x 56x56 96->96 13.96 instead of
+// 13.81, ResNet-18 at batch 5 186.7 instead of 185.6.
+inline bool activates_half(const ContractionCore &a) {
+  if (a.out_dtype == DT_F32) return false;
+  for (int o = 0; o < a.epi.n_ops; ++o) {
+    const int kind = a.epi.ops[o].kind;
+    if (kind == TRACEA_EPI_OP_GELU || kind == TRACEA_EPI_OP_SILU || kind == TRACEA_EPI_OP_BIAS_ADD_SILU) return true;
+  }
+  return false;
 }
 
 // Applies one operator to V consecutive channels n..n+V-1 of output row m
@@ -364,14 +390,22 @@ __device__ __forceinline__ ChainPlan chain_plan(const EpilogueChain &chain) {
 // the LDS table (tab points at this lane's first channel, vectors bn apart),
 // the first residual tensor through the plan, any further one from the
 // kernel arguments.  The operator loop is a real loop (its body is emitted
-// once) over kinds held in one scalar.
+// once) over kinds held in one scalar.  ACT: see activates_half.
+template <bool ACT>
 __device__ __forceinline__ void apply_epilogue_tab(float (&v)[8], long long m, int n, int nvalid,
                                                    const EpilogueChain &chain, const ChainPlan &plan,
-                                                   const float *tab, int bn, bool half_out) {
+                                                   const float *tab, int bn) {
 #pragma nounroll
   for (int o = 0; o < plan.n_ops; ++o) {
     const int kind = (int)((plan.kinds >> (4 * o)) & 15u);
-    if (kind == TRACEA_EPI_OP_RELU) {
+    if (ACT && (kind == TRACEA_EPI_OP_SILU || kind == TRACEA_EPI_OP_BIAS_ADD_SILU)) {
+      float t[1][8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) t[0][e] = kind == TRACEA_EPI_OP_SILU ? v[e] : v[e] + tab[(o * 2) * bn + e];
+      silu_half(t);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[e] = t[0][e];
+    } else if (kind == TRACEA_EPI_OP_RELU) {
 #pragma unroll
       for (int e = 0; e < 8; ++e) v[e] = fmaxf(0.0f, v[e]);
     } else if (kind == TRACEA_EPI_OP_BIAS_ADD || kind == TRACEA_EPI_OP_BIAS_ADD_SILU ||
@@ -386,23 +420,14 @@ __device__ __forceinline__ void apply_epilogue_tab(float (&v)[8], long long m, i
         for (int e = 0; e < 8; ++e) v[e] = v[e] + a[e];
       } else if (kind == TRACEA_EPI_OP_BIAS_ADD_SILU) {
 #pragma unroll
-        for (int e = 0; e < 8; ++e) v[e] = v[e] + a[e];
-        if (half_out) {
-          const HalfActivation f = half_activation(kind);
-#pragma unroll
-          for (int e = 0; e < 8; ++e) v[e] = activate_half(v[e], f);
-        } else {
-#pragma unroll
-          for (int e = 0; e < 8; ++e) v[e] = v[e] / (1.0f + expf(-v[e]));
-        }
+        for (int e = 0; e < 8; ++e) v[e] = silu(v[e] + a[e]);
       } else {
 #pragma unroll
         for (int e = 0; e < 8; ++e) v[e] = v[e] * a[e] + b[e];
       }
-    } else if (half_out && (kind == TRACEA_EPI_OP_GELU || kind == TRACEA_EPI_OP_SILU)) {
-      const HalfActivation f = half_activation(kind);
+    } else if (ACT && kind == TRACEA_EPI_OP_GELU) {
 #pragma unroll
-      for (int e = 0; e < 8; ++e) v[e] = activate_half(v[e], f);
+      for (int e = 0; e < 8; ++e) v[e] = gelu_half(v[e]);
     } else if (kind == TRACEA_EPI_OP_RESIDUAL_ADD && o == plan.res_index) {
       float t[8];
       load_as_float<8>(plan.res_ptr, plan.res_dtype, m * plan.res_ld + n, nvalid, t);
@@ -420,9 +445,10 @@ __device__ __forceinline__ void apply_epilogue_tab(float (&v)[8], long long m, i
 // thousand instructions and hundreds of branches per row, more than the
 // instruction cache holds.  Nearly every call needs none of it: all 8 channels
 // of every lane exist, rows of C (and of the residual) are 16-byte aligned, and
-// the chain is made of bias / scale-shift / BatchNorm / ReLU / GELU / SiLU / one residual.
+// the chain is made of bias / scale-shift / BatchNorm / ReLU / one residual (ACT: GELU and SiLU as well).
 // Whether that holds is the same for the whole workgroup, so it is decided
 // once and the row loops are emitted twice, each behind a uniform branch.
+template <bool ACT>
 __device__ __forceinline__ bool chain_is_simple(const ChainPlan &plan, const ContractionCore &args, int n0, int bn) {
   bool ok = n0 + bn <= args.N && (args.ldc & 7) == 0 && (((uintptr_t)args.C) & 15) == 0;
 #pragma unroll
@@ -430,22 +456,12 @@ __device__ __forceinline__ bool chain_is_simple(const ChainPlan &plan, const Con
     const int kind = (int)((plan.kinds >> (4 * o)) & 15u);
     ok = ok && (kind == TRACEA_EPI_OP_NONE || kind == TRACEA_EPI_OP_BIAS_ADD || kind == TRACEA_EPI_OP_RELU ||
                 kind == TRACEA_EPI_OP_SCALE_SHIFT || kind == TRACEA_EPI_OP_BATCHNORM ||
-                (args.out_dtype != DT_F32 && (kind == TRACEA_EPI_OP_GELU || kind == TRACEA_EPI_OP_SILU || kind == TRACEA_EPI_OP_BIAS_ADD_SILU)) ||
+                (ACT && (kind == TRACEA_EPI_OP_GELU || kind == TRACEA_EPI_OP_SILU || kind == TRACEA_EPI_OP_BIAS_ADD_SILU)) ||
                 (kind == TRACEA_EPI_OP_RESIDUAL_ADD && o == plan.res_index));
   }
   if (plan.res_index >= 0)
     ok = ok && plan.res_dtype != DT_F32 && (plan.res_ld & 7) == 0 && (((uintptr_t)plan.res_ptr) & 15) == 0;
   return ok;
-}
-
-__device__ __forceinline__ bool chain_activates(const ChainPlan &plan) {
-  bool any = false;
-#pragma unroll
-  for (int o = 0; o < TRACEA_MAX_EPILOGUE_OPS; ++o) {
-    const int kind = (int)((plan.kinds >> (4 * o)) & 15u);
-    any = any || kind == TRACEA_EPI_OP_GELU || kind == TRACEA_EPI_OP_SILU || kind == TRACEA_EPI_OP_BIAS_ADD_SILU;
-  }
-  return any;
 }
 
 // The specialised path for the 32 staged rows of one accumulator block: the
@@ -456,20 +472,22 @@ __device__ __forceinline__ bool chain_activates(const ChainPlan &plan) {
 // its staged values and one more per operator, back to back.
 // row_of(r) gives the output row of staged row r, or -1 if it does not exist.
 // F32OUT: C holds fp32 (two 16-byte stores per lane and row) instead of DT.
-// ACT: GELU and SiLU among the operators (in every launch's body they cost ResNet-18 at batch 5 one percent).
-template <int DT, int TN, bool F32OUT = false, bool ACT = false, typename RowOf>
+// ACT: GELU and SiLU among the operators (see activates_half); one group there, from the lane's row it_first on (active_rows).
+template <int DT, int TN, bool F32OUT, bool ACT, int GROUP_MAX = 4, typename RowOf>
 __device__ __forceinline__ void simple_rows(const float *stage, int lane, int n, const ContractionCore &args,
-                                            const ChainPlan &plan, const float *tab, int bn, RowOf row_of) {
+                                            const ChainPlan &plan, const float *tab, int bn, RowOf row_of,
+                                            [[maybe_unused]] int it_first = 0) {
   constexpr int EP_PITCH = TN + 4, LPR = TN / 8, RPI = 64 / LPR, NIT = 32 / RPI;
-  constexpr int GROUP = NIT < 4 ? NIT : 4;
+  constexpr int GROUP = NIT < GROUP_MAX ? NIT : GROUP_MAX;
   const int er = lane / LPR, ec = (lane % LPR) * 8;
-  static_for<0, NIT / GROUP>([&](auto grp) {
+  static_for<0, ACT ? 1 : NIT / GROUP>([&](auto grp) {
     constexpr int it0 = decltype(grp)::value * GROUP;
     float v[GROUP][8];
     long long m[GROUP];
 #pragma unroll
     for (int g = 0; g < GROUP; ++g) {
-      const int r = er + (it0 + g) * RPI;
+      int r = er + (it0 + g) * RPI;
+      if constexpr (ACT) r += it_first * RPI;
       m[g] = row_of(r);
       const f32x4 lo = *(const f32x4 *)(stage + r * EP_PITCH + ec);
       const f32x4 hi = *(const f32x4 *)(stage + r * EP_PITCH + ec + 4);
@@ -524,14 +542,9 @@ __device__ __forceinline__ void simple_rows(const float *stage, int lane, int n,
             for (int e = 0; e < 8; ++e) v[g][e] = v[g][e] * a[e] + b[e];
         }
       }
-      if constexpr (ACT) {  // (chain_is_simple lets these through for 16-bit results only)
-        if (kind == TRACEA_EPI_OP_GELU || kind == TRACEA_EPI_OP_SILU || kind == TRACEA_EPI_OP_BIAS_ADD_SILU) {
-          const HalfActivation f = half_activation(kind);
-#pragma unroll
-          for (int g = 0; g < GROUP; ++g)
-#pragma unroll
-            for (int e = 0; e < 8; ++e) v[g][e] = activate_half(v[g][e], f);
-        }
+      if constexpr (ACT) {
+        if (kind == TRACEA_EPI_OP_GELU) gelu_half(v);
+        else if (kind == TRACEA_EPI_OP_SILU || kind == TRACEA_EPI_OP_BIAS_ADD_SILU) silu_half(v);
       }
     }
 #pragma unroll
@@ -557,6 +570,14 @@ __device__ __forceinline__ void simple_rows(const float *stage, int lane, int n,
       }
     }
   });
+}
+// (one copy of the code for all rows of a block)
+template <int DT, int TN, int GROUP_MAX, typename RowOf>
+__device__ __forceinline__ void active_rows(const float *stage, int lane, int n, const ContractionCore &args, const ChainPlan &plan,
+                                            const float *tab, int bn, RowOf row_of) {
+  constexpr int NIT = TN / 16, GROUP = NIT < GROUP_MAX ? NIT : GROUP_MAX;
+#pragma nounroll
+  for (int it = 0; it < NIT; it += GROUP) simple_rows<DT, TN, false, true, GROUP_MAX>(stage, lane, n, args, plan, tab, bn, row_of, it);
 }
 
 // ---- tile order ---------------------------------------------------------------
@@ -623,7 +644,7 @@ struct Sequenced {
 // EXT: what few launches need and the others do not carry.  GEMM: blockIdx.z names one of several products (batch_*; in
 // every kernel these three fields cost 3072x1024x768 11.22 us against 10.95, 1536x1536x2048 23.6 against 23.4).
 // Convolution: a bank in place (b_taps; in every kernel with an N-contiguous B, N8 56x56 128->512 1x1 17.0 against 16.6).
-template <int DT, int BM, int BN, int BK, int WM, int WN, int NS, int PIPE, int MS, bool CONV, bool B_NCONTIG, bool EXT>
+template <int DT, int BM, int BN, int BK, int WM, int WN, int NS, int PIPE, int MS, bool CONV, bool B_NCONTIG, bool EXT, bool ACT>
 __global__ void __launch_bounds__(WM *WN * 64) contraction_kernel(const std::conditional_t<EXT, ContractionArgs, ContractionCore> args) {
   static_assert(MS == 32 || (MS == 16 && PIPE == 2 && !CONV && BK % 32 == 0), "the 16x16x32 form exists for a GEMM on pipeline 2");
   constexpr int NT = WM * WN * 64;
@@ -784,8 +805,8 @@ __global__ void __launch_bounds__(WM *WN * 64) contraction_kernel(const std::con
   // (fp32 output takes it only where a wave holds at most 8 accumulator blocks: with 16,
   // a second copy of the row body costs the compiler its register allocation.)
   constexpr bool F32_SIMPLE = FM * FN <= 8;
-  const bool out_f32 = F32_SIMPLE && args.out_dtype == DT_F32;
-  const bool simple = chain_is_simple(plan, args, n0, BN) && (args.out_dtype == DT || out_f32);
+  const bool out_f32 = F32_SIMPLE && !ACT && args.out_dtype == DT_F32;
+  const bool simple = chain_is_simple<ACT>(plan, args, n0, BN) && (args.out_dtype == DT || out_f32);
 
   // This thread's entries of the epilogue operand table (see chain_table_value):
   // requested here so that they arrive under the main loop.
@@ -807,7 +828,9 @@ __global__ void __launch_bounds__(WM *WN * 64) contraction_kernel(const std::con
       tabr[i] = idx < TAB_ENTRIES ? chain_table_value(args.epi, idx / (2 * BN), (idx / BN) & 1, n0 + idx % BN, N) : 0.0f;       \
     }                                                                                                                           \
   }
-  if constexpr (PIPE != 2 || !CONV) {
+  // (The four-wave 256x256 kernel of an N-contiguous B with ACT has no registers to hold them: behind the main loop there.)
+  constexpr bool TABLE_LATE = ACT && MS == 16 && B_NCONTIG && FM * FN >= 16;
+  if constexpr ((PIPE != 2 || !CONV) && !TABLE_LATE) {
     TRACEA_REQUEST_TABLE()
   }
 
@@ -1316,7 +1339,6 @@ __global__ void __launch_bounds__(WM *WN * 64) contraction_kernel(const std::con
     if constexpr (CONV) {
       TRACEA_REQUEST_TABLE()
     }
-#undef TRACEA_REQUEST_TABLE
     __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): this wave's share of tile 0 is in LDS
     __syncthreads();
     read_operands(0, smem, smem + A_STAGE, 0);
@@ -1555,11 +1577,15 @@ __global__ void __launch_bounds__(WM *WN * 64) contraction_kernel(const std::con
   // the end of the kernel with the stores taken out, 11.2 k with them.  (Decided per block of 32 rows, inside
   // the loop below: as a path of its own in front of the loop it cost the register allocation a hundred spills.)
   // (four-wave kernels: the eight-wave 256x256 member has 256 registers and spills 16 with this path in it)
-  constexpr bool REG_EPILOGUE = MS == 16 && !CONV && WM * WN == 4;
+  constexpr bool REG_EPILOGUE = MS == 16 && !CONV && WM * WN == 4 && !ACT;
   const bool from_registers = REG_EPILOGUE && simple && plan.n_ops == 0 && args.out_dtype == DT;
   float *stage = (float *)smem + wave * (32 * EP_PITCH);
   float *table = (float *)smem + STAGING_FLOATS;
   const int er = lane / LPR, ec = (lane % LPR) * 8;
+  if constexpr (TABLE_LATE) {
+    TRACEA_REQUEST_TABLE()
+  }
+#undef TRACEA_REQUEST_TABLE
 #pragma unroll
   for (int i = 0; i < TPT; ++i)
     if (tid + i * NT < TAB_ENTRIES) table[tid + i * NT] = tabr[i];
@@ -1573,41 +1599,39 @@ __global__ void __launch_bounds__(WM *WN * 64) contraction_kernel(const std::con
   const unsigned om_hw_m = args.hw_m, om_hw_s = args.hw_s, om_w_m = args.w_m, om_w_s = args.w_s;
   const int om_hw = args.h_out * args.w_out, om_w = args.w_out, om_sh = args.o_sh, om_sw = args.o_sw, om_wo = args.o_wo;
   const long long om_img = args.o_img;
-  static_for<0, FM>([&](auto blk) {
+  auto leave_from_registers = [&](auto blk) __attribute__((always_inline)) {
     constexpr int i = decltype(blk)::value;
-    if constexpr (REG_EPILOGUE) {
-      if (from_registers) {
-        const int q = lane >> 4;
-        unsigned short *cbase = (unsigned short *)args.C + n0 + wn * TN + (q & 1) * 16 + (q >> 1) * 8;
-        auto pack2 = [](float x, float y) __attribute__((always_inline)) -> unsigned {
-          if constexpr (DT == DT_F16) {
-            const f16x2 h = {(_Float16)x, (_Float16)y};
-            return __builtin_bit_cast(unsigned, h);
-          } else {
-            const bf16x2 h = {(__bf16)x, (__bf16)y};
-            return __builtin_bit_cast(unsigned, h);
-          }
-        };
+    const int q = lane >> 4;
+    unsigned short *cbase = (unsigned short *)args.C + n0 + wn * TN + (q & 1) * 16 + (q >> 1) * 8;
+    auto pack2 = [](float x, float y) __attribute__((always_inline)) -> unsigned {
+      if constexpr (DT == DT_F16) {
+        const f16x2 h = {(_Float16)x, (_Float16)y};
+        return __builtin_bit_cast(unsigned, h);
+      } else {
+        const bf16x2 h = {(__bf16)x, (__bf16)y};
+        return __builtin_bit_cast(unsigned, h);
+      }
+    };
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
-          const int m = m0 + wm * TM + i * 32 + h * 16 + (lane & 15);
-          unsigned short *crow = cbase + (zrow + m) * args.ldc;
+    for (int h = 0; h < 2; ++h) {
+      const int m = m0 + wm * TM + i * 32 + h * 16 + (lane & 15);
+      unsigned short *crow = cbase + (zrow + m) * args.ldc;
 #pragma unroll
-          for (int j = 0; j < FN; ++j) {
-            const f32x4 a4 = acc16[2 * i + h][2 * j], b4 = acc16[2 * i + h][2 * j + 1];
-            unsigned a_lo = pack2(a4[0], a4[1]), a_hi = pack2(a4[2], a4[3]);
-            unsigned b_lo = pack2(b4[0], b4[1]), b_hi = pack2(b4[2], b4[3]);
-            // (as instructions: the compiler's builtin for the swap returns its first result twice; the s_nop
-            // is the wait the hardware asks for between a vector-ALU write of an operand and the swap)
-            asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %1" : "+v"(a_lo), "+v"(b_lo));
-            asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %1" : "+v"(a_hi), "+v"(b_hi));
-            const u32x4 row8 = {a_lo, a_hi, b_lo, b_hi};
-            if (m < M) *(u32x4 *)(crow + j * 32) = row8;
-          }
-        }
-        return;
+      for (int j = 0; j < FN; ++j) {
+        const f32x4 a4 = acc16[2 * i + h][2 * j], b4 = acc16[2 * i + h][2 * j + 1];
+        unsigned a_lo = pack2(a4[0], a4[1]), a_hi = pack2(a4[2], a4[3]);
+        unsigned b_lo = pack2(b4[0], b4[1]), b_hi = pack2(b4[2], b4[3]);
+        // (as instructions: the compiler's builtin for the swap returns its first result twice; the s_nop
+        // is the wait the hardware asks for between a vector-ALU write of an operand and the swap)
+        asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %1" : "+v"(a_lo), "+v"(b_lo));
+        asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %1" : "+v"(a_hi), "+v"(b_hi));
+        const u32x4 row8 = {a_lo, a_hi, b_lo, b_hi};
+        if (m < M) *(u32x4 *)(crow + j * 32) = row8;
       }
     }
+  };
+  auto stage_block = [&](auto blk) __attribute__((always_inline)) {
+    constexpr int i = decltype(blk)::value;
     static_for<0, FN>([&](auto col) {
       constexpr int j = decltype(col)::value;
       if constexpr (MS == 16) {
@@ -1629,6 +1653,8 @@ __global__ void __launch_bounds__(WM *WN * 64) contraction_kernel(const std::con
         }
       }
     });
+  };
+  auto finish_block = [&](int i) __attribute__((always_inline)) {
     // The staging area is private to the wave and a wave's LDS operations
     // complete in program order: a compiler-level fence is all that is needed
     // between the writes above and the reads below (and before the next pass
@@ -1652,12 +1678,14 @@ __global__ void __launch_bounds__(WM *WN * 64) contraction_kernel(const std::con
     if (simple) {
       const int mb = m0 + wm * TM + i * 32;
       auto row_of = [&](int r) -> long long { return mb + r < M ? out_row(mb + r) : -1ll; };
-      if constexpr (F32_SIMPLE) {
-        if (out_f32) simple_rows<DT, TN, true>(stage, lane, n0 + wn * TN + ec, args, plan, tab, BN, row_of);
-        else if (chain_activates(plan)) simple_rows<DT, TN, false, true>(stage, lane, n0 + wn * TN + ec, args, plan, tab, BN, row_of);
-        else simple_rows<DT, TN, false>(stage, lane, n0 + wn * TN + ec, args, plan, tab, BN, row_of);
+      if constexpr (F32_SIMPLE && !ACT) {
+        if (out_f32) simple_rows<DT, TN, true, false>(stage, lane, n0 + wn * TN + ec, args, plan, tab, BN, row_of);
+        else simple_rows<DT, TN, false, false>(stage, lane, n0 + wn * TN + ec, args, plan, tab, BN, row_of);
+      } else if constexpr (ACT) {
+        active_rows<DT, TN, FM * FN * WM * WN == 64 && WM * WN == 8 ? 2 : 4>(  // (eight waves of 256 registers: four rows spill)
+            stage, lane, n0 + wn * TN + ec, args, plan, tab, BN, row_of);
       } else {
-        simple_rows<DT, TN, false, true>(stage, lane, n0 + wn * TN + ec, args, plan, tab, BN, row_of);  // (one copy, see above)
+        simple_rows<DT, TN, false, false>(stage, lane, n0 + wn * TN + ec, args, plan, tab, BN, row_of);
       }
     } else {
       for (int r = er; r < 32; r += RPI) {
@@ -1674,14 +1702,35 @@ __global__ void __launch_bounds__(WM *WN * 64) contraction_kernel(const std::con
           }
           const int nvalid = N - n;
           const long long row = out_row(m);
-          apply_epilogue_tab(v, row, n, nvalid, args.epi, plan, tab, BN, args.out_dtype != DT_F32);
+          apply_epilogue_tab<ACT>(v, row, n, nvalid, args.epi, plan, tab, BN);
           store_from_float<8>(args.C, args.out_dtype, row * args.ldc + n, nvalid, v);
         }
       }
     }
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     __builtin_amdgcn_wave_barrier();
-  });
+  };
+  if constexpr (ACT) {
+    // (one copy of the rows for all blocks: GELU and SiLU are long, and a copy each is more than the instruction cache holds)
+#pragma nounroll
+    for (int i = 0; i < FM; ++i) {
+      static_for<0, FM>([&](auto blk) {
+        if (i == decltype(blk)::value) stage_block(blk);
+      });
+      finish_block(i);
+    }
+  } else {
+    static_for<0, FM>([&](auto blk) {
+      if constexpr (REG_EPILOGUE) {
+        if (from_registers) {
+          leave_from_registers(blk);
+          return;
+        }
+      }
+      stage_block(blk);
+      finish_block(decltype(blk)::value);
+    });
+  }
 }
 
 template <int BM, int BN, int BK, int WM, int WN, int NS, int PIPE, int MS = 32>
@@ -1692,6 +1741,7 @@ int launch_contraction(const ContractionArgs &a, bool conv, int dtype, bool b_nc
   constexpr bool BATCHES = PIPE >= 2 && BM * BN <= 128 * 128, TAPS = PIPE >= 2 && MS == 32;
   if (ext && !(conv ? TAPS && b_ncontig : BATCHES)) return (int)hipErrorInvalidValue;
   constexpr size_t lds = (size_t)NS * (BM + BN) * BK * 2;
+  const bool act = activates_half(a);
   const bool listed = !conv && a.tile_list != nullptr;  // one workgroup per record, no split grid
   const dim3 grid((unsigned)(listed ? a.tile_count : a.grid_m * a.grid_n),
                   (unsigned)(!listed && a.k_split > 0 ? (a.K + a.k_split - 1) / a.k_split : 1),
@@ -1699,7 +1749,12 @@ int launch_contraction(const ContractionArgs &a, bool conv, int dtype, bool b_nc
       block(WM * WN * 64);
 #define TRACEA_LAUNCH(DTV, CONVV, NCV, EXTV)                                                 \
   do {                                                                                       \
-    auto kfn = contraction_kernel<DTV, BM, BN, BK, WM, WN, NS, PIPE, MS, (CONVV) && MS == 32, NCV, EXTV>; \
+    if (act) TRACEA_LAUNCH_ONE(DTV, CONVV, NCV, EXTV, true);                                 \
+    TRACEA_LAUNCH_ONE(DTV, CONVV, NCV, EXTV, false);                                         \
+  } while (0)
+#define TRACEA_LAUNCH_ONE(DTV, CONVV, NCV, EXTV, ACTV)                                       \
+  do {                                                                                       \
+    auto kfn = contraction_kernel<DTV, BM, BN, BK, WM, WN, NS, PIPE, MS, (CONVV) && MS == 32, NCV, EXTV, ACTV>; \
     static bool attr_done = false;                                                           \
     if (!attr_done) {                                                                        \
       hipError_t e = hipFuncSetAttribute((const void *)kfn,                                  \
@@ -1724,6 +1779,7 @@ int launch_contraction(const ContractionArgs &a, bool conv, int dtype, bool b_nc
   TRACEA_LAUNCH_FORM(DT_BF16);
 #undef TRACEA_LAUNCH_FORM
 #undef TRACEA_LAUNCH
+#undef TRACEA_LAUNCH_ONE
 }
 
 }  // namespace tracea_amd

@@ -50,10 +50,6 @@ struct Epilogue16 {
   }
   static __device__ __forceinline__ f32x4 finish(f32x4 v, f32x4 a, f32x4 b, const float (&r)[4]) {
     if constexpr (AFF) v = v * a + b;
-    if constexpr (ACT) {
-#pragma unroll
-      for (int e = 0; e < 4; ++e) v[e] = activate_half(v[e], form_activation<F>());
-    }
     if constexpr (RELU1_F32) {
 #pragma unroll
       for (int e = 0; e < 4; ++e) v[e] = fmaxf(0.0f, v[e]);
@@ -67,6 +63,22 @@ struct Epilogue16 {
       for (int e = 0; e < 4; ++e) v[e] = fmaxf(0.0f, v[e]);
     }
     return v;
+  }
+  // GELU and SiLU of N filter blocks of a pixel block at once, behind the affine part; what is left of the form is Plain.
+  using Plain = Epilogue16<DT, 0>;
+  template <int N>
+  static __device__ __forceinline__ void activate(const f32x4 *acc, const f32x4 *ta, const f32x4 *tb, f32x4 (&out)[N]) {
+    float v[N][4];
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      f32x4 t = acc[i];
+      if constexpr (AFF) t = t * ta[i] + tb[i];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[i][e] = t[e];
+    }
+    form_activation<F>(v);
+#pragma unroll
+    for (int i = 0; i < N; ++i) out[i] = f32x4{v[i][0], v[i][1], v[i][2], v[i][3]};
   }
   // One pixel block x two filter blocks fa, fb (accumulators acc_a, acc_b): after the swap the lanes of
   // 16-lane group q hold channels (q>>1)*8 .. +7 of block (q&1 ? fb : fa), one 16-byte store per lane.
@@ -87,6 +99,13 @@ struct Epilogue16 {
   static __device__ __forceinline__ void pair_block_with(f32x4 acc_a, f32x4 acc_b, int fa, int fb, f32x4 ta_a, f32x4 tb_a,
                                                          f32x4 ta_b, f32x4 tb_b, int prow, int q, __amdgpu_buffer_rsrc_t rsrc_c,
                                                          int row_c, u32x4 r8) {
+    if constexpr (ACT) {
+      const f32x4 acc[2] = {acc_a, acc_b}, ta[2] = {ta_a, ta_b}, tb[2] = {tb_a, tb_b};
+      f32x4 v[2];
+      activate(acc, ta, tb, v);
+      Plain::pair_block_with(v[0], v[1], fa, fb, ta_a, tb_a, ta_b, tb_b, prow, q, rsrc_c, row_c, r8);
+      return;
+    }
     float ra[4] = {0, 0, 0, 0}, rb[4] = {0, 0, 0, 0};
     if constexpr (RES) {
       unsigned r0 = r8[0], r1 = r8[1], r2 = r8[2], r3 = r8[3];
@@ -119,6 +138,12 @@ struct Epilogue16 {
   static __device__ __forceinline__ void pixel_block(const f32x4 (&acc)[4], const int (&fb)[4], const f32x4 (&ta)[4],
                                                      const f32x4 (&tb)[4], int prow, int q, __amdgpu_buffer_rsrc_t rsrc_c,
                                                      __amdgpu_buffer_rsrc_t rsrc_r, int row_c, int row_r) {
+    if constexpr (ACT) {
+      f32x4 v[4];
+      activate(acc, ta, tb, v);
+      Plain::pixel_block(v, fb, ta, tb, prow, q, rsrc_c, rsrc_r, row_c, row_r);
+      return;
+    }
 #pragma unroll
     for (int j = 0; j < 2; ++j)
       pair_block(acc[2 * j], acc[2 * j + 1], fb[2 * j], fb[2 * j + 1], ta[2 * j], tb[2 * j], ta[2 * j + 1], tb[2 * j + 1], prow, q, rsrc_c,
@@ -128,6 +153,12 @@ struct Epilogue16 {
   static __device__ __forceinline__ void pixel_block_with(const f32x4 (&acc)[4], const int (&fb)[4], const f32x4 (&ta)[4],
                                                           const f32x4 (&tb)[4], int prow, int q, __amdgpu_buffer_rsrc_t rsrc_c,
                                                           int row_c, const u32x4 (&res)[2]) {
+    if constexpr (ACT) {
+      f32x4 v[4];
+      activate(acc, ta, tb, v);
+      Plain::pixel_block_with(v, fb, ta, tb, prow, q, rsrc_c, row_c, res);
+      return;
+    }
 #pragma unroll
     for (int j = 0; j < 2; ++j)
       pair_block_with(acc[2 * j], acc[2 * j + 1], fb[2 * j], fb[2 * j + 1], ta[2 * j], tb[2 * j], ta[2 * j + 1], tb[2 * j + 1], prow, q,
@@ -140,6 +171,12 @@ struct Epilogue16 {
   }
   static __device__ __forceinline__ void single_block_with(f32x4 acc, f32x4 ta, f32x4 tb, int ch, int prow,
                                                            __amdgpu_buffer_rsrc_t rsrc_c, int row_c, u32x2 r4) {
+    if constexpr (ACT) {
+      f32x4 t[1];
+      activate(&acc, &ta, &tb, t);
+      Plain::single_block_with(t[0], ta, tb, ch, prow, rsrc_c, row_c, r4);
+      return;
+    }
     float rr[4] = {0, 0, 0, 0};
     if constexpr (RES) {
       unpack2(r4[0], rr[0], rr[1]);
@@ -158,12 +195,14 @@ struct Epilogue16 {
   }
 };
 
-// switch (sig) over the forms: BODY(F) with F a compile-time constant; MORE: further cases
-#define TRACEA_EPILOGUE16_ACTIVATIONS(BODY)                                                                             \
-    case 16: BODY(16); break; case 17: BODY(17); break; case 32: BODY(32); break; case 33: BODY(33); break;
-#define TRACEA_EPILOGUE16_FORMS(sig, BODY, MORE)                                                                        \
+// switch (sig) over the forms of a kernel with and without activations: BODY(F) with F a compile-time constant
+#define TRACEA_EPILOGUE16_ACTIVATIONS(sig, BODY)                                                                        \
   switch (sig) {                                                                                                        \
-    MORE                                                                                                                \
+    case 16: BODY(16); break; case 17: BODY(17); break; case 32: BODY(32); break; case 33: BODY(33); break;             \
+    default: break;                                                                                                     \
+  }
+#define TRACEA_EPILOGUE16_FORMS(sig, BODY)                                                                              \
+  switch (sig) {                                                                                                        \
     case 0: BODY(0); break;  case 1: BODY(1); break;  case 2: BODY(2); break;  case 3: BODY(3); break;                  \
     case 4: BODY(4); break;  case 5: BODY(5); break;  case 6: BODY(6); break;  case 7: BODY(7); break;                  \
     case 8: BODY(8); break;  case 9: BODY(9); break;  case 10: BODY(10); break; case 11: BODY(11); break;               \

@@ -33,7 +33,7 @@ constexpr int CK_THREADS = 512;
 constexpr int CK_TABLE_BYTES = TRACEA_MAX_EPILOGUE_OPS * 2 * 64 * 4;
 constexpr int CK_STAGE_BYTES = 64 * 256;  // 64 filters x 128 channels
 
-template <int DT, int CIN, int NPB, int RING>
+template <int DT, int CIN, int NPB, int RING, bool ACT>
 __global__ void __launch_bounds__(CK_THREADS) conv_ksplit16_kernel(const ContractionCore args) {
   constexpr int NT = CK_THREADS, BN = 64, NW = NT / 64;
   constexpr int CPT = CIN / 128;  // stages (128-channel chunks) per filter tap
@@ -396,7 +396,8 @@ __global__ void __launch_bounds__(CK_THREADS) conv_ksplit16_kernel(const Contrac
         });
       };
 #define TRACEA_CK_FORM(F) run_form(std::integral_constant<int, F>{})
-      TRACEA_EPILOGUE16_FORMS(sig, TRACEA_CK_FORM, TRACEA_EPILOGUE16_ACTIVATIONS(TRACEA_CK_FORM))
+      if constexpr (ACT) { TRACEA_EPILOGUE16_ACTIVATIONS(sig, TRACEA_CK_FORM) }
+      else { TRACEA_EPILOGUE16_FORMS(sig, TRACEA_CK_FORM) }
 #undef TRACEA_CK_FORM
       return;
     }
@@ -432,7 +433,7 @@ __global__ void __launch_bounds__(CK_THREADS) conv_ksplit16_kernel(const Contrac
       }
       const int nvalid = N - n;
       const long long m = m_img + pr;
-      apply_epilogue_tab(v, m, n, nvalid, args.epi, plan, table + ec, BN, args.out_dtype != DT_F32);
+      apply_epilogue_tab<ACT>(v, m, n, nvalid, args.epi, plan, table + ec, BN);
       store_from_float<8>(args.C, args.out_dtype, m * args.ldc + n, nvalid, v);
     }
   }
@@ -451,9 +452,9 @@ int launch_conv_ksplit16(const ContractionArgs &a, bool conv, int dtype, bool b_
   const size_t lds = (operands > staging ? operands : staging) + CK_TABLE_BYTES;
   if (lds > 160 * 1024) return (int)hipErrorInvalidValue;
   const dim3 grid((unsigned)(a.grid_m * a.grid_n)), block(CK_THREADS);
-#define TRACEA_LAUNCH_CK(DTV)                                                                        \
+#define TRACEA_LAUNCH_CK(DTV, ACTV)                                                                  \
   do {                                                                                               \
-    auto kfn = conv_ksplit16_kernel<DTV, CIN, NPB, RING>;                                             \
+    auto kfn = conv_ksplit16_kernel<DTV, CIN, NPB, RING, ACTV>;                                           \
     static bool attr_done = false;                                                                   \
     if (!attr_done) {                                                                                \
       hipError_t e = hipFuncSetAttribute((const void *)kfn, hipFuncAttributeMaxDynamicSharedMemorySize, \
@@ -464,8 +465,9 @@ int launch_conv_ksplit16(const ContractionArgs &a, bool conv, int dtype, bool b_
     hipLaunchKernelGGL(kfn, grid, block, lds, stream, a);                                            \
     return (int)hipGetLastError();                                                                   \
   } while (0)
-  if (dtype == DT_F16) TRACEA_LAUNCH_CK(DT_F16);
-  else TRACEA_LAUNCH_CK(DT_BF16);
+  const bool act = activates_half(a);
+  if (dtype == DT_F16) { if (act) TRACEA_LAUNCH_CK(DT_F16, true); else TRACEA_LAUNCH_CK(DT_F16, false); }
+  else { if (act) TRACEA_LAUNCH_CK(DT_BF16, true); else TRACEA_LAUNCH_CK(DT_BF16, false); }
 #undef TRACEA_LAUNCH_CK
   return (int)hipErrorInvalidValue;
 }

@@ -23,7 +23,7 @@
 
 namespace tracea_amd {
 
-template <int DT, int TM, int BN, int WM, int WN, int NSB, bool FULL>
+template <int DT, int TM, int BN, int WM, int WN, int NSB, bool FULL, bool ACT>
 __global__ void __launch_bounds__(WM *WN * 64) conv_patch_kernel(const ContractionCore args) {
   constexpr int NT = WM * WN * 64;
   constexpr int BK = 64, CH = 8, ROW_BYTES = 128, RP = 2;  // filter tile: BN rows x 64 k, XOR-swizzled
@@ -130,7 +130,7 @@ __global__ void __launch_bounds__(WM *WN * 64) conv_patch_kernel(const Contracti
 
   // chain description and choice of the row body: read here, under the main loop
   const ChainPlan plan = chain_plan(args.epi);
-  const bool simple = chain_is_simple(plan, args, n0, BN) && args.out_dtype == DT;
+  const bool simple = chain_is_simple<ACT>(plan, args, n0, BN) && args.out_dtype == DT;
 
   // this thread's entries of the epilogue operand table, requested under the main loop
   constexpr int TAB_ENTRIES = TRACEA_MAX_EPILOGUE_OPS * 2 * BN;
@@ -280,7 +280,8 @@ __global__ void __launch_bounds__(WM *WN * 64) conv_patch_kernel(const Contracti
     if (simple) {
       const int pb = wm * TMW + i * 32;
       auto row_of = [&](int r) -> long long { return pb + r < npix ? m_img + pb + r : -1ll; };
-      simple_rows<DT, TN, false, true>(stage, lane, n0 + wn * TN + ec, args, plan, tab, BN, row_of);  // (a second copy: 133 registers)
+      if constexpr (ACT) active_rows<DT, TN, 4>(stage, lane, n0 + wn * TN + ec, args, plan, tab, BN, row_of);
+      else simple_rows<DT, TN, false, false>(stage, lane, n0 + wn * TN + ec, args, plan, tab, BN, row_of);
     } else {
       for (int r = er; r < 32; r += RPI) {
         const int pr = wm * TMW + i * 32 + r;
@@ -296,7 +297,7 @@ __global__ void __launch_bounds__(WM *WN * 64) conv_patch_kernel(const Contracti
           }
           const int nvalid = N - n;
           const long long m = m_img + pr;
-          apply_epilogue_tab(v, m, n, nvalid, args.epi, plan, tab, BN, args.out_dtype != DT_F32);
+          apply_epilogue_tab<ACT>(v, m, n, nvalid, args.epi, plan, tab, BN);
           store_from_float<8>(args.C, args.out_dtype, m * args.ldc + n, nvalid, v);
         }
       }
@@ -317,7 +318,12 @@ int launch_conv_patch(const ContractionArgs &a, bool conv, int dtype, bool b_nco
   const dim3 grid((unsigned)(a.grid_m * a.grid_n)), block(WM * WN * 64);
 #define TRACEA_LAUNCH_PATCH(DTV, FULLV)                                                             \
   do {                                                                                              \
-    auto kfn = conv_patch_kernel<DTV, TM, BN, WM, WN, NSB, FULLV>;                                  \
+    if (act) TRACEA_LAUNCH_PATCH_ONE(DTV, FULLV, true);                                             \
+    TRACEA_LAUNCH_PATCH_ONE(DTV, FULLV, false);                                                     \
+  } while (0)
+#define TRACEA_LAUNCH_PATCH_ONE(DTV, FULLV, ACTV)                                                   \
+  do {                                                                                              \
+    auto kfn = conv_patch_kernel<DTV, TM, BN, WM, WN, NSB, FULLV, ACTV>;                            \
     static bool attr_done = false;                                                                  \
     if (!attr_done) {                                                                               \
       hipError_t e = hipFuncSetAttribute((const void *)kfn, hipFuncAttributeMaxDynamicSharedMemorySize, \
@@ -328,10 +334,12 @@ int launch_conv_patch(const ContractionArgs &a, bool conv, int dtype, bool b_nco
     hipLaunchKernelGGL(kfn, grid, block, lds, stream, a);                                           \
     return (int)hipGetLastError();                                                                  \
   } while (0)
+  const bool act = activates_half(a);
   const bool full = a.K % 64 == 0;  // every filter tile holds all of its k-steps
   if (dtype == DT_F16) { if (full) TRACEA_LAUNCH_PATCH(DT_F16, true); else TRACEA_LAUNCH_PATCH(DT_F16, false); }
   else { if (full) TRACEA_LAUNCH_PATCH(DT_BF16, true); else TRACEA_LAUNCH_PATCH(DT_BF16, false); }
 #undef TRACEA_LAUNCH_PATCH
+#undef TRACEA_LAUNCH_PATCH_ONE
   return (int)hipErrorInvalidValue;
 }
 

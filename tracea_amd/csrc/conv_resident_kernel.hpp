@@ -48,7 +48,7 @@ constexpr int rs_filter_bytes(int ks) { return rs_filter_iters(ks) * RS_THREADS 
 constexpr int RS_TABLE_BYTES = TRACEA_MAX_EPILOGUE_OPS * 2 * 64 * 4;
 
 // KS: 16-wide k-steps (K / 16); KPT: k-steps per filter tap (C / 16).
-template <int DT, int KS, int KPT>
+template <int DT, int KS, int KPT, bool ACT>
 __global__ void __launch_bounds__(RS_THREADS) conv_resident_kernel(const ContractionCore args) {
   constexpr int NT = RS_THREADS, BN = 64, NW = NT / 64;
   constexpr int CPB = rs_cpb(KS), FIT = rs_filter_iters(KS);
@@ -387,15 +387,13 @@ __global__ void __launch_bounds__(RS_THREADS) conv_resident_kernel(const Contrac
 #pragma unroll
         for (int u = 0; u < UN; ++u) {
           const int pr = pr0 + u * PPS;
-          float v[8] = {lo[u][0], lo[u][1], lo[u][2], lo[u][3], hi[u][0], hi[u][1], hi[u][2], hi[u][3]};
+          float v1[1][8] = {{lo[u][0], lo[u][1], lo[u][2], lo[u][3], hi[u][0], hi[u][1], hi[u][2], hi[u][3]}};
+          float(&v)[8] = v1[0];
           if constexpr (AFF) {
 #pragma unroll
             for (int e = 0; e < 8; ++e) v[e] = v[e] * ta[e] + tb[e];
           }
-          if constexpr ((F & (FORM_SILU | FORM_GELU)) != 0) {
-#pragma unroll
-            for (int e = 0; e < 8; ++e) v[e] = activate_half(v[e], form_activation<F>());
-          }
+          if constexpr ((F & (FORM_SILU | FORM_GELU)) != 0) form_activation<F>(v1);
           if constexpr (RELU1) {
 #pragma unroll
             for (int e = 0; e < 8; ++e) v[e] = fmaxf(0.0f, v[e]);
@@ -429,15 +427,21 @@ __global__ void __launch_bounds__(RS_THREADS) conv_resident_kernel(const Contrac
         }
       }
     };
-    switch (sig) {
 #define TRACEA_RS_FORM(F) case F: run_form(std::integral_constant<int, F>{}); break;
-      TRACEA_RS_FORM(0) TRACEA_RS_FORM(1) TRACEA_RS_FORM(2) TRACEA_RS_FORM(3) TRACEA_RS_FORM(4) TRACEA_RS_FORM(5)
-      TRACEA_RS_FORM(6) TRACEA_RS_FORM(7) TRACEA_RS_FORM(8) TRACEA_RS_FORM(9) TRACEA_RS_FORM(10) TRACEA_RS_FORM(11)
-      TRACEA_RS_FORM(12) TRACEA_RS_FORM(13) TRACEA_RS_FORM(14) TRACEA_RS_FORM(15)
-      TRACEA_RS_FORM(16) TRACEA_RS_FORM(17) TRACEA_RS_FORM(32) TRACEA_RS_FORM(33)
-#undef TRACEA_RS_FORM
-      default: break;
+    if constexpr (ACT) {
+      switch (sig) {
+        TRACEA_RS_FORM(16) TRACEA_RS_FORM(17) TRACEA_RS_FORM(32) TRACEA_RS_FORM(33)
+        default: break;
+      }
+    } else {
+      switch (sig) {
+        TRACEA_RS_FORM(0) TRACEA_RS_FORM(1) TRACEA_RS_FORM(2) TRACEA_RS_FORM(3) TRACEA_RS_FORM(4) TRACEA_RS_FORM(5)
+        TRACEA_RS_FORM(6) TRACEA_RS_FORM(7) TRACEA_RS_FORM(8) TRACEA_RS_FORM(9) TRACEA_RS_FORM(10) TRACEA_RS_FORM(11)
+        TRACEA_RS_FORM(12) TRACEA_RS_FORM(13) TRACEA_RS_FORM(14) TRACEA_RS_FORM(15)
+        default: break;
+      }
     }
+#undef TRACEA_RS_FORM
   } else {
     // every other case (partial channel groups, unaligned rows, fp32 output, GELU / SiLU among
     // others, further residuals): the general operator chain on the staged values
@@ -456,7 +460,7 @@ __global__ void __launch_bounds__(RS_THREADS) conv_resident_kernel(const Contrac
         }
         const int nvalid = N - n;
         const long long m = m_img + pr;
-        apply_epilogue_tab(v, m, n, nvalid, args.epi, plan, table + ec, BN, args.out_dtype != DT_F32);
+        apply_epilogue_tab<ACT>(v, m, n, nvalid, args.epi, plan, table + ec, BN);
         store_from_float<8>(args.C, args.out_dtype, m * args.ldc + n, nvalid, v);
       }
     }
@@ -470,9 +474,9 @@ int launch_conv_resident(const ContractionArgs &a, bool conv, int dtype, bool b_
   // the general epilogue stages p_tm x 68 floats in front of the table
   if (lds > 160 * 1024 || (size_t)a.p_tm * 68 * 4 > lds - RS_TABLE_BYTES) return (int)hipErrorInvalidValue;
   const dim3 grid((unsigned)(a.grid_m * a.grid_n)), block(RS_THREADS);
-#define TRACEA_LAUNCH_RS(DTV)                                                                        \
+#define TRACEA_LAUNCH_RS(DTV, ACTV)                                                                      \
   do {                                                                                               \
-    auto kfn = conv_resident_kernel<DTV, KS, KPT>;                                                    \
+    auto kfn = conv_resident_kernel<DTV, KS, KPT, ACTV>;                                                    \
     static bool attr_done = false;                                                                   \
     if (!attr_done) {                                                                                \
       hipError_t e = hipFuncSetAttribute((const void *)kfn, hipFuncAttributeMaxDynamicSharedMemorySize, \
@@ -483,8 +487,9 @@ int launch_conv_resident(const ContractionArgs &a, bool conv, int dtype, bool b_
     hipLaunchKernelGGL(kfn, grid, block, lds, stream, a);                                            \
     return (int)hipGetLastError();                                                                   \
   } while (0)
-  if (dtype == DT_F16) TRACEA_LAUNCH_RS(DT_F16);
-  else TRACEA_LAUNCH_RS(DT_BF16);
+  const bool act = activates_half(a);
+  if (dtype == DT_F16) { if (act) TRACEA_LAUNCH_RS(DT_F16, true); else TRACEA_LAUNCH_RS(DT_F16, false); }
+  else { if (act) TRACEA_LAUNCH_RS(DT_BF16, true); else TRACEA_LAUNCH_RS(DT_BF16, false); }
 #undef TRACEA_LAUNCH_RS
   return (int)hipErrorInvalidValue;
 }

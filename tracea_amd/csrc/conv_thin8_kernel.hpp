@@ -43,7 +43,7 @@ __host__ __device__ constexpr int ct_aux_bytes(int r, int p_tm, int patch_bytes)
   return staging > spill ? staging : spill;
 }
 
-template <int DT, int R>
+template <int DT, int R, bool ACT>
 __global__ void __launch_bounds__(CT_THREADS) conv_thin8_kernel(const ContractionCore args) {
   constexpr int NT = CT_THREADS, BN = 64, NW = NT / 64, C = 8, PBW = 2, STEPS = 2 * R;
   asm volatile("" ::"s"(args.A), "s"(args.B), "s"(args.N), "s"(args.ldb), "s"(args.b_bytes), "s"(args.grid_n), "s"(args.h_in),
@@ -265,7 +265,8 @@ __global__ void __launch_bounds__(CT_THREADS) conv_thin8_kernel(const Contractio
         }
       };
 #define TRACEA_CT_FORM(F) run_form(std::integral_constant<int, F>{})
-      TRACEA_EPILOGUE16_FORMS(sig, TRACEA_CT_FORM, )
+      if constexpr (ACT) { TRACEA_EPILOGUE16_ACTIVATIONS(sig, TRACEA_CT_FORM) }
+      else { TRACEA_EPILOGUE16_FORMS(sig, TRACEA_CT_FORM) }
 #undef TRACEA_CT_FORM
     } else {
       // any other chain: accumulators through the staging area, then the general operator loop over whole pixels
@@ -294,7 +295,7 @@ __global__ void __launch_bounds__(CT_THREADS) conv_thin8_kernel(const Contractio
           }
           const int nvalid = N - n;
           const long long m = m_img + pr;
-          apply_epilogue_tab(v, m, n, nvalid, args.epi, plan, table + ec, BN, args.out_dtype != DT_F32);
+          apply_epilogue_tab<ACT>(v, m, n, nvalid, args.epi, plan, table + ec, BN);
           store_from_float<8>(args.C, args.out_dtype, m * args.ldc + n, nvalid, v);
         }
       }
@@ -318,9 +319,9 @@ int launch_conv_thin8(const ContractionArgs &a, bool conv, int dtype, bool b_nco
   const size_t lds = (size_t)2 * a.p_np_bytes + ct_aux_bytes(R, a.p_tm, a.p_np_bytes) + CT_TABLE_BYTES;
   if (lds > 160 * 1024) return (int)hipErrorInvalidValue;
   const dim3 grid((unsigned)(a.p_iters * a.grid_n)), block(CT_THREADS);
-#define TRACEA_LAUNCH_CT(DTV)                                                                        \
+#define TRACEA_LAUNCH_CT(DTV, ACTV)                                                                  \
   do {                                                                                               \
-    auto kfn = conv_thin8_kernel<DTV, R>;                                                            \
+    auto kfn = conv_thin8_kernel<DTV, R, ACTV>;                                                      \
     static bool attr_done = false;                                                                   \
     if (!attr_done) {                                                                                \
       hipError_t e = hipFuncSetAttribute((const void *)kfn, hipFuncAttributeMaxDynamicSharedMemorySize, \
@@ -331,8 +332,9 @@ int launch_conv_thin8(const ContractionArgs &a, bool conv, int dtype, bool b_nco
     hipLaunchKernelGGL(kfn, grid, block, lds, stream, a);                                            \
     return (int)hipGetLastError();                                                                   \
   } while (0)
-  if (dtype == DT_F16) TRACEA_LAUNCH_CT(DT_F16);
-  else TRACEA_LAUNCH_CT(DT_BF16);
+  const bool act = activates_half(a);
+  if (dtype == DT_F16) { if (act) TRACEA_LAUNCH_CT(DT_F16, true); else TRACEA_LAUNCH_CT(DT_F16, false); }
+  else { if (act) TRACEA_LAUNCH_CT(DT_BF16, true); else TRACEA_LAUNCH_CT(DT_BF16, false); }
 #undef TRACEA_LAUNCH_CT
   return (int)hipErrorInvalidValue;
 }

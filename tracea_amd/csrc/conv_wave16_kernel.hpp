@@ -50,7 +50,7 @@ constexpr int cw_ring_stage_bytes(int cin) { return cw_ring_iters(cin) * 256 * 1
 // (the resident slab: tap t of the 64 filters at t * 64 * 2 * CIN bytes, without padding)
 inline int cw_resident_filter_bytes(int k) { return 64 * k * 2; }
 
-template <int DT, int CIN, int PBW, int RING, int WK = 4>
+template <int DT, int CIN, int PBW, int RING, int WK, bool ACT>
 __global__ void __launch_bounds__(CW_THREADS) conv_wave16_kernel(const ContractionCore args) {
   static_assert(WK == 4 || (WK == 8 && RING == 0), "eight multiplying waves only with the resident filter slab");
   static_assert(RING != 0 || CIN == 64, "the resident slab's layout: one load instruction per thread and tap");
@@ -557,7 +557,8 @@ __global__ void __launch_bounds__(CW_THREADS) conv_wave16_kernel(const Contracti
       }
     };
 #define TRACEA_CW_FORM(F) run_form(std::integral_constant<int, F>{})
-    TRACEA_EPILOGUE16_FORMS(form_sig, TRACEA_CW_FORM, TRACEA_EPILOGUE16_ACTIVATIONS(TRACEA_CW_FORM))
+    if constexpr (ACT) { TRACEA_EPILOGUE16_ACTIVATIONS(form_sig, TRACEA_CW_FORM) }
+    else { TRACEA_EPILOGUE16_FORMS(form_sig, TRACEA_CW_FORM) }
 #undef TRACEA_CW_FORM
     return;
   }
@@ -595,7 +596,7 @@ __global__ void __launch_bounds__(CW_THREADS) conv_wave16_kernel(const Contracti
       }
       const int nvalid = N - n;
       const long long m = m_img + pr;
-      apply_epilogue_tab(v, m, n, nvalid, args.epi, plan, table + ec, BN, args.out_dtype != DT_F32);
+      apply_epilogue_tab<ACT>(v, m, n, nvalid, args.epi, plan, table + ec, BN);
       store_from_float<8>(args.C, args.out_dtype, m * args.ldc + n, nvalid, v);
     }
   }
@@ -614,9 +615,9 @@ int launch_conv_wave16(const ContractionArgs &a, bool conv, int dtype, bool b_nc
   if ((size_t)a.p_tm * 68 * 4 > lds - CW_TABLE_BYTES) lds = (size_t)a.p_tm * 68 * 4 + CW_TABLE_BYTES;
   if (lds > 160 * 1024) return (int)hipErrorInvalidValue;
   const dim3 grid((unsigned)(a.grid_m * a.grid_n)), block(CW_THREADS);
-#define TRACEA_LAUNCH_CW(DTV)                                                                        \
+#define TRACEA_LAUNCH_CW(DTV, ACTV)                                                                  \
   do {                                                                                               \
-    auto kfn = conv_wave16_kernel<DTV, CIN, PBW, RING, WK>;                                               \
+    auto kfn = conv_wave16_kernel<DTV, CIN, PBW, RING, WK, ACTV>;                                    \
     static bool attr_done = false;                                                                   \
     if (!attr_done) {                                                                                \
       hipError_t e = hipFuncSetAttribute((const void *)kfn, hipFuncAttributeMaxDynamicSharedMemorySize, \
@@ -627,8 +628,9 @@ int launch_conv_wave16(const ContractionArgs &a, bool conv, int dtype, bool b_nc
     hipLaunchKernelGGL(kfn, grid, block, lds, stream, a);                                            \
     return (int)hipGetLastError();                                                                   \
   } while (0)
-  if (dtype == DT_F16) TRACEA_LAUNCH_CW(DT_F16);
-  else TRACEA_LAUNCH_CW(DT_BF16);
+  const bool act = activates_half(a);
+  if (dtype == DT_F16) { if (act) TRACEA_LAUNCH_CW(DT_F16, true); else TRACEA_LAUNCH_CW(DT_F16, false); }
+  else { if (act) TRACEA_LAUNCH_CW(DT_BF16, true); else TRACEA_LAUNCH_CW(DT_BF16, false); }
 #undef TRACEA_LAUNCH_CW
   return (int)hipErrorInvalidValue;
 }

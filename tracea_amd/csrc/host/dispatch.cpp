@@ -2046,11 +2046,9 @@ bool plan_conv_thin8(const ConvGeometry &g, const ContractionVariant &v, bool w_
 // SiLU], each part at most once and in this order, affine = bias / scale-shift / BatchNorm; every tile has all 64
 // channels, output rows and residual rows are 8-byte aligned and addressable with 32-bit byte offsets
 // inside a tile, output and residual have the operand type.  Anything else: sig = -1 (general path).
-// activations: whether the kernel has the forms with GELU and SiLU.  The one for 8 channels does not: its epilogue runs once per
-// tile of a persistent workgroup, and four more forms cost the others there (16x 112x112 8->64 7x7 with bias and ReLU 9.85 ->
-// 9.95 us, 10.15 behind a test of their own).  Elsewhere, bias and SiLU, us, before (general path) / now: 32x 56x56 64->64 3x3 18.8 / 12.4,
-// 32x 14x14 256->256 14.8 / 12.2.
-void fast_epilogue_form(const EpilogueChain &chain, int dtype, bool activations, ContractionArgs *a) {
+// Bias and SiLU, us, general path / this: 32x 56x56 64->64 3x3 17.9 / 12.1, 32x 14x14 256->256 14.8 / 12.5, 16x 112x112 8->64 7x7
+// 13.9 / 10.6.
+void fast_epilogue_form(const EpilogueChain &chain, int dtype, ContractionArgs *a) {
   ContractionArgs::FastEpilogue fe{};
   fe.sig = -1;
   a->fe = fe;
@@ -2064,7 +2062,6 @@ void fast_epilogue_form(const EpilogueChain &chain, int dtype, bool activations,
                      op.kind == TRACEA_EPI_OP_BATCHNORM;
     int part;
     if (op.kind == TRACEA_EPI_OP_NONE) continue;
-    else if (act && !activations) { ok = false; break; }
     else if (aff) part = 0;
     else if (act) part = 1;
     else if (op.kind == TRACEA_EPI_OP_RELU) part = stage <= 2 ? 1 : 3;
@@ -2272,8 +2269,7 @@ TraceaStatus run_conv(const ConvPlan &plan, const EpilogueChain &chain, hipStrea
   const long long w_extent = (long long)g.n_gemm * g.k_gemm * 2;
   const bool small = x_extent < (1ll << 31) && w_extent < (1ll << 31);
   if (conv_only(contraction_variant(vi)) && plan_conv_resident(g, contraction_variant(vi), plan.w_ncontig, &a)) {
-    if (contraction_variant(vi).pipeline == 5 || (contraction_variant(vi).pipeline >= 7 && contraction_variant(vi).pipeline <= 10)) 
-      fast_epilogue_form(chain, plan.x.dtype, contraction_variant(vi).pipeline != 10, &a);
+    if (contraction_variant(vi).pipeline == 5 || (contraction_variant(vi).pipeline >= 7 && contraction_variant(vi).pipeline <= 10)) fast_epilogue_form(chain, plan.x.dtype, &a);
     const int e = contraction_variant(vi).launch(a, true, plan.x.dtype, false, stream);
     // a member that refuses the arguments its plan accepted (it launched nothing) gives way to the
     // selector's choice below, like one whose plan failed
