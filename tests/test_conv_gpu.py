@@ -383,7 +383,7 @@ def test_filter_resident_variant_operator_chains(tracea_gpu, member, cin):
 def test_conv_activations_in_the_epilogue_from_registers(tracea_gpu, member, cin, r, stride, dtype):
     """GELU and SiLU with and without an affine part in front, which the kernels with an epilogue from registers take there,
     and chains that must not be taken for these: parts before or behind the activation.  Scores from -60 to 60 reach both
-    ends of the activations.  Tolerance: that of the sum and of the stored result's rounding, and as
+    ends of the activations, some from -480 to 480 go beyond the range of SiLU's short form.  Tolerance: that of the sum and of the stored result's rounding, and as
     much again for the slopes of two activations (at most 1.13 each) and a second rounding."""
     from tracea_amd import capi
     rng = np.random.default_rng(5)
@@ -398,13 +398,14 @@ def test_conv_activations_in_the_epilogue_from_registers(tracea_gpu, member, cin
     dx, dw = _dev(x, td), _dev(w_rsck, td).permute(3, 0, 1, 2).contiguous()
     O, E = capi, oracle
     bias_op = ((O.OP_BIAS_ADD, _dev(bias)), (E.EPI_BIAS_ADD, bias))
+    wide = ((O.OP_BIAS_ADD, _dev(bias * 8)), (E.EPI_BIAS_ADD, bias * 8))
     ss = ((O.OP_SCALE_SHIFT, _dev(scale), _dev(shift)), (E.EPI_SCALE_SHIFT, scale, shift))
     bn = ((O.OP_BATCHNORM, _dev(gamma), _dev(beta), _dev(mean), _dev(var), 1e-5), (E.EPI_BATCHNORM, gamma, beta, mean, var, 1e-5))
     relu, gelu, silu = ((O.OP_RELU,), (E.EPI_RELU,)), ((O.OP_GELU,), (E.EPI_GELU,)), ((O.OP_SILU,), (E.EPI_SILU,))
     resid = ((O.OP_RESIDUAL_ADD, _dev(res, td)), (E.EPI_RESIDUAL_ADD, res))
     capi.force_variant("conv2d", member)
     try:
-        for chain in ([gelu], [silu], [bias_op, gelu], [bias_op, silu], [ss, gelu], [bn, silu], [relu, gelu], [gelu, relu], [silu, resid],
+        for chain in ([gelu], [silu], [bias_op, gelu], [bias_op, silu], [wide, gelu], [wide, silu], [ss, gelu], [bn, silu], [relu, gelu], [gelu, relu], [silu, resid],
                       [resid, silu], [bias_op, silu, gelu], [silu, bias_op], [bias_op, relu, silu]):
             want = oracle.epilogue_apply(acc, [c[1] for c in chain])
             y = tracea_gpu.conv2d_ex(dx, dw, [c[0] for c in chain], stride=stride, padding=r // 2)

@@ -486,27 +486,32 @@ def test_output_over_an_operand(tracea_gpu, dtype, shape):
 @pytest.mark.parametrize("n", [128, 120])  # whole tiles (the row body with the short forms) and partial ones (the general one)
 def test_activations_over_the_whole_range(tracea_gpu, dtype, kind, n):
     """Every row holds one value x in all columns: zero, tiny, the range in which the activation bends, where its exponential
-    leaves fp32, the type's largest, infinities and NaN, against the formula in float64.  Three units of fp32 in the
-    exponential's argument (up to 2^8 before it overflows) and half a unit of the stored type; results below the
-    smallest normal number of fp32 or the type count as that small."""
+    leaves fp32 (GELU near -10, SiLU near -87), the type's largest, infinities and NaN; with a bias, columns that differ by
+    less than the type resolves.  Against the formulas in float64, written without their cancellation below zero.  Bounds: half
+    a unit of the stored type; 2^-24 six times (two each for the power and the reciprocal or quotient, one for the sum and the
+    product), and for GELU three times more per power of two in its exponent (square, sum, product and the two constants, times
+    ln 2) as far as the power counts in the sum; half the smallest number of the type; and where the power is beyond fp32 (SiLU) or its reciprocal
+    below fp32's normal numbers (GELU) |x| times that, which is nothing against the others elsewhere."""
     big = torch.finfo(dtype).max
     x = torch.cat([torch.tensor([0.0, -0.0, big, -big, float("inf"), float("-inf"), float("nan")]), torch.linspace(-20, 20, 641),
+                   torch.linspace(-11, -9, 65), torch.linspace(-128, -64, 129), torch.linspace(64, 128, 65),
                    torch.tensor([1.0, -1.0]).repeat_interleave(20) * torch.logspace(-6, 4, 20).repeat(2)]).to(dtype)
     a = torch.zeros(x.numel(), 64, dtype=dtype)
     a[:, 3] = x
     b = torch.zeros(64, n, dtype=dtype)
     b[3] = 1
-    kw = {"bias": torch.zeros(n).cuda()} if "bias" in kind else {}
+    bias = torch.linspace(-0.25, 0.25, n) if "bias" in kind else torch.zeros(n)
+    kw = {"bias": bias.cuda()} if "bias" in kind else {}
     got = tracea_gpu.gemm(a.cuda(), b.cuda(), epilogue=kind, **kw).double().cpu()
-    v = x.double()
-    want = 0.5 * v * (1 + torch.tanh(0.79788456 * (v + 0.044715 * v ** 3))) if kind == "gelu" else v / (1 + torch.exp(-v))
-    v, want = v[:, None].expand_as(got), want[:, None].expand_as(got)
+    v = (x.float()[:, None] + bias).double()
+    power = -2 * 0.79788456 * (v + 0.044715 * v ** 3) if kind == "gelu" else -v
+    want = v / (1 + torch.exp(power))
     assert torch.equal(torch.isnan(got), torch.isnan(want))
     assert torch.equal(got[torch.isinf(want)], want[torch.isinf(want)])
     fin = torch.isfinite(want)
     half_unit = 2.0 ** -11 if dtype == torch.float16 else 2.0 ** -8
-    # (1 + tanh cancels below zero in the general body: an absolute error of two units of fp32 times |x|)
-    bound = want.abs() * (half_unit + 3 * 2.0 ** -16) + v.abs() * 2.0 ** -22 + max(torch.finfo(dtype).tiny * half_unit, 2.0 ** -126)
+    units, lost = (6 + 3 * power.abs() / np.log(2) * torch.sigmoid(power), 2.0 ** -126) if kind == "gelu" else (6.0, 2.0 ** -128)
+    bound = want.abs() * (half_unit + units * 2.0 ** -24) * (1 + half_unit) + torch.finfo(dtype).tiny * half_unit + v.abs() * lost
     assert bool(((got - want).abs() <= bound)[fin].all())
 
 

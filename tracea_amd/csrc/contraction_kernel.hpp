@@ -162,13 +162,46 @@ __device__ __forceinline__ float gelu_half(float x) {
 }
 __device__ __forceinline__ float silu(float x) { return x / (1.0f + expf(-x)); }
 
-// SiLU in the same way, x / (1 + 2^(x c1)).
+// SiLU of G x V values of one lane, for the fast row bodies: expf's own steps (2^n times the hardware's exp2 of what is left
+// of x log2(e) in two parts) and the quotient with its remainder added back, eleven instructions a value and half a one to find
+// the largest, where expf with its range checks and the division take 25.  Largest relative error 1.8e-7, root
+// mean square 3.7e-8 to 4.4e-8 from -80 to 80: those of the library.  Only while no power or reciprocal leaves the normal
+// numbers, that is up to silu_in_range: beyond (infinities among them) the library.  NaN stays NaN.  bf16 2048x5632x2048 55.7 us, with
+// expf and the division for all values 67.7.
 template <int G, int V>
-__device__ __forceinline__ void silu_half(float (&v)[G][V]) {
+__device__ __forceinline__ bool silu_in_range(const float (&v)[G][V]) {
+  float top = 0.0f;
 #pragma unroll
   for (int g = 0; g < G; ++g)
 #pragma unroll
-    for (int e = 0; e < V; ++e) v[g][e] = v[g][e] * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(v[g][e] * -1.4426950f));
+    for (int e = 0; e < V; ++e) top = fmaxf(top, fabsf(v[g][e]));
+  return top <= 86.0f;
+}
+template <int G, int V>
+__device__ __forceinline__ void silu_half_in_range(float (&v)[G][V]) {
+#pragma unroll
+  for (int g = 0; g < G; ++g)
+#pragma unroll
+    for (int e = 0; e < V; ++e) {
+      const float x = v[g][e];
+      const float m = fmaf(x, -1.44269502f, 12582912.0f);  // n in the low bits: 1.5 * 2^23 has a unit of one
+      const float n = m - 12582912.0f;
+      const float p = __builtin_amdgcn_exp2f(fmaf(x, -1.92596303e-8f, fmaf(x, -1.44269502f, -n)));
+      const float d = 1.0f + __builtin_bit_cast(float, __builtin_bit_cast(unsigned, p) + (__builtin_bit_cast(unsigned, m) << 23));
+      const float r = __builtin_amdgcn_rcpf(d), y = x * r;
+      v[g][e] = fmaf(fmaf(-d, y, x), r, y);
+    }
+}
+template <int G, int V>
+__device__ __forceinline__ void silu_half(float (&v)[G][V]) {
+  if (__builtin_expect(silu_in_range(v), 1)) {
+    silu_half_in_range(v);
+  } else {
+#pragma unroll
+    for (int g = 0; g < G; ++g)
+#pragma unroll
+      for (int e = 0; e < V; ++e) v[g][e] = silu(v[g][e]);
+  }
 }
 template <int G, int V>
 __device__ __forceinline__ void gelu_half(float (&v)[G][V]) {
@@ -1711,7 +1744,7 @@ __global__ void __launch_bounds__(WM *WN * 64) contraction_kernel(const std::con
     __builtin_amdgcn_wave_barrier();
   };
   if constexpr (ACT) {
-    // (one copy of the rows for all blocks: GELU and SiLU are long, and a copy each is more than the instruction cache holds)
+    // (one copy of the rows for all blocks: with one each, bf16 2048x5632x2048 with SiLU waited for its code, 62.4 us against 55.7)
 #pragma nounroll
     for (int i = 0; i < FM; ++i) {
       static_for<0, FM>([&](auto blk) {
