@@ -400,17 +400,48 @@ def test_rule_and_block_order(tracea_gpu, case, causal):
     assert_close_scaled(got.float().cpu().numpy(), oracle.attention_bhsd(q, k, v, 1.0 / np.sqrt(d), causal), _tol(d, "f16"), str(case))
 
 
+# Under a causal mask beyond one workgroup per CU, both sides of each line: groups over the keys up to two workgroups per CU from 2048
+# keys on (384 and 512 workgroups, 520 of them, 2040 keys, a third head dimension that has no such member); heads no multiple of 4 (up
+# to 9/8 per CU, fewer than 8 heads, above in pairs, an odd number of blocks); above D 64 nearly two per CU on short walks; pairs in whole
+# rounds up to 2048 keys, at one per CU, beyond 2048 keys and wherever 4 divides no heads
+@pytest.mark.parametrize("b,h,s,d,member", [
+    (1, 12, 4096, 64, "q128_kv64_d64_k2"), (1, 12, 4096, 128, "q128_kv64_d128_k2"), (1, 16, 4090, 64, "q128_kv64_d64_k2"),
+    (1, 20, 3300, 64, "q128_kv64_d64_pipe2"), (1, 32, 1900, 64, "q128_kv64_d64_pipe2"), (1, 12, 4096, 96, "q128_kv64_part96"),
+    (1, 9, 4096, 64, "q128_kv64_d64_k2"), (1, 9, 4100, 64, "q128_kv64_d64_pipe2"), (1, 7, 6100, 64, "q128_kv64_d64_k2"),
+    (1, 7, 7100, 64, "q128_kv64_d64_pipe2_x2"), (1, 30, 2048, 64, "q128_kv64_d64_pipe2_x2"), (1, 18, 2048, 128, "q128_kv64_d128_k2"),
+    (1, 19, 2048, 128, "q128_kv64_d128_pipe2_x2"), (1, 26, 2100, 128, "q128_kv64_d128_pipe2"),
+    (1, 32, 2048, 128, "q128_kv64_d128_pipe2_x2"), (1, 28, 2304, 128, "q128_kv64_d128_pipe2_x2"), (1, 28, 2048, 128, "q128_kv64_d128_k2"), (1, 32, 1921, 128, "q128_kv64_d128_pipe2_x2"),
+    (1, 16, 4096, 128, "q128_kv64_d128_k2"), (1, 32, 2048, 64, "q128_kv64_d64_k2"),
+    (2, 32, 1024, 128, "q128_kv64_d128_pipe2"), (8, 32, 512, 64, "q128_kv64_d64_pipe2_x2"), (4, 32, 2048, 128, "q128_kv64_d128_pipe2_x2"),
+    (4, 32, 2304, 64, "q128_kv64_d64_pipe2"), (3, 31, 1024, 64, "q128_kv64_d64_pipe2_x2")])
+def test_causal_rule_beyond_one_workgroup_per_cu(tracea_gpu, b, h, s, d, member):
+    """The member that the rule takes, and its rows as the bits that the same member gives for single heads."""
+    from tracea_amd import capi
+    g = torch.Generator(device="cuda").manual_seed(b * h + s + d)
+    q, k, v = (torch.randn(b, h, s, d, device="cuda", generator=g).half() for _ in range(3))
+    out = tracea_gpu.attention(q, k, v, causal=True)
+    assert capi.last_variant("attention") == "fa2_" + member
+    capi.force_variant("attention", "fa2_" + member)
+    try:
+        for bi, hi in ((0, 0), (b // 2, h // 2), (b - 1, h - 1)):
+            one = [t[bi:bi + 1, hi:hi + 1] for t in (q, k, v)]
+            assert torch.equal(tracea_gpu.attention(*one, causal=True)[0, 0], out[bi, hi]), (bi, hi)
+    finally:
+        capi.force_variant("attention", -1)
+
+
 # Causal launches beyond one workgroup per CU take the last query block of 64 heads at a time first.  One group of heads and a
 # smaller one, several groups with 4 heads left, numbers that 4 but not 8 divides, and one that keeps the old order (67): each
 # head's rows are the bits that a launch of that head alone gives, so every block ran once and in its place.
 @pytest.mark.parametrize("b,h,s", [(1, 12, 2900), (1, 36, 1030), (1, 68, 600), (2, 66, 300), (3, 64, 200), (1, 67, 600)])
-@pytest.mark.parametrize("d", [64, 96, 128])
-def test_heaviest_blocks_first(tracea_gpu, b, h, s, d):
+@pytest.mark.parametrize("member", ["q128_kv64_d64_pipe2", "q128_kv64_part96", "q128_kv64_d128_pipe2", "q128_kv64_d64_k2", "q128_kv64_d128_k2"])
+def test_heaviest_blocks_first(tracea_gpu, b, h, s, member):
     from tracea_amd import capi
+    d = 96 if "part96" in member else 64 if "d64" in member else 128
     g = torch.Generator(device="cuda").manual_seed(b * h + s + d)
     q, k, v = (torch.randn(b, h, s, d, device="cuda", generator=g).half() for _ in range(3))
     out = torch.full_like(q, float("nan"))
-    capi.force_variant("attention", "fa2_q128_kv64_part96" if d == 96 else "fa2_q128_kv64_d%d_pipe2" % d)
+    capi.force_variant("attention", "fa2_" + member)
     try:
         tracea_gpu.attention(q, k, v, causal=True, out=out)
         for bi in range(b):

@@ -130,7 +130,7 @@ def test_tune_fa2_returns_a_flash_variant(tracea_gpu, cache_file):
     assert ("q%d_" % cfg["m_tile"]) in ran and cfg["intrinsic_shape"] == shape
     assert cfg["fusion_count"] == (2 if ran.endswith("_x2") else 1)  # query blocks per workgroup
     # without a record: dense attention over a long sequence takes 256 queries on eight waves, one block per
-    # workgroup; under a causal mask, with a pair of query blocks per CU or more, 128 on four, two blocks each
+    # workgroup; under a causal mask, with pairs of query blocks in whole rounds of two per CU, 128 on four, two blocks each
     q, k, v = [torch.randn(4, 32, 2048, 128, device="cuda").bfloat16() for _ in range(3)]
     tracea_gpu.attention(q, k, v, causal=False)
     assert capi.last_variant("attention") == "fa2_q256_kv64_d128_s2_pipe2"

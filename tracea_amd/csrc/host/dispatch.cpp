@@ -2946,20 +2946,32 @@ TraceaStatus dispatch_attention(const TraceaTensorView &tq, const TraceaTensorVi
   if (vi < 0 && blocks64 <= cus && S > from64) vi = D <= 64 ? member(64, 8, 1, 4) : member(64, 4, 1, 2);
   if (vi < 0 && blocks128 <= cus && S > from128) vi = member(128, 8, 1, 2);
   // Under a causal mask, up to two workgroups per CU over a long sequence: the last block's walk over its keys is longer than
-  // a SIMD's share of all the work, so two groups share that as well.  H12 S4096 D64 45.2 / 36.7, D128 67.7 / 58.0, H8 S8192
-  // D64 95.5 / 79.0, H32 S2048 27.2 / 26.5 and 42.1 / 41.7, but H36 S1500 20.3 / 21.5, H40 S1024 14.3 / 15.1.
-  if (vi < 0 && a.causal && S >= 2048 && blocks128 > cus && blocks128 <= 2 * cus) vi = member(128, 8, 1, 2);
+  // a SIMD's share of all the work, so two groups share that as well.  Single blocks / groups, us: H12 S4096 D64 44.6 / 36.0, D128
+  // 68.3 / 58.4, H8 S8192 D64 95.4 / 78.5, but H36 S1500 20.3 / 21.5, H40 S1024 14.3 / 15.1.  Two places of the range belong to
+  // pairs of blocks, which come in one round there.  Heads that are no multiple of 4 keep their order (the kernel's comment), so the
+  // heavy blocks of the last heads end a launch of groups: groups / pairs / single blocks, D64 H30 S2048 34.0 / 26.8 / 30.1, H15 S4096 61.8 /
+  // 45.2 / 54.2, H13 S3072 36.9 / 35.0 / 35.9, D128 H19 S2048 40.6 / 36.0 / 41.1, and odd numbers of blocks, which have no pairs, H9 S4224
+  // 58.8 / - / 49.9, H26 S2176 34.8 / - / 30.1; few blocks per CU or heads that fill no XCD twice stay: H9 S4096 40.4 / 43.6 / 50.9, H13
+  // S2560 23.2 / 30.7 / 27.3, H6 S8192 73.2 / 80.1 / 89.0.  And above D 64 nearly two workgroups per CU on short walks: D128 H32 S2048 42.0 /
+  // 41.2 / 42.4, S1980 41.7 / 41.0 / 41.6, H28 S2304 46.4 / 45.1 / 46.7, but H28 S2048 39.5 / 39.4 / 39.8, H24 S2304 41.4 / 41.6 / 43.4, H20 S3072
+  // 55.2 / 55.3 / 58.7, H16 S4096 72.2 / 73.6 / 79.0.
+  if (vi < 0 && a.causal && S > 1920 && blocks128 > cus && blocks128 <= 2 * cus) {
+    const bool late_heavy = bh % 4 != 0 && blocks128 * 8 > cus * (bh < 8 ? 12 : 9);
+    const bool short_and_full = D > 64 && S < 3072 && blocks128 * 4 > cus * 7;
+    if (short_and_full || (late_heavy && S >= 2048)) vi = member(128, 4, 2);
+    else if (S >= 2048) vi = member(128, 8, 1, 2);
+  }
   // Two query blocks per workgroup, a heavy one paired with a light one, fill the device evenly where their number is a
   // multiple of two per CU, and start the second block on tiles already requested.  Single blocks, the heaviest first,
-  // need no such number.  Replayed graphs, pairs / single blocks, us: B4 H12 S1500 D64 29.0 / 22.2, D128 44.7 / 35.5, B4 H32
+  // need no such number, and are ahead at one pair per CU: B2 H32 S1024 D64 20.0 / 17.8, D128 26.7 / 25.5, B4 H32 S512 13.2 / 12.6 and
+  // 18.7 / 18.6.  Replayed graphs, pairs / single blocks, us: B4 H12 S1500 D64 29.0 / 22.2, D128 44.7 / 35.5, B4 H32
   // S700 D128 32.4 / 29.6, B2 H18 S4096 D64 114.1 / 88.2, B4 H32 S4096 D128 492.7 / 487.9; in full rounds over sequences up
   // to 2048 the pairs are ahead or level: B8 H32 S512 D64 19.8 / 21.2, D128 32.1 / 33.1, S1024 D128 82.8 / 84.7, B4 H32 S2048
   // 135.2 / 135.5.
   // Heads that are no multiple of 4 come in their old order, and in pairs wherever these fill the device (B3 H31 S2048 D128
   // 105.6 against 136.8 with the heaviest blocks of all heads first).
-  // (Dense attention does not take the pairs by rule: with the softmax shift folded into the score product,
-  // which the paired members at head dimension 128 have no registers for, the one-block eight-wave member below
-  // is ahead -- B4 H32 S4096 D128 904 us against 964, B8 H32 S2048 D64 294 against 302, same box.)
+  // (Dense attention does not take the pairs by rule: the one-block eight-wave member below is ahead --
+  // B4 H32 S4096 D128 935 us against 956 and 974 for its pairs and those of four waves, B8 H32 S2048 D64 293 against 294 and 297.)
   const long long pairs = bh * (((S + 127) / 128) / 2);
   if (vi < 0 && a.causal && pairs >= cus && (bh % 4 != 0 || (S <= 2048 && pairs % (2 * cus) == 0))) vi = member(128, 4, 2);
   // Dense attention over a long sequence with enough workgroups to go round: 256 queries on eight waves share
