@@ -432,9 +432,15 @@ __device__ __forceinline__ void apply_epilogue_tab(float (&v)[8], long long m, i
   for (int o = 0; o < plan.n_ops; ++o) {
     const int kind = (int)((plan.kinds >> (4 * o)) & 15u);
     if (ACT && (kind == TRACEA_EPI_OP_SILU || kind == TRACEA_EPI_OP_BIAS_ADD_SILU)) {
-      float t[1][8];
+      float t[1][8] = {{v[0], v[1], v[2], v[3], v[4], v[5], v[6], v[7]}};
+      if (kind == TRACEA_EPI_OP_BIAS_ADD_SILU) {
+        const f32x4 a0 = *(const f32x4 *)(tab + (o * 2) * bn), a1 = *(const f32x4 *)(tab + (o * 2) * bn + 4);
 #pragma unroll
-      for (int e = 0; e < 8; ++e) t[0][e] = kind == TRACEA_EPI_OP_SILU ? v[e] : v[e] + tab[(o * 2) * bn + e];
+        for (int e = 0; e < 4; ++e) {
+          t[0][e] += a0[e];
+          t[0][4 + e] += a1[e];
+        }
+      }
       silu_half(t);
 #pragma unroll
       for (int e = 0; e < 8; ++e) v[e] = t[0][e];
