@@ -481,7 +481,7 @@ fa2_fwd_pipe_kernel(const AttentionArgs a) {
   // workgroups lost what they gain: H36 S400 D128 15.2 us against 11.7 on blocks of 128, now 11.5.  Under a causal mask
   // beyond one workgroup per CU a ragged total stays in order: the run's last blocks are heavy ones and meet heavy ones
   // on their CU (261 blocks, H9 S3600 D128, 63 us against 52).
-  const bool runs = (total & 7) == 0 || !a.causal || total <= 256;
+  const bool runs = (total & 7) == 0 || !a.causal || total <= a.cus;
   const int xcd = blockIdx.x & 7;
   const int vid = runs ? xcd * (total >> 3) + min(xcd, total & 7) + ((int)blockIdx.x >> 3) : (int)blockIdx.x;
   // Under a causal mask and beyond one workgroup per CU: the last query block of every head, then the one before, and so on,
@@ -491,7 +491,7 @@ fa2_fwd_pipe_kernel(const AttentionArgs a) {
   // against 279).
   const int heads = a.B * a.H;
   int bh, slot;
-  if (ITEMS == 1 && a.causal && total > 256 && (heads & 3) == 0) {
+  if (ITEMS == 1 && a.causal && total > a.cus && (heads & 3) == 0) {
     const int first = (int)blockIdx.x / (64 * per_bh) * 64, r = (int)blockIdx.x - first * per_bh, n = min(64, heads - first);
     slot = r / n;
     bh = first + r - slot * n;

@@ -120,6 +120,7 @@ struct AttentionArgs {
   long long o_sb, o_sh, o_ss;
   float scale_log2;  // softmax scale * log2(e)
   int causal;
+  int cus;  // of the device: the order of the blocks changes where a launch has more workgroups
 };
 
 // A precompiled kernel variant and the rule that says when it applies.

@@ -2918,6 +2918,7 @@ TraceaStatus dispatch_attention(const TraceaTensorView &tq, const TraceaTensorVi
   a.o_sb = o.stride[0]; a.o_sh = o.stride[1]; a.o_ss = o.stride[2];
   a.scale_log2 = scale * 1.4426950408889634f;
   a.causal = params.causal ? 1 : 0;
+  a.cus = (int)device_limits().cus;
 
   // Choice of the family member: a forced one, else the tuner's record of this problem, else by rule.
   int vi = forced_variant("attention");
