@@ -518,9 +518,12 @@ def test_activations_over_the_whole_range(tracea_gpu, dtype, kind, n):
 # four to eight elements in an operand, K on and off the 32-deep tiles, a last row of B within 4 elements of the end in the tile
 # before the last (N 1 and 3), two groups of waves with an even and an odd number of K tiles, more tiles than CUs (1100 x 1090)
 @pytest.mark.parametrize("shape", [(1, 5, 4), (4, 1, 33), (2, 3, 34), (65, 3, 66), (63, 65, 64), (64, 64, 95), (3, 130, 127), (70, 67, 321),
-                                   (129, 65, 577), (1100, 1090, 403)])
+                                   (129, 65, 577), (1100, 1090, 403), (70, 67, 31)])
 def test_fp32_operands_at_any_element_alignment(tracea_gpu, shape):
-    """As above for fp32 with both operands by rows."""
+    """As above for fp32 with both operands by rows.  That they are read in place: two groups of waves where the rule says so (padded
+    copies of a K below 512 are not split, and their product has a K of its own), and the bits of the entry point that makes no copies
+    (which otherwise sums in one chain; four products or fewer may round alike in both)."""
+    from tracea_amd import capi
     m, n, k = shape
     rng = np.random.default_rng(m + 3 * n + 7 * k)
     a = (rng.standard_normal((m, k)) / np.sqrt(k)).astype(np.float32)
@@ -538,7 +541,15 @@ def test_fp32_operands_at_any_element_alignment(tracea_gpu, shape):
     for gap, first in ((0, 1), (1, 0), (3, 2), (5, 3)):
         for junk in (float("nan"), float("inf")):
             out = torch.full((m + 1, n + 3), 7.0, device="cuda")
-            tracea_gpu.gemm(placed(a, gap, first, junk), placed(b, gap, first, junk), bias=_dev(bias), epilogue="bias+relu", out=out[:m, :n])
+            args = placed(a, gap, first, junk), placed(b, gap, first, junk)
+            tracea_gpu.gemm(*args, bias=_dev(bias), epilogue="bias+relu", out=out[:m, :n])
+            tiles = -(-m // 64) * -(-n // 64)
+            groups = 2 if 32 < k and tiles <= torch.cuda.get_device_properties(0).multi_processor_count else 1
+            assert (capi.lib().tracea_last_split_k(), capi.lib().tracea_last_split_k_launches()) == (groups, 1)
+            if k >= 30:
+                other = torch.empty(m, n, device="cuda")
+                tracea_gpu.gemm_noalloc(*args, other, bias=_dev(bias), epilogue="bias+relu")
+                assert torch.equal(other, out[:m, :n]), "ran from copies"
             got = out.cpu().numpy()
             # (k products and sums rounded to fp32, about 3 in absolute value at most for a row of A of unit length)
             assert np.abs(got[:m, :n] - ref).max() <= 2.0 ** -24 * 2 * (k + 8) * max(1.0, np.abs(ref).max()), (gap, first)
