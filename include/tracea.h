@@ -321,10 +321,10 @@ TraceaStatus tracea_linear(TraceaTensorView a, TraceaTensorView w, const TraceaT
  * form the calling thread's latest gemm / conv2d launch took (1 or 2).  (The reference has no split along K:
  * its GEMM grid is one block per output tile, src/emitter/cuda/gemm.rs:92-207.) */
 /* Operands of tracea_gemm / tracea_gemm_ex whose rows are not whole 16-byte pieces or do not start on 16 bytes:
- * half precision with A along K and B along N or K is read in place, at any element alignment, except where a
- * short, deep or very large product is faster from copies.  The rest -- fp32 with such rows, operands strided
- * along K -- is copied into padded, zero-filled rows of a second per-(device, stream) buffer (at most 1 GiB,
- * same rules as the one above) and multiplied from there.  Where that buffer cannot be had
+ * half precision with A along K and B along N or K, and fp32 with A along K and B along N, are read in place, at any
+ * element alignment, except where a deep product of few tiles or a large one is faster from copies.  Those and the rest
+ * (fp32 with B along K, operands strided along K) are copied into padded, zero-filled rows of a second
+ * per-(device, stream) buffer (at most 1 GiB, same rules as the one above) and multiplied from there.  Where that buffer cannot be had
  * (tracea_gemm_noalloc, a stream under capture that made no such call before, A and B of different types) a
  * kernel on the vector ALU that reads any layout runs instead: same results, far slower.  (The reference's
  * kernels take M, N, K as they come: src/emitter/cuda/gemm.rs:92-207 guards every element.) */

@@ -144,9 +144,9 @@ __global__ void __launch_bounds__(RS_THREADS) conv_resident_kernel(const Contrac
   // part at most once and in this order, where affine is a bias, a scale-shift or a BatchNorm (all three
   // become v*a + b with per-channel a, b: a bias is a = 1); every channel of every tile exists, rows are
   // 8-byte aligned, output and residual have the operand type.  sig says which parts are present (bit 0
-  // affine, 1 first ReLU, 2 residual, 3 second ReLU) and selects one of 16 straight-line epilogues; sig < 0:
-  // any other chain, the general path.  Table: fast form entries [0..63] = a, [64..127] = b; general path
-  // the layout of chain_table_value.
+  // affine, 1 first ReLU, 2 residual, 3 second ReLU; in the kernel with ACT bit 4 SiLU or 5 GELU behind the affine part) and
+  // selects one of 16 straight-line epilogues (4 with ACT); sig < 0: any other chain, the general path.  Table: fast form
+  // entries [0..63] = a, [64..127] = b; general path the layout of chain_table_value.
   const int sig = args.fe.sig;
   constexpr int TPT = RS_TABLE_BYTES / 4 / NT;  // table entries per thread on the general path
   float tabr = 0.0f, tabg[TPT];
@@ -443,8 +443,8 @@ __global__ void __launch_bounds__(RS_THREADS) conv_resident_kernel(const Contrac
     }
 #undef TRACEA_RS_FORM
   } else {
-    // every other case (partial channel groups, unaligned rows, fp32 output, GELU / SiLU among
-    // others, further residuals): the general operator chain on the staged values
+    // every other case (partial channel groups, unaligned rows, fp32 output, GELU / SiLU among other
+    // operators, further residuals): the general operator chain on the staged values
     const ChainPlan plan = chain_plan(args.epi);
     for (int idx = tid; idx < npix * (BN / 8); idx += NT) {
       const int pr = idx >> 3;

@@ -115,8 +115,8 @@ __global__ void __launch_bounds__(CW_THREADS) conv_wave16_kernel(const Contracti
 
   // ---- epilogue form ----
   // sig >= 0: the chain reads [affine] [ReLU] [residual] [ReLU] (bit 0 affine, 1 first ReLU, 2 residual,
-  // 3 second ReLU), affine = v*a + b per channel; table [0..63] = a, [64..127] = b.  sig < 0: any other
-  // chain, table in the layout of chain_table_value.
+  // 3 second ReLU) or, in the kernel with ACT, [affine] and SiLU (bit 4) or GELU (bit 5), affine = v*a + b per channel; table
+  // [0..63] = a, [64..127] = b.  sig < 0: any other chain, table in the layout of chain_table_value.
   const int sig = args.fe.sig;
   // the resident slab's nine taps are awaited in two groups (the general chain's table takes the old road)
   const bool prog = RING == 0 && taps == 9 && sig >= 0;

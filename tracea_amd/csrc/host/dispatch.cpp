@@ -1166,8 +1166,8 @@ TraceaStatus run_gemm(const View &a, const View &b, const View &c, const Epilogu
     const int groups = ragged_f32_groups(M, N, K);
     if (groups != 0) return run_gemm_f32_any_alignment(a, b, c, chain, g_split_k_enabled.load() ? groups : 1, stream);
   }
-  // Operands none of these kernels reads in place -- fp32 with a K that is not a whole number of 16-byte pieces or rows
-  // that do not start on 16 bytes, strides along K, and half precision where ragged_tile says so -- are copied once into
+  // Operands none of these kernels reads in place -- rows off 16 bytes where ragged_tile (half precision) or ragged_f32_groups
+  // says so, fp32 with a B by columns, strides along K -- are copied once into
   // padded, zero-filled rows and multiplied from there: two copy launches in front of a tile kernel instead of
   // the any-layout kernel on the vector ALU (fp32 1000 x 900 x 1030: 794 us there).  Half precision: both as
   // K-contiguous rows (a row-major B is transposed on the way); fp32: A by rows, B row-major.  Not for the entry
