@@ -86,6 +86,38 @@ def test_small_shapes_every_variant_both_filter_layouts(tracea_gpu, variant):
         capi.force_variant("conv2d", -1)
 
 
+@pytest.mark.parametrize("variant", range(40))
+def test_activations_every_variant_both_filter_layouts(tracea_gpu, variant):
+    """The kernels with activations are others than those without: both filter layouts, whole and partial tiles (64, 128, 72
+    filters), a stride, and scores beyond 86 in some channels only."""
+    from tracea_amd import capi
+    names = capi.variants("conv2d")
+    if variant >= len(names):
+        pytest.skip("no such variant")
+    capi.force_variant("conv2d", variant)
+    try:
+        for n, h, w, c, k, r, stride, pad in ((2, 20, 20, 64, 64, 3, 1, 1), (3, 14, 14, 64, 128, 3, 2, 1), (1, 33, 17, 32, 72, 3, 1, 1), (2, 9, 7, 16, 24, 1, 1, 0)):
+            rng = np.random.default_rng(variant * 100 + h + c)
+            x = round_bf16(rng.standard_normal((n, h, w, c)))
+            w_rsck = round_bf16(rng.standard_normal((r, r, c, k)) * np.sqrt(2.0 / (r * r * c)))
+            bias = np.where(rng.random(k) < 0.1, rng.uniform(-200, 200, k), rng.standard_normal(k) * 3).astype(np.float32)
+            acc = oracle.conv2d_nhwc(x, w_rsck, stride, pad, 1)
+            res = round_bf16(rng.standard_normal(acc.shape))
+            dx, dbias, dres = _dev(x, torch.bfloat16), _dev(bias), _dev(res, torch.bfloat16)
+            dw = _dev(w_rsck, torch.bfloat16)
+            tol = 1.13 * tol_half(r * r * c, "bf16")  # (an activation's slope)
+            silu = oracle.epilogue_apply(acc, [(oracle.EPI_BIAS_ADD_SILU, bias)])
+            chain = oracle.epilogue_apply(acc, [(oracle.EPI_BIAS_ADD, bias), (oracle.EPI_GELU,), (oracle.EPI_RESIDUAL_ADD, res)])
+            for bank, layout in ((dw.permute(3, 0, 1, 2).contiguous(), "krsc"), (dw, "rsck")):
+                y = tracea_gpu.conv2d(dx, bank, bias=dbias, stride=stride, padding=pad, epilogue="bias+silu", weight_layout=layout)
+                assert_close_scaled(y.float().cpu().numpy(), silu, tol, "%s %s bias+silu" % (names[variant], layout))
+                y = tracea_gpu.conv2d_ex(dx, bank, [(capi.OP_BIAS_ADD, dbias), (capi.OP_GELU,), (capi.OP_RESIDUAL_ADD, dres)], stride=stride, padding=pad,
+                                         weight_layout=layout)
+                assert_close_scaled(y.float().cpu().numpy(), chain, tol, "%s %s bias, gelu, residual" % (names[variant], layout))
+    finally:
+        capi.force_variant("conv2d", -1)
+
+
 PATCH_SHAPES = [  # n, h, w, c, k, r, s, stride, pad, dilation: all with C % 16 == 0
     (2, 20, 20, 64, 64, 3, 3, 1, 1, 1),    # 400 pixels: several tiles per image, last one partial
     (1, 33, 17, 32, 72, 3, 3, 1, 1, 1),    # K = 288: partial last filter tile, N not a tile multiple

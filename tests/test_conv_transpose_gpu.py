@@ -267,6 +267,22 @@ def test_filter_cache_reuses_the_regrouped_bank_until_it_is_cleared(tracea_gpu):
         capi.lib().tracea_conv_transpose_filter_cache_clear()
 
 
+@pytest.mark.parametrize("shape", [(3, 17, 15, 256, 64, 4, 4, 2, 1, 0), (2, 9, 7, 128, 72, 3, 3, 2, 1, 1), (2, 7, 5, 64, 136, 3, 3, 1, 1, 0)])
+def test_activations_of_the_phase_kernels(tracea_gpu, shape):
+    """GELU and SiLU, with scores beyond 86 in some channels, on the bank read where it lies and on the regrouped one."""
+    n, h, w, c, k, r, s, stride, pad, opad = shape
+    x, wt = _operands(shape, 11, round_f16)
+    rng = np.random.default_rng(12)
+    bias = np.where(rng.random(k) < 0.1, rng.uniform(-200, 200, k), rng.standard_normal(k) * 3).astype(np.float32)
+    acc = oracle.conv_transpose2d_nhwc(x, wt, stride, pad, opad)
+    dx = _dev(x, torch.float16)
+    tol = 1.13 * tol_half(c * r * s, "f16")  # (an activation's slope)
+    for bank, layout in ((_dev(wt, torch.float16), "crsk"), (_dev(wt.transpose(3, 1, 2, 0), torch.float16), "krsc")):
+        for kw, chain in (({"epilogue": "gelu"}, [(oracle.EPI_GELU,)]), ({"epilogue": "bias+silu", "bias": _dev(bias)}, [(oracle.EPI_BIAS_ADD_SILU, bias)])):
+            y = tracea_gpu.conv_transpose2d(dx, bank, stride=stride, padding=pad, output_padding=opad, weight_layout=layout, **kw)
+            assert_close_scaled(y.float().cpu().numpy(), oracle.epilogue_apply(acc, chain), tol, "%s %s" % (layout, kw["epilogue"]))
+
+
 # like phases in one launch (2x2 and 4x4 at stride 2), unlike ones (3x3, 5x3 at 3x2), one phase (stride 1); K tiles of one
 # and of several to a tap (C 64, 128, 192), K off the 64-column tiles, more rows than one tile
 @pytest.mark.parametrize("shape", [(1, 5, 6, 64, 24, 4, 4, 2, 1, 0), (2, 9, 7, 128, 72, 3, 3, 2, 1, 1), (1, 6, 6, 192, 40, 2, 2, 2, 0, 0),

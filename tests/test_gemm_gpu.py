@@ -7,7 +7,7 @@ import numpy as np
 import pytest
 
 import oracle
-from helpers import assert_close_scaled, round_bf16, round_f16, tol_for_k, tol_half
+from helpers import assert_close_scaled, launches, round_bf16, round_f16, tol_for_k, tol_half
 
 torch = pytest.importorskip("torch")
 pytestmark = pytest.mark.gpu
@@ -515,14 +515,53 @@ def test_activations_over_the_whole_range(tracea_gpu, dtype, kind, n):
     assert bool(((got - want).abs() <= bound)[fin].all())
 
 
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+@pytest.mark.parametrize("shape", [(300, 384, 200), (64, 512, 2304)])  # whole tiles of every size and partial ones; K split over workgroups
+def test_activations_on_every_member(tracea_gpu, dtype, shape):
+    """The kernels with activations are others than those without: each member, both layouts of B, chains that end in one, go on
+    behind it and hold scores beyond 86 in some columns only, and a batch in one launch."""
+    from tracea_amd import capi
+    tdt, rnd = (torch.float16, round_f16) if dtype == "f16" else (torch.bfloat16, round_bf16)
+    m, n, k = shape
+    rng = np.random.default_rng(m + n)
+    a = rnd(rng.standard_normal((m, k)) / np.sqrt(k))
+    bt = rnd(rng.standard_normal((n, k)))
+    bias = np.where(rng.random(n) < 0.1, rng.uniform(-200, 200, n), rng.standard_normal(n) * 3).astype(np.float32)
+    res = rnd(rng.standard_normal((m, n)))
+    acc = oracle.gemm_f64(a, bt.T).astype(np.float32)
+    da, dbt, dbias, dres = _dev(a, tdt), _dev(bt, tdt), _dev(bias), _dev(res, tdt)
+    O, E = capi, oracle
+    chains = [([(O.OP_BIAS_ADD, dbias), (O.OP_GELU,)], [(E.EPI_BIAS_ADD, bias), (E.EPI_GELU,)]),
+              ([(O.OP_BIAS_ADD, dbias), (O.OP_SILU,), (O.OP_RESIDUAL_ADD, dres)], [(E.EPI_BIAS_ADD, bias), (E.EPI_SILU,), (E.EPI_RESIDUAL_ADD, res)]),
+              ([(O.OP_RESIDUAL_ADD, dres), (O.OP_GELU,), (O.OP_BIAS_ADD, dbias), (O.OP_SILU,)], [(E.EPI_RESIDUAL_ADD, res), (E.EPI_GELU,), (E.EPI_BIAS_ADD, bias), (E.EPI_SILU,)])]
+    wants = [oracle.epilogue_apply(acc, e) for _, e in chains]
+    fused = oracle.epilogue_apply(acc, [(E.EPI_BIAS_ADD_SILU, bias)])
+    # (the sum's tolerance through slopes of at most 1.13 each, and the stored rounding)
+    tol = 1.13 ** 2 * tol_half(k, dtype)
+    try:
+        for name in capi.variants("gemm"):
+            capi.force_variant("gemm", name)
+            for b in (dbt.t(), dbt.t().contiguous()):
+                for (ops, _), want in zip(chains, wants):
+                    got = tracea_gpu.gemm_ex(da, b, ops).float().cpu().numpy()
+                    assert_close_scaled(got, want, tol, "%s %s" % (name, [o[0] for o in ops]))
+                got = tracea_gpu.gemm(da, b, bias=dbias, epilogue="bias+silu").float().cpu().numpy()
+                assert_close_scaled(got, fused, tol, "%s bias+silu" % name)
+    finally:
+        capi.force_variant("gemm", -1)
+    for kw, want in (({"epilogue": "gelu"}, oracle.epilogue_apply(acc, [(E.EPI_GELU,)])), ({"epilogue": "bias+silu", "bias": dbias}, fused)):
+        got = tracea_gpu.linear(torch.stack([da] * 3), torch.stack([dbt.t().contiguous()] * 3), **kw)
+        for z in range(3):
+            assert_close_scaled(got[z].float().cpu().numpy(), want, tol, "batch %s" % kw["epilogue"])
+
+
 # four to eight elements in an operand, K on and off the 32-deep tiles, a last row of B within 4 elements of the end in the tile
 # before the last (N 1 and 3), two groups of waves with an even and an odd number of K tiles, more tiles than CUs (1100 x 1090)
 @pytest.mark.parametrize("shape", [(1, 5, 4), (4, 1, 33), (2, 3, 34), (65, 3, 66), (63, 65, 64), (64, 64, 95), (3, 130, 127), (70, 67, 321),
                                    (129, 65, 577), (1100, 1090, 403), (70, 67, 31)])
 def test_fp32_operands_at_any_element_alignment(tracea_gpu, shape):
-    """As above for fp32 with both operands by rows.  That they are read in place: two groups of waves where the rule says so (padded
-    copies of a K below 512 are not split, and their product has a K of its own), and the bits of the entry point that makes no copies
-    (which otherwise sums in one chain; four products or fewer may round alike in both)."""
+    """As above for fp32 with both operands by rows: in one launch (copies would be two more), on two groups of waves where the
+    rule says so."""
     from tracea_amd import capi
     m, n, k = shape
     rng = np.random.default_rng(m + 3 * n + 7 * k)
@@ -546,11 +585,9 @@ def test_fp32_operands_at_any_element_alignment(tracea_gpu, shape):
             tiles = -(-m // 64) * -(-n // 64)
             groups = 2 if 32 < k and tiles <= torch.cuda.get_device_properties(0).multi_processor_count else 1
             assert (capi.lib().tracea_last_split_k(), capi.lib().tracea_last_split_k_launches()) == (groups, 1)
-            if k >= 30:
-                other = torch.empty(m, n, device="cuda")
-                tracea_gpu.gemm_noalloc(*args, other, bias=_dev(bias), epilogue="bias+relu")
-                assert torch.equal(other, out[:m, :n]), "ran from copies"
             got = out.cpu().numpy()
             # (k products and sums rounded to fp32, about 3 in absolute value at most for a row of A of unit length)
             assert np.abs(got[:m, :n] - ref).max() <= 2.0 ** -24 * 2 * (k + 8) * max(1.0, np.abs(ref).max()), (gap, first)
             assert (got[m] == 7.0).all() and (got[:, n:] == 7.0).all(), "outside the output"
+    dbias = _dev(bias)
+    assert launches(lambda: tracea_gpu.gemm(*args, bias=dbias, epilogue="bias+relu", out=out[:m, :n])) == 1
